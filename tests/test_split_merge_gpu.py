@@ -1,0 +1,70 @@
+"""The merge of split keys at the edges of its two forms (up to 16 parts a row, and more), with columns that
+do not fill its last group of threads and with parts that hold no live key.
+
+Bounds: a probability and an output element are each rounded to the input dtype once (2^-9 relative for
+bfloat16), which in the 2-norm of a row stays below 2 * 2^-9 = 4e-3 with room for the sums; float32 rows carry
+the exponent's rounding, 2e-7 per unit of a log-sum-exp of about 10, and 1e-5 covers it."""
+
+import math
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def amd(gpu_device):
+    import torch_neuronx_amd as amd
+
+    return amd
+
+
+def _want(q, k, v, lens):
+    rep = q.shape[1] // k.shape[1]
+    q, k, v = q.double(), k.double().repeat_interleave(rep, 1), v.double().repeat_interleave(rep, 1)
+    s = (q @ k.transpose(-1, -2).contiguous()) / math.sqrt(q.shape[-1])
+    if lens is not None:
+        s = s.masked_fill(torch.arange(k.shape[2], device=q.device)[None, None, None] >= lens[:, None, None, None], -math.inf)
+    return torch.softmax(s, -1) @ v, torch.logsumexp(s, -1)
+
+
+def _rel(a, b):
+    return float((a.double() - b).norm() / b.norm())
+
+
+# (parts of the call on 256 compute units: bf16 2, 16, 17, 64, 33; float32 2, 16, 17, 512, 64)
+@pytest.mark.parametrize("dtype,B,Hq,Hkv,S,D,Dv,ragged", [
+    (torch.bfloat16, 32, 8, 8, 513, 64, 64, False),
+    (torch.bfloat16, 4, 8, 8, 4096, 128, 128, False),
+    (torch.float16, 1, 32, 8, 17 * 256, 128, 72, False),
+    (torch.bfloat16, 1, 32, 8, 32768, 128, 128, False),
+    (torch.bfloat16, 2, 8, 8, 33 * 256, 256, 200, True),
+    (torch.float32, 32, 16, 16, 512, 64, 40, True),
+    (torch.float32, 8, 8, 8, 2048, 128, 128, False),
+    (torch.float32, 3, 8, 4, 17 * 128, 128, 104, True),
+    (torch.float32, 1, 2, 1, 65536, 64, 64, False),
+    (torch.float32, 2, 8, 8, 8192, 256, 136, True),
+])
+def test_split_keys_of_the_forward(amd, gpu_device, dtype, B, Hq, Hkv, S, D, Dv, ragged):
+    g = torch.Generator(device=gpu_device).manual_seed(S + D)
+    q, k, v = (torch.randn(s, generator=g, device=gpu_device).to(dtype) for s in ((B, Hq, 1, D), (B, Hkv, S, D), (B, Hkv, S, Dv)))
+    # (the last batch keeps 100 keys: most of its parts have none)
+    lens = torch.tensor([S - 1] * (B - 1) + [100], device=gpu_device, dtype=torch.int32) if ragged else None
+    out, lse = amd.sdpa_forward(q, k, v, kv_lens=lens)
+    want, want_lse = _want(q, k, v, lens)
+    assert _rel(out, want) <= (1e-5 if dtype is torch.float32 else 4e-3)
+    assert float((lse.double() - want_lse).abs().max()) <= (1e-5 if dtype is torch.float32 else 2e-3)
+
+
+@pytest.mark.parametrize("B,Hkv,S,D", [(1, 8, 128, 128), (1, 8, 16 * 128, 64), (1, 4, 20000, 128), (2, 1, 131072, 256), (70, 4, 4096, 128)])
+def test_partials_of_the_fp8_decode(amd, gpu_device, B, Hkv, S, D):
+    g = torch.Generator(device=gpu_device).manual_seed(S)
+    q = torch.randn(B, 2 * Hkv, 1, D, generator=g, device=gpu_device, dtype=torch.bfloat16)
+    k, v = ((torch.randn(B, Hkv, S, D, generator=g, device=gpu_device) * 32).to(torch.float8_e4m3fn) for _ in range(2))
+    sc = torch.full((B, Hkv), 1.0 / 32, device=gpu_device)
+    lens = torch.randint(1, S + 1, (B,), generator=g, device=gpu_device, dtype=torch.int32)
+    out, lse = amd.decode_fp8kv(q, k, v, sc, sc, lens)
+    want, want_lse = _want(q, k.float() / 32, v.float() / 32, lens)
+    assert _rel(out, want) <= 4e-3
+    assert float((lse.double() - want_lse).abs().max()) <= 2e-3

@@ -34,6 +34,7 @@
 #include <type_traits>
 
 #include "common.h"
+#include "split_merge.h"
 
 // Scratch of the entry point that allocates nothing (mi355_sdpa_decode_fp8kv_static): partial
 // results and step counts of one decode call.  Every GPU the library runs on holds its own copy
@@ -44,8 +45,6 @@ static __device__ __align__(256) unsigned char scratch[MI355_SDPA_DECODE_STATIC_
 namespace mi355 {
 namespace {
 
-typedef __attribute__((ext_vector_type(4))) float f32x4;
-typedef __attribute__((ext_vector_type(4))) uint32_t u32x4;
 typedef __attribute__((ext_vector_type(2))) float f32x2;
 
 constexpr float kLog2e = 1.4426950408889634f;
@@ -123,7 +122,6 @@ __device__ __forceinline__ long as_long(uint32_t lo, uint32_t hi) {
   return (long)(((uint64_t)hi << 32) | lo);
 }
 
-typedef __attribute__((ext_vector_type(2))) uint32_t u32x2;
 // Head dims 64, 128 and 256: a K row is D/64 pieces of 64 bytes, of which lane group g takes 16 each
 // (two contraction steps of 32 per piece); a V row is 16 pieces of D/16 bytes, one per lane n.
 template <int D>
@@ -454,84 +452,35 @@ __global__ __launch_bounds__(64, dec_occ(D)) void decode_kernel(DecP p) {
   }
 }
 
-// Merge the partials of one (batch, kv head, query row); D threads = D output columns.
-// The wavefronts that touched this (batch, kv head) follow from the step numbering alone, and
-// their partials sit in consecutive slots.
-template <typename TQ, int D>
-__global__ __launch_bounds__(D) void decode_merge_kernel(DecP p) {
-  constexpr int NW = D / 64;  // wavefronts of the workgroup
-  __shared__ float s_red[2][4];
-  __shared__ float w_s[kMaxSimds * 2];  // weights of the partials (at most one per wavefront of the streaming kernel)
+// Merge the partials of one (batch, kv head, query row), see split_merge.h.  The wavefronts that touched
+// this (batch, kv head) follow from the step numbering alone, and their partials sit in consecutive slots.
+template <typename TQ, int D, int SLICES>
+__global__ __launch_bounds__(SLICES * D / 4) void decode_merge_kernel(DecP p) {
+  __shared__ MergeLds<SLICES, D / 4> lds;
   const int row = blockIdx.x % p.R;
   const int hk = (blockIdx.x / p.R) % p.Hkv;
   const int b = blockIdx.x / (p.R * p.Hkv);
-  const int d = threadIdx.x;
   const int pref = p.ws_steps[b], nb = p.ws_steps[b + 1] - pref;
   const int T = steps_per_wave(p.ws_steps[p.B] * p.Hkv, p.n_waves, p.t_min);
   const int g0 = pref * p.Hkv + hk * nb;
   const int w0 = g0 / T;
   const int npart = nb > 0 ? (g0 + nb - 1) / T - w0 + 1 : 0;
   const int64_t slot0 = (int64_t)(b * p.Hkv + hk + w0) * p.R + row;  // partial c sits at slot0 + c*R
-  float M = -INFINITY, L = 0.f, O = 0.f;
-  constexpr int kFew = 8;
-  if (npart <= kFew) {
-    // few partials: fetch every (max, sum) pair and output value at once, then combine; each
-    // thread repeats the scalar part, which costs less than a second round trip to memory
-    float m[kFew], l[kFew], o[kFew];
-#pragma unroll
-    for (int c = 0; c < kFew; ++c) {
-      const int64_t s = slot0 + (int64_t)min(c, max(npart - 1, 0)) * p.R;
-      const bool live = c < npart;
-      m[c] = live ? p.ws_ml[s * 2] : -INFINITY;
-      l[c] = live ? p.ws_ml[s * 2 + 1] : 0.f;
-      o[c] = live ? p.ws_o[s * D + d] : 0.f;
-    }
-#pragma unroll
-    for (int c = 0; c < kFew; ++c) M = fmaxf(M, m[c]);
-#pragma unroll
-    for (int c = 0; c < kFew; ++c) {
-      const float w = c < npart ? __builtin_amdgcn_exp2f(m[c] - M) : 0.f;
-      L = fmaf(l[c], w, L);
-      O = fmaf(o[c], w, O);
-    }
-  } else {
-    // many partials (a long sequence in a small batch: up to one per wavefront of the chip): their
-    // (max, sum) pairs a thread each, the weights left in LDS, and the partial outputs requested eight
-    // at a time - read one after the other, 256 partials were 256 trips to the L2 in a row, and a
-    // single sequence of 32768 keys spent two thirds of its decode step here
-    for (int c = d; c < npart; c += D) M = fmaxf(M, p.ws_ml[(slot0 + (int64_t)c * p.R) * 2]);
-    M = wave_max(M);
-    if ((d & 63) == 0) s_red[0][d >> 6] = M;
-    __syncthreads();
-    M = s_red[0][0];
-#pragma unroll
-    for (int w = 1; w < NW; ++w) M = fmaxf(M, s_red[0][w]);
-    for (int c = d; c < npart; c += D) {
-      const int64_t s = slot0 + (int64_t)c * p.R;
-      const float w = __builtin_amdgcn_exp2f(p.ws_ml[s * 2] - M);
-      w_s[c] = w;
-      L += p.ws_ml[s * 2 + 1] * w;
-    }
-    L = wave_sum(L);
-    if ((d & 63) == 0) s_red[1][d >> 6] = L;
-    __syncthreads();
-    L = s_red[1][0];
-#pragma unroll
-    for (int w = 1; w < NW; ++w) L += s_red[1][w];
-    const float* po = p.ws_o + slot0 * D + d;
-    const int64_t stride = (int64_t)p.R * D;
-    for (int c0 = 0; c0 < npart; c0 += 8) {
-      float o[8];
-#pragma unroll
-      for (int j = 0; j < 8; ++j) o[j] = c0 + j < npart ? po[(c0 + j) * stride] : 0.f;
-#pragma unroll
-      for (int j = 0; j < 8; ++j) O = fmaf(o[j], c0 + j < npart ? w_s[c0 + j] : 0.f, O);
-    }
-  }
+  const float* const po = p.ws_o + slot0 * D + (threadIdx.x % (D / 4)) * 4;
+  const float* const pml = p.ws_ml + slot0 * 2;
+  float O, M, L;
+  merge_parts<SLICES, D / 4>(
+      lds, npart,
+      [&](int c, float& m, float& l) {
+        const f32x2 w = *(const f32x2*)(pml + (int64_t)c * p.R * 2);
+        m = w[0], l = w[1];
+      },
+      [&](int c) { return *(const f32x4*)(po + (int64_t)c * p.R * D); }, O, M, L);
   const int rep = p.Hq / p.Hkv;
   const int h = hk * rep + row % rep, lq = row / rep;
+  const int d = threadIdx.x;
   TQ* o = (TQ*)p.out + b * p.o_sb + h * p.o_sh + lq * p.o_sl;
-  o[d] = (TQ)(L > 0.f ? O / L : 0.f);
+  if (d < D) o[d] = (TQ)(L > 0.f ? O / L : 0.f);
   if (p.lse && d == 0)
     p.lse[((int64_t)b * p.Hq + h) * p.Lq + lq] = L > 0.f ? (M + __builtin_amdgcn_logf(L)) * kLn2 : -INFINITY;
 }
@@ -581,7 +530,12 @@ int launch_td(const DecP& g, hipStream_t s) {
 #undef DECODE
   int rc = check_launch("decode_kernel");
   if (rc) return rc;
-  hipLaunchKernelGGL((decode_merge_kernel<TQ, D>), dim3(g.B * g.Hkv * g.R), dim3(D), 0, s, g);
+  // (a (batch, kv head) has about its share of the wavefronts as partials)
+  const dim3 rows(g.B * g.Hkv * g.R);
+  if (merge_slices_for(g.n_waves / ((int64_t)g.B * g.Hkv)) == kMergeMany)
+    hipLaunchKernelGGL((decode_merge_kernel<TQ, D, kMergeMany>), rows, dim3(kMergeMany * D / 4), 0, s, g);
+  else
+    hipLaunchKernelGGL((decode_merge_kernel<TQ, D, kMergeFew>), rows, dim3(kMergeFew * D / 4), 0, s, g);
   return check_launch("decode_merge_kernel");
 }
 template <typename TQ>

@@ -163,7 +163,7 @@ __global__ __launch_bounds__(64 * WAVES, 1) void fwd_f32_kernel(FwdM p) {
     }
   }
   // (few rows against many keys: the key tiles are split over blockIdx.y, each part leaves its normalised
-  // rows and their log-sum-exp in the workspace for fwd_f32_merge_kernel; no causal flag, no window then)
+  // rows and their log-sum-exp in the workspace for fwd_split_merge_kernel; no causal flag, no window then)
   const int split = p.split_tiles ? blockIdx.y : 0;
   int t_first = 0;
   if (!FUNC && p.split_tiles) {
@@ -291,70 +291,6 @@ __global__ __launch_bounds__(64 * WAVES, 1) void fwd_f32_kernel(FwdM p) {
       p.lse[((int64_t)b * p.Hq + h) * p.L + qrow] = lse_row;
     }
   }
-}
-
-// Merge of the parts of a call whose keys were split: out = sum_s w_s O_s with w_s = exp(lse_s - lse),
-// lse = log sum_s exp(lse_s).  One workgroup per query row, a thread per output column (two at widths
-// above 128); the parts' lse are read side by side and their weights left in LDS, the parts' rows are
-// requested eight at a time.
-__global__ __launch_bounds__(128) void fwd_f32_merge_kernel(FwdM p) {
-  constexpr int MAXP = 512;  // (fwd_f32_plan never makes more parts)
-  __shared__ float w_s[MAXP];
-  __shared__ float red_s[4];
-  const int64_t row = blockIdx.x;  // (b * Hq + h) * L + l
-  const int l = (int)(row % p.L);
-  const int64_t bh = row / p.L;
-  const int b = (int)(bh / p.Hq), h = (int)(bh % p.Hq);
-  const float* pl = p.part_lse + bh * p.n_split * p.L + l;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  float ls[MAXP / 128];
-  float m = -INFINITY;
-#pragma unroll
-  for (int i = 0; i < MAXP / 128; ++i) {
-    const int sp = tid + 128 * i;
-    ls[i] = sp < p.n_split ? pl[(int64_t)sp * p.L] : -INFINITY;
-    m = fmaxf(m, ls[i]);
-  }
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) m = fmaxf(m, __shfl_xor(m, off, 64));
-  if (lane == 0) red_s[wave] = m;
-  __syncthreads();
-  m = fmaxf(red_s[0], red_s[1]);
-  float sum = 0.f;
-#pragma unroll
-  for (int i = 0; i < MAXP / 128; ++i) {
-    const int sp = tid + 128 * i;
-    const float w = ls[i] == -INFINITY ? 0.f : __expf(ls[i] - m);  // (a part without live keys: weight 0)
-    w_s[sp] = w;  // (every slot: the loop below multiplies the slots past the last part by a zero, which a stale NaN would survive)
-    sum += w;
-  }
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) sum += __shfl_xor(sum, off, 64);
-  if (lane == 0) red_s[2 + wave] = sum;
-  __syncthreads();
-  sum = red_s[2] + red_s[3];
-  float acc[2] = {0.f, 0.f};
-  const int d = tid;
-  const float* po = p.part_o + (bh * p.n_split * p.L + l) * p.dv_real;
-  const int64_t part_stride = (int64_t)p.L * p.dv_real;
-  for (int s0 = 0; s0 < p.n_split; s0 += 8) {
-    float x[2][8];
-#pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      const bool on = s0 + j < p.n_split && w_s[min(s0 + j, MAXP - 1)] > 0.f;
-#pragma unroll
-      for (int i = 0; i < 2; ++i) x[i][j] = (on && d + 128 * i < p.dv_real) ? po[(s0 + j) * part_stride + d + 128 * i] : 0.f;
-    }
-#pragma unroll
-    for (int j = 0; j < 8; ++j)
-#pragma unroll
-      for (int i = 0; i < 2; ++i) acc[i] = fmaf(s0 + j < p.n_split ? w_s[min(s0 + j, MAXP - 1)] : 0.f, x[i][j], acc[i]);
-  }
-#pragma unroll
-  for (int i = 0; i < 2; ++i)
-    if (d + 128 * i < p.dv_real)
-      ((float*)p.out)[b * p.o_sb + h * p.o_sh + (int64_t)l * p.o_sl + d + 128 * i] = sum > 0.f ? acc[i] / sum : 0.f;
-  if (d == 0 && p.lse) p.lse[row] = sum > 0.f ? m + __builtin_logf(sum) : -INFINITY;
 }
 
 template <int D, int WAVES, int MODE>
@@ -722,7 +658,7 @@ namespace {
 // become the rows of one head (they read the same K and V; a view of q, out and the log-sum-exp, nothing
 // moves) where no causal flag, functor or per-head bias tells the heads apart, and where that still
 // leaves compute units short of workgroups the key tiles are split over blockIdx.y, at least 4
-// tiles (128 keys) per part, into the caller's workspace (fwd_f32_merge_kernel adds the parts up).
+// tiles (128 keys) per part, into the caller's workspace (fwd_split_merge_kernel adds the parts up).
 void fwd_f32_plan(FwdM& g, const mi355_sdpa_fwd_params& p, int mode) {
   g.split_tiles = 0, g.n_split = 1;
   const int rep = g.Hq / g.Hkv;
@@ -825,8 +761,7 @@ int launch_fwd_f32_mfma(const mi355_sdpa_fwd_params& p, hipStream_t s) {
 #undef LAUNCH
   const int rc = check_launch("fwd_f32_kernel");
   if (rc != MI355_SDPA_OK || !g.split_tiles) return rc;
-  hipLaunchKernelGGL(fwd_f32_merge_kernel, dim3((unsigned)((int64_t)g.B * g.Hq * g.L)), dim3(128), 0, s, g);
-  return check_launch("fwd_f32_merge_kernel");
+  return launch_fwd_split_merge(g, MI355_SDPA_F32, s);
 }
 
 bool bwd_f32_mfma_supported(const mi355_sdpa_bwd_params& p, const char** why) {

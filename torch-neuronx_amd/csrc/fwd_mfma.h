@@ -102,6 +102,8 @@ __device__ __forceinline__ void decode_block(const FwdM& p, int& b, int& h, int&
 // head_dim 64, 128 or 256: the width the kernel is built for (g.d_real: the width of the data);
 // waves = 4 or 8 wavefronts (128 or 256 query rows) per workgroup, 4 only at head dim 256
 int launch_fwd_mfma_w32(const FwdM& g, int dtype, int head_dim, int waves, hipStream_t s);
+// adds up the parts that a call with split keys left in g.part_o / g.part_lse (any of the three dtypes)
+int launch_fwd_split_merge(const FwdM& g, int dtype, hipStream_t s);
 // bytes of workspace with which that launch would split the keys of the call (0: it would not)
 size_t fwd_w32_workspace(const FwdM& g, int head_dim, int waves);
 

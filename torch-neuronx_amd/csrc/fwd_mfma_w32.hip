@@ -30,6 +30,7 @@
 #include <type_traits>
 
 #include "fwd_mfma.h"
+#include "split_merge.h"
 
 namespace mi355 {
 namespace {
@@ -929,72 +930,41 @@ __global__ __launch_bounds__(64 * WAVES, D > 128 ? 1 : 8 / WAVES) void fwd_w32_k
   fwd_w32_body<T, D, WAVES, MASK>(p, ma);
 }
 
-// Merge of the parts of a call whose keys were split: out = sum_s w_s O_s with w_s = exp(lse_s - lse),
-// lse = log sum_s exp(lse_s).  One workgroup per query row, one thread per output element.  The parts'
-// lse are read side by side (a thread per part) and their weights left in LDS; the rows of the parts
-// are then requested eight at a time: read one after the other, each of the two passes was a chain of
-// trips to the L2, and a call with 64 parts spent as long here as in the attention kernel.
-template <typename T>
-__global__ __launch_bounds__(128) void fwd_split_merge_kernel(FwdM p) {
-  constexpr int MAXP = 512;  // (fwd_w32_plan never makes more parts)
-  __shared__ float w_s[MAXP];
-  __shared__ float red_s[4];
+// Merge of the parts of a call whose keys were split (see split_merge.h): normalised rows and their
+// log-sum-exp, so a part's statistics are (lse in the log2 domain, 1).
+template <typename T, int TPR, int SLICES>
+__global__ __launch_bounds__(SLICES * TPR) void fwd_split_merge_kernel(FwdM p) {
+  __shared__ MergeLds<SLICES, TPR> lds;
   const int64_t row = blockIdx.x;  // (b * Hq + h) * L + l
   const int l = (int)(row % p.L);
   const int64_t bh = row / p.L;
   const int b = (int)(bh / p.Hq), h = (int)(bh % p.Hq);
-  const float* pl = p.part_lse + bh * p.n_split * p.L + l;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  float ls[MAXP / 128];
-  float m = -INFINITY;
-#pragma unroll
-  for (int i = 0; i < MAXP / 128; ++i) {
-    const int sp = tid + 128 * i;
-    ls[i] = sp < p.n_split ? pl[(int64_t)sp * p.L] : -INFINITY;
-    m = fmaxf(m, ls[i]);
-  }
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) m = fmaxf(m, __shfl_xor(m, off, 64));
-  if (lane == 0) red_s[wave] = m;
-  __syncthreads();
-  m = fmaxf(red_s[0], red_s[1]);
-  float sum = 0.f;
-#pragma unroll
-  for (int i = 0; i < MAXP / 128; ++i) {
-    const int sp = tid + 128 * i;
-    const float w = ls[i] == -INFINITY ? 0.f : __expf(ls[i] - m);  // (a part without keys: weight 0, its rows were never written)
-    w_s[sp] = w;  // (every slot: the loop below multiplies the slots past the last part by a zero, which a stale NaN would survive)
-    sum += w;
-  }
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) sum += __shfl_xor(sum, off, 64);
-  if (lane == 0) red_s[2 + wave] = sum;
-  __syncthreads();
-  sum = red_s[2] + red_s[3];
-  float acc[2] = {0.f, 0.f};
-  const int d = tid;  // columns d and d + 128 (head dims up to 256)
-  const float* po = p.part_o + (bh * p.n_split * p.L + l) * p.dv_real;
+  const float* const pl = p.part_lse + bh * p.n_split * p.L + l;
+  const int d4 = min((int)(threadIdx.x % TPR) * 4, p.dv_real - 4);  // (a multiple of 8; columns past it are not written)
+  const float* const po = p.part_o + (bh * p.n_split * p.L + l) * p.dv_real + d4;
   const int64_t part_stride = (int64_t)p.L * p.dv_real;
-  for (int s0 = 0; s0 < p.n_split; s0 += 8) {
-    float x[2][8];
-#pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      const bool on = s0 + j < p.n_split && w_s[min(s0 + j, MAXP - 1)] > 0.f;
-#pragma unroll
-      for (int i = 0; i < 2; ++i) x[i][j] = (on && d + 128 * i < p.dv_real) ? po[(s0 + j) * part_stride + d + 128 * i] : 0.f;
-    }
-#pragma unroll
-    for (int j = 0; j < 8; ++j)
-#pragma unroll
-      for (int i = 0; i < 2; ++i) acc[i] = fmaf(s0 + j < p.n_split ? w_s[min(s0 + j, MAXP - 1)] : 0.f, x[i][j], acc[i]);
+  float O, M, L;
+  merge_parts<SLICES, TPR>(
+      lds, p.n_split, [&](int c, float& m, float& w) { m = pl[(int64_t)c * p.L] * kLog2eF, w = 1.f; },
+      [&](int c) { return *(const f32x4*)(po + c * part_stride); }, O, M, L);
+  const int d = threadIdx.x;
+  if (d < p.dv_real) ((T*)p.out)[b * p.o_sb + h * p.o_sh + (int64_t)l * p.o_sl + d] = (T)(L > 0.f ? O / L : 0.f);
+  if (d == 0 && p.lse) p.lse[row] = L > 0.f ? M / kLog2eF + __builtin_logf(L) : -INFINITY;
+}
+
+template <typename T>
+void launch_merge(const FwdM& g, hipStream_t s) {
+  const dim3 rows((unsigned)((int64_t)g.B * g.Hq * g.L));
+  const bool many = merge_slices_for(g.n_split) == kMergeMany;
+#define MERGE(TPR, SLICES) hipLaunchKernelGGL((fwd_split_merge_kernel<T, TPR, SLICES>), rows, dim3(SLICES * TPR), 0, s, g)
+  if (g.dv_real > 128) {
+    if (many) MERGE(64, kMergeMany);
+    else MERGE(64, kMergeFew);
+  } else {
+    if (many) MERGE(32, kMergeMany);
+    else MERGE(32, kMergeFew);
   }
-#pragma unroll
-  for (int i = 0; i < 2; ++i)
-    if (d + 128 * i < p.dv_real) {
-      T* o = (T*)p.out + b * p.o_sb + h * p.o_sh + (int64_t)l * p.o_sl + d + 128 * i;
-      *(uint16_t*)o = (uint16_t)Mma<T>::pack(sum > 0.f ? acc[i] / sum : 0.f, 0.f);
-    }
-  if (d == 0 && p.lse) p.lse[row] = sum > 0.f ? m + __builtin_logf(sum) : -INFINITY;
+#undef MERGE
 }
 
 // one instantiation; head dim 256 and the variant with a bias need more than the 64 KB of LDS a kernel may declare
@@ -1068,7 +1038,7 @@ void fwd_w32_plan(FwdM& g, int head_dim, int& waves) {
   if (g.grouped && (head_dim <= 128 || g.bias_kind == 0) && !g.causal && g.window == 0 && !g.sink_logit && !g.sm.any) {
     const int64_t groups = (int64_t)g.B * g.Hkv * (g.Hq / g.Hkv / g.grouped);
     const int nt = (g.S + BN - 1) / BN;
-    const int want = (int)std::min<int64_t>((512 + groups - 1) / groups, nt / 8);  // (at most 512 parts: fwd_split_merge_kernel's limit)
+    const int want = (int)std::min<int64_t>((512 + groups - 1) / groups, nt / 8);  // (at most 512 parts)
     if (groups < 256 && want >= 2) {
       g.split_tiles = (nt + want - 1) / want;
       g.n_split = (nt + g.split_tiles - 1) / g.split_tiles;
@@ -1083,6 +1053,13 @@ size_t fwd_w32_workspace(const FwdM& g0, int head_dim, int waves) {
   fwd_w32_plan(g, head_dim, waves);
   if (!g.split_tiles) return 0;
   return (size_t)g.B * g.Hq * g.n_split * g.L * (g.dv_real + 1) * sizeof(float);
+}
+
+int launch_fwd_split_merge(const FwdM& g, int dtype, hipStream_t s) {
+  if (dtype == MI355_SDPA_BF16) launch_merge<bf16_t>(g, s);
+  else if (dtype == MI355_SDPA_F16) launch_merge<f16_t>(g, s);
+  else launch_merge<float>(g, s);
+  return check_launch("fwd_split_merge_kernel");
 }
 
 int launch_fwd_mfma_w32(const FwdM& g0, int dtype, int head_dim, int waves, hipStream_t s) {
@@ -1115,10 +1092,7 @@ int launch_fwd_mfma_w32(const FwdM& g0, int dtype, int head_dim, int waves, hipS
   if (rc != MI355_SDPA_OK) return rc;
   rc = check_launch("fwd_w32_kernel");
   if (rc != MI355_SDPA_OK || !g.split_tiles) return rc;
-  const dim3 rows((unsigned)((int64_t)g.B * g.Hq * g.L));
-  if (dtype == MI355_SDPA_BF16) hipLaunchKernelGGL((fwd_split_merge_kernel<bf16_t>), rows, dim3(128), 0, s, g);
-  else hipLaunchKernelGGL((fwd_split_merge_kernel<f16_t>), rows, dim3(128), 0, s, g);
-  return check_launch("fwd_split_merge_kernel");
+  return launch_fwd_split_merge(g, dtype, s);
 }
 
 }  // namespace mi355
