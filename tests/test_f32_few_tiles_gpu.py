@@ -1,0 +1,56 @@
+"""Float32 forward with few query tiles: 32-row workgroups whose four wavefronts share out the key tiles.
+Sizes around a tile, around four tiles (one per wavefront) and around the number of workgroups at which the
+128-row kernel takes over, ragged key counts (none at all included), narrow V, grouped heads, L != S.
+
+Bound: the tolerance of the float32 gate, 1e-5 on values of order 1 (float32 sums of at most 128 products and
+1000 keys: about 3e-7 relative measured, and the rows are compared absolutely)."""
+
+import pytest
+import torch
+
+from tests.helpers import max_abs, oracle_fwd, qkv
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def amd(gpu_device):
+    import torch_neuronx_amd as amd
+
+    return amd
+
+
+@pytest.mark.parametrize("B,Hq,Hkv,L,S,E,Dv,causal", [
+    (1, 2, 2, 33, 33, 64, 64, False),
+    (1, 2, 2, 31, 33, 64, 64, True),
+    (2, 4, 4, 128, 128, 64, 64, False),
+    (2, 4, 2, 127, 129, 64, 64, True),
+    (1, 4, 1, 65, 97, 128, 128, True),
+    (1, 2, 2, 200, 161, 128, 72, True),
+    (1, 3, 3, 1, 257, 40, 40, False),
+    (2, 2, 2, 150, 500, 104, 8, False),
+    (1, 4, 4, 1000, 1000, 64, 64, True),
+    (20, 4, 4, 130, 130, 64, 64, False),   # 160 workgroups of 128 rows: the last size here
+    (23, 4, 4, 129, 129, 64, 64, False),   # ... and past it
+    (15, 8, 8, 150, 150, 64, 64, True),    # 240, causal
+])
+def test_against_the_oracle(amd, gpu_device, B, Hq, Hkv, L, S, E, Dv, causal):
+    q, k, v = qkv(B, Hq, Hkv, L, S, E, Dv, seed=L + S)
+    out, lse = amd.sdpa_forward(*(t.to(gpu_device) for t in (q, k, v)), is_causal=causal)
+    ro, rl = oracle_fwd(q, k, v, is_causal=causal)
+    assert max_abs(out, ro) <= 1e-5 and max_abs(lse, rl) <= 1e-5
+
+
+@pytest.mark.parametrize("causal", [False, True])
+def test_key_counts(amd, gpu_device, causal):
+    B, H, S, D = 4, 2, 140, 64
+    q, k, v = qkv(B, H, H, S, S, D, seed=5)
+    lens = torch.tensor([140, 0, 1, 97], dtype=torch.int32)
+    k[2, :, 1:], v[2, :, 1:] = float("nan"), float("nan")  # (keys past a batch's count are never used)
+    out, lse = amd.sdpa_forward(*(t.to(gpu_device) for t in (q, k, v)), is_causal=causal, kv_lens=lens.to(gpu_device))
+    for b, n in enumerate(lens.tolist()):
+        if n == 0:
+            assert not out[b].any() and torch.isneginf(lse[b]).all()
+            continue
+        ro, rl = oracle_fwd(q[b:b + 1], k[b:b + 1, :, :n], v[b:b + 1, :, :n], is_causal=causal)
+        assert max_abs(out[b:b + 1], ro) <= 1e-5 and max_abs(lse[b:b + 1], rl) <= 1e-5

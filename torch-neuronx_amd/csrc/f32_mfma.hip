@@ -16,6 +16,7 @@
 // room: these kernels are not pipelined by hand.
 //
 //   fwd_f32_kernel        128 query rows per workgroup (4 wavefronts x 32), 32-key tiles
+//   fwd_f32_few_kernel    32 query rows per workgroup, its wavefronts share out the key tiles (few query tiles)
 //   bwd_f32_dq_kernel     the same shape; also leaves delta = rowsum(dO * O) and the log2-domain
 //                         log-sum-exp in the workspace
 //   bwd_f32_dkdv_kernel   128 keys per workgroup; loops over the query heads of the group (the GQA
@@ -291,6 +292,122 @@ __global__ __launch_bounds__(64 * WAVES, 1) void fwd_f32_kernel(FwdM p) {
       p.lse[((int64_t)b * p.Hq + h) * p.L + qrow] = lse_row;
     }
   }
+}
+
+// Few query tiles (a small batch, short sequences): 128-row workgroups would leave compute units empty and
+// each of the busy ones walking all of its keys in one chain of 64-cycle matrix ops.  Here a workgroup is
+// 32 query rows and its four wavefronts take every fourth key tile each; the four partial results meet
+// in LDS.  What bounds such a call is that chain and the trips to memory in front of it, not bytes: K and V
+// go from global memory straight into the registers that feed the matrix op (a lane supplies one
+// element per operand, so a K row is plain 16-byte loads of its own row and a V column one 4-byte load per
+// key), the next tile's under the current one's ops, and nothing in the loop waits for another wavefront.
+// Plain and causal calls with per-batch key counts, head dims up to 128.  B=2, 4 heads, S=128, D=64: 14.9 us
+// in fwd_f32_kernel, 8.2 here; B=1, 8 heads, S=1024, D=128: 161 -> 64 (where each pays: few_query_tiles).
+template <int D>
+__global__ __launch_bounds__(256, 1) void fwd_f32_few_kernel(FwdM p) {
+  constexpr int KW = 4, DB = D / 32, PITCH = D + 4;
+  __shared__ float m_s[KW][32], l_s[KW][32];
+  float* const o_s = wide_f32_lds;  // [KW][32][PITCH]
+  const int n_rb = (p.L + 31) / 32;
+  const int rb = n_rb - 1 - blockIdx.x / (p.B * p.Hq);  // heavy row blocks first
+  const int bh = blockIdx.x % (p.B * p.Hq), b = bh / p.Hq, h = bh % p.Hq, hk = h / (p.Hq / p.Hkv);
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, col = lane & 31, half = lane >> 5;
+  const int q0 = rb * 32, qrow = q0 + col, qc = min(qrow, p.L - 1);
+  const float* kp = (const float*)p.k + b * p.k_sb + hk * p.k_sh;
+  const float* vp = (const float*)p.v + b * p.v_sb + hk * p.v_sh;
+  const int S = p.kv_lens ? min(p.S, max(p.kv_lens[b], 0)) : p.S;
+  int nt = (S + BT - 1) / BT;
+  if (p.causal) nt = min(nt, (min(q0 + 32, p.L) - 1) / BT + 1);
+  const int lim = p.causal ? min(qrow, S - 1) : S - 1;
+  const float c = p.scale * kLog2eF;
+  float qf[D / 2];
+  load_half_row<D>(qf, (const float*)p.q + b * p.q_sb + h * p.q_sh + (int64_t)qc * p.q_sl, half, p.d_real);
+  float kf[D / 2], vf[16][DB];
+  auto fetch_k = [&](int t) {  // (rows past the keys: the last one again, their scores are masked)
+    load_half_row<D>(kf, kp + (int64_t)min(t * BT + col, S - 1) * p.k_sl, half, p.d_real);
+  };
+  auto fetch_v = [&](int t) {  // (... and zeros, which the zero probabilities leave finite)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      const int kv = t * BT + (r >> 2) * 8 + half * 4 + (r & 3);
+      const float* row = vp + (int64_t)kv * p.v_sl + col;
+#pragma unroll
+      for (int db = 0; db < DB; ++db) vf[r][db] = (kv < S && db * 32 + col < p.dv_real) ? row[db * 32] : 0.f;
+    }
+  };
+  f32x16 oacc[DB];
+#pragma unroll
+  for (int i = 0; i < DB; ++i) zero(oacc[i]);
+  float m_run = -INFINITY, l_run = 0.f;
+  if (wave < nt) fetch_k(wave), fetch_v(wave);
+  for (int t = wave; t < nt; t += KW) {
+    f32x16 s = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int i = 0; i < D / 2; ++i) s = mma(kf[i], qf[i], s);
+    if (t + KW < nt) fetch_k(t + KW);
+    float tm = -INFINITY;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      if (t * BT + (r >> 2) * 8 + half * 4 + (r & 3) > lim) s[r] = -INFINITY;
+      tm = fmaxf(tm, s[r]);
+    }
+    tm = fmaxf(tm, __shfl_xor(tm, 32, 64));
+    const float m_new = fmaxf(m_run, tm);
+    const float m_use = m_new == -INFINITY ? 0.f : m_new;
+    const float alpha = __builtin_amdgcn_exp2f((m_run - m_use) * c);
+    m_run = m_new;
+    float psum = 0.f;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      s[r] = __builtin_amdgcn_exp2f((s[r] - m_use) * c);
+      psum += s[r];
+    }
+    l_run = l_run * alpha + psum;
+#pragma unroll
+    for (int i = 0; i < DB; ++i)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) oacc[i][r] *= alpha;
+#pragma unroll
+    for (int r = 0; r < 16; ++r)
+#pragma unroll
+      for (int db = 0; db < DB; ++db) oacc[db] = mma(vf[r][db], s[r], oacc[db]);
+    if (t + KW < nt) fetch_v(t + KW);
+  }
+  // the four parts of a row: every wavefront leaves (maximum, sum, O) and a row is put together by 8 threads
+  const float l_tot = l_run + __shfl_xor(l_run, 32, 64);
+  if (half == 0) m_s[wave][col] = m_run, l_s[wave][col] = l_tot;
+  float* const o_w = o_s + (wave * 32 + col) * PITCH + half * 4;
+#pragma unroll
+  for (int db = 0; db < DB; ++db)
+#pragma unroll
+    for (int g = 0; g < 4; ++g)
+      *(f32x4*)(o_w + db * 32 + g * 8) = f32x4{oacc[db][g * 4], oacc[db][g * 4 + 1], oacc[db][g * 4 + 2], oacc[db][g * 4 + 3]};
+  __syncthreads();
+  const int r = tid >> 3, c4 = (tid & 7) * 4;
+  float mt = -INFINITY, lt = 0.f, w[KW];
+#pragma unroll
+  for (int i = 0; i < KW; ++i) mt = fmaxf(mt, m_s[i][r]);
+#pragma unroll
+  for (int i = 0; i < KW; ++i) {
+    w[i] = mt == -INFINITY ? 0.f : __builtin_amdgcn_exp2f((m_s[i][r] - mt) * c);
+    lt = fmaf(l_s[i][r], w[i], lt);
+  }
+  const float inv = lt > 0.f ? 1.f / lt : 0.f;
+  if (q0 + r >= p.L) return;
+  float* const orow = (float*)p.out + b * p.o_sb + h * p.o_sh + (int64_t)(q0 + r) * p.o_sl;
+#pragma unroll
+  for (int d0 = 0; d0 < D; d0 += 32) {
+    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int i = 0; i < KW; ++i) {
+      const f32x4 x = *(const f32x4*)(o_s + (i * 32 + r) * PITCH + d0 + c4);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) acc[e] = fmaf(x[e], w[i], acc[e]);
+    }
+    if (d0 + c4 < p.dv_real) *(f32x4*)(orow + d0 + c4) = f32x4{acc[0] * inv, acc[1] * inv, acc[2] * inv, acc[3] * inv};
+  }
+  if (p.lse && (tid & 7) == 0)
+    p.lse[((int64_t)b * p.Hq + h) * p.L + q0 + r] = lt > 0.f ? mt * p.scale + __builtin_logf(lt) : -INFINITY;
 }
 
 template <int D, int WAVES, int MODE>
@@ -682,6 +799,18 @@ void fwd_f32_plan(FwdM& g, const mi355_sdpa_fwd_params& p, int mode) {
   }
 }
 
+// Which plain calls run in fwd_f32_few_kernel (32-row workgroups whose wavefronts share out the key tiles)
+// instead of fwd_f32_kernel (128-row workgroups that share every tile).  By the number of 128-row
+// workgroups: a compute unit holds one of them at a time, so up to 256 they all take as long as the one with
+// the most keys, while the 32-row ones cost 1.3 times the work (no tile is shared) spread over four times as
+// many workgroups.  Measured, 128-row / 32-row in us (8 heads, D=64; D=128 gives the same ratios):
+//   B=2, 4 heads, S=128 (8) 14.9 / 8.2;  B=1, S=1024 (64) 92 / 35;  B=2, S=1024 (128) 93 / 66, causal 92 / 41;
+//   B=4, S=1024 (256) 97 / 126, causal 93 / 79;  B=8, S=512 (256) 52 / 74, causal 50 / 52;  B=8, S=1024 (512) 160 / 251
+// A single key tile has nothing to share out (S=16: 5.8 / 6.6).
+bool few_query_tiles(const FwdM& g) {
+  return g.S > BT && (int64_t)g.B * g.Hq * ((g.L + 127) / 128) <= (g.causal ? 240 : 160);
+}
+
 void fwd_f32_fill(FwdM& g, const mi355_sdpa_fwd_params& p, int& mode) {
   g.q = p.q.data, g.k = p.k.data, g.v = p.v.data, g.out = p.out.data, g.lse = p.lse;
   g.q_sb = p.q.stride[0], g.q_sh = p.q.stride[1], g.q_sl = p.q.stride[2];
@@ -729,8 +858,24 @@ int launch_fwd_f32_mfma(const mi355_sdpa_fwd_params& p, hipStream_t s) {
     else
       g.split_tiles = 0, g.n_split = 1;
   }
-  // rows per workgroup: 128 (a workgroup is one wavefront per 32 rows; 64- and 32-row workgroups
-  // measured slower even when 128-row ones leave compute units without work)
+  if (mode == 0 && !g.split_tiles && g.d_real <= 128 && few_query_tiles(g)) {
+#define LAUNCH_FEW(DD)                                                                                          \
+  do {                                                                                                          \
+    constexpr int kLds = 4 * 32 * (DD + 4) * (int)sizeof(float);                                                \
+    static LdsOnce once;                                                                                        \
+    const hipError_t e = reserve_lds(once, (const void*)fwd_f32_few_kernel<DD>, kLds);                          \
+    if (e != hipSuccess) {                                                                                      \
+      set_error("SDPA: cannot reserve %d bytes of LDS for fwd_f32_few_kernel: %s", kLds, hipGetErrorString(e)); \
+      return MI355_SDPA_ERR_LAUNCH;                                                                             \
+    }                                                                                                           \
+    hipLaunchKernelGGL((fwd_f32_few_kernel<DD>), dim3((unsigned)((int64_t)g.B * g.Hq * ((g.L + 31) / 32))), dim3(256), kLds, s, g); \
+  } while (0)
+    if (g.d_real <= 64) LAUNCH_FEW(64);
+    else LAUNCH_FEW(128);
+#undef LAUNCH_FEW
+    return check_launch("fwd_f32_few_kernel");
+  }
+  // rows per workgroup: 128 (a workgroup is one wavefront per 32 rows)
   const int waves = pick_waves((int64_t)g.B * g.Hq, g.L);
   g.n_qt = (g.L + 32 * waves - 1) / (32 * waves);
   const dim3 grid((unsigned)((int64_t)g.B * g.Hq * g.n_qt), (unsigned)g.n_split), block(64 * waves);
