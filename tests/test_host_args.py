@@ -1,0 +1,56 @@
+"""The native argument marshalling: what it refuses, and the block it writes against the tensors it was given."""
+
+import ctypes as C
+
+import pytest
+import torch
+
+
+@pytest.fixture(scope="module")
+def amd():
+    import torch_neuronx_amd as amd
+
+    return amd
+
+
+def test_refuses_what_is_no_gpu_tensor(amd):
+    p = amd._lib.FwdParams()
+    t = torch.zeros(1, 1, 2, 8)
+    with pytest.raises(ValueError, match="query"):
+        amd._lib.host().forward(C.addressof(p), t, t, t, None, True, False, 1.0, 0, False)
+    with pytest.raises(TypeError):
+        amd._lib.host().forward(C.addressof(p), None, t, t, None, True, False, 1.0, 0, False)
+    with pytest.raises(TypeError, match="arguments"):
+        amd._lib.host().backward(C.addressof(p), t)
+    with pytest.raises(ValueError):
+        amd.decode_fp8kv(t, t.to(torch.float8_e4m3fn), t.to(torch.float8_e4m3fn), t, t)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("layout", ["plain", "seq_major_view", "expanded_kv", "strided_head_dim", "one_row"])
+def test_block_and_outputs_of_a_call(amd, gpu_device, layout):
+    B, Hq, Hkv, L, S, E, Dv = 2, 4, 2, 5, 7, 16, 8
+    if layout == "one_row":
+        L = 1
+    q, k, v = (torch.randn(s, device=gpu_device) for s in ((B, Hq, L, E), (B, Hkv, S, E), (B, Hkv, S, Dv)))
+    if layout == "seq_major_view":
+        q, k, v = (t.transpose(1, 2).contiguous().transpose(1, 2) for t in (q, k, v))
+    elif layout == "expanded_kv":
+        k, v = k[:, :1].expand(B, Hkv, S, E), v[:, :1].expand(B, Hkv, S, Dv)
+    elif layout == "strided_head_dim":
+        q = q.transpose(2, 3).contiguous().transpose(2, 3)
+    p = amd._lib.FwdParams()
+    out, lse, hold = amd._lib.host().forward(C.addressof(p), q, k, v, None, True, True, 0.25, 2, False)
+    assert tuple(out.shape) == (B, Hq, L, Dv) and out.dtype == q.dtype and tuple(lse.shape) == (B, Hq, L)
+    want = amd.ops.empty_like_layout(q, (B, Hq, L, Dv))
+    assert out.stride() == (want.stride() if want.stride(3) == 1 else torch.empty(out.shape).stride())
+    assert len(hold) == (layout == "strided_head_dim" and L > 1)
+    for t, f in ((hold[0] if hold else q, p.q), (k, p.k), (v, p.v), (out, p.out)):
+        assert f.data == t.data_ptr() and tuple(f.size) == tuple(t.shape) and tuple(f.stride) == t.stride()
+    assert (p.lse, p.bias.data, p.dtype, p.is_causal, p.scale, p.force_kernel) == (lse.data_ptr(), None, amd._lib.F32, 1, 0.25, 2)
+    b = amd._lib.BwdParams()
+    go = torch.randn(out.shape, device=gpu_device)
+    dq, dk, dv, hold = amd._lib.host().backward(C.addressof(b), go, q, k, v, out, lse.double(), None, None, False, 0.5, 0, True)
+    for g, x, f in ((dq, q, b.grad_q), (dk, k, b.grad_k), (dv, v, b.grad_v)):
+        assert g.shape == x.shape and g.transpose(1, 2).is_contiguous() and f.data == g.data_ptr() and tuple(f.stride) == g.stride()
+    assert hold[-1].dtype == torch.float32 and b.lse == hold[-1].data_ptr()  # (a float64 log-sum-exp is converted)

@@ -1,4 +1,5 @@
-"""Builds libmi355_sdpa.so (hand-written gfx950 HIP kernels + C ABI) with hipcc, in-tree."""
+"""Builds, in-tree, libmi355_sdpa.so (hand-written gfx950 HIP kernels + C ABI, hipcc) and the extension
+module _host_args.so (argument marshalling on torch's C++ tensors, g++)."""
 
 from __future__ import annotations
 
@@ -6,12 +7,14 @@ import os
 import shutil
 import subprocess
 import sys
+import sysconfig
 from concurrent.futures import ThreadPoolExecutor
 
 PKG_DIR = os.path.dirname(os.path.abspath(__file__))
 CSRC_DIR = os.path.join(os.path.dirname(PKG_DIR), "csrc")
 LIB_DIR = os.path.join(PKG_DIR, "lib")
 LIB_PATH = os.path.join(LIB_DIR, "libmi355_sdpa.so")
+HOST_PATH = os.path.join(LIB_DIR, "_host_args.so")
 OBJ_DIR = os.path.join(LIB_DIR, "obj")
 
 SOURCES = ["api", "fwd_generic", "fwd_mfma", "fwd_mfma_w32", "bwd_generic", "bwd_mfma", "bwd_dkdv_w32", "bwd_dq_w32", "bwd_wide", "decode_fp8kv", "mask_rows", "f32_mfma"]
@@ -85,8 +88,33 @@ def _run(cmd, verbose):
     return _resource_lines(proc.stderr)
 
 
+def _host_flags():
+    import torch
+    from torch.utils.cpp_extension import include_paths
+
+    torch_lib = os.path.join(os.path.dirname(torch.__file__), "lib")
+    compile_flags = ["-O2", "-std=c++17", "-fPIC", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+                     *(f"-I{d}" for d in include_paths()), "-I" + sysconfig.get_path("include")]
+    link_flags = ["-shared", "-L" + LIB_DIR, "-l:" + os.path.basename(LIB_PATH), "-Wl,-rpath,$ORIGIN",
+                  "-L" + torch_lib, "-ltorch_python", "-ltorch_cpu", "-lc10"]
+    return compile_flags, link_flags
+
+
+def build_host(verbose: bool = False, compile_only: bool = False) -> None:
+    """The extension module; its link needs the library."""
+    compile_flags, link_flags = _host_flags()
+    obj = os.path.join(OBJ_DIR, "host_args.o")
+    if compile_only:
+        _run(["g++", *compile_flags, "-c", os.path.join(CSRC_DIR, "host_args.cpp"), "-o", obj], verbose)
+        return
+    tmp = HOST_PATH + ".tmp"
+    _run(["g++", obj, "-o", tmp, *link_flags], verbose)
+    os.replace(tmp, HOST_PATH)
+
+
 def build(verbose: bool = False, jobs: int = 6) -> str:
-    """Compile every HIP source for gfx950 and link the shared library.  Always recompiles."""
+    """Compile every HIP source for gfx950 and link the shared library, then the extension module.  Always
+    recompiles."""
     os.makedirs(OBJ_DIR, exist_ok=True)
     hipcc = _hipcc()
 
@@ -96,7 +124,9 @@ def build(verbose: bool = False, jobs: int = 6) -> str:
         return obj, _run([hipcc, *HIPCC_FLAGS, "-c", src, "-o", obj], verbose)
 
     with ThreadPoolExecutor(max_workers=jobs) as pool:
+        host = pool.submit(build_host, verbose, True)
         results = list(pool.map(compile_one, SOURCES))
+        host.result()
     objs = [o for o, _ in results]
     with open(RESOURCE_PATH + ".tmp", "w") as f:
         for name, (_, lines) in zip(SOURCES, results):
@@ -106,6 +136,7 @@ def build(verbose: bool = False, jobs: int = 6) -> str:
     tmp = LIB_PATH + ".tmp"
     _run([hipcc, "--offload-arch=gfx950", "-shared", "-fPIC", "-o", tmp, *objs], verbose)
     os.replace(tmp, LIB_PATH)
+    build_host(verbose)
     return LIB_PATH
 
 

@@ -7,12 +7,12 @@ missing the import of any op raises, so a GPU run can never silently take anothe
 from __future__ import annotations
 
 import ctypes as C
-import struct
+import importlib.util
 import os
 
 import torch
 
-from ._build import LIB_PATH
+from ._build import HOST_PATH, LIB_PATH
 
 F32, F16, BF16, F64, BOOL, FP8_E4M3, OTHER = 0, 1, 2, 3, 4, 5, 99
 KERNEL_NONE, KERNEL_GENERIC, KERNEL_MFMA, KERNEL_MFMA_T128, KERNEL_MFMA_T256 = 0, 1, 2, 3, 4
@@ -136,6 +136,27 @@ def load() -> C.CDLL:
     return _lib
 
 
+_host = None
+
+
+def host():
+    """The extension module that allocates a call's outputs and writes its parameter block
+    (csrc/host_args.cpp), loaded once.  Raises if it has not been built for these structures."""
+    global _host
+    if _host is None:
+        load()
+        if not os.path.exists(HOST_PATH):
+            raise RuntimeError(f"{HOST_PATH} is missing: build the extension first "
+                               "(python -m torch_neuronx_amd._build, or __graft_entry__.build()). There is no fallback path.")
+        spec = importlib.util.spec_from_file_location("_host_args", HOST_PATH)
+        mod = importlib.util.module_from_spec(spec)
+        spec.loader.exec_module(mod)
+        if (mod.FWD_BYTES, mod.BWD_BYTES, mod.DECODE_BYTES) != (C.sizeof(FwdParams), C.sizeof(BwdParams), C.sizeof(DecodeParams)):
+            raise RuntimeError(f"{HOST_PATH} was built for other structures than this binding's: rebuild it")
+        _host = mod
+    return _host
+
+
 def last_error() -> str:
     return load().mi355_sdpa_last_error().decode()
 
@@ -148,22 +169,6 @@ def tensor4(t) -> Tensor4:
         return Tensor4()
     assert t.dim() == 4
     return Tensor4(t.data_ptr(), _I64x4(*t.shape), _I64x4(*t.stride()))
-
-
-_T4 = struct.Struct("@P4q4q")
-assert _T4.size == C.sizeof(Tensor4)
-
-
-def put4(params, field, t) -> None:
-    """Write tensor ``t`` (4-D, or None: left zero) into the Tensor4 member ``field`` (a descriptor such
-    as ``FwdParams.q``) of the parameter block ``params``: one packed write, a third of the time of
-    building a Tensor4 and assigning it, which counts on calls whose kernels take microseconds."""
-    if t is None:
-        return
-    sh, st = t.shape, t.stride()
-    if len(sh) != 4:
-        raise ValueError("expected a 4-D tensor")
-    _T4.pack_into(params, field.offset, t.data_ptr(), sh[0], sh[1], sh[2], sh[3], st[0], st[1], st[2], st[3])
 
 
 _raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)

@@ -1,8 +1,8 @@
 """Host side of the fused attention path: marshals torch tensors into the C ABI.
 
-Everything here is plumbing - allocation of outputs with the layout rules of the operator
-contract, argument normalisation and error mapping.  All arithmetic happens in the HIP
-kernels behind ``libmi355_sdpa.so``.
+Everything here is plumbing - argument normalisation and error mapping; the outputs are allocated and
+the parameter blocks written natively (``_lib.host()``).  All arithmetic happens in the HIP kernels
+behind ``libmi355_sdpa.so``.
 """
 
 from __future__ import annotations
@@ -13,11 +13,6 @@ import math
 import torch
 
 from . import _lib
-
-
-def _require_cuda(t: torch.Tensor, name: str) -> None:
-    if t.device.type != "cuda":
-        raise ValueError(f"Expected a GPU tensor for {name}, got {t.device}")
 
 
 def make_desc(query, key, value, attn_bias=None, dropout_p=0.0, is_causal=False,
@@ -80,14 +75,8 @@ def out_strides(ref_sizes, ref_strides, out_sizes):
 
 def empty_like_layout(ref: torch.Tensor, shape, dtype=None) -> torch.Tensor:
     """New tensor of ``shape`` whose dimension order follows ``ref`` (stride-0 dims never alias)."""
-    if ref.is_contiguous() and 0 not in ref.shape:  # the common case needs no stride arithmetic
-        return torch.empty(tuple(shape), dtype=dtype or ref.dtype, device=ref.device)
     st = out_strides(ref.shape, ref.stride(), shape)
     return torch.empty_strided(tuple(shape), st, dtype=dtype or ref.dtype, device=ref.device)
-
-
-def _unit_last(t: torch.Tensor) -> torch.Tensor:
-    return t if t.stride(-1) == 1 or t.size(-1) <= 1 else t.contiguous()
 
 
 def _bias_view(attn_bias, B, Hq, L, S, repack_for=None):
@@ -293,27 +282,17 @@ def sdpa_forward(query, key, value, attn_bias=None, is_causal=False, scale=None,
 
     ``seq_major_out``: ``out`` is laid out ``(B,L,Hq,Dv)`` in memory whatever the query's layout, which
     is what upstream's memory-efficient operator promises its callers."""
-    score_mods = _score_mods(score_mods)
-    for t, n in ((query, "query"), (key, "key"), (value, "value")):
-        _require_cuda(t, n)
-    B, Hq, L, E = query.shape
-    S, Dv = key.shape[2], value.shape[3]
+    score_mods = _score_mods(score_mods) if score_mods else None
+    L = query.shape[2]
     if scale is None:
-        scale = 1.0 / math.sqrt(E)
-    q, k, v = _unit_last(query), _unit_last(key), _unit_last(value)
-    if seq_major_out:
-        out = torch.empty((B, L, Hq, Dv), dtype=query.dtype, device=query.device).transpose(1, 2)
-    else:
-        out = empty_like_layout(query, (B, Hq, L, Dv))
-        if out.stride(-1) != 1 and Dv > 1:
-            out = torch.empty((B, Hq, L, Dv), dtype=query.dtype, device=query.device)
-    lse = torch.empty((B, Hq, L), dtype=torch.float32, device=query.device) if need_lse else None
-    bias, bias_dt = _bias_view(attn_bias, B, Hq, L, S, repack_for=None if force_kernel == _lib.KERNEL_GENERIC else query.dtype)
-    p, P = _lib.FwdParams(), _lib.FwdParams
-    for f, t in ((P.q, q), (P.k, k), (P.v, v), (P.out, out), (P.bias, bias)):
-        _lib.put4(p, f, t)
-    p.lse = lse.data_ptr() if lse is not None else None
-    p.bias_dtype = bias_dt
+        scale = 1.0 / math.sqrt(query.shape[3])
+    bias = attn_bias
+    if bias is not None:
+        B, Hq, S = query.shape[0], query.shape[1], key.shape[2]
+        bias = _bias_view(attn_bias, B, Hq, L, S, repack_for=None if force_kernel == _lib.KERNEL_GENERIC else query.dtype)[0]
+    p = _lib.FwdParams()
+    out, lse, _hold = _lib.host().forward(C.addressof(p), query, key, value, bias, need_lse, bool(is_causal), scale,  # noqa: F841
+                                          force_kernel, seq_major_out)  # (_hold: copies that the launch reads)
     if kv_lens is not None:
         kv_lens = kv_lens.to(device=query.device, dtype=torch.int32).contiguous()
         p.kv_lens = kv_lens.data_ptr()
@@ -325,25 +304,25 @@ def sdpa_forward(query, key, value, attn_bias=None, is_causal=False, scale=None,
         if dropout_keep.numel() <= 1:
             dropout_p = 0.0  # a mask of one element is the reference's placeholder for none (torch_neuronx/_sdpa_math.py:42-45)
         else:
-            dropout_keep = _keep_rows(dropout_keep, B, Hq, L, S, query.dtype)
+            dropout_keep = _keep_rows(dropout_keep, query.shape[0], query.shape[1], L, key.shape[2], query.dtype)
             p.dropout_keep, p.dropout_keep_ld = dropout_keep.data_ptr(), dropout_keep.stride(2)
-    p.dropout_p = float(dropout_p)
-    p.dtype = _lib.dtype_id(query.dtype)
-    p.is_causal, p.scale, p.force_kernel = int(bool(is_causal)), float(scale), int(force_kernel)
+    if dropout_p:
+        p.dropout_p = float(dropout_p)
     if live_tiles is True:
-        live_tiles = mask_tile_maps(attn_bias, B, Hq, L, S)
-    _z = _mask_spec(p.mask, query, S, window, sink_keys, sink_logit, live_tiles, score_mods)  # noqa: F841 (kept alive over the launch)
+        live_tiles = mask_tile_maps(attn_bias, query.shape[0], query.shape[1], L, key.shape[2])
+    if window or sink_keys or sink_logit is not None or live_tiles is not None or score_mods:
+        _z = _mask_spec(p.mask, query, key.shape[2], window, sink_keys, sink_logit, live_tiles, score_mods)  # noqa: F841 (kept alive over the launch)
     if mask_verdict is not None:
         p.mask.mask_verdict = mask_verdict.data_ptr()
-    ws = None
+    lib, dev = _lib.load(), query.device
     if L <= 128:
         # few query rows: the library may want to split the keys over more workgroups
-        need = _lib.load().mi355_sdpa_fwd_workspace_bytes(C.byref(p))
+        need = lib.mi355_sdpa_fwd_workspace_bytes(C.byref(p))
         if need:
-            ws = torch.empty(need, dtype=torch.uint8, device=query.device)
+            ws = torch.empty(need, dtype=torch.uint8, device=dev)
             p.workspace, p.workspace_bytes = ws.data_ptr(), need
-    with _lib.on_device(query.device):
-        rc = _lib.load().mi355_sdpa_fwd(C.byref(p), _lib.current_stream(query.device))
+    with _lib.on_device(dev):
+        rc = lib.mi355_sdpa_fwd(C.byref(p), _lib.current_stream(dev))
     _lib.check(rc)
     return out, lse
 
@@ -361,37 +340,21 @@ def sdpa_backward(grad_out, query, key, value, out, lse, attn_bias=None, is_caus
     ``seq_major_grads``: dq, dk and dv are laid out ``(B,L,H,D)`` in memory whatever the inputs' layouts,
     and ``grad_bias_row_pad = 16`` leaves the bias gradient as a view of rows padded to 16 keys: the
     layouts upstream's memory-efficient backward promises its callers."""
-    score_mods = _score_mods(score_mods)
-    for t, n in ((grad_out, "grad_out"), (query, "query"), (key, "key"), (value, "value")):
-        _require_cuda(t, n)
-    B, Hq, L, E = query.shape
-    Hkv, S, Dv = key.shape[1], key.shape[2], value.shape[3]
+    score_mods = _score_mods(score_mods) if score_mods else None
+    L = query.shape[2]
     if scale is None:
-        scale = 1.0 / math.sqrt(E)
-    go, q, k, v, o = (_unit_last(t) for t in (grad_out, query, key, value, out))
-    lse = lse.to(torch.float32).contiguous()
-
-    def grad_like(ref, shape):
-        if seq_major_grads:
-            return torch.empty((shape[0], shape[2], shape[1], shape[3]), dtype=ref.dtype, device=ref.device).transpose(1, 2)
-        g = empty_like_layout(ref, shape)
-        if g.stride(-1) != 1 and shape[-1] > 1:
-            g = torch.empty(shape, dtype=ref.dtype, device=ref.device)
-        return g
-
-    dq, dk, dv = grad_like(query, (B, Hq, L, E)), grad_like(key, (B, Hkv, S, E)), grad_like(value, (B, Hkv, S, Dv))
-    bias, bias_dt = _bias_view(attn_bias, B, Hq, L, S, repack_for=None if force_kernel == _lib.KERNEL_GENERIC else query.dtype)
-    dbias = None
-    if want_grad_bias and bias is not None:
-        # (the matrix-op kernels for 16-bit inputs write the gradient four keys at a time: rows padded to that)
-        S4 = S if (query.dtype == torch.float32 or L == 1) and grad_bias_row_pad <= 4 else -(-S // grad_bias_row_pad) * grad_bias_row_pad
-        dbias = torch.empty((B, Hq, L, S4), dtype=query.dtype, device=query.device)[..., :S]
-    p, P = _lib.BwdParams(), _lib.BwdParams
-    for f, t in ((P.grad_out, go), (P.q, q), (P.k, k), (P.v, v), (P.out, o), (P.grad_q, dq), (P.grad_k, dk),
-                 (P.grad_v, dv), (P.bias, bias), (P.grad_bias, dbias)):
-        _lib.put4(p, f, t)
-    p.lse = lse.data_ptr()
-    p.bias_dtype = bias_dt
+        scale = 1.0 / math.sqrt(query.shape[3])
+    bias, dbias = attn_bias, None
+    if bias is not None:
+        B, Hq, S = query.shape[0], query.shape[1], key.shape[2]
+        bias = _bias_view(attn_bias, B, Hq, L, S, repack_for=None if force_kernel == _lib.KERNEL_GENERIC else query.dtype)[0]
+        if want_grad_bias:
+            # (the matrix-op kernels for 16-bit inputs write the gradient four keys at a time: rows padded to that)
+            S4 = S if (query.dtype == torch.float32 or L == 1) and grad_bias_row_pad <= 4 else -(-S // grad_bias_row_pad) * grad_bias_row_pad
+            dbias = torch.empty((B, Hq, L, S4), dtype=query.dtype, device=query.device)[..., :S]
+    p = _lib.BwdParams()
+    dq, dk, dv, _hold = _lib.host().backward(C.addressof(p), grad_out, query, key, value, out, lse, bias, dbias,  # noqa: F841
+                                             bool(is_causal), scale, force_kernel, seq_major_grads)
     if kv_lens is not None:
         kv_lens = kv_lens.to(device=query.device, dtype=torch.int32).contiguous()
         p.kv_lens = kv_lens.data_ptr()
@@ -403,26 +366,27 @@ def sdpa_backward(grad_out, query, key, value, out, lse, attn_bias=None, is_caus
         if dropout_keep.numel() <= 1:
             dropout_p = 0.0  # a mask of one element is the reference's placeholder for none (torch_neuronx/_sdpa_math.py:42-45)
         else:
-            dropout_keep = _keep_rows(dropout_keep, B, Hq, L, S, query.dtype)
+            dropout_keep = _keep_rows(dropout_keep, query.shape[0], query.shape[1], L, key.shape[2], query.dtype)
             p.dropout_keep, p.dropout_keep_ld = dropout_keep.data_ptr(), dropout_keep.stride(2)
-    p.dropout_p = float(dropout_p)
-    p.dtype = _lib.dtype_id(query.dtype)
-    p.is_causal, p.scale, p.force_kernel = int(bool(is_causal)), float(scale), int(force_kernel)
+    if dropout_p:
+        p.dropout_p = float(dropout_p)
     if live_tiles is True:
-        live_tiles = mask_tile_maps(attn_bias, B, Hq, L, S)
-    _z, _keep = _mask_spec(p.mask, query, S, window, sink_keys, sink_logit, live_tiles, score_mods)
+        live_tiles = mask_tile_maps(attn_bias, query.shape[0], query.shape[1], L, key.shape[2])
+    _z = None
+    if window or sink_keys or sink_logit is not None or live_tiles is not None or score_mods:
+        _z, _keep = _mask_spec(p.mask, query, key.shape[2], window, sink_keys, sink_logit, live_tiles, score_mods)  # noqa: F841
     if mask_verdict is not None:
         p.mask.mask_verdict = mask_verdict.data_ptr()
     dsink = None
     if _z is not None:
         dsink = torch.empty(_z.shape, dtype=torch.float32, device=query.device)
         p.grad_sink_logit = dsink.data_ptr()
-    lib = _lib.load()
+    lib, dev = _lib.load(), query.device
     nbytes = lib.mi355_sdpa_bwd_workspace_bytes(C.byref(p))
-    ws = torch.empty((max(nbytes, 1),), dtype=torch.uint8, device=query.device)
+    ws = torch.empty(max(nbytes, 1), dtype=torch.uint8, device=dev)
     p.workspace, p.workspace_bytes = ws.data_ptr(), nbytes
-    with _lib.on_device(query.device):
-        rc = lib.mi355_sdpa_bwd(C.byref(p), _lib.current_stream(query.device))
+    with _lib.on_device(dev):
+        rc = lib.mi355_sdpa_bwd(C.byref(p), _lib.current_stream(dev))
     _lib.check(rc)
     if dbias is not None and dbias.stride(2) != S and L > 1 and grad_bias_row_pad <= 4:
         dbias = dbias.contiguous()  # (rows were padded for the kernel)
@@ -439,13 +403,10 @@ def decode_fp8kv(query, k_fp8, v_fp8, k_scale, v_scale, kv_lens=None, scale=None
     allocates nothing: the caller passes ``out`` (and ``lse`` if wanted), ``k_scale`` / ``v_scale`` /
     ``kv_lens`` must already be contiguous float32 / int32 device tensors, and nothing is allocated
     here either."""
-    for t, n in ((query, "query"), (k_fp8, "key"), (v_fp8, "value")):
-        _require_cuda(t, n)
     if k_fp8.dtype != torch.float8_e4m3fn or v_fp8.dtype != torch.float8_e4m3fn:
         raise RuntimeError("decode_fp8kv: key and value must be float8_e4m3fn")
-    B, Hq, Lq, D = query.shape
     if scale is None:
-        scale = 1.0 / math.sqrt(D)
+        scale = 1.0 / math.sqrt(query.shape[3])
     if static_scratch:
         if out is None:
             raise ValueError("decode_fp8kv: static_scratch=True needs a preallocated out")
@@ -456,39 +417,19 @@ def decode_fp8kv(query, k_fp8, v_fp8, k_scale, v_scale, kv_lens=None, scale=None
         for t, n in ((query, "query"), (k_fp8, "key"), (v_fp8, "value"), (out, "out")):
             if t.stride(-1) != 1:
                 raise ValueError(f"decode_fp8kv: with static_scratch=True {n} must have unit stride on the head dim")
-        q, k, v, ks, vs = query, k_fp8, v_fp8, k_scale, v_scale
-    else:
-        q, k, v = _unit_last(query), _unit_last(k_fp8), _unit_last(v_fp8)
-        if out is None:
-            out = torch.empty((B, Hq, Lq, v.shape[3]), dtype=query.dtype, device=query.device)
-        if lse is None and need_lse:
-            lse = torch.empty((B, Hq, Lq), dtype=torch.float32, device=query.device)
-        ks = k_scale.to(device=query.device, dtype=torch.float32).contiguous()
-        vs = v_scale.to(device=query.device, dtype=torch.float32).contiguous()
-        if kv_lens is not None:
-            kv_lens = kv_lens.to(device=query.device, dtype=torch.int32).contiguous()
-    if tuple(out.shape) != (B, Hq, Lq, v.shape[3]) or out.dtype != query.dtype:
-        raise ValueError("decode_fp8kv: out must have shape (B, Hq, Lq, D) and the query's dtype")
-    if lse is not None and (tuple(lse.shape) != (B, Hq, Lq) or lse.dtype != torch.float32 or not lse.is_contiguous()):
-        raise ValueError("decode_fp8kv: lse must be a contiguous float32 (B, Hq, Lq) tensor")
-    p, P = _lib.DecodeParams(), _lib.DecodeParams
-    for f, t in ((P.q, q), (P.k, k), (P.v, v), (P.out, out)):
-        _lib.put4(p, f, t)
-    p.k_scale, p.v_scale = ks.data_ptr(), vs.data_ptr()
-    if kv_lens is not None:
-        p.kv_lens = kv_lens.data_ptr()
-    p.lse = lse.data_ptr() if lse is not None else None
-    p.q_dtype, p.scale, p.num_splits = _lib.dtype_id(query.dtype), float(scale), int(num_splits)
-    lib = _lib.load()
+    p = _lib.DecodeParams()
+    out, lse, _hold = _lib.host().decode(C.addressof(p), query, k_fp8, v_fp8, k_scale, v_scale, kv_lens, out, lse,  # noqa: F841
+                                         need_lse and not static_scratch, scale, num_splits)
+    lib, dev = _lib.load(), query.device
     if static_scratch:
-        with _lib.on_device(query.device):
-            rc = lib.mi355_sdpa_decode_fp8kv_static(C.byref(p), _lib.current_stream(query.device))
+        with _lib.on_device(dev):
+            rc = lib.mi355_sdpa_decode_fp8kv_static(C.byref(p), _lib.current_stream(dev))
         _lib.check(rc)
         return out, lse
     nbytes = lib.mi355_sdpa_decode_workspace_bytes(C.byref(p))
-    ws = torch.empty((max(nbytes, 1),), dtype=torch.uint8, device=query.device)
+    ws = torch.empty(max(nbytes, 1), dtype=torch.uint8, device=dev)
     p.workspace, p.workspace_bytes = ws.data_ptr(), nbytes
-    with _lib.on_device(query.device):
-        rc = lib.mi355_sdpa_decode_fp8kv(C.byref(p), _lib.current_stream(query.device))
+    with _lib.on_device(dev):
+        rc = lib.mi355_sdpa_decode_fp8kv(C.byref(p), _lib.current_stream(dev))
     _lib.check(rc)
     return out, lse

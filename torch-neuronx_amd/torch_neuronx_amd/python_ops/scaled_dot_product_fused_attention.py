@@ -49,19 +49,17 @@ def _empty_rng(device):
     return pair
 
 
-_validated = set()
+_debug_masks = {}
 
 
-def _validate_once(query, key, value, attn_bias, dropout_p, is_causal, scale):
-    """Boundary checks of the call; a signature that passed is not checked again."""
-    sig = (query.shape, key.shape, value.shape, query.dtype, key.dtype, value.dtype, key.device.type,
-           value.device.type, attn_bias is None, dropout_p, is_causal, scale,
-           query.stride(-1), key.stride(-1), value.stride(-1))
-    if sig in _validated:
-        return
-    ops.validate(ops.make_desc(query, key, value, attn_bias, dropout_p, is_causal, False, scale))
-    if len(_validated) < 4096 and all(isinstance(d, int) for t in (query, key, value) for d in t.shape):
-        _validated.add(sig)
+def _no_debug_mask(query):
+    # upstream's debug mask when none is asked for: an empty tensor of the query's dtype, never written,
+    # so one per device and dtype serves every call
+    key = (query.device, query.dtype)
+    mask = _debug_masks.get(key)
+    if mask is None:
+        mask = _debug_masks[key] = torch.empty((0,), dtype=query.dtype, device=query.device)
+    return mask
 
 
 def _dropout_keep(query, S, dropout_p):
@@ -197,15 +195,15 @@ def _forward(query, key, value, attn_bias, dropout_p, is_causal, return_debug_ma
     attn_bias = _present(attn_bias)
     if return_debug_mask:
         raise NotImplementedError("Debug mask not supported in Neuron implementation.")
-    _validate_once(query, key, value, attn_bias, dropout_p, is_causal, scale)
+    _lib.host().validate(query, key, value, attn_bias is not None, dropout_p, is_causal)
     orig_dtype = query.dtype
     if orig_dtype == torch.float64:  # computed as float32, result restored to the caller's dtype
         query, key, value = query.float(), key.float(), value.float()  # (no-ops for float32 key / value)
         if attn_bias is not None and attn_bias.dtype == torch.float64:
             attn_bias = attn_bias.float()
-    S = key.shape[2]
     keep = None
     if dropout_p > 0.0:
+        S = key.shape[2]
         if upstream is not None and not torch.cuda.is_current_stream_capturing():
             remember = torch.is_grad_enabled() and (query.requires_grad or key.requires_grad or value.requires_grad)
             keep, seed, offset = _seeded_keep(query, S, dropout_p, remember)
@@ -214,8 +212,10 @@ def _forward(query, key, value, attn_bias, dropout_p, is_causal, return_debug_ma
             seed, offset = keep, torch.empty((0,), dtype=torch.int32, device=query.device)
     else:
         seed, offset = _empty_rng(query.device) if upstream is None else _scalar_rng()
-    attn_bias, is_causal, functor = _recover_pattern(attn_bias, is_causal, query, key, dropout_p=dropout_p)
-    functor = _skip_tables(functor, attn_bias, is_causal, dropout_p, query, key)
+    functor = {}
+    if attn_bias is not None:
+        attn_bias, is_causal, functor = _recover_pattern(attn_bias, is_causal, query, key, dropout_p=dropout_p)
+        functor = _skip_tables(functor, attn_bias, is_causal, dropout_p, query, key)
     out, lse = ops.sdpa_forward(query, key, value, attn_bias=attn_bias, is_causal=is_causal, scale=scale,
                                 dropout_p=dropout_p, dropout_keep=keep, need_lse=need_lse,
                                 force_kernel=_force_kernel(), seq_major_out=upstream == "efficient", **functor)
@@ -253,8 +253,10 @@ def _backward(grad_out, query, key, value, attn_bias, out, logsumexp, dropout_p,
             dropout_p = 0.0  # a placeholder carries no mask: treated as absent (_sdpa_math.py:42-45)
         else:
             keep = philox_seed
-    attn_bias, is_causal, functor = _recover_pattern(attn_bias, is_causal, query, key, want_grad_bias, dropout_p=dropout_p)
-    functor = _skip_tables(functor, attn_bias, is_causal, dropout_p, query, key)
+    functor = {}
+    if attn_bias is not None:
+        attn_bias, is_causal, functor = _recover_pattern(attn_bias, is_causal, query, key, want_grad_bias, dropout_p=dropout_p)
+        functor = _skip_tables(functor, attn_bias, is_causal, dropout_p, query, key)
     dq, dk, dv, dbias = ops.sdpa_backward(
         grad_out, query, key, value, out, logsumexp, attn_bias=attn_bias, is_causal=is_causal, scale=scale,
         dropout_p=dropout_p, dropout_keep=keep, want_grad_bias=want_grad_bias, force_kernel=_force_kernel(),
@@ -283,8 +285,7 @@ def scaled_dot_product_flash_attention(
     the (empty) debug mask as upstream's operator returns them."""
     out, lse, seed, offset = _forward(query, key, value, None, dropout_p, is_causal, return_debug_mask, scale,
                                       upstream="flash")
-    return (out, lse, None, None, query.shape[2], key.shape[2], seed, offset,
-            torch.empty((0,), dtype=query.dtype, device=query.device))
+    return out, lse, None, None, query.shape[2], key.shape[2], seed, offset, _no_debug_mask(query)
 
 
 def scaled_dot_product_flash_attention_backward(
