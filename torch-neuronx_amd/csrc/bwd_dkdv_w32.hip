@@ -1,4 +1,5 @@
-// Flash-attention backward, dK and dV, for gfx950, head dim 64 or 128, bf16/f16.
+// Flash-attention backward, dK and dV, for gfx950, head dim 64 or 128, bf16/f16 (at 64 the calls with a bias, a
+// window, a functor or split dQ keys: bwd_d64.hip has the others).
 //
 // One workgroup = 8 wavefronts = 128 keys of one (batch, kv head); it loops over the query
 // heads of the group (the GQA sum of decompositions.py:2595-2598 happens in registers) and over
@@ -870,7 +871,11 @@ int launch_m(const BwdM& g, hipStream_t s) {
       set_error("SDPA: dropout in bwd_dkdv_w32_kernel needs a keep-mask and no tile table");
       return MI355_SDPA_ERR_UNSUPPORTED;
     }
-    if (!g.bias_kind) return launch_t<T, D, 3>(g, s);
+    if (!g.bias_kind) {
+      if constexpr (D != 64) return launch_t<T, D, 3>(g, s);
+      set_error("SDPA: dropout without a bias at head dims up to 64 belongs to bwd_d64.hip");
+      return MI355_SDPA_ERR_UNSUPPORTED;
+    }
     if (g.verdict) {  // (see bwd_dkdv_w32_kernel: the pair with dropout)
       if (int rc = launch_t<T, D, 3, true>(g, s)) return rc;
     }
@@ -926,18 +931,16 @@ int launch_bwd_dkdv_merge(const BwdM& g, int dtype, hipStream_t s) {
   return check_launch("bwd_dkdv_merge_kernel");
 }
 
-int launch_bwd_dkdv_w32(const BwdM& g0, int dtype, int head_dim, hipStream_t s) {
-  BwdM g = g0;
-  if (g.d_real <= 0 || g.d_real > head_dim) g.d_real = head_dim;
-  g.dv_real = g.d_real;
+// the split of a call's items as the kernels and bwd_dkdv_merge_kernel read it (g.parts = 1 without room for the parts)
+bool bwd_dkdv_plan_parts(BwdM& g) {
   g.parts_h = 1, g.chunk_items = 0;
   if (!g.part_dk || !g.part_dv) g.parts = 1;
   if (g.parts > 1) {
     int parts;
     bwd_dkdv_w32_plan(g, g.parts_h, parts);
     if (parts != g.parts) {
-      set_error("SDPA: bwd_dkdv_w32_kernel was given %d parts where its plan has %d", g.parts, parts);
-      return MI355_SDPA_ERR_INVALID;
+      set_error("SDPA: the dK/dV kernel was given %d parts where its plan has %d", g.parts, parts);
+      return false;
     }
     // the heaviest workgroup (every query tile of its heads) fills all the tile shares
     const int parts_q = g.parts / g.parts_h;
@@ -946,6 +949,14 @@ int launch_bwd_dkdv_w32(const BwdM& g0, int dtype, int head_dim, hipStream_t s) 
     // count: every key block then deals its items to all the parts in equal shares)
     if (g.sm.doc_sorted) g.chunk_items = 0;
   }
+  return true;
+}
+
+int launch_bwd_dkdv_w32(const BwdM& g0, int dtype, int head_dim, hipStream_t s) {
+  BwdM g = g0;
+  if (g.d_real <= 0 || g.d_real > head_dim) g.d_real = head_dim;
+  g.dv_real = g.d_real;
+  if (!bwd_dkdv_plan_parts(g)) return MI355_SDPA_ERR_INVALID;
   if (!g.sm.doc_sorted || g.n_kt > 1024) g.kt_order = nullptr;  // (the ranking kernel holds 1024 weights)
   if (head_dim == 128) return dtype == MI355_SDPA_BF16 ? launch_m<bf16_t, 128>(g, s) : launch_m<f16_t, 128>(g, s);
   return dtype == MI355_SDPA_BF16 ? launch_m<bf16_t, 64>(g, s) : launch_m<f16_t, 64>(g, s);

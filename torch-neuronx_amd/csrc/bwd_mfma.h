@@ -87,6 +87,8 @@ struct BwdM {
 // parts the dK/dV kernel of bwd_dkdv_w32.hip / of bwd_wide.hip would use for this call
 int bwd_dkdv_w32_parts(const BwdM& g);
 int bwd_wide_parts(const BwdM& g);
+// fills in the split of a call's items (false: the parts given are not the plan's)
+bool bwd_dkdv_plan_parts(BwdM& g);
 // adds up the parts' rows (g.parts, g.part_dk with d_real columns, g.part_dv with dv_real) into dK and dV
 int launch_bwd_dkdv_merge(const BwdM& g, int dtype, hipStream_t s);
 
@@ -132,6 +134,10 @@ int launch_bwd_dkdv_w32(const BwdM& g, int dtype, int head_dim, hipStream_t s);
 // dQ with two wavefronts per SIMD (bwd_dq_w32.hip), same convention
 bool bwd_dq_w32_fits(const BwdM& g, int head_dim);
 int launch_bwd_dq_w32(const BwdM& g, int dtype, int head_dim, hipStream_t s);
+// both kernels at head dims up to 64 for the calls they take; the bits of a dropout mask live in the workspace
+bool bwd_d64_takes(const BwdM& g);
+size_t bwd_d64_bits_bytes(const BwdM& g);
+int launch_bwd_d64(const BwdM& g, int dtype, uint32_t* keep_bits, hipStream_t s);
 // head dims above 128 and D_qk != D_v (D_v <= D_qk <= 256), without masks (bwd_wide.hip)
 int launch_bwd_wide(const BwdM& g, int dtype, hipStream_t s);
 

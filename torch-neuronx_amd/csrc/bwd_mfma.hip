@@ -677,8 +677,9 @@ size_t bwd_mfma_workspace(const mi355_sdpa_bwd_params& p) {
   if (p.dtype != MI355_SDPA_BF16 && p.dtype != MI355_SDPA_F16) return row_terms_bytes(p);
   BwdM g;
   fill(g, p);
-  int split_tiles;
-  return row_terms_bytes(p) + part_rows_bytes(g, parts_of(g, p)) + dq_part_bytes(g, dq_splits(g, p, &split_tiles));
+  g.dq_n_split = dq_splits(g, p, &g.dq_split_tiles);
+  // (dQ parts and the bits of a dropout mask never come together)
+  return row_terms_bytes(p) + part_rows_bytes(g, parts_of(g, p)) + std::max(dq_part_bytes(g, g.dq_n_split), bwd_d64_bits_bytes(g));
 }
 
 int launch_bwd_mfma(const mi355_sdpa_bwd_params& p, hipStream_t s) {
@@ -705,7 +706,10 @@ int launch_bwd_mfma(const mi355_sdpa_bwd_params& p, hipStream_t s) {
   if (key_order_bytes(p) && p.workspace_bytes >= row_terms_bytes(p)) g.kt_order = (int32_t*)((char*)p.workspace + row_stats_bytes(p));
   const int D = p.q.size[3] <= 64 ? 64 : 128;  // the kernels' width
   int rc;
-  if (p.q.size[3] > 128 || p.v.size[3] != p.q.size[3]) rc = launch_bwd_wide(g, p.dtype, s);
+  if (bwd_d64_takes(g)) {
+    const size_t at = row_terms_bytes(p) + part_rows_bytes(g, parts);
+    rc = launch_bwd_d64(g, p.dtype, p.workspace_bytes >= at + bwd_d64_bits_bytes(g) ? (uint32_t*)((char*)p.workspace + at) : nullptr, s);
+  } else if (p.q.size[3] > 128 || p.v.size[3] != p.q.size[3]) rc = launch_bwd_wide(g, p.dtype, s);
   else if (p.dtype == MI355_SDPA_BF16) rc = D == 128 ? launch_td<bf16_t, 128>(g, s) : launch_td<bf16_t, 64>(g, s);
   else rc = D == 128 ? launch_td<f16_t, 128>(g, s) : launch_td<f16_t, 64>(g, s);
   // (a sink logit changes nothing in these kernels: the probabilities come from the saved
