@@ -1,0 +1,75 @@
+"""The forward with a soft cap and no other score functor (its variant of the 32-row kernels):
+sizes around its 32-key tiles, windows, key counts that leave tiles and rows without a key, scores far beyond the
+cap, a cap far beyond the scores, infinite scores.
+
+Bounds, against the same attention in float64 on the kernel's inputs: the capped score is cap (1 - 2 r) with r
+to 2^-22 relative, so a score is off by at most 2^-21 cap and what the float32 sum of its products loses
+(2^-21 scale sum |q||k|), in lse as well (plus 2^-20 |lse| of its own sum); the output carries that, the rounding of P
+(2^-9 in bf16, 2^-12 in f16) and its own: 2.5 roundings and twice the score's error times the largest |v|."""
+
+import math
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def amd(gpu_device):
+    import torch_neuronx_amd as amd
+
+    return amd
+
+
+CASES = [
+    # B, Hq, Hkv, L, S, D, causal, window, lens, cap, strength of the scores
+    (1, 2, 2, 31, 33, 128, False, None, None, 5.0, 1.0),
+    (1, 4, 2, 65, 127, 256, True, None, None, 50.0, 4.0),
+    (2, 2, 1, 130, 130, 256, True, 40, None, 2.0, 1.0),
+    (3, 2, 2, 100, 193, 160, False, None, [193, 0, 65], 5.0, 30.0),
+    (2, 4, 4, 300, 300, 128, True, 64, [300, 129], 50.0, 1.0),
+    (1, 2, 2, 40, 600, 256, True, 100, None, 30.0, 1.0),   # rows whose first tiles lie outside the window
+    (1, 8, 2, 513, 513, 128, True, None, None, 1e4, 1.0),
+    (2, 2, 1, 97, 225, 64, True, 50, [225, 96], 5.0, 2.0),
+    (1, 3, 3, 200, 64, 40, False, None, None, 50.0, 8.0),
+    (1, 1, 1, 2, 700, 256, False, None, None, 5.0, 1.0),
+]
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("case", CASES, ids=lambda c: "L%d_S%d_D%d_c%d_w%s_cap%g_x%g" % (c[3:8] + c[9:]))
+def test_against_float64(amd, gpu_device, case, dtype):
+    B, Hq, Hkv, L, S, D, causal, window, lens, cap, strong = case
+    dev = gpu_device
+    g = torch.Generator(device=dev).manual_seed(L * 7 + S)
+    q, k, v = (torch.randn(s, generator=g, device=dev) for s in ((B, Hq, L, D), (B, Hkv, S, D), (B, Hkv, S, D)))
+    q, k, v = (q * strong).to(dtype), k.to(dtype), v.to(dtype)
+    q[0, 0, 0], k[0, 0, 0] = math.inf, k[0, 0, 0].abs() + 0.5  # that row's scores: +inf at key 0, NaN at the others
+    kw = dict(is_causal=causal, softcap=cap)
+    if window:
+        kw["window"] = window
+    lens_t = torch.full((B,), S, device=dev) if lens is None else torch.tensor(lens, device=dev)
+    if lens is not None:
+        kw["kv_lens"] = lens_t.to(torch.int32)
+    out, lse = amd.sdpa_forward(q, k, v, **kw)
+    Q, (K, V) = q.double(), (t.double().repeat_interleave(Hq // Hkv, 1) for t in (k, v))
+    s = cap * torch.tanh(Q @ K.transpose(-1, -2).contiguous() / math.sqrt(D) / cap)
+    i, j = torch.arange(L, device=dev)[:, None], torch.arange(S, device=dev)[None]
+    dead = (j[None] >= lens_t[:, None, None])[:, None].expand(B, 1, L, S).clone()
+    if causal:
+        dead |= j > i
+    if window:
+        dead |= j < i - window + 1
+    s = s.masked_fill(dead, -math.inf)
+    want, want_lse = torch.softmax(s, -1).nan_to_num(0.0) @ V, torch.logsumexp(s, -1)
+    poisoned = torch.zeros(B, Hq, L, dtype=torch.bool, device=dev)
+    poisoned[0, 0, 0] = bool(torch.isnan(s[0, 0, 0]).any())  # (a causal row 0 sees key 0 alone: its score is the cap)
+    empty = dead.all(-1).expand(B, Hq, L)
+    assert (out[empty & ~poisoned] == 0).all() and (lse[empty & ~poisoned] == -math.inf).all()
+    ok = ~empty & ~poisoned
+    products = (Q.abs() @ K.abs().transpose(-1, -2).contiguous() / math.sqrt(D)).masked_fill(torch.isinf(Q).any(-1, keepdim=True), 0.0)
+    score_err = 2.0**-21 * (cap + float(products.max()))
+    assert ((lse.double() - want_lse)[ok].abs() <= score_err + 2.0**-20 * want_lse[ok].abs() + 2.0**-20).all()
+    eps = 2.0**-9 if dtype is torch.bfloat16 else 2.0**-12
+    assert float((out.double() - want)[ok].abs().max()) <= (2.5 * eps + 2 * score_err) * float(V.abs().max())

@@ -27,6 +27,7 @@
 //
 // Numerics: torch_neuronx/_sdpa_math.py:51-95 (float32 accumulation and softmax, probabilities
 // rounded to the input dtype for P*V only, dead rows give zeros and lse = -inf).
+#include <algorithm>
 #include <type_traits>
 
 #include "fwd_mfma.h"
@@ -52,6 +53,11 @@ constexpr float kLazy = 8.f;  // log2 headroom before the accumulator is rescale
 // MASK = 4 is MASK = 1 plus the score functors and document ids of score_mod.h:
 // they rewrite the raw score tile in a block of its own right after the matrix ops that produce it,
 // where the bias of MASK = 2 is folded in, so the softmax behind them is the common code.
+// MASK = 5 is MASK = 1 plus a soft cap and no other functor: s -> cap tanh(s / cap)
+// rides on the matrix ops as part of the softmax, two stages more per score (see cap_e, cap_x).  As the block
+// of MASK = 4 it ran with the matrix pipe idle, at head dim 256 with nobody on the SIMD to fill it (B=2, 16 heads,
+// S=4096, D=256, window 1024: 264 -> 206 us, the same call without a cap 180; causal, no window 411 -> 318; D=128,
+// 32 heads, causal 377 -> 327; D=64, 32 heads, causal 270 -> 247, 16 heads, S=1000, B=4 46.5 -> 37).
 template <typename T, int D, int WAVES, int MASK>
 __device__ __forceinline__ void fwd_w32_body(const FwdM& p, const MaskArgs ma) {
   constexpr int BM = 32 * WAVES, NT = 64 * WAVES;
@@ -69,7 +75,8 @@ __device__ __forceinline__ void fwd_w32_body(const FwdM& p, const MaskArgs ma) {
   // Tiles go from global memory straight into LDS (see the staging section): four unpadded,
   // swizzled buffers per operand, tile t in buffer t % 4.
   // mask functors (window, sink keys, sink logit): in the masked variant without a bias
-  constexpr bool FUNC = MASK == 1 || MASK == 4;
+  constexpr bool FUNC = MASK == 1 || MASK == 4 || MASK == 5;
+  constexpr bool CAP = MASK == 5;
   constexpr bool SMOD = MASK == 4;  // score functors, document ids
   constexpr int NBUF = 4, TILE = BN * D;
   __shared__ __attribute__((aligned(16))) uint16_t k_static[DYN ? 8 : NBUF * TILE];
@@ -311,9 +318,13 @@ __device__ __forceinline__ void fwd_w32_body(const FwdM& p, const MaskArgs ma) {
   const u32x4 kd_rsrc = descriptor(kp, k_bytes), vd_rsrc = descriptor(vp, v_bytes);
   const int d_wave = DSPLIT ? wave % KL : wave;  // this wavefront's first 1 KB slice of a tile
   const bool dma_k = !DSPLIT || wave < KL, dma_v = !DSPLIT || wave >= KL;  // (uniform per wavefront)
-  uint32_t kd_off[NL], vd_off[NL];
+  // (rows 16 apart share a swizzle: such loads share an offset register, the rows between them travel in the
+  // uniform part of the offset)
+  constexpr int LROWS = WAVES * 64 / CH, UNQ = LROWS >= 16 ? 1 : std::min(NL, 16 / LROWS);
+  const uint32_t k_step = (uint32_t)(UNQ * LROWS * p.k_sl * 2), v_step = (uint32_t)(UNQ * LROWS * p.v_sl * 2);
+  uint32_t kd_off[UNQ], vd_off[UNQ];
 #pragma unroll
-  for (int i = 0; i < NL; ++i) {
+  for (int i = 0; i < UNQ; ++i) {
     const int ch = (d_wave + i * WAVES) * 64 + lane, row = ch / CH, gch = (ch % CH) ^ tile_swz<D>(row);
     kd_off[i] = (uint32_t)((row * p.k_sl + gch * 8) * 2);
     vd_off[i] = (uint32_t)((row * p.v_sl + gch * 8) * 2);
@@ -335,14 +346,14 @@ __device__ __forceinline__ void fwd_w32_body(const FwdM& p, const MaskArgs ma) {
     const uint32_t g = (uint32_t)(tile_of(min(t, nt - 1)) * k_tile_bytes), l = lds_kd + (uint32_t)((t & (NBUF - 1)) * TILE * 2);
     if (dma_k) {
 #pragma unroll
-      for (int i = 0; i < NL; ++i) tile_load(kd_rsrc, kd_off[i] + g, l + i * WAVES * 1024);
+      for (int i = 0; i < NL; ++i) tile_load(kd_rsrc, kd_off[i % UNQ] + (g + (i / UNQ) * k_step), l + i * WAVES * 1024);
     }
   };
   auto request_v = [&](int t) {
     const uint32_t g = (uint32_t)(tile_of(min(t, nt - 1)) * v_tile_bytes), l = lds_vd + (uint32_t)((t & (NBUF - 1)) * TILE * 2);
     if (dma_v) {
 #pragma unroll
-      for (int i = 0; i < NL; ++i) tile_load(vd_rsrc, vd_off[i] + g, l + i * WAVES * 1024);
+      for (int i = 0; i < NL; ++i) tile_load(vd_rsrc, vd_off[i % UNQ] + (g + (i / UNQ) * v_step), l + i * WAVES * 1024);
     }
   };
   auto request_pair = [&](int j) { request_k(j + 1), request_v(j); };
@@ -627,13 +638,21 @@ __device__ __forceinline__ void fwd_w32_body(const FwdM& p, const MaskArgs ma) {
   // tile's probabilities.  Exact arithmetic: numerator and row sum always carry the same
   // reference, and lse = reference * scale + ln(sum).
   constexpr float kTrig = 8192.f;  // 16 probabilities of at most 2^kLazy stay below this
+  // Soft cap (MASK = 5): with e = 2^(2 log2(e) scale s / cap) and r = 1 / (1 + e) the capped score is
+  // cap (1 - 2 r), so its exponent in the log2 domain, reference subtracted, is one multiply-add on r.  A
+  // masked score (-inf) would come out as -cap: the minimum with s + 1e30 keeps it (and a NaN).
+  auto scalar = [](float x) { return __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, x))); };
+  const float cap_k = CAP ? scalar(2.f * kLog2eF * p.scale / p.sm.softcap) : 0.f, cap_2l = CAP ? scalar(-2.f * kLog2eF * p.sm.softcap) : 0.f;
+  const float cap_raw = CAP ? scalar(p.sm.softcap / p.scale) : 0.f;  // the cap in units of the raw scores
+  auto cap_r = [&](float s) { return __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(s * cap_k)); };
   auto raise_reference = [&](float t0) {
-    const float tm = fmaxf(t0, __shfl_xor(t0, 32, 64));
+    float tm = fmaxf(t0, __shfl_xor(t0, 32, 64));
+    if constexpr (CAP) tm = fminf(fmaf(cap_r(tm), -2.f * cap_raw, cap_raw), tm + 1e30f);  // (the cap is monotonic)
     const bool up = (tm - m_run) * c > kLazy;  // false for NaN (-inf minus -inf)
     m_new = up ? tm : m_run;
     const float m_use = (m_new == -INFINITY) ? 0.f : m_new;
     alpha = __builtin_amdgcn_exp2f((m_run - m_use) * c);
-    mc = m_use * c;
+    mc = CAP ? fmaf(-0.5f, cap_2l, -m_use * c) : m_use * c;  // (soft cap: what is left of the cap's exponent above the reference)
     need_rescale = __builtin_amdgcn_ballot_w64(up) != 0;
   };
 
@@ -641,9 +660,22 @@ __device__ __forceinline__ void fwd_w32_body(const FwdM& p, const MaskArgs ma) {
   // hand (the chain read S -> fma -> exp2 -> add/pack is strictly dependent and a wavefront
   // issues in order).  Pair j of 8: accumulator registers 2 j, 2 j + 1.
   float xs[2][2], pv[2][2];
+  float ce[2];  // (soft cap) 2^(...) of the pair on its way
+  auto cap_e = [&](const f32x16& sv, int j) {
+    ce[0] = __builtin_amdgcn_exp2f(sv[2 * j] * cap_k);
+    ce[1] = __builtin_amdgcn_exp2f(sv[2 * j + 1] * cap_k);
+  };
+  auto cap_x = [&](const f32x16& sv, int j) {
+    xs[j & 1][0] = fminf(fmaf(__builtin_amdgcn_rcpf(1.f + ce[0]), cap_2l, mc), sv[2 * j] + 1e30f);
+    xs[j & 1][1] = fminf(fmaf(__builtin_amdgcn_rcpf(1.f + ce[1]), cap_2l, mc), sv[2 * j + 1] + 1e30f);
+  };
   auto stage1 = [&](const f32x16& sv, int j) {
-    xs[j & 1][0] = fmaf(sv[2 * j], c, -mc);
-    xs[j & 1][1] = fmaf(sv[2 * j + 1], c, -mc);
+    if constexpr (CAP) {
+      cap_e(sv, j), cap_x(sv, j);
+    } else {
+      xs[j & 1][0] = fmaf(sv[2 * j], c, -mc);
+      xs[j & 1][1] = fmaf(sv[2 * j + 1], c, -mc);
+    }
   };
   auto stage2 = [&](int j) {
     pv[j & 1][0] = __builtin_amdgcn_exp2f(xs[j & 1][0]);
@@ -663,7 +695,19 @@ __device__ __forceinline__ void fwd_w32_body(const FwdM& p, const MaskArgs ma) {
   // Pairs 0..3 hold the tile's first 16 keys (the first contraction step of P*V), pairs 4..7 the
   // last 16.  Four pairs are spread over the eight matrix ops of a phase:
   //   slot 2q: exp2 of pair q, scaling of pair q+1     slot 2q+1: sum and packing of pair q
+  // with a soft cap in sixteen steps: exp2 of pair q, cap_e of q+1, sum and packing of q, cap_x of q+1
+  constexpr int STEPS = CAP ? 16 : 8;
   auto softmax_slot = [&](const f32x16& sv, int base, int slot, uint32_t (&pk)[8], float& ps) {
+    if constexpr (CAP) {
+      const int q = slot >> 2, r = slot & 3;
+      if (r == 0) stage2(base + q);
+      else if (r == 2) stage3(base + q, pk, ps);
+      else if (q + 1 < 4) {
+        if (r == 1) cap_e(sv, base + q + 1);
+        else cap_x(sv, base + q + 1);
+      }
+      return;
+    }
     const int q = slot >> 1;
     if ((slot & 1) == 0) {
       stage2(base + q);
@@ -749,7 +793,7 @@ __device__ __forceinline__ void fwd_w32_body(const FwdM& p, const MaskArgs ma) {
       else ring[(ks + AHEAD) & 7] = read_v(ks + AHEAD - KS);
       snext = Mma<T>::run(ring[ks & 7], qf[ks], ks == 0 ? zero16 : snext);
 #pragma unroll
-      for (int hs = ks * 8 / KS; hs < (ks + 1) * 8 / KS; ++hs) softmax_slot(scur, 4, hs, pk, ps);
+      for (int hs = ks * STEPS / KS; hs < (ks + 1) * STEPS / KS; ++hs) softmax_slot(scur, 4, hs, pk, ps);
       __builtin_amdgcn_sched_barrier(0);
     }
     // ---- check ---------------------------------------------------------------------------------
@@ -786,7 +830,7 @@ __device__ __forceinline__ void fwd_w32_body(const FwdM& p, const MaskArgs ma) {
     // so the wait for the last op of phase A is spent on the matrix pipe.  The barrier sits two
     // slots before the end: by then every wavefront has stored its share of tiles t+2 (K) and
     // t+1 (V) and has issued its last read of V(t); behind it the first K fragments of the next
-    // phase A are requested.  The eight half-steps of the softmax are spread over the slots, the
+    // phase A are requested.  The steps of the softmax are spread over the slots, the
     // last one trailing the loop.
 #pragma unroll
     for (int i = 0; i < NPV; ++i) {  // i = DB * (16-key step) + d block
@@ -814,13 +858,13 @@ __device__ __forceinline__ void fwd_w32_body(const FwdM& p, const MaskArgs ma) {
         if (__builtin_expect(edge(t + 1), 0)) mask_tile(snext, tile_of(t + 1) * BN);  // rare
         stage1(snext, 0);
       }
-      // half-steps 0 .. 6 spread over the slots (the last one trails the loop)
+      // all steps but the last spread over the slots (that one trails the loop)
 #pragma unroll
-      for (int hs = (i == 0 ? 0 : max((i * 8) / NPV - 1, 0)); hs < max(((i + 1) * 8) / NPV - 1, 0); ++hs)
+      for (int hs = (i == 0 ? 0 : max((i * STEPS) / NPV - 1, 0)); hs < max(((i + 1) * STEPS) / NPV - 1, 0); ++hs)
         softmax_slot(snext, 0, hs, pkn, psn);
       __builtin_amdgcn_sched_barrier(0);
     }
-    softmax_slot(snext, 0, 7, pkn, psn);
+    softmax_slot(snext, 0, STEPS - 1, pkn, psn);
   };
   // a wavefront whose rows lie above the causal diagonal of the remaining tiles only feeds LDS
   auto idle_step = [&](int t) {
@@ -973,7 +1017,7 @@ int launch_one(const FwdM& g, dim3 grid, hipStream_t s) {
   int bytes = 0;
   if constexpr (D > 128 || MASK == 2 || MASK == 3) {
     // (four buffers per operand, 4 KB of bias tile per wavefront, and the tile list of a call with a skip table)
-    constexpr int kBase = 2 * 4 * BN * D * 2 + (MASK >= 2 ? WAVES * 4096 : 0) + (MASK == 3 ? WAVES * 1024 : 0);
+    constexpr int kBase = 2 * 4 * BN * D * 2 + (MASK == 2 || MASK == 3 ? WAVES * 4096 : 0) + (MASK == 3 ? WAVES * 1024 : 0);
     constexpr int kBytes = kBase + (MASK == 2 ? 2048 + 16 : 0);
     static LdsOnce once;
     const hipError_t attr = reserve_lds(once, (const void*)fwd_w32_kernel<T, D, WAVES, MASK, PATTERN>, kBytes);
@@ -988,6 +1032,7 @@ int launch_one(const FwdM& g, dim3 grid, hipStream_t s) {
 }
 template <typename T, int D, int WAVES>
 int launch_mask(const FwdM& g, int mask, dim3 grid, hipStream_t s) {
+  if (mask == 5) return launch_one<T, D, WAVES, 5>(g, grid, s);
   if (mask == 4) return launch_one<T, D, WAVES, 4>(g, grid, s);
   if (mask == 3) return launch_one<T, D, WAVES, 3>(g, grid, s);
   if (mask == 2) {
@@ -1077,7 +1122,7 @@ int launch_fwd_mfma_w32(const FwdM& g0, int dtype, int head_dim, int waves, hipS
     return MI355_SDPA_ERR_UNSUPPORTED;
   }
   const dim3 grid((unsigned)blocks);
-  // kernel variant: 3 with a keep-mask (and a bias or none), 2 with a bias, 1 with key counts or rows narrower than the kernel's head dim
+  // kernel variant: 5 with a soft cap alone, 4 with the other score functors, 3 with a keep-mask (and a bias or none), 2 with a bias, 1 with key counts or rows narrower than the kernel's head dim
   if (g.keep_scale != 0.f && (!g.keep || g.live_tiles)) {
     set_error("SDPA: dropout in fwd_w32_kernel needs a keep-mask and no tile table");
     return MI355_SDPA_ERR_UNSUPPORTED;
@@ -1086,7 +1131,8 @@ int launch_fwd_mfma_w32(const FwdM& g0, int dtype, int head_dim, int waves, hipS
     set_error("SDPA: score functors in fwd_w32_kernel go with no bias and no dropout");
     return MI355_SDPA_ERR_UNSUPPORTED;
   }
-  const int mask = g.sm.any ? 4 : g.keep_scale != 0.f ? 3 : g.bias_kind != 0 ? 2 : (g.kv_lens != nullptr || g.d_real != head_dim || g.dv_real != head_dim || g.window > 0 || g.sink_logit || g.split_tiles) ? 1 : 0;
+  const bool cap_only = g.sm.softcap > 0.f && !g.sm.alibi && !g.sm.key_bias && !g.sm.key_weight && !g.sm.doc_q;
+  const int mask = cap_only ? 5 : g.sm.any ? 4 : g.keep_scale != 0.f ? 3 : g.bias_kind != 0 ? 2 : (g.kv_lens != nullptr || g.d_real != head_dim || g.dv_real != head_dim || g.window > 0 || g.sink_logit || g.split_tiles) ? 1 : 0;
   int rc = dtype == MI355_SDPA_BF16 ? launch_dims<bf16_t>(g, head_dim, waves, mask, grid, s)
                                           : launch_dims<f16_t>(g, head_dim, waves, mask, grid, s);
   if (rc != MI355_SDPA_OK) return rc;
