@@ -73,3 +73,18 @@ def test_against_float64(amd, gpu_device, case, dtype):
     assert ((lse.double() - want_lse)[ok].abs() <= score_err + 2.0**-20 * want_lse[ok].abs() + 2.0**-20).all()
     eps = 2.0**-9 if dtype is torch.bfloat16 else 2.0**-12
     assert float((out.double() - want)[ok].abs().max()) <= (2.5 * eps + 2 * score_err) * float(V.abs().max())
+
+
+def test_lse_of_a_large_cap_keeps_the_reference(amd, gpu_device):
+    # A row's reference must not be rounded to the precision of the cap (cap log2(e) = 1443: 2^-14 of rounding step, 2.4e-5
+    # of the lse by root mean square, from row to row).  What the scores carry themselves is at most 2^-22 cap each:
+    # a common part (the reciprocal's rounding has a side it prefers), and one that averages out over the
+    # keys, S / e of which carry the weight.
+    g = torch.Generator(device=gpu_device).manual_seed(11)
+    S, cap = 4096, 1000.0
+    q, k, v = (torch.randn(1, 4, n, 128, generator=g, device=gpu_device).to(torch.bfloat16) for n in (300, S, S))
+    lse = amd.sdpa_forward(q, k, v, softcap=cap)[1]
+    s = cap * torch.tanh(q.double() @ k.double().transpose(-1, -2).contiguous() / math.sqrt(128) / cap)
+    off = lse.double() - torch.logsumexp(s, -1)
+    assert abs(float(off.mean())) <= 2.0**-22 * cap
+    assert float(off.std()) <= 2.0**-22 * cap / math.sqrt(S / math.e) + 2.0**-22 * float(lse.abs().max())

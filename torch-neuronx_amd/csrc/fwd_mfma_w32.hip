@@ -639,20 +639,22 @@ __device__ __forceinline__ void fwd_w32_body(const FwdM& p, const MaskArgs ma) {
   // reference, and lse = reference * scale + ln(sum).
   constexpr float kTrig = 8192.f;  // 16 probabilities of at most 2^kLazy stay below this
   // Soft cap (MASK = 5): with e = 2^(2 log2(e) scale s / cap) and r = 1 / (1 + e) the capped score is
-  // cap (1 - 2 r), so its exponent in the log2 domain, reference subtracted, is one multiply-add on r.  A
+  // cap (1 - 2 r): 1 - 2 r is exact but for r, and its exponent in the log2 domain, reference subtracted, one
+  // multiply-add more.  (Both in one, r times -2 cap plus the rest of the reference, rounds that rest to the precision of
+  // the cap, for a whole row: lse 1.2e-7 -> 2.9e-7 off at a cap of 50.)  A
   // masked score (-inf) would come out as -cap: the minimum with s + 1e30 keeps it (and a NaN).
   auto scalar = [](float x) { return __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, x))); };
-  const float cap_k = CAP ? scalar(2.f * kLog2eF * p.scale / p.sm.softcap) : 0.f, cap_2l = CAP ? scalar(-2.f * kLog2eF * p.sm.softcap) : 0.f;
+  const float cap_k = CAP ? scalar(2.f * kLog2eF * p.scale / p.sm.softcap) : 0.f, cap_l = CAP ? scalar(kLog2eF * p.sm.softcap) : 0.f;
   const float cap_raw = CAP ? scalar(p.sm.softcap / p.scale) : 0.f;  // the cap in units of the raw scores
   auto cap_r = [&](float s) { return __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(s * cap_k)); };
   auto raise_reference = [&](float t0) {
     float tm = fmaxf(t0, __shfl_xor(t0, 32, 64));
-    if constexpr (CAP) tm = fminf(fmaf(cap_r(tm), -2.f * cap_raw, cap_raw), tm + 1e30f);  // (the cap is monotonic)
+    if constexpr (CAP) tm = fminf(fmaf(cap_r(tm), -2.f, 1.f) * cap_raw, tm + 1e30f);  // (the cap is monotonic)
     const bool up = (tm - m_run) * c > kLazy;  // false for NaN (-inf minus -inf)
     m_new = up ? tm : m_run;
     const float m_use = (m_new == -INFINITY) ? 0.f : m_new;
     alpha = __builtin_amdgcn_exp2f((m_run - m_use) * c);
-    mc = CAP ? fmaf(-0.5f, cap_2l, -m_use * c) : m_use * c;  // (soft cap: what is left of the cap's exponent above the reference)
+    mc = m_use * c;
     need_rescale = __builtin_amdgcn_ballot_w64(up) != 0;
   };
 
@@ -666,8 +668,8 @@ __device__ __forceinline__ void fwd_w32_body(const FwdM& p, const MaskArgs ma) {
     ce[1] = __builtin_amdgcn_exp2f(sv[2 * j + 1] * cap_k);
   };
   auto cap_x = [&](const f32x16& sv, int j) {
-    xs[j & 1][0] = fminf(fmaf(__builtin_amdgcn_rcpf(1.f + ce[0]), cap_2l, mc), sv[2 * j] + 1e30f);
-    xs[j & 1][1] = fminf(fmaf(__builtin_amdgcn_rcpf(1.f + ce[1]), cap_2l, mc), sv[2 * j + 1] + 1e30f);
+    xs[j & 1][0] = fminf(fmaf(fmaf(__builtin_amdgcn_rcpf(1.f + ce[0]), -2.f, 1.f), cap_l, -mc), sv[2 * j] + 1e30f);
+    xs[j & 1][1] = fminf(fmaf(fmaf(__builtin_amdgcn_rcpf(1.f + ce[1]), -2.f, 1.f), cap_l, -mc), sv[2 * j + 1] + 1e30f);
   };
   auto stage1 = [&](const f32x16& sv, int j) {
     if constexpr (CAP) {
