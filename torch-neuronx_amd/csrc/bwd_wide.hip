@@ -18,21 +18,15 @@
 // Tiles sit in LDS row-major, unpadded and XOR swizzled; transposed operands come out of the
 // transposing LDS read.  Math follows torch_neuronx/_sdpa_math.py:98-176: float32 accumulation, rows with
 // lse = -inf give zero gradients, scale multiplies dQ and dK once at the end.
-#include "bwd_mfma.h"
+//
+// At the full width the dK/dV of calls without a bias or dropout come from bwd_wide_pair.hip.
+#include "bwd_wide.h"
 
 namespace mi355 {
 namespace {
 
-constexpr int DW = 256;           // the width the kernels are built for
 constexpr int KS = DW / 16;       // contraction steps over the head dim
 constexpr int DB = DW / 32;       // 32-row blocks of a transposed product
-constexpr int BT = 32;            // rows of a staged tile
-
-typedef short s16x4 __attribute__((ext_vector_type(4)));
-__device__ __forceinline__ u32x2 tr_read(const uint16_t* ptr) {
-  const s16x4 v = __builtin_amdgcn_ds_read_tr16_b64_v4i16((s16x4 __attribute__((address_space(3)))*)(ptr));
-  return __builtin_bit_cast(u32x2, v);
-}
 
 // Both kernels stage their 32-row tiles from global memory straight into LDS (buffer loads with the
 // LDS bit, 16 bytes per lane, 1 KB of contiguous LDS per wavefront and instruction), one tile ahead,
@@ -42,7 +36,6 @@ __device__ __forceinline__ u32x2 tr_read(const uint16_t* ptr) {
 // of four consecutive rows overlap in their banks).  16 loads cover a tile; a chunk past a narrow
 // row's end asks for an offset beyond the buffer and gets zeros, and so do rows past the buffer's end.
 constexpr int TILE_LOADS = BT * (DW / 8) / 64;
-constexpr int TILE_ELEMS = BT * DW;
 constexpr int WIDE_DKDV_LDS = 2 * 2 * TILE_ELEMS * 2 + 2 * 2 * BT * 4;
 constexpr int WIDE_DQ_LDS = 2 * 2 * TILE_ELEMS * 2;
 constexpr int WIDE_LIST_LDS = 2048 + 16;   // masked dQ instances: the list of live key tiles (1024 entries and the count)
@@ -78,34 +71,6 @@ struct TrOffSwz {
 // element offset of the row read of contraction step j (this lane: row col, 8 elements at 16 j + 8 half)
 __device__ __forceinline__ int wide_row_off(int j, int col, int half, int swz_col) {
   return col * DW + (((2 * (j % 8) + half) ^ swz_col) << 3) + (j / 8) * WIN;
-}
-
-// raw buffer resource, in scalar registers
-__device__ __forceinline__ u32x4 wide_descriptor(const void* base, int64_t bytes) {
-  const uint64_t a = (uint64_t)base;
-  return u32x4{(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)a),
-               (uint32_t)__builtin_amdgcn_readfirstlane((int)((uint32_t)(a >> 32) & 0xffffu)),
-               (uint32_t)__builtin_amdgcn_readfirstlane((int)bytes), 0x00020000u};
-}
-// (m0 holds the LDS address of such a load, one wait state after it is written)
-__device__ __forceinline__ void wide_tile_load(const u32x4& rsrc, uint32_t voffset, uint32_t lds_addr) {
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds"
-               :: "s"(__builtin_amdgcn_readfirstlane((int)lds_addr)), "v"(voffset), "s"(rsrc) : "memory", "m0");
-}
-// byte offset of this lane's chunk of load `ld` inside a tile whose first row is the buffer's base
-__device__ __forceinline__ uint32_t wide_chunk_off(int ld, int lane, int row_stride, int width) {
-  const int pos = ld * 64 + lane, r = pos / (DW / 8), ch = (pos % (DW / 8)) ^ tile_swz<DW>(r);
-  return ch * 8 < width ? (uint32_t)((r * row_stride + ch * 8) * 2) : 0xfffffff0u;
-}
-
-// compile-time loop: f(std::integral_constant<int, 0>{}) ... f(std::integral_constant<int, N - 1>{})
-template <typename F, int... I>
-__device__ __forceinline__ void static_for_impl(F&& f, std::integer_sequence<int, I...>) {
-  (f(std::integral_constant<int, I>{}), ...);
-}
-template <int N, typename F>
-__device__ __forceinline__ void static_for(F&& f) {
-  static_for_impl(f, std::make_integer_sequence<int, N>{});
 }
 
 // The kernels are instantiated for the widths they serve, ER for Q / K and DVR for V / dO / O
@@ -1029,7 +994,8 @@ int launch_t(const BwdM& g, hipStream_t s) {
   hipLaunchKernelGGL((bwd_wide_dq_kernel<T, ER, DVR, MODE>), dim3((unsigned)q_blocks), dim3(256), kDqLds, s, g);
   int rc = check_launch("bwd_wide_dq_kernel");
   if (rc) return rc;
-  rc = launch_dkdv<T, ER, DVR, MODE, MODE == 1 && !(NO_TABLES && ER + DVR > 320)>(g, k_blocks, s);
+  if constexpr (ER + DVR > 320 && (MODE == 0 || MODE == 2)) rc = launch_bwd_wide_pair(g, std::is_same<T, bf16_t>::value ? MI355_SDPA_BF16 : MI355_SDPA_F16, s);
+  else rc = launch_dkdv<T, ER, DVR, MODE, MODE == 1 && !(NO_TABLES && ER + DVR > 320)>(g, k_blocks, s);
   if (rc || g.parts == 1) return rc;
   return launch_bwd_dkdv_merge(g, std::is_same<T, bf16_t>::value ? MI355_SDPA_BF16 : MI355_SDPA_F16, s);
 }
@@ -1047,9 +1013,10 @@ int launch_w(const BwdM& g, hipStream_t s) {
     return drop ? launch_t<T, 192, 128, 3>(g, s)
            : func ? launch_t<T, 192, 128, 2>(g, s) : masked ? launch_t<T, 192, 128, 1>(g, s) : launch_t<T, 192, 128, 0>(g, s);
   if (drop) return launch_t<T, 256, 256, 3>(g, s);
-  if (func) return launch_t<T, 256, 256, 2>(g, s);
-  if (masked && g.parts > 1) return launch_t<T, 256, 256, 1, true>(g, s);  // (bwd_wide_parts: no skip table then)
-  return masked ? launch_t<T, 256, 256, 1>(g, s) : launch_t<T, 256, 256, 0>(g, s);
+  // (key counts alone take the functor instance: its dQ kernel tests only the tiles at an edge, and its dK/dV is the pair kernel's)
+  if (!g.bias_kind) return func || g.kv_lens ? launch_t<T, 256, 256, 2>(g, s) : launch_t<T, 256, 256, 0>(g, s);
+  if (g.parts > 1) return launch_t<T, 256, 256, 1, true>(g, s);  // (bwd_wide_parts: no skip table then)
+  return launch_t<T, 256, 256, 1>(g, s);
 }
 
 }  // namespace

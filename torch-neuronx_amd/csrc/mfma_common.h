@@ -111,6 +111,7 @@ struct MmaV<f16_t> {
 // the matrix ops that write them are inline assembly, whose hazard the compiler does not know, so
 // nothing else would keep it from placing a read of an accumulator between the last op and the idle
 // cycles.
+__device__ __forceinline__ void mfma_to_valu_gap(f32x16& a) { asm volatile("s_nop 15\n\ts_nop 7" : "+v"(a) :: "memory"); }
 __device__ __forceinline__ void mfma_to_valu_gap(f32x16& a, f32x16& b) {
   asm volatile("s_nop 15\n\ts_nop 7" : "+v"(a), "+v"(b) :: "memory");
 }
