@@ -126,9 +126,14 @@ constexpr WideOp dkdv_op(int k) {  // S steps and dP steps (in turns where both 
 // MODE 2 (FUNC): per-batch key counts, a sliding window with sink keys (the tiles it drops whole are not
 // walked) and the score functors and document ids of score_mod.h, each score through score_mod_at where
 // its probability is formed; the derivative of the functors multiplies the gradient of the scores.
+// MODE 4 (CAP, dQ kernel only): MODE 2 with a soft cap and no other functor.  What bounds this kernel is one wavefront's
+// chain with nobody else on its SIMD; the block of MODE 2 between S and dP (nine instructions per score, two of
+// them quarter-rate) ran with the matrix pipe idle.  Here the cap is part of the probability and rides on the
+// dP products.  dQ, B=2, 16 heads, S=4096, cap 50, MODE 2 / MODE 4: D=256 with a window of 1024 416 / 319 us (forward and backward
+// 924 / 831), causal 715 / 528, 192/128 causal 592 / 397.
 template <typename T, int ER, int DVR, int MODE>
 __global__ __launch_bounds__(256, 1) void bwd_wide_dq_kernel(BwdM p) {
-  constexpr bool MASKED = MODE == 1 || MODE == 3, FUNC = MODE == 2, DROP = MODE == 3;
+  constexpr bool MASKED = MODE == 1 || MODE == 3, CAP = MODE == 4, FUNC = MODE == 2 || CAP, DROP = MODE == 3;
   constexpr int KSE = ER / 16, KSV = DVR / 16, DBE = ER / 32;
   extern __shared__ __attribute__((aligned(16))) uint16_t wide_lds[];
   uint16_t* const k_buf = wide_lds;                    // [2][TILE_ELEMS]
@@ -137,7 +142,9 @@ __global__ __launch_bounds__(256, 1) void bwd_wide_dq_kernel(BwdM p) {
   const int n_qt = (p.L + 127) / 128;
   const int qt = n_qt - 1 - blockIdx.x / (p.B * p.Hq);  // heavy query tiles first
   const int bh = blockIdx.x % (p.B * p.Hq), b = bh / p.Hq, h = bh % p.Hq, hk = h / (p.Hq / p.Hkv);
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, col = lane & 31, half = lane >> 5;
+  const int tid = threadIdx.x, lane = tid & 63, col = lane & 31, half = lane >> 5;
+  // (CAP: in a scalar register, so that the test for an edge is a branch)
+  const int wave = CAP ? __builtin_amdgcn_readfirstlane(tid >> 6) : tid >> 6;
   const int q0 = qt * 128, qw0 = q0 + wave * 32, qrow = qw0 + col, qc = min(qrow, p.L - 1);
   const int er = p.d_real, dvr = p.dv_real;
 
@@ -241,10 +248,12 @@ __global__ __launch_bounds__(256, 1) void bwd_wide_dq_kernel(BwdM p) {
   // (FUNC) the window of this lane's row, and what the derivative of the functors needs
   const int lo_w = (FUNC && p.window > 0) ? qrow - p.window + 1 : (int)0x80000000;
   const int n_sink = FUNC ? p.sink_keys : 0;
-  const float inv_scale = FUNC ? 1.f / p.scale : 0.f;
-  const float icap = (FUNC && p.sm.softcap > 0.f) ? p.scale / p.sm.softcap : 0.f;
-  const float* const f_kw = (FUNC && p.sm.key_weight) ? p.sm.key_weight + (int64_t)h * p.S : nullptr;
-  const bool need_dfac = FUNC && (p.sm.softcap > 0.f || p.sm.key_weight != nullptr);
+  const float inv_scale = MODE == 2 ? 1.f / p.scale : 0.f;
+  const float icap = (MODE == 2 && p.sm.softcap > 0.f) ? p.scale / p.sm.softcap : 0.f;
+  const float* const f_kw = (MODE == 2 && p.sm.key_weight) ? p.sm.key_weight + (int64_t)h * p.S : nullptr;
+  const bool need_dfac = MODE == 2 && (p.sm.softcap > 0.f || p.sm.key_weight != nullptr);
+  // (CAP) with r = 1 / (1 + 2^(cap_k s)) the capped score is cap (1 - 2 r), in the log2 domain cap_l (1 - 2 r)
+  const float cap_k = CAP ? 2.f * c / p.sm.softcap : 0.f, cap_l = CAP ? p.sm.softcap * kLog2eF : 0.f;
 
   // the buffers end with the last key row: rows of a ragged last tile beyond it read as zeros
   const u32x4 k_rsrc = wide_descriptor(kp, S > 0 ? ((int64_t)(S - 1) * p.k_sl + er) * 2 : 0);
@@ -338,6 +347,7 @@ __global__ __launch_bounds__(256, 1) void bwd_wide_dq_kernel(BwdM p) {
     // (FUNC: GENERAL is the tile as the functors, a window's edge or the diagonal need it; a tile inside
     // the window of every row of a call without score functors is the plain tile, at the plain speed: tests
     // per score, even uniform ones, cost this kernel a third of its time)
+    bool edge = false;  // (CAP) the tile crosses the diagonal, the end of the keys or the edge of a window
     auto tile = [&](auto general_c) {
       constexpr bool GENERAL = decltype(general_c)::value;
       const uint16_t* k_t = k_buf + (t & 1) * TILE_ELEMS;
@@ -367,14 +377,14 @@ __global__ __launch_bounds__(256, 1) void bwd_wide_dq_kernel(BwdM p) {
       // is formed under the dQ ops of the first 16.
       float bl[16], pr[16];
       uint32_t pS[8];
-      if constexpr (FUNC && GENERAL) {
+      if constexpr (MODE == 2 && GENERAL) {
 #pragma unroll
         for (int r = 0; r < 16; ++r) bl[r] = 1.f;
       }
       auto prob = [&](int r) {
         const int kv = ta * BT + (r >> 2) * 8 + half * 4 + (r & 3);
         float x;
-        if constexpr (FUNC && GENERAL) {
+        if constexpr (MODE == 2 && GENERAL) {
           // (the scores went through the functors in a block of their own, see below; only dS is formed
           // from this probability, so the functors' derivative rides on it: 1 - tanh^2 of the soft cap,
           // recovered from the capped score, times the key's weight)
@@ -392,6 +402,23 @@ __global__ __launch_bounds__(256, 1) void bwd_wide_dq_kernel(BwdM p) {
         else x = fmaf(sacc[r], c, -lse2);
         pr[r] = __builtin_amdgcn_exp2f(kv > lim ? -INFINITY : x);  // (masked before the exponential: no branch)
       };
+      // (CAP) a probability in three stages, each of them one dP slot behind the one before: a chain of three quarter-rate
+      // instructions has nobody else on the SIMD to hide behind, so a slot works on three scores at once
+      auto cap_stage = [&](int stage, int group) {
+        constexpr int PER = 16 / KSV;  // scores per slot
+        if (group < 0 || group >= KSV) return;
+#pragma unroll
+        for (int r = group * PER; r < (group + 1) * PER; ++r) {
+          if (stage == 0) {
+            sacc[r] = __builtin_amdgcn_exp2f(sacc[r] * cap_k);
+          } else if (stage == 1) {
+            sacc[r] = __builtin_amdgcn_rcpf(1.f + sacc[r]);
+          } else {
+            const float th = fmaf(sacc[r], -2.f, 1.f);
+            pr[r] = __builtin_amdgcn_exp2f(fmaf(th, cap_l, -lse2)) * fmaf(-th, th, 1.f);
+          }
+        }
+      };
       auto form_ds = [&](int r) {  // elements r, r + 1
         if constexpr (DROP) {
           const float k0 = (float)((kraw[r >> 2] >> (8 * (r & 3))) & 0xffu), k1 = (float)((kraw[r >> 2] >> (8 * (r & 3) + 8)) & 0xffu);
@@ -407,7 +434,7 @@ __global__ __launch_bounds__(256, 1) void bwd_wide_dq_kernel(BwdM p) {
         if constexpr (op.kind) {
           dpacc = Mma<T>::run(ring[k & 7], dof[op.j], dpacc);
           if constexpr (op.j == 0 && MASKED) bias_log2(bl);
-          if constexpr (op.j == 0 && FUNC && GENERAL) {
+          if constexpr (op.j == 0 && MODE == 2 && GENERAL) {
             // every score through the functors, in one block behind one test: s = mod(scale * s) / scale,
             // so that the code around it is the common one (a call with a window alone skips the block)
             // (one loop per functor behind one test each: tested per score, even a uniform test costs this
@@ -448,13 +475,29 @@ __global__ __launch_bounds__(256, 1) void bwd_wide_dq_kernel(BwdM p) {
               for (int r = 0; r < 16; ++r) sacc[r] *= inv_scale;
             }
           }
+          if constexpr (CAP) {
+            cap_stage(2, op.j - 2), cap_stage(1, op.j - 1), cap_stage(0, op.j);
+          } else {
 #pragma unroll
-          for (int r = (op.j * 16) / KSV; r < ((op.j + 1) * 16) / KSV; ++r) prob(r);
+            for (int r = (op.j * 16) / KSV; r < ((op.j + 1) * 16) / KSV; ++r) prob(r);
+          }
         } else {
           sacc = Mma<T>::run(ring[k & 7], qf[op.j], sacc);
         }
         __builtin_amdgcn_sched_barrier(0);
       });
+      if constexpr (CAP) {
+        cap_stage(2, KSV - 2), cap_stage(1, KSV - 1), cap_stage(2, KSV - 1);
+        // (one test for all of the scores, here where their registers are all that is alive of them; as a second copy of the
+        // tile it costs a second set of accumulators, 128 moves a tile)
+        if (edge) {
+#pragma unroll
+          for (int r = 0; r < 16; ++r) {
+            const int kv = ta * BT + (r >> 2) * 8 + half * 4 + (r & 3);
+            pr[r] = ((kv > lim) | ((kv < lo_w) & (kv >= n_sink))) ? 0.f : pr[r];
+          }
+        }
+      }
 #pragma unroll
       for (int r = 0; r < 8; r += 2) form_ds(r);
       __builtin_amdgcn_sched_barrier(0);
@@ -484,7 +527,9 @@ __global__ __launch_bounds__(256, 1) void bwd_wide_dq_kernel(BwdM p) {
         // does the tile cross the diagonal, the end of the keys or the edge of a window of this wavefront's rows?
         const int k_lo = tile_of(t) * BT, k_hi = k_lo + BT - 1;
         const bool edge_t = k_hi >= S || (p.causal && k_hi > qw0) || (p.window > 0 && k_lo < qw0 + 31 - p.window + 1 && k_hi >= p.sink_keys);
-        if (edge_t || need_dfac || p.sm.any) tile(std::true_type{});
+        edge = edge_t;
+        if constexpr (CAP) tile(std::false_type{});
+        else if (edge_t || need_dfac || p.sm.any) tile(std::true_type{});
         else tile(std::false_type{});
       } else {
         tile(std::true_type{});
@@ -994,8 +1039,8 @@ int launch_t(const BwdM& g, hipStream_t s) {
   hipLaunchKernelGGL((bwd_wide_dq_kernel<T, ER, DVR, MODE>), dim3((unsigned)q_blocks), dim3(256), kDqLds, s, g);
   int rc = check_launch("bwd_wide_dq_kernel");
   if (rc) return rc;
-  if constexpr (ER + DVR > 320 && (MODE == 0 || MODE == 2)) rc = launch_bwd_wide_pair(g, std::is_same<T, bf16_t>::value ? MI355_SDPA_BF16 : MI355_SDPA_F16, s);
-  else rc = launch_dkdv<T, ER, DVR, MODE, MODE == 1 && !(NO_TABLES && ER + DVR > 320)>(g, k_blocks, s);
+  if constexpr (ER + DVR > 320 && (MODE == 0 || MODE == 2 || MODE == 4)) rc = launch_bwd_wide_pair(g, std::is_same<T, bf16_t>::value ? MI355_SDPA_BF16 : MI355_SDPA_F16, s);
+  else rc = launch_dkdv<T, ER, DVR, MODE == 4 ? 2 : MODE, MODE == 1 && !(NO_TABLES && ER + DVR > 320)>(g, k_blocks, s);
   if (rc || g.parts == 1) return rc;
   return launch_bwd_dkdv_merge(g, std::is_same<T, bf16_t>::value ? MI355_SDPA_BF16 : MI355_SDPA_F16, s);
 }
@@ -1004,6 +1049,7 @@ template <typename T>
 int launch_w(const BwdM& g, hipStream_t s) {
   const bool func = g.window > 0 || g.sm.any;  // (never together with a bias: refused before)
   const bool masked = g.bias_kind || g.kv_lens;  // (a bias gradient comes with a bias)
+  const bool cap_only = g.sm.softcap > 0.f && !g.sm.alibi && !g.sm.key_bias && !g.sm.key_weight && !g.sm.doc_q;
   const bool drop = g.keep_scale != 0.f;          // (never together with a functor or a skip table: refused before)
   if (drop && (!g.keep || func || g.live_t || g.live_tiles)) {
     set_error("SDPA: dropout in the wide backward kernels needs a keep-mask, no functor and no tile table");
@@ -1011,8 +1057,9 @@ int launch_w(const BwdM& g, hipStream_t s) {
   }
   if (g.d_real <= 192 && g.dv_real <= 128)
     return drop ? launch_t<T, 192, 128, 3>(g, s)
-           : func ? launch_t<T, 192, 128, 2>(g, s) : masked ? launch_t<T, 192, 128, 1>(g, s) : launch_t<T, 192, 128, 0>(g, s);
+           : cap_only ? launch_t<T, 192, 128, 4>(g, s) : func ? launch_t<T, 192, 128, 2>(g, s) : masked ? launch_t<T, 192, 128, 1>(g, s) : launch_t<T, 192, 128, 0>(g, s);
   if (drop) return launch_t<T, 256, 256, 3>(g, s);
+  if (cap_only) return launch_t<T, 256, 256, 4>(g, s);
   // (key counts alone take the functor instance: its dQ kernel tests only the tiles at an edge, and its dK/dV is the pair kernel's)
   if (!g.bias_kind) return func || g.kv_lens ? launch_t<T, 256, 256, 2>(g, s) : launch_t<T, 256, 256, 0>(g, s);
   if (g.parts > 1) return launch_t<T, 256, 256, 1, true>(g, s);  // (bwd_wide_parts: no skip table then)
