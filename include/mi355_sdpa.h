@@ -254,7 +254,8 @@ size_t mi355_sdpa_fwd_workspace_bytes(const mi355_sdpa_fwd_params* p);
 int mi355_sdpa_bwd(const mi355_sdpa_bwd_params* p, void* stream);
 /* Bytes of workspace this backward call needs: the row terms (rowsum(dO * O) and the log-sum-exp in
  * the log2 domain), and for a call with few key blocks the float32 partial dK / dV rows of the
- * workgroups that share a key block.  Ask per call: the size depends on every shape. */
+ * workgroups that share a key block, and for dropout at head dims up to 64 the keep-mask as bits (whole
+ * 128-key blocks per query row).  Ask per call: the size depends on every shape. */
 size_t mi355_sdpa_bwd_workspace_bytes(const mi355_sdpa_bwd_params* p);
 
 /* Decode-step attention over an fp8 e4m3 K/V cache with per-sequence lengths.
