@@ -80,3 +80,28 @@ CASES = [
 def test_against_float64(amd, gpu_device, case, dtype):
     B, Hq, Hkv, L, S, D, causal, lens, p = case
     _check(amd, gpu_device, B, Hq, Hkv, L, S, D, causal, dtype, lens, p)
+
+
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("which", ["q", "do"])
+def test_a_batch_beyond_32_bit_offsets(amd, gpu_device, which, causal):
+    """Q or dO of one batch spans 2 GiB (two heads that far apart in one allocation), K and V do not: not
+    these kernels' case, the 64-bit ones have it.  L: 256 workgroups of 256 rows."""
+    B, H, L, S, D = 1, 2, 32768, 96, 64
+    g = torch.Generator(device=gpu_device).manual_seed(3)
+    q, k, v, do = (torch.randn(B, H, n, D, generator=g, device=gpu_device).to(torch.bfloat16) for n in (L, S, S, L))
+    far = torch.empty((1 << 30) + L * D, dtype=torch.bfloat16, device=gpu_device).as_strided((B, H, L, D), ((1 << 30) + L * D, 1 << 30, D, 1))
+    far.copy_(q if which == "q" else do)
+    q, do = (far, do) if which == "q" else (q, far)
+    out, lse = amd.sdpa_forward(q, k, v, is_causal=causal)
+    dq, dk, dv, _ = amd.sdpa_backward(do, q, k, v, out, lse, is_causal=causal)
+    for h in range(H):
+        Q, K, V, DO = (t[0, h].double() for t in (q, k, v, do))
+        s = Q @ K.t() / math.sqrt(D)
+        if causal:
+            s = s.masked_fill(~torch.ones(L, S, dtype=torch.bool, device=gpu_device).tril(), -math.inf)
+        P = torch.softmax(s, -1)
+        dS = P * (DO @ V.t() - (DO * (P @ V)).sum(-1, keepdim=True)) / math.sqrt(D)
+        for name, a, r in (("dq", dq, dS @ K), ("dk", dk, dS.t() @ Q), ("dv", dv, P.t() @ DO)):
+            off = float((a[0, h].double() - r).norm() / r.norm())
+            assert off <= 8e-3, (name, h, off)

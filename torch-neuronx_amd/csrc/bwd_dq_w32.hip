@@ -1,5 +1,5 @@
 // Flash-attention backward, dQ, for gfx950, head dim 64 or 128, bf16/f16 (at 64 the calls with a bias, a window, a
-// functor or split keys: bwd_d64.hip has the others).
+// functor or split keys, and those whose Q or dO of one batch is beyond 32-bit offsets: bwd_d64.hip has the others).
 //
 // One workgroup = 8 wavefronts of 32 query rows each (256 rows of one (batch, query head)), one
 // workgroup per compute unit, two wavefronts per SIMD with 256 registers each; it walks the keys
@@ -825,7 +825,7 @@ int launch_bwd_dq_w32(const BwdM& g, int dtype, int head_dim, hipStream_t s) {
     else if (mask == 3) LAUNCH(TT, DD, 3);                                   \
     else if (mask == 2) LAUNCH(TT, DD, 2);                                   \
     else if (mask == 1) LAUNCH(TT, DD, 1);                                   \
-    else if constexpr (DD != 64) LAUNCH(TT, DD, 0); /* (64: bwd_d64.hip) */  \
+    else LAUNCH(TT, DD, 0);                                                  \
   } while (0)
 #define LAUNCH_D(DD)                                                         \
   do {                                                                       \
