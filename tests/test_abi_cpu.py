@@ -207,6 +207,18 @@ def test_entry_points_reject_bad_arguments_without_a_gpu(amd):
     assert lib.mi355_sdpa_bwd_workspace_bytes(None) == 0
 
 
+@pytest.mark.parametrize("Hq,L,S,ld", [(16, 512, 512, 0), (64, 16384, 16384, 0), (32, 32768, 32768, 0), (1, 4096, 100, 1 << 20)])
+def test_every_dropout_call_at_head_dim_64_gets_room_for_its_keep_bits(amd, Hq, L, S, ld):
+    """Whatever the matrix-op backward accepts: the kernels that take such a call read the keep-mask as bits."""
+    p, D = amd._lib.BwdParams(), 64
+    for f, n in (("grad_out", L), ("q", L), ("out", L), ("grad_q", L), ("k", S), ("v", S), ("grad_k", S), ("grad_v", S)):
+        setattr(p, f, amd._lib.Tensor4(4096, (C.c_int64 * 4)(1, Hq, n, D), (C.c_int64 * 4)(Hq * n * D, n * D, D, 1)))
+    p.lse, p.dtype, p.scale = 4096, amd._lib.BF16, 0.125
+    plain = amd._lib.load().mi355_sdpa_bwd_workspace_bytes(C.byref(p))
+    p.dropout_p, p.dropout_keep, p.dropout_keep_ld = 0.1, 4096, ld
+    assert amd._lib.load().mi355_sdpa_bwd_workspace_bytes(C.byref(p)) >= plain + Hq * L * -(-S // 128) * 16
+
+
 def test_host_ops_refuse_cpu_tensors(amd):
     q = torch.randn(1, 2, 4, 8)
     with pytest.raises(ValueError):

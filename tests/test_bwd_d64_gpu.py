@@ -105,3 +105,36 @@ def test_a_batch_beyond_32_bit_offsets(amd, gpu_device, which, causal):
         for name, a, r in (("dq", dq, dS @ K), ("dk", dk, dS.t() @ Q), ("dv", dv, P.t() @ DO)):
             off = float((a[0, h].double() - r).norm() / r.norm())
             assert off <= 8e-3, (name, h, off)
+
+
+def _check_heads(amd, q, k, v, do, keep, p, heads):
+    L, S, D = q.shape[2], k.shape[2], q.shape[3]
+    kw = dict(dropout_p=p, dropout_keep=keep)
+    out, lse = amd.sdpa_forward(q, k, v, **kw)
+    dq, dk, dv, _ = amd.sdpa_backward(do, q, k, v, out, lse, **kw)
+    for h in heads:
+        Q, K, V, DO, kp = *(t[0, h].double() for t in (q, k, v, do)), keep[0, h].double() / (1 - p)
+        P = torch.softmax(Q @ K.t() / math.sqrt(D), -1)
+        dP = (DO @ V.t()) * kp
+        dS = P * (dP - (DO * ((P * kp) @ V)).sum(-1, keepdim=True)) / math.sqrt(D)
+        for name, a, r in (("dq", dq, dS @ K), ("dk", dk, dS.t() @ Q), ("dv", dv, (P * kp).t() @ DO)):
+            off = float((a[0, h].double() - r).norm() / r.norm())
+            assert off <= 8e-3, (name, h, off)
+
+
+def test_keep_bits_of_a_batch_beyond_2_gib(amd, gpu_device):
+    """Hq * L * ceil(S / 128) * 16 bytes of keep bits reach 2 GiB (every head reads the same Q, K, V and dO)."""
+    H, L, S, D = 512, 1 << 18, 4, 8
+    g = torch.Generator(device=gpu_device).manual_seed(4)
+    q, k, v, do = (torch.randn(1, 1, n, D, generator=g, device=gpu_device).to(torch.bfloat16).expand(1, H, n, D) for n in (L, S, S, L))
+    keep = torch.empty(1, H, L, S, dtype=torch.uint8, device=gpu_device).bernoulli_(0.75, generator=g)
+    _check_heads(amd, q, k, v, do, keep, 0.25, (0, 300, 511))
+
+
+def test_keep_mask_rows_far_apart(amd, gpu_device):
+    """The rows of a keep-mask lie 1 MiB apart: 2.5 GiB from the first to the last."""
+    L, S, D, ld = 2560, 100, 64, 1 << 20
+    g = torch.Generator(device=gpu_device).manual_seed(5)
+    q, k, v, do = (torch.randn(1, 1, n, D, generator=g, device=gpu_device).to(torch.bfloat16) for n in (L, S, S, L))
+    keep = torch.empty(L * ld, dtype=torch.uint8, device=gpu_device).as_strided((1, 1, L, S), (L * ld, L * ld, ld, 1)).bernoulli_(0.75, generator=g)
+    _check_heads(amd, q, k, v, do, keep, 0.25, (0,))

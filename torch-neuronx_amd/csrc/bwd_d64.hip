@@ -22,7 +22,10 @@
 //
 // Dropout: the keep-mask is bytes.  The dQ kernel reads them (16 of a row per lane, the halves of a wavefront
 // exchange what the other one needs) and leaves one BIT per score behind for the dK/dV kernel, whose lanes
-// are keys: read as bytes there the mask is a load per score.  Rows of bits, 32 keys per word.
+// are keys: read as bytes there the mask is a load per score.  32 keys per word, four words per query row and
+// block of 128 keys, laid out [batch][kv head][block][head of the group][row]: a dK/dV workgroup reads one run of
+// them, at 32-bit offsets however many there are in all.  (Rows of bits over all keys: a load's 64 lanes touch as
+// many lines, backward of B=4, 16 heads, S=2048 causal 217 us against 189, of B=2, 16/4 heads, S=4096 688 / 636.)
 //
 // Math follows torch_neuronx/_sdpa_math.py:98-176: float32 accumulation, rows with lse = -inf give zero
 // gradients, scale multiplies dQ and dK once at the end.
@@ -100,8 +103,8 @@ __device__ __forceinline__ void chunk_offsets(uint32_t (&off)[NCH], int tid, int
   for (int n = 0; n < NCH; ++n) off[n] = ch * 8 < width ? (uint32_t)(((row + (256 / CH) * n) * row_stride + ch * 8) * 2) : 0x7ffffff0u;
 }
 
-// words of keep bits per query row: whole blocks of 128 keys
-__host__ __device__ __forceinline__ int bit_words(int S) { return (S + 127) / 128 * 4; }
+// words of keep bits of one block of 128 keys of one (batch, kv head): four per query row of the group's heads
+__host__ __device__ __forceinline__ int64_t block_words(const BwdM& p) { return (int64_t)(p.Hq / p.Hkv) * p.L * 4; }
 
 // this lane's 16 elements of an accumulator packed to the input dtype, in B-operand order
 template <typename T>
@@ -190,11 +193,13 @@ __global__ __launch_bounds__(256, 3) void bwd_d64_dq_kernel(BwdM p, uint32_t* ke
       lds_load16(v_rsrc, v_off[n] >= 0x7ffffff0u ? v_off[n] : v_off[n] + vb, lds_v + (uint32_t)(buf * TILE_BYTES + n * 4096));
     }
   };
-  // (dropout) keep bytes of this lane's row: keys 16 half .. +15 of each 32-key block of tile t
+  // (dropout) keep bytes of this lane's row: keys 16 half .. +15 of each 32-key block of tile t, through a
+  // buffer of this wavefront's rows (rows past L: the last one again)
+  const int keep_rows = min(32, p.L - qw0), qw0c = min(qw0, p.L - 1);
   const __amdgpu_buffer_rsrc_t keep_rsrc = __builtin_amdgcn_make_buffer_rsrc(
-      uniform_ptr((const char*)p.keep + (DROP ? (((int64_t)b * p.Hq + h) * p.L) * p.keep_ld : 0)), 0,
-      __builtin_amdgcn_readfirstlane(DROP ? (int)((int64_t)p.L * p.keep_ld) : 0), 0x00020000);
-  const uint32_t keep_off = DROP ? (uint32_t)((int64_t)qc * p.keep_ld + half * 16) : 0u;
+      uniform_ptr((const char*)p.keep + (DROP ? (((int64_t)b * p.Hq + h) * p.L + qw0c) * p.keep_ld : 0)), 0,
+      __builtin_amdgcn_readfirstlane(DROP ? (int)((int64_t)max(keep_rows, 1) * p.keep_ld) : 0), 0x00020000);
+  const uint32_t keep_off = DROP ? (uint32_t)((int64_t)(qc - qw0c) * p.keep_ld + half * 16) : 0u;
   u32x4 kraw[DROP ? 2 : 1];
   auto load_keep = [&](int t) {
     if constexpr (DROP) {
@@ -238,7 +243,7 @@ __global__ __launch_bounds__(256, 3) void bwd_d64_dq_kernel(BwdM p, uint32_t* ke
 #pragma unroll
   for (int i = 0; i < DB; ++i) zero(acc[i]);
   const float c = p.scale * kLog2eF;
-  uint32_t* const bit_row = DROP ? keep_bits + (((int64_t)b * p.Hq + h) * p.L + qc) * bit_words(p.S) : nullptr;
+  uint32_t* const bit_row = DROP ? keep_bits + (int64_t)bm.stream * p.n_kt * block_words(p) + ((int64_t)bm.unit * p.L + qc) * 4 : nullptr;
 
   wait_loads();
   await_keep();
@@ -283,7 +288,7 @@ __global__ __launch_bounds__(256, 3) void bwd_d64_dq_kernel(BwdM p, uint32_t* ke
         }
         bits <<= 4 * half;
         bits |= __shfl_xor(bits, 32, 64);
-        if (qrow < p.L && half == 0) bit_row[kv0 >> 5] = bits;
+        if (qrow < p.L && half == 0) bit_row[(t >> 1) * block_words(p) + (t & 1) * 2 + mb] = bits;
       }
       float ds[16];
 #pragma unroll
@@ -367,8 +372,7 @@ __global__ __launch_bounds__(256, OCC) void bwd_d64_dkdv_kernel(BwdM p, const ui
   const u32x4 go_rsrc = descriptor((const uint16_t*)p.go + b * p.go_sb, ((int64_t)(p.Hq - 1) * p.go_sh + (int64_t)(p.L - 1) * p.go_sl + dr) * 2);
   const u32x4 lse_rsrc = descriptor(p.lse2 + (int64_t)b * p.Hq * p.L, (int64_t)p.Hq * p.L * 4);
   const u32x4 dl_rsrc = descriptor(p.delta + (int64_t)b * p.Hq * p.L, (int64_t)p.Hq * p.L * 4);
-  const int words = bit_words(p.S);
-  const u32x4 bit_rsrc = descriptor(DROP ? keep_bits + (int64_t)b * p.Hq * p.L * words : nullptr, DROP ? (int64_t)p.Hq * p.L * words * 4 : 0);
+  const u32x4 bit_rsrc = descriptor(DROP ? keep_bits + ((int64_t)st * p.n_kt + kt) * block_words(p) : nullptr, DROP ? block_words(p) * 4 : 0);
   uint32_t q_off[NCH], go_off[NCH];
   chunk_offsets(q_off, tid, p.q_sl, dr);
   chunk_offsets(go_off, tid, p.go_sl, dr);
@@ -384,7 +388,7 @@ __global__ __launch_bounds__(256, OCC) void bwd_d64_dkdv_kernel(BwdM p, const ui
     const uint32_t row = (uint32_t)(h * p.L + q0 + lane);
     if (wave == 0) lds_load4(lse_rsrc, row * 4, lds_address(lse_s[buf]));
     if (wave == 1) lds_load4(dl_rsrc, row * 4, lds_address(dl_s[buf]));
-    if constexpr (DROP) lds_load4(bit_rsrc, (row * words + (uint32_t)(kt * 4 + wave)) * 4, lds_address(bit_s[buf][wave]));
+    if constexpr (DROP) lds_load4(bit_rsrc, (uint32_t)((h - hk * rep_all) * p.L + q0 + lane) * 16 + wave * 4, lds_address(bit_s[buf][wave]));
   };
   auto finish_item = [&](int it, int buf) {  // (the tile's loads have landed)
     const int q0 = item_q0(it);
@@ -544,14 +548,14 @@ int launch_t(const BwdM& g, uint32_t* bits, hipStream_t s) {
 
 bool bwd_d64_takes(const BwdM& g) {
   if (g.d_real > 64 || g.dv_real != g.d_real || g.bias_kind || g.gbias || g.window > 0 || g.sm.any || g.dq_split_tiles) return false;
-  // (32-bit byte offsets from the start of a batch or of a (batch, head))
-  if (!bwd_dkdv_w32_fits(g, 64) || !bwd_dq_w32_fits(g, 64)) return false;
-  return g.keep_scale == 0.f || ((int64_t)g.L * g.keep_ld < (1ll << 31) && (int64_t)g.Hq * g.L * bit_words(g.S) * 4 < (1ll << 31));
+  // (32-bit byte offsets from the start of a batch, and of a key block's keep bits; the latter are the smaller ones
+  // but for heads expanded from one)
+  return bwd_dkdv_w32_fits(g, 64) && bwd_dq_w32_fits(g, 64) && (g.keep_scale == 0.f || block_words(g) * 4 < (1ll << 32));
 }
 
 size_t bwd_d64_bits_bytes(const BwdM& g) {
   if (g.keep_scale == 0.f || !bwd_d64_takes(g)) return 0;
-  return ((size_t)g.B * g.Hq * g.L * bit_words(g.S) * sizeof(uint32_t) + 255) & ~(size_t)255;
+  return ((size_t)g.B * g.Hkv * g.n_kt * block_words(g) * sizeof(uint32_t) + 255) & ~(size_t)255;
 }
 
 int launch_bwd_d64(const BwdM& g0, int dtype, uint32_t* keep_bits, hipStream_t s) {

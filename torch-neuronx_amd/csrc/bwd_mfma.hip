@@ -627,6 +627,7 @@ bool bwd_mfma_supported(const mi355_sdpa_bwd_params& p, const char** why) {
     fill(g, p);
     const int D = E <= 64 ? 64 : 128;
     if (!bwd_dkdv_w32_fits(g, D) || !bwd_dq_w32_fits(g, D)) return *why = "masked call / padded head dim beyond 32-bit offsets", false;
+    if (D == 64 && g.keep_scale != 0.f && !g.bias_kind && !bwd_d64_takes(g)) return *why = "dropout keep bits beyond 32-bit offsets", false;
   }
   return true;
 }
