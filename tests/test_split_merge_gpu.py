@@ -68,3 +68,15 @@ def test_partials_of_the_fp8_decode(amd, gpu_device, B, Hkv, S, D):
     want, want_lse = _want(q, k.float() / 32, v.float() / 32, lens)
     assert _rel(out, want) <= 4e-3
     assert float((lse.double() - want_lse).abs().max()) <= 2e-3
+
+
+@pytest.mark.parametrize("H,S", [(64, 4096), (8, 65536)])
+def test_a_large_lse_is_rounded_twice_and_no_more(amd, gpu_device, H, S):
+    """Every score of a row is the same float32 value c between 512 and 1000, exactly: a part's lse is c + ln(keys),
+    the row's that plus ln(parts), each sum rounded once to half a unit of 2^-14 (2^-20 for the two logarithms)."""
+    c = 512.0 + 488.0 * torch.rand(H, generator=torch.Generator(device=gpu_device).manual_seed(H), device=gpu_device)
+    q, k = torch.zeros(1, H, 1, 64, device=gpu_device), torch.zeros(1, H, S, 64, device=gpu_device)
+    q[0, :, 0, 5], k[..., 5] = c, 1.0
+    out, lse = amd.sdpa_forward(q, k, torch.ones_like(k), scale=1.0)
+    assert float((lse[0, :, 0].double() - c.double() - math.log(S)).abs().max()) <= 2 * 2.0**-15 + 2.0**-20
+    assert float((out - 1).abs().max()) <= 1e-5

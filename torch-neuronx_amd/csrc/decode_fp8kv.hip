@@ -469,7 +469,7 @@ __global__ __launch_bounds__(SLICES * D / 4) void decode_merge_kernel(DecP p) {
   const float* const po = p.ws_o + slot0 * D + (threadIdx.x % (D / 4)) * 4;
   const float* const pml = p.ws_ml + slot0 * 2;
   float O, M, L;
-  merge_parts<SLICES, D / 4>(
+  merge_parts<false, SLICES, D / 4>(
       lds, npart,
       [&](int c, float& m, float& l) {
         const f32x2 w = *(const f32x2*)(pml + (int64_t)c * p.R * 2);

@@ -977,7 +977,7 @@ __global__ __launch_bounds__(64 * WAVES, D > 128 ? 1 : 8 / WAVES) void fwd_w32_k
 }
 
 // Merge of the parts of a call whose keys were split (see split_merge.h): normalised rows and their
-// log-sum-exp, so a part's statistics are (lse in the log2 domain, 1).
+// log-sum-exp, so a part's statistics are (lse, 1).
 template <typename T, int TPR, int SLICES>
 __global__ __launch_bounds__(SLICES * TPR) void fwd_split_merge_kernel(FwdM p) {
   __shared__ MergeLds<SLICES, TPR> lds;
@@ -990,12 +990,12 @@ __global__ __launch_bounds__(SLICES * TPR) void fwd_split_merge_kernel(FwdM p) {
   const float* const po = p.part_o + (bh * p.n_split * p.L + l) * p.dv_real + d4;
   const int64_t part_stride = (int64_t)p.L * p.dv_real;
   float O, M, L;
-  merge_parts<SLICES, TPR>(
-      lds, p.n_split, [&](int c, float& m, float& w) { m = pl[(int64_t)c * p.L] * kLog2eF, w = 1.f; },
+  merge_parts<true, SLICES, TPR>(
+      lds, p.n_split, [&](int c, float& m, float& w) { m = pl[(int64_t)c * p.L], w = 1.f; },
       [&](int c) { return *(const f32x4*)(po + c * part_stride); }, O, M, L);
   const int d = threadIdx.x;
   if (d < p.dv_real) ((T*)p.out)[b * p.o_sb + h * p.o_sh + (int64_t)l * p.o_sl + d] = (T)(L > 0.f ? O / L : 0.f);
-  if (d == 0 && p.lse) p.lse[row] = L > 0.f ? M / kLog2eF + __builtin_logf(L) : -INFINITY;
+  if (d == 0 && p.lse) p.lse[row] = L > 0.f ? M + __builtin_logf(L) : -INFINITY;
 }
 
 template <typename T>

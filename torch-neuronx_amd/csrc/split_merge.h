@@ -1,5 +1,5 @@
 // Merge of the partial rows that a call with split keys leaves in its workspace (fwd_mfma_w32.hip,
-// f32_mfma.hip, decode_fp8kv.hip): out = sum_c w_c O_c / sum_c w_c l_c with w_c = 2^(m_c - max m).
+// f32_mfma.hip, decode_fp8kv.hip): out = sum_c w_c O_c / sum_c w_c l_c with w_c = 2^(m_c - max m), or e^ of it.
 //
 // One workgroup per output row.  What bounds it is not the bytes (a few MB, in L2) but the trips to
 // them: it is a launch between two others whose work is one chain of dependent loads.  So the parts are
@@ -25,14 +25,17 @@ struct MergeLds {
   float m[SLICES], l[SLICES];
 };
 
-// ml(c, m, l): statistics of part c, log2 domain (m = -inf: a part without keys, its row is never used
-// whatever it holds).  row(c): this thread's four columns of part c.  Workgroup of SLICES * TPR threads;
+// ml(c, m, l): statistics of part c, m in the log2 domain or (LN) the natural one (m = -inf: a part without
+// keys, its row is never used whatever it holds).  (The domain is the caller's: a log-sum-exp turned into the other
+// one and back takes two roundings of its own size, lse 4.1e-7 -> 4.4e-7 off at float32, 8 heads, S=2048; here only
+// differences are converted.)  row(c): this thread's four columns of part c.  Workgroup of SLICES * TPR threads;
 // on return thread d < 4 * TPR holds column d of the weighted sum (O), and M and L are those of the row.
-template <int SLICES, int TPR, typename ML, typename ROW>
+template <bool LN, int SLICES, int TPR, typename ML, typename ROW>
 __device__ __forceinline__ void merge_parts(MergeLds<SLICES, TPR>& lds, int np, ML ml, ROW row, float& O, float& M, float& L) {
   static_assert(SLICES >= 4, "one thread per column at the end");
   constexpr int BATCH = 8;
   const int slice = threadIdx.x / TPR, quad = threadIdx.x % TPR;
+  auto weight = [](float d) { return __builtin_amdgcn_exp2f(LN ? d * kLog2eF : d); };
   float ms = -INFINITY, ls = 0.f;
   f32x4 os = {0.f, 0.f, 0.f, 0.f};
   for (int c0 = slice; c0 < np; c0 += SLICES * BATCH) {
@@ -51,11 +54,11 @@ __device__ __forceinline__ void merge_parts(MergeLds<SLICES, TPR>& lds, int np, 
 #pragma unroll
     for (int i = 0; i < BATCH; ++i) mn = fmaxf(mn, m[i]);
     if (mn == -INFINITY) continue;
-    const float f = __builtin_amdgcn_exp2f(ms - mn);  // (no part yet: 0)
+    const float f = weight(ms - mn);  // (no part yet: 0)
     ls *= f, os *= f;
 #pragma unroll
     for (int i = 0; i < BATCH; ++i) {
-      const float w = __builtin_amdgcn_exp2f(m[i] - mn);
+      const float w = weight(m[i] - mn);
       ls = fmaf(l[i], w, ls);
 #pragma unroll
       for (int e = 0; e < 4; ++e) os[e] = m[i] == -INFINITY ? os[e] : fmaf(o[i][e], w, os[e]);
@@ -72,7 +75,7 @@ __device__ __forceinline__ void merge_parts(MergeLds<SLICES, TPR>& lds, int np, 
   const int d = min((int)threadIdx.x, 4 * TPR - 1);
 #pragma unroll
   for (int s = 0; s < SLICES; ++s) {
-    const float w = __builtin_amdgcn_exp2f(lds.m[s] - M);
+    const float w = weight(lds.m[s] - M);
     L = fmaf(lds.l[s], w, L);
     O = fmaf(lds.o[s][d], w, O);
   }
