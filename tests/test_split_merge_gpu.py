@@ -80,3 +80,18 @@ def test_a_large_lse_is_rounded_twice_and_no_more(amd, gpu_device, H, S):
     out, lse = amd.sdpa_forward(q, k, torch.ones_like(k), scale=1.0)
     assert float((lse[0, :, 0].double() - c.double() - math.log(S)).abs().max()) <= 2 * 2.0**-15 + 2.0**-20
     assert float((out - 1).abs().max()) <= 1e-5
+
+
+@pytest.mark.parametrize("B,S,part,every", [(1, 8192, 8192, 1), (1, 8192, 100, 3), (1, 1024, 128, 4), (1, 1024, 128, 8), (16, 1024, 128, 4), (1, 32768, 256, 16)])
+def test_nan_keys_of_the_fp8_decode_are_not_dropped(amd, gpu_device, B, S, part, every):
+    """A cache with NaN keys gives rows without a sum (zeros, lse = -inf), whether the NaNs share their parts with
+    ordinary keys or fill whole parts (of 128 keys, in the last case 256), those that one group of the merge's
+    threads takes among them: never what the other keys alone would give."""
+    g = torch.Generator(device=gpu_device).manual_seed(S)
+    q = torch.randn(B, 16, 1, 128, generator=g, device=gpu_device, dtype=torch.bfloat16)
+    k, v = (torch.randn(B, 8, S, 128, generator=g, device=gpu_device) for _ in range(2))
+    k[:, :, torch.arange(S, device=gpu_device) // part % every == every - 1] = math.nan
+    k, v = k.to(torch.float8_e4m3fn), v.to(torch.float8_e4m3fn)
+    one = torch.ones(B, 8, device=gpu_device)
+    out, lse = amd.decode_fp8kv(q, k, v, one, one)
+    assert not out.any() and torch.isneginf(lse).all()

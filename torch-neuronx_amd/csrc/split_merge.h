@@ -53,12 +53,14 @@ __device__ __forceinline__ void merge_parts(MergeLds<SLICES, TPR>& lds, int np, 
     float mn = ms;
 #pragma unroll
     for (int i = 0; i < BATCH; ++i) mn = fmaxf(mn, m[i]);
-    if (mn == -INFINITY) continue;
-    const float f = weight(ms - mn);  // (no part yet: 0)
+    // (no part with a score so far: the reference is 0, the weights are too, and a NaN among the sums - a part whose
+    // scores are all NaN has no maximum - still makes the row's sum one)
+    const float ref = mn == -INFINITY ? 0.f : mn;
+    const float f = weight(ms - ref);
     ls *= f, os *= f;
 #pragma unroll
     for (int i = 0; i < BATCH; ++i) {
-      const float w = weight(m[i] - mn);
+      const float w = weight(m[i] - ref);
       ls = fmaf(l[i], w, ls);
 #pragma unroll
       for (int e = 0; e < 4; ++e) os[e] = m[i] == -INFINITY ? os[e] : fmaf(o[i][e], w, os[e]);
