@@ -138,3 +138,38 @@ def test_keep_mask_rows_far_apart(amd, gpu_device):
     q, k, v, do = (torch.randn(1, 1, n, D, generator=g, device=gpu_device).to(torch.bfloat16) for n in (L, S, S, L))
     keep = torch.empty(L * ld, dtype=torch.uint8, device=gpu_device).as_strided((1, 1, L, S), (L * ld, L * ld, ld, 1)).bernoulli_(0.75, generator=g)
     _check_heads(amd, q, k, v, do, keep, 0.25, (0,))
+
+
+@pytest.mark.parametrize("p", [0.0, 0.25])
+@pytest.mark.parametrize("L,causal", [(100, False), (97, True), (33, False)])
+def test_nan_of_one_head_stays_in_it(amd, gpu_device, L, causal, p):
+    """The rows past L of a head's last tile are the next head's in memory: a NaN there must not meet this head's
+    zero probabilities.  (Heads are independent, so the others' gradients are the same bits.)"""
+    B, H, S, D = 2, 3, 130, 64
+    g = torch.Generator(device=gpu_device).manual_seed(L)
+    q, k, v, do = (torch.randn(B, H, n, D, generator=g, device=gpu_device).to(torch.bfloat16) for n in (L, S, S, L))
+    kw = dict(is_causal=causal)
+    if p:
+        kw.update(dropout_p=p, dropout_keep=amd.ops.padded_keep_mask(B, H, L, S, gpu_device).bernoulli_(1 - p, generator=g))
+
+    def grads():
+        out, lse = amd.sdpa_forward(q, k, v, **kw)
+        return amd.sdpa_backward(do, q, k, v, out, lse, **kw)[:3]
+
+    want = grads()
+    q[:, 1], do[:, 1] = math.nan, math.inf
+    for name, a, w in zip(("dq", "dk", "dv"), grads(), want):
+        assert torch.isfinite(a[:, ::2]).all() and torch.equal(a[:, ::2], w[:, ::2]), name
+        assert torch.isnan(a[:, 1]).any(), name
+
+
+@pytest.mark.parametrize("L", [64, 100])
+def test_every_row_of_the_gradient_in_one_place(amd, gpu_device, L):
+    """dO with row stride 0 (a mean over the rows leaves such a gradient): rows past L are live data there."""
+    B, H, S, D = 2, 2, 130, 64
+    g = torch.Generator(device=gpu_device).manual_seed(L)
+    q, k, v = (torch.randn(B, H, n, D, generator=g, device=gpu_device).to(torch.bfloat16) for n in (L, S, S))
+    do = torch.randn(B, H, 1, D, generator=g, device=gpu_device).to(torch.bfloat16).expand(B, H, L, D)
+    out, lse = amd.sdpa_forward(q, k, v)
+    for a, w in zip(amd.sdpa_backward(do, q, k, v, out, lse)[:3], amd.sdpa_backward(do.contiguous(), q, k, v, out, lse)[:3]):
+        assert torch.equal(a, w)

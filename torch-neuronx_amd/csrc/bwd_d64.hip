@@ -366,33 +366,33 @@ __global__ __launch_bounds__(256, OCC) void bwd_d64_dkdv_kernel(BwdM p, const ui
   auto item_head = [&](int it) { return h0 + (it + it0 - item_tile(it) * rep); };
   auto item_q0 = [&](int it) { return (nqs - 1 - item_tile(it)) * BQ; };
 
-  // staging: the buffers end with the last row of the batch; rows past L read as zeros or as another head's
-  // rows and are switched off through lse = +inf
-  const u32x4 q_rsrc = descriptor((const uint16_t*)p.q + b * p.q_sb, ((int64_t)(p.Hq - 1) * p.q_sh + (int64_t)(p.L - 1) * p.q_sl + dr) * 2);
-  const u32x4 go_rsrc = descriptor((const uint16_t*)p.go + b * p.go_sb, ((int64_t)(p.Hq - 1) * p.go_sh + (int64_t)(p.L - 1) * p.go_sl + dr) * 2);
-  const u32x4 lse_rsrc = descriptor(p.lse2 + (int64_t)b * p.Hq * p.L, (int64_t)p.Hq * p.L * 4);
-  const u32x4 dl_rsrc = descriptor(p.delta + (int64_t)b * p.Hq * p.L, (int64_t)p.Hq * p.L * 4);
   const u32x4 bit_rsrc = descriptor(DROP ? keep_bits + ((int64_t)st * p.n_kt + kt) * block_words(p) : nullptr, DROP ? block_words(p) * 4 : 0);
   uint32_t q_off[NCH], go_off[NCH];
   chunk_offsets(q_off, tid, p.q_sl, dr);
   chunk_offsets(go_off, tid, p.go_sl, dr);
   const uint32_t lds_q = lds_address(q_t) + wave * 1024, lds_do = lds_address(do_t) + wave * 1024;
+  // (the buffers of an item are its tile's own and end with the head's last row: a row past L must not be another
+  // head's, whose NaN would survive the zero probabilities)
   auto load_item = [&](int it, int buf) {
-    const int h = item_head(it), q0 = item_q0(it);
-    const uint32_t qb = (uint32_t)((h * p.q_sh + (int64_t)q0 * p.q_sl) * 2), gb = (uint32_t)((h * p.go_sh + (int64_t)q0 * p.go_sl) * 2);
+    const int h = item_head(it), q0 = item_q0(it), rows = min(p.L - q0, BQ);
+    const u32x4 q_rsrc = descriptor((const uint16_t*)p.q + b * p.q_sb + h * p.q_sh + (int64_t)q0 * p.q_sl, ((int64_t)(rows - 1) * p.q_sl + dr) * 2);
+    const u32x4 go_rsrc = descriptor((const uint16_t*)p.go + b * p.go_sb + h * p.go_sh + (int64_t)q0 * p.go_sl, ((int64_t)(rows - 1) * p.go_sl + dr) * 2);
 #pragma unroll
     for (int n = 0; n < NCH; ++n) {
-      lds_load16(q_rsrc, q_off[n] >= 0x7ffffff0u ? q_off[n] : q_off[n] + qb, lds_q + (uint32_t)(buf * TILE_BYTES + n * 4096));
-      lds_load16(go_rsrc, go_off[n] >= 0x7ffffff0u ? go_off[n] : go_off[n] + gb, lds_do + (uint32_t)(buf * TILE_BYTES + n * 4096));
+      lds_load16(q_rsrc, q_off[n], lds_q + (uint32_t)(buf * TILE_BYTES + n * 4096));
+      lds_load16(go_rsrc, go_off[n], lds_do + (uint32_t)(buf * TILE_BYTES + n * 4096));
     }
-    const uint32_t row = (uint32_t)(h * p.L + q0 + lane);
-    if (wave == 0) lds_load4(lse_rsrc, row * 4, lds_address(lse_s[buf]));
-    if (wave == 1) lds_load4(dl_rsrc, row * 4, lds_address(dl_s[buf]));
+    if (wave < 2) {  // the rows' statistics: wavefront 0 log-sum-exps, wavefront 1 deltas
+      const u32x4 st_rsrc = descriptor((wave == 0 ? p.lse2 : p.delta) + ((int64_t)b * p.Hq + h) * p.L + q0, rows * 4);
+      lds_load4(st_rsrc, lane * 4, wave == 0 ? lds_address(lse_s[buf]) : lds_address(dl_s[buf]));
+    }
     if constexpr (DROP) lds_load4(bit_rsrc, (uint32_t)((h - hk * rep_all) * p.L + q0 + lane) * 16 + wave * 4, lds_address(bit_s[buf][wave]));
   };
-  auto finish_item = [&](int it, int buf) {  // (the tile's loads have landed)
+  // rows past L: no probability whatever stands there (wavefront 0, which loaded the values it writes over and has
+  // waited for them)
+  auto finish_item = [&](int it, int buf) {
     const int q0 = item_q0(it);
-    if (q0 + BQ > p.L && tid < BQ && q0 + tid >= p.L) lse_s[buf][tid] = INFINITY, dl_s[buf][tid] = 0.f;
+    if (q0 + BQ > p.L && tid < BQ && q0 + tid >= p.L) lse_s[buf][tid] = INFINITY;
   };
   if (n_items > 0) load_item(0, 0);
   u32x4 kf[KS], vf[KS];  // this lane's key as B operand
