@@ -1,6 +1,6 @@
 """The forward with a soft cap and no other score functor (its variant of the 32-row kernels):
 sizes around its 32-key tiles, windows, key counts that leave tiles and rows without a key, scores far beyond the
-cap, a cap far beyond the scores, infinite scores.
+cap, a cap far beyond the scores, infinite scores of either sign.
 
 Bounds, against the same attention in float64 on the kernel's inputs: the capped score is cap (1 - 2 r) with r
 to 2^-22 relative, so a score is off by at most 2^-21 cap and what the float32 sum of its products loses
@@ -88,3 +88,37 @@ def test_lse_of_a_large_cap_keeps_the_reference(amd, gpu_device):
     off = lse.double() - torch.logsumexp(s, -1)
     assert abs(float(off.mean())) <= 2.0**-22 * cap
     assert float(off.std()) <= 2.0**-22 * cap / math.sqrt(S / math.e) + 2.0**-22 * float(lse.abs().max())
+
+
+@pytest.mark.parametrize("D", [64, 128, 256])
+@pytest.mark.parametrize("L,S,causal,window,lens", [(70, 160, False, None, None), (97, 97, True, None, None), (130, 130, True, 40, None), (40, 193, False, None, [100, 65])])
+def test_scores_of_minus_infinity_are_minus_the_cap(amd, gpu_device, D, L, S, causal, window, lens):
+    """-cap like any score far below it, in tiles with a mask and without one: a row all of whose scores are -inf
+    (or finite beyond -1e30) is the mean of the values it sees, a single such key keeps its share."""
+    B, H, cap, dev = 2, 2, 5.0, gpu_device
+    g = torch.Generator(device=dev).manual_seed(D + S)
+    q, k, v = (torch.randn(B, H, n, D, generator=g, device=dev).to(torch.bfloat16) for n in (L, S, S))
+    k[..., 0] = k[..., 0].abs() + 0.5
+    q[0, :, ::3, 0] = -math.inf
+    q[0, :, 1::3, 0] = -3e38                         # (scores of about -1e37 and below)
+    q[1, :, :, 1], k[1, :, :, 1] = -1.0, 0.0
+    k[1, :, 5::40, 1] = math.inf                     # keys whose score is -inf for every row
+    kw = dict(is_causal=causal, softcap=cap)
+    if window:
+        kw["window"] = window
+    lens_t = torch.tensor(lens or [S] * B, device=dev)
+    if lens:
+        kw["kv_lens"] = lens_t.to(torch.int32)
+    out, lse = amd.sdpa_forward(q, k, v, **kw)
+    i, j = torch.arange(L, device=dev)[:, None], torch.arange(S, device=dev)[None]
+    dead = (j[None] >= lens_t[:, None, None])[:, None].expand(B, 1, L, S).clone()
+    if causal:
+        dead |= j > i
+    if window:
+        dead |= j < i - window + 1
+    raw = q.double() @ k.double().transpose(-1, -2).contiguous() / math.sqrt(D)
+    assert not torch.isnan(raw).any()
+    s = (cap * torch.tanh(raw / cap)).masked_fill(dead, -math.inf)
+    score_err = 2.0**-21 * (cap + 4 * math.sqrt(D))
+    assert float((lse.double() - torch.logsumexp(s, -1)).abs().max()) <= score_err + 2.0**-19
+    assert float((out.double() - torch.softmax(s, -1) @ v.double()).abs().max()) <= (2.5 * 2.0**-9 + 2 * score_err) * float(v.double().abs().max())

@@ -27,6 +27,8 @@
 //
 // Numerics: torch_neuronx/_sdpa_math.py:51-95 (float32 accumulation and softmax, probabilities
 // rounded to the input dtype for P*V only, dead rows give zeros and lse = -inf).
+#include <float.h>
+
 #include <algorithm>
 #include <type_traits>
 
@@ -418,6 +420,7 @@ __device__ __forceinline__ void fwd_w32_body(const FwdM& p, const MaskArgs ma) {
       const int kv = kv0 + (r >> 2) * 8 + half * 4 + (r & 3);
       // (bitwise on purpose: with || and && every element gets a cascade of branches)
       const bool dead = FUNC ? (kv > lim) | ((kv < lo_w) & (kv >= n_sink)) : kv > lim;
+      if constexpr (CAP) s[r] = s[r] == -INFINITY ? -FLT_MAX : s[r];  // (the cap gives a live score of -inf -cap, see cap_x)
       s[r] = dead ? -INFINITY : s[r];
     }
   };
@@ -642,14 +645,17 @@ __device__ __forceinline__ void fwd_w32_body(const FwdM& p, const MaskArgs ma) {
   // cap (1 - 2 r): 1 - 2 r is exact but for r, and its exponent in the log2 domain, reference subtracted, one
   // multiply-add more.  (Both in one, r times -2 cap plus the rest of the reference, rounds that rest to the precision of
   // the cap, for a whole row: lse 1.2e-7 -> 2.9e-7 off at a cap of 50.)  A
-  // masked score (-inf) would come out as -cap: the minimum with s + 1e30 keeps it (and a NaN).
+  // masked score (-inf) would come out as -cap: in a tile that mask_tile went over (w_mask = 1e-10) the minimum with
+  // s w_mask + 1e30 keeps it; that is far above every exponent for any other score, a -inf that is no mask's included
+  // (-FLT_MAX there), and for the tiles without a mask (w_mask = 0: 1e30, or a NaN, which a minimum drops).
   auto scalar = [](float x) { return __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, x))); };
   const float cap_k = CAP ? scalar(2.f * kLog2eF * p.scale / p.sm.softcap) : 0.f, cap_l = CAP ? scalar(kLog2eF * p.sm.softcap) : 0.f;
   const float cap_raw = CAP ? scalar(p.sm.softcap / p.scale) : 0.f;  // the cap in units of the raw scores
   auto cap_r = [&](float s) { return __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(s * cap_k)); };
-  auto raise_reference = [&](float t0) {
+  auto mask_weight = [&](bool masked) { return CAP && masked ? 1e-10f : 0.f; };
+  auto raise_reference = [&](float t0, float w_mask) {
     float tm = fmaxf(t0, __shfl_xor(t0, 32, 64));
-    if constexpr (CAP) tm = fminf(fmaf(cap_r(tm), -2.f, 1.f) * cap_raw, tm + 1e30f);  // (the cap is monotonic)
+    if constexpr (CAP) tm = fminf(fmaf(cap_r(tm), -2.f, 1.f) * cap_raw, fmaf(tm, w_mask, 1e30f));  // (the cap is monotonic)
     const bool up = (tm - m_run) * c > kLazy;  // false for NaN (-inf minus -inf)
     m_new = up ? tm : m_run;
     const float m_use = (m_new == -INFINITY) ? 0.f : m_new;
@@ -667,13 +673,13 @@ __device__ __forceinline__ void fwd_w32_body(const FwdM& p, const MaskArgs ma) {
     ce[0] = __builtin_amdgcn_exp2f(sv[2 * j] * cap_k);
     ce[1] = __builtin_amdgcn_exp2f(sv[2 * j + 1] * cap_k);
   };
-  auto cap_x = [&](const f32x16& sv, int j) {
-    xs[j & 1][0] = fminf(fmaf(fmaf(__builtin_amdgcn_rcpf(1.f + ce[0]), -2.f, 1.f), cap_l, -mc), sv[2 * j] + 1e30f);
-    xs[j & 1][1] = fminf(fmaf(fmaf(__builtin_amdgcn_rcpf(1.f + ce[1]), -2.f, 1.f), cap_l, -mc), sv[2 * j + 1] + 1e30f);
+  auto cap_x = [&](const f32x16& sv, int j, float w_mask) {
+    xs[j & 1][0] = fminf(fmaf(fmaf(__builtin_amdgcn_rcpf(1.f + ce[0]), -2.f, 1.f), cap_l, -mc), fmaf(sv[2 * j], w_mask, 1e30f));
+    xs[j & 1][1] = fminf(fmaf(fmaf(__builtin_amdgcn_rcpf(1.f + ce[1]), -2.f, 1.f), cap_l, -mc), fmaf(sv[2 * j + 1], w_mask, 1e30f));
   };
-  auto stage1 = [&](const f32x16& sv, int j) {
+  auto stage1 = [&](const f32x16& sv, int j, float w_mask) {
     if constexpr (CAP) {
-      cap_e(sv, j), cap_x(sv, j);
+      cap_e(sv, j), cap_x(sv, j, w_mask);
     } else {
       xs[j & 1][0] = fmaf(sv[2 * j], c, -mc);
       xs[j & 1][1] = fmaf(sv[2 * j + 1], c, -mc);
@@ -699,21 +705,21 @@ __device__ __forceinline__ void fwd_w32_body(const FwdM& p, const MaskArgs ma) {
   //   slot 2q: exp2 of pair q, scaling of pair q+1     slot 2q+1: sum and packing of pair q
   // with a soft cap in sixteen steps: exp2 of pair q, cap_e of q+1, sum and packing of q, cap_x of q+1
   constexpr int STEPS = CAP ? 16 : 8;
-  auto softmax_slot = [&](const f32x16& sv, int base, int slot, uint32_t (&pk)[8], float& ps) {
+  auto softmax_slot = [&](const f32x16& sv, int base, int slot, uint32_t (&pk)[8], float& ps, float w_mask) {
     if constexpr (CAP) {
       const int q = slot >> 2, r = slot & 3;
       if (r == 0) stage2(base + q);
       else if (r == 2) stage3(base + q, pk, ps);
       else if (q + 1 < 4) {
         if (r == 1) cap_e(sv, base + q + 1);
-        else cap_x(sv, base + q + 1);
+        else cap_x(sv, base + q + 1, w_mask);
       }
       return;
     }
     const int q = slot >> 1;
     if ((slot & 1) == 0) {
       stage2(base + q);
-      if (q + 1 < 4) stage1(sv, base + q + 1);
+      if (q + 1 < 4) stage1(sv, base + q + 1, w_mask);
     } else {
       stage3(base + q, pk, ps);
     }
@@ -731,6 +737,7 @@ __device__ __forceinline__ void fwd_w32_body(const FwdM& p, const MaskArgs ma) {
   f32x16 s_a, s_b;
   uint32_t pk_a[8], pk_b[8];
   float ps_a = 0.f, ps_b = 0.f;
+  float w_cur = mask_weight(edge(0));  // of the tile whose scores iteration() finds in scur
   {
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks) {
@@ -741,11 +748,11 @@ __device__ __forceinline__ void fwd_w32_body(const FwdM& p, const MaskArgs ma) {
     load_bias(1);
     apply_smod(s_a, tile_of(0));
     if (edge(0)) mask_tile(s_a, tile_of(0) * BN);
-    raise_reference(tile_max(s_a));  // the first reference is the maximum of the first tile
+    raise_reference(tile_max(s_a), w_cur);  // the first reference is the maximum of the first tile
     m_run = m_new;
 #pragma unroll
     for (int j = 0; j < 4; ++j) {  // first half of tile 0
-      stage1(s_a, j);
+      stage1(s_a, j, w_cur);
       stage2(j);
       stage3(j, pk_a, ps_a);
     }
@@ -781,7 +788,7 @@ __device__ __forceinline__ void fwd_w32_body(const FwdM& p, const MaskArgs ma) {
       return u32x4{lo[0], lo[1], hi[0], hi[1]};
     };
     __builtin_amdgcn_sched_barrier(0);
-    stage1(scur, 4);
+    stage1(scur, 4, w_cur);
     __builtin_amdgcn_sched_barrier(0);
     // ---- phase A -------------------------------------------------------------------------------
     // (the scores are on the critical path - probabilities, then the second product wait for them -
@@ -795,7 +802,7 @@ __device__ __forceinline__ void fwd_w32_body(const FwdM& p, const MaskArgs ma) {
       else ring[(ks + AHEAD) & 7] = read_v(ks + AHEAD - KS);
       snext = Mma<T>::run(ring[ks & 7], qf[ks], ks == 0 ? zero16 : snext);
 #pragma unroll
-      for (int hs = ks * STEPS / KS; hs < (ks + 1) * STEPS / KS; ++hs) softmax_slot(scur, 4, hs, pk, ps);
+      for (int hs = ks * STEPS / KS; hs < (ks + 1) * STEPS / KS; ++hs) softmax_slot(scur, 4, hs, pk, ps, w_cur);
       __builtin_amdgcn_sched_barrier(0);
     }
     // ---- check ---------------------------------------------------------------------------------
@@ -806,7 +813,7 @@ __device__ __forceinline__ void fwd_w32_body(const FwdM& p, const MaskArgs ma) {
     bool trig = !(ps <= kTrig);
     if constexpr (MASK) trig |= m_run == -INFINITY;
     if (__builtin_expect(__builtin_amdgcn_ballot_w64(trig) != 0, 0)) {
-      raise_reference(tile_max(scur));
+      raise_reference(tile_max(scur), w_cur);
       if (need_rescale) {
         l_run *= alpha;
 #pragma unroll
@@ -818,7 +825,7 @@ __device__ __forceinline__ void fwd_w32_body(const FwdM& p, const MaskArgs ma) {
       ps = 0.f;
 #pragma unroll
       for (int j = 0; j < 8; ++j) {  // the whole tile again, against the new reference
-        stage1(scur, j);
+        stage1(scur, j, w_cur);
         stage2(j);
         stage3(j, pk, ps);
       }
@@ -857,16 +864,18 @@ __device__ __forceinline__ void fwd_w32_body(const FwdM& p, const MaskArgs ma) {
         apply_bias(snext, true);
         load_bias(t + 2);
         apply_smod(snext, tile_of(t + 1));
-        if (__builtin_expect(edge(t + 1), 0)) mask_tile(snext, tile_of(t + 1) * BN);  // rare
-        stage1(snext, 0);
+        const bool masked = edge(t + 1);
+        if (__builtin_expect(masked, 0)) mask_tile(snext, tile_of(t + 1) * BN);  // rare
+        w_cur = mask_weight(masked);
+        stage1(snext, 0, w_cur);
       }
       // all steps but the last spread over the slots (that one trails the loop)
 #pragma unroll
       for (int hs = (i == 0 ? 0 : max((i * STEPS) / NPV - 1, 0)); hs < max(((i + 1) * STEPS) / NPV - 1, 0); ++hs)
-        softmax_slot(snext, 0, hs, pkn, psn);
+        softmax_slot(snext, 0, hs, pkn, psn, w_cur);
       __builtin_amdgcn_sched_barrier(0);
     }
-    softmax_slot(snext, 0, STEPS - 1, pkn, psn);
+    softmax_slot(snext, 0, STEPS - 1, pkn, psn, w_cur);
   };
   // a wavefront whose rows lie above the causal diagonal of the remaining tiles only feeds LDS
   auto idle_step = [&](int t) {
