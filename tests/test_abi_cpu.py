@@ -207,13 +207,31 @@ def test_entry_points_reject_bad_arguments_without_a_gpu(amd):
     assert lib.mi355_sdpa_bwd_workspace_bytes(None) == 0
 
 
+def _bwd_params(amd, Hq, Hkv, L, S, D):
+    p = amd._lib.BwdParams()
+    for f, h, n in (("grad_out", Hq, L), ("q", Hq, L), ("out", Hq, L), ("grad_q", Hq, L),
+                    ("k", Hkv, S), ("v", Hkv, S), ("grad_k", Hkv, S), ("grad_v", Hkv, S)):
+        setattr(p, f, amd._lib.Tensor4(4096, (C.c_int64 * 4)(1, h, n, D), (C.c_int64 * 4)(h * n * D, n * D, D, 1)))
+    p.lse, p.dtype, p.scale = 4096, amd._lib.BF16, 0.125
+    return p
+
+
+@pytest.mark.parametrize("empty", ["Hq", "Hkv", "L", "S", "D"])
+@pytest.mark.parametrize("dropout", [False, True])
+def test_a_backward_without_elements_is_sized_and_refused(amd, empty, dropout):
+    """The size of the workspace is asked for before the shapes are checked (no division by what is not there)."""
+    p = _bwd_params(amd, **{**dict(Hq=4, Hkv=2, L=64, S=64, D=64), empty: 0})
+    if dropout:
+        p.dropout_p, p.dropout_keep = 0.1, 4096
+    assert amd._lib.load().mi355_sdpa_bwd_workspace_bytes(C.byref(p)) < 1 << 20
+    if empty == "Hkv":
+        assert amd._lib.load().mi355_sdpa_bwd(C.byref(p), None) == amd._lib.ERR_INVALID
+
+
 @pytest.mark.parametrize("Hq,L,S,ld", [(16, 512, 512, 0), (64, 16384, 16384, 0), (32, 32768, 32768, 0), (1, 4096, 100, 1 << 20)])
 def test_every_dropout_call_at_head_dim_64_gets_room_for_its_keep_bits(amd, Hq, L, S, ld):
     """Whatever the matrix-op backward accepts: the kernels that take such a call read the keep-mask as bits."""
-    p, D = amd._lib.BwdParams(), 64
-    for f, n in (("grad_out", L), ("q", L), ("out", L), ("grad_q", L), ("k", S), ("v", S), ("grad_k", S), ("grad_v", S)):
-        setattr(p, f, amd._lib.Tensor4(4096, (C.c_int64 * 4)(1, Hq, n, D), (C.c_int64 * 4)(Hq * n * D, n * D, D, 1)))
-    p.lse, p.dtype, p.scale = 4096, amd._lib.BF16, 0.125
+    p = _bwd_params(amd, Hq, Hq, L, S, 64)
     plain = amd._lib.load().mi355_sdpa_bwd_workspace_bytes(C.byref(p))
     p.dropout_p, p.dropout_keep, p.dropout_keep_ld = 0.1, 4096, ld
     assert amd._lib.load().mi355_sdpa_bwd_workspace_bytes(C.byref(p)) >= plain + Hq * L * -(-S // 128) * 16

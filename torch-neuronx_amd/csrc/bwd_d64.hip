@@ -547,6 +547,7 @@ int launch_t(const BwdM& g, uint32_t* bits, hipStream_t s) {
 }  // namespace
 
 bool bwd_d64_takes(const BwdM& g) {
+  if (g.Hkv < 1) return false;  // (asked for the size of a workspace before anything is checked)
   if (g.d_real > 64 || g.dv_real != g.d_real || g.bias_kind || g.gbias || g.window > 0 || g.sm.any || g.dq_split_tiles) return false;
   // (32-bit byte offsets from the start of a batch, and of a key block's keep bits; the latter are the smaller ones
   // but for heads expanded from one)
