@@ -237,6 +237,21 @@ def test_every_dropout_call_at_head_dim_64_gets_room_for_its_keep_bits(amd, Hq, 
     assert amd._lib.load().mi355_sdpa_bwd_workspace_bytes(C.byref(p)) >= plain + Hq * L * -(-S // 128) * 16
 
 
+@pytest.mark.parametrize("D,ld", [(64, 1 << 26), (128, 1 << 21), (256, 1 << 21)])
+def test_keep_mask_rows_too_far_apart_for_the_matrix_op_kernels(amd, D, ld):
+    """The limits are those of the mask's own pitch, not of S: past them a call is the generic kernels'."""
+    b = _bwd_params(amd, 2, 2, 4096, 100, D)
+    b.dropout_p, b.dropout_keep, b.dropout_keep_ld, b.force_kernel = 0.1, 4096, ld, amd._lib.KERNEL_MFMA
+    b.workspace, b.workspace_bytes = 4096, 1 << 40
+    assert amd._lib.load().mi355_sdpa_bwd(C.byref(b), None) == amd._lib.ERR_UNSUPPORTED
+    assert "keep-mask rows beyond" in amd._lib.last_error()
+    if 32 * ld >= 1 << 31:
+        f = amd._lib.FwdParams(q=b.q, k=b.k, v=b.v, out=b.out, dtype=b.dtype, scale=b.scale)
+        f.dropout_p, f.dropout_keep, f.dropout_keep_ld, f.force_kernel = 0.1, 4096, ld, amd._lib.KERNEL_MFMA
+        assert amd._lib.load().mi355_sdpa_fwd(C.byref(f), None) == amd._lib.ERR_UNSUPPORTED
+        assert "keep-mask rows beyond" in amd._lib.last_error()
+
+
 def test_host_ops_refuse_cpu_tensors(amd):
     q = torch.randn(1, 2, 4, 8)
     with pytest.raises(ValueError):

@@ -606,10 +606,13 @@ bool bwd_mfma_supported(const mi355_sdpa_bwd_params& p, const char** why) {
   }
   if (p.dropout_p > 0.f) {
     // the keep-mask takes a bool bias's way into the kernels (one dword = four keys of a row)
-    const int64_t S = p.k.size[2];
+    const int64_t S = p.k.size[2], ld = p.dropout_keep_ld > 0 ? p.dropout_keep_ld : S;
     if (p.mask.window > 0) return *why = "dropout together with a window functor", false;
-    if (!p.dropout_keep || ((uintptr_t)p.dropout_keep & 3) != 0 || (p.dropout_keep_ld > 0 ? p.dropout_keep_ld : p.k.size[2]) % 4 != 0) return *why = "dropout keep-mask rows do not start on dwords", false;
-    if ((p.q.size[2] + 64) * S + S + 64 >= (1ll << 31)) return *why = "dropout keep-mask rows beyond 32-bit offsets", false;
+    if (!p.dropout_keep || ((uintptr_t)p.dropout_keep & 3) != 0 || ld % 4 != 0) return *why = "dropout keep-mask rows do not start on dwords", false;
+    // (bwd_d64.hip addresses the mask from the 32 rows of a wavefront, the others from a head's first row)
+    const bool near = !wide && E <= 64 && !p.bias.data;
+    if ((p.q.size[2] + 64) * S + S + 64 >= (1ll << 31) || 32 * ld >= (1ll << 31) || (!near && (p.q.size[2] + 64) * ld + S + 64 >= (1ll << 32)))
+      return *why = "dropout keep-mask rows beyond 32-bit offsets", false;
   }
   if (!(p.scale > 0.f)) return *why = "scale <= 0", false;
   if (p.q.size[2] < 1 || p.k.size[2] < 1) return *why = "empty sequence", false;
