@@ -252,6 +252,15 @@ def test_keep_mask_rows_too_far_apart_for_the_matrix_op_kernels(amd, D, ld):
         assert "keep-mask rows beyond" in amd._lib.last_error()
 
 
+@pytest.mark.parametrize("name", ["k", "v", "grad_k", "grad_v"])
+def test_keys_of_a_head_beyond_32_bit_offsets_above_head_dim_128(amd, name):
+    b = _bwd_params(amd, 2, 2, 64, 1 << 18, 256)
+    getattr(b, name).stride[2] = 1 << 13
+    b.force_kernel, b.workspace, b.workspace_bytes = amd._lib.KERNEL_MFMA, 4096, 1 << 40
+    assert amd._lib.load().mi355_sdpa_bwd(C.byref(b), None) == amd._lib.ERR_UNSUPPORTED
+    assert "beyond 32-bit" in amd._lib.last_error()
+
+
 def test_host_ops_refuse_cpu_tensors(amd):
     q = torch.randn(1, 2, 4, 8)
     with pytest.raises(ValueError):

@@ -625,6 +625,10 @@ bool bwd_mfma_supported(const mi355_sdpa_bwd_params& p, const char** why) {
       if (t->size[i] > 1 && (t->stride[i] % 8) != 0) return *why = "stride not a multiple of 8 elements", false;
   }
   if ((int64_t)p.q.size[0] * p.q.size[1] * ((p.q.size[2] + 127) / 128) > 0x7fffffff) return *why = "too many tiles", false;
+  // (their K, V, dK and dV of one head are addressed with unsigned 32-bit byte offsets)
+  if (wide)
+    for (const mi355_sdpa_tensor* t : {&p.k, &p.v, &p.grad_k, &p.grad_v})
+      if (t->size[2] > 1 && (t->size[2] + 32) * t->stride[2] * 2 + 512 >= (1ll << 32)) return *why = "keys of a head beyond 32-bit offsets", false;
   if (!wide && (p.bias.data || p.kv_lens || padded || p.mask.window > 0 || p.dropout_p > 0.f || smod)) {
     BwdM g;
     fill(g, p);
