@@ -54,3 +54,17 @@ def test_block_and_outputs_of_a_call(amd, gpu_device, layout):
     for g, x, f in ((dq, q, b.grad_q), (dk, k, b.grad_k), (dv, v, b.grad_v)):
         assert g.shape == x.shape and g.transpose(1, 2).is_contiguous() and f.data == g.data_ptr() and tuple(f.stride) == g.stride()
     assert hold[-1].dtype == torch.float32 and b.lse == hold[-1].data_ptr()  # (a float64 log-sum-exp is converted)
+
+
+@pytest.mark.gpu
+def test_the_debug_mask_of_a_call_is_its_own(amd, gpu_device):
+    """The flash operator's (empty) debug mask: changed by one caller, or made under inference mode, it is no other
+    call's."""
+    q = torch.randn(1, 2, 8, 64, device=gpu_device, dtype=torch.bfloat16)
+    call = lambda: torch.ops.aten._scaled_dot_product_flash_attention(q, q, q)[8]
+    with torch.inference_mode():
+        first = call()
+    second = call()
+    assert first.is_inference() and not second.is_inference()
+    second.resize_(3)
+    assert call().shape == (0,)

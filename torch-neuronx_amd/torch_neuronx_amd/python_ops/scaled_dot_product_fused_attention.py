@@ -49,19 +49,6 @@ def _empty_rng(device):
     return pair
 
 
-_debug_masks = {}
-
-
-def _no_debug_mask(query):
-    # upstream's debug mask when none is asked for: an empty tensor of the query's dtype, never written,
-    # so one per device and dtype serves every call
-    key = (query.device, query.dtype)
-    mask = _debug_masks.get(key)
-    if mask is None:
-        mask = _debug_masks[key] = torch.empty((0,), dtype=query.dtype, device=query.device)
-    return mask
-
-
 def _dropout_keep(query, S, dropout_p):
     """Keep-mask drawn on the device; it travels to the backward in the philox_seed slot, the
     way the reference carries its mask (decompositions.py:2354-2356)."""
@@ -285,7 +272,8 @@ def scaled_dot_product_flash_attention(
     the (empty) debug mask as upstream's operator returns them."""
     out, lse, seed, offset = _forward(query, key, value, None, dropout_p, is_causal, return_debug_mask, scale,
                                       upstream="flash")
-    return out, lse, None, None, query.shape[2], key.shape[2], seed, offset, _no_debug_mask(query)
+    return (out, lse, None, None, query.shape[2], key.shape[2], seed, offset,
+            torch.empty((0,), dtype=query.dtype, device=query.device))
 
 
 def scaled_dot_product_flash_attention_backward(
