@@ -26,6 +26,16 @@ def test_refuses_what_is_no_gpu_tensor(amd):
         amd.decode_fp8kv(t, t.to(torch.float8_e4m3fn), t.to(torch.float8_e4m3fn), t, t)
 
 
+def test_placeholders_made_under_inference_mode_serve_training(amd, monkeypatch):
+    from torch_neuronx_amd.python_ops import scaled_dot_product_fused_attention as ops
+
+    monkeypatch.setattr(ops, "_rng_placeholders", {})
+    monkeypatch.setattr(ops, "_scalar_rng_pair", None)
+    with torch.inference_mode():
+        pairs = ops._empty_rng(torch.device("cpu")) + ops._scalar_rng()
+    assert not any(t.is_inference() for t in pairs)
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("layout", ["plain", "seq_major_view", "expanded_kv", "strided_head_dim", "one_row"])
 def test_block_and_outputs_of_a_call(amd, gpu_device, layout):

@@ -43,8 +43,9 @@ def _empty_rng(device):
     # never written, so one pair per device serves every call
     pair = _rng_placeholders.get(device)
     if pair is None:
-        pair = (torch.empty((0,), dtype=torch.int32, device=device),
-                torch.empty((0,), dtype=torch.int32, device=device))
+        with torch.inference_mode(False):  # (an inference tensor could not be saved for a later backward)
+            pair = (torch.empty((0,), dtype=torch.int32, device=device),
+                    torch.empty((0,), dtype=torch.int32, device=device))
         _rng_placeholders[device] = pair
     return pair
 
@@ -71,7 +72,8 @@ def _scalar_rng():
     is applied."""
     global _scalar_rng_pair
     if _scalar_rng_pair is None:
-        _scalar_rng_pair = (torch.zeros((), dtype=torch.int64), torch.zeros((), dtype=torch.int64))
+        with torch.inference_mode(False):  # (see _empty_rng)
+            _scalar_rng_pair = (torch.zeros((), dtype=torch.int64), torch.zeros((), dtype=torch.int64))
     return _scalar_rng_pair
 
 
