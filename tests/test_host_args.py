@@ -26,6 +26,25 @@ def test_refuses_what_is_no_gpu_tensor(amd):
         amd.decode_fp8kv(t, t.to(torch.float8_e4m3fn), t.to(torch.float8_e4m3fn), t, t)
 
 
+@pytest.mark.parametrize("block,error", [(0, ValueError), (None, TypeError), ("0", TypeError), (-1 << 80, OverflowError)])
+def test_refuses_what_is_no_block(amd, block, error):
+    t, host = torch.zeros(1, 1, 2, 8), amd._lib.host()
+    with pytest.raises(error):
+        host.forward(block, t, t, t, None, True, False, 1.0, 0, False)
+    with pytest.raises(error):
+        host.backward(block, t, t, t, t, t, t, None, None, False, 1.0, 0, False)
+    with pytest.raises(error):
+        host.decode(block, t, t, t, t, t, None, None, None, True, 1.0, 0)
+
+
+def test_refuses_a_scale_that_is_no_number(amd):
+    p, t = amd._lib.FwdParams(), torch.zeros(1, 1, 2, 8)
+    with pytest.raises(TypeError, match="real number"):
+        amd._lib.host().forward(C.addressof(p), t, t, t, None, True, False, "1", 0, False)
+    with pytest.raises(TypeError, match="real number"):
+        amd._lib.host().validate(t, t, t, False, "0", False)
+
+
 def test_placeholders_made_under_inference_mode_serve_training(amd, monkeypatch):
     from torch_neuronx_amd.python_ops import scaled_dot_product_fused_attention as ops
 

@@ -33,6 +33,29 @@ const at::Tensor& tensor(PyObject* o) {
   TORCH_CHECK_TYPE(THPVariable_Check(o), "expected a tensor, got ", Py_TYPE(o)->tp_name);
   return THPVariable_Unpack(o);
 }
+// the caller's parameter block (never written through before it is known to be one)
+template <typename P>
+P* block(PyObject* o) {
+  void* const p = PyLong_AsVoidPtr(o);
+  if (PyErr_Occurred()) throw python_error();
+  TORCH_CHECK_VALUE(p, "null parameter block");
+  return (P*)p;
+}
+float real(PyObject* o) {
+  const double x = PyFloat_AsDouble(o);
+  if (PyErr_Occurred()) throw python_error();
+  return (float)x;
+}
+int32_t whole(PyObject* o) {
+  const long x = PyLong_AsLong(o);
+  if (PyErr_Occurred()) throw python_error();
+  return (int32_t)x;
+}
+bool truth(PyObject* o) {
+  const int x = PyObject_IsTrue(o);
+  if (x < 0) throw python_error();
+  return x;
+}
 at::Tensor optional(PyObject* o) { return o == Py_None ? at::Tensor() : tensor(o); }
 
 void on_gpu(const at::Tensor& t, const char* name) {
@@ -88,23 +111,23 @@ void arity(Py_ssize_t got, Py_ssize_t want, const char* name) {
 PyObject* forward(PyObject*, PyObject* const* a, Py_ssize_t n) {
   HANDLE_TH_ERRORS
   arity(n, 10, "forward");
-  auto* p = (mi355_sdpa_fwd_params*)PyLong_AsVoidPtr(a[0]);
-  const at::Tensor &query = tensor(a[1]), &key = tensor(a[2]), &value = tensor(a[3]);
+  auto* p = block<mi355_sdpa_fwd_params>(a[0]);
+  const at::Tensor &query = tensor(a[1]), &key = tensor(a[2]), &value = tensor(a[3]), bias = optional(a[4]);
+  const bool need_lse = truth(a[5]), is_causal = truth(a[6]), seq_major = truth(a[9]);
+  const float scale = real(a[7]);
+  const int32_t force_kernel = whole(a[8]);
   on_gpu(query, "query"), on_gpu(key, "key"), on_gpu(value, "value");
   std::vector<at::Tensor> hold;
-  const at::Tensor q = unit_last(query, hold), k = unit_last(key, hold), v = unit_last(value, hold), bias = optional(a[4]);
+  const at::Tensor q = unit_last(query, hold), k = unit_last(key, hold), v = unit_last(value, hold);
   const int64_t B = q.size(0), H = q.size(1), L = q.size(2);
-  const at::Tensor out = like(query, {B, H, L, v.size(3)}, PyObject_IsTrue(a[9]));
+  const at::Tensor out = like(query, {B, H, L, v.size(3)}, seq_major);
   at::Tensor lse;
-  if (PyObject_IsTrue(a[5])) lse = at::empty({B, H, L}, query.options().dtype(at::kFloat));
+  if (need_lse) lse = at::empty({B, H, L}, query.options().dtype(at::kFloat));
   put(p->q, q), put(p->k, k), put(p->v, v), put(p->out, out), put(p->bias, bias);
   p->lse = lse.defined() ? (float*)lse.mutable_data_ptr() : nullptr;
   p->bias_dtype = bias.defined() ? dtype_id(bias.scalar_type()) : 0;
   p->dtype = dtype_id(query.scalar_type());
-  p->is_causal = PyObject_IsTrue(a[6]);
-  p->scale = (float)PyFloat_AsDouble(a[7]);
-  p->force_kernel = (int32_t)PyLong_AsLong(a[8]);
-  if (PyErr_Occurred()) return nullptr;
+  p->is_causal = is_causal, p->scale = scale, p->force_kernel = force_kernel;
   return result({out, lse}, hold);
   END_HANDLE_TH_ERRORS
 }
@@ -114,15 +137,18 @@ PyObject* forward(PyObject*, PyObject* const* a, Py_ssize_t n) {
 PyObject* backward(PyObject*, PyObject* const* a, Py_ssize_t n) {
   HANDLE_TH_ERRORS
   arity(n, 13, "backward");
-  auto* p = (mi355_sdpa_bwd_params*)PyLong_AsVoidPtr(a[0]);
-  const at::Tensor &grad_out = tensor(a[1]), &query = tensor(a[2]), &key = tensor(a[3]), &value = tensor(a[4]), &out = tensor(a[5]);
+  auto* p = block<mi355_sdpa_bwd_params>(a[0]);
+  const at::Tensor &grad_out = tensor(a[1]), &query = tensor(a[2]), &key = tensor(a[3]), &value = tensor(a[4]), &out = tensor(a[5]),
+                   bias = optional(a[7]), dbias = optional(a[8]);
+  at::Tensor lse = tensor(a[6]);
+  const bool is_causal = truth(a[9]), seq_major = truth(a[12]);
+  const float scale = real(a[10]);
+  const int32_t force_kernel = whole(a[11]);
   on_gpu(grad_out, "grad_out"), on_gpu(query, "query"), on_gpu(key, "key"), on_gpu(value, "value");
   std::vector<at::Tensor> hold;
   const at::Tensor go = unit_last(grad_out, hold), q = unit_last(query, hold), k = unit_last(key, hold), v = unit_last(value, hold),
-                   o = unit_last(out, hold), bias = optional(a[7]), dbias = optional(a[8]);
-  at::Tensor lse = tensor(a[6]);
+                   o = unit_last(out, hold);
   if (lse.scalar_type() != at::kFloat || !lse.is_contiguous()) hold.push_back(lse = lse.to(at::kFloat).contiguous());
-  const bool seq_major = PyObject_IsTrue(a[12]);
   const int64_t B = q.size(0), Hq = q.size(1), L = q.size(2), E = q.size(3), Hkv = k.size(1), S = k.size(2), Dv = v.size(3);
   const at::Tensor dq = like(query, {B, Hq, L, E}, seq_major), dk = like(key, {B, Hkv, S, E}, seq_major), dv = like(value, {B, Hkv, S, Dv}, seq_major);
   put(p->grad_out, go), put(p->q, q), put(p->k, k), put(p->v, v), put(p->out, o);
@@ -130,10 +156,7 @@ PyObject* backward(PyObject*, PyObject* const* a, Py_ssize_t n) {
   p->lse = (const float*)lse.const_data_ptr();
   p->bias_dtype = bias.defined() ? dtype_id(bias.scalar_type()) : 0;
   p->dtype = dtype_id(query.scalar_type());
-  p->is_causal = PyObject_IsTrue(a[9]);
-  p->scale = (float)PyFloat_AsDouble(a[10]);
-  p->force_kernel = (int32_t)PyLong_AsLong(a[11]);
-  if (PyErr_Occurred()) return nullptr;
+  p->is_causal = is_causal, p->scale = scale, p->force_kernel = force_kernel;
   return result({dq, dk, dv}, hold);
   END_HANDLE_TH_ERRORS
 }
@@ -142,33 +165,34 @@ PyObject* backward(PyObject*, PyObject* const* a, Py_ssize_t n) {
 PyObject* decode(PyObject*, PyObject* const* a, Py_ssize_t n) {
   HANDLE_TH_ERRORS
   arity(n, 12, "decode");
-  auto* p = (mi355_sdpa_decode_params*)PyLong_AsVoidPtr(a[0]);
+  auto* p = block<mi355_sdpa_decode_params>(a[0]);
   const at::Tensor &query = tensor(a[1]), &key = tensor(a[2]), &value = tensor(a[3]);
+  const at::Tensor k_scale = optional(a[4]), v_scale = optional(a[5]), kv_lens = optional(a[6]);
+  at::Tensor out = optional(a[7]), lse = optional(a[8]);
+  const bool need_lse = truth(a[9]);
+  const float scale = real(a[10]);
+  const int32_t num_splits = whole(a[11]);
   on_gpu(query, "query"), on_gpu(key, "key"), on_gpu(value, "value");
   std::vector<at::Tensor> hold;
   const at::Tensor q = unit_last(query, hold), k = unit_last(key, hold), v = unit_last(value, hold);
-  auto vec = [&](PyObject* o, at::ScalarType dt) -> const void* {  // contiguous, on the query's device
-    at::Tensor t = optional(o);
+  auto vec = [&](at::Tensor t, at::ScalarType dt) -> const void* {  // contiguous, on the query's device
     if (!t.defined()) return nullptr;
     if (t.scalar_type() != dt || !t.is_contiguous() || t.device() != query.device()) hold.push_back(t = t.to(query.device(), dt).contiguous());
     return t.const_data_ptr();
   };
   const int64_t B = q.size(0), H = q.size(1), L = q.size(2), D = v.size(3);
-  at::Tensor out = optional(a[7]), lse = optional(a[8]);
   if (!out.defined()) out = at::empty({B, H, L, D}, query.options());
-  if (!lse.defined() && PyObject_IsTrue(a[9])) lse = at::empty({B, H, L}, query.options().dtype(at::kFloat));
+  if (!lse.defined() && need_lse) lse = at::empty({B, H, L}, query.options().dtype(at::kFloat));
   TORCH_CHECK_VALUE(out.sizes() == at::IntArrayRef({B, H, L, D}) && out.scalar_type() == query.scalar_type(),
                     "decode_fp8kv: out must have shape (B, Hq, Lq, D) and the query's dtype");
   TORCH_CHECK_VALUE(!lse.defined() || (lse.sizes() == at::IntArrayRef({B, H, L}) && lse.scalar_type() == at::kFloat && lse.is_contiguous()),
                     "decode_fp8kv: lse must be a contiguous float32 (B, Hq, Lq) tensor");
   put(p->q, q), put(p->k, k), put(p->v, v), put(p->out, out);
-  p->k_scale = (const float*)vec(a[4], at::kFloat), p->v_scale = (const float*)vec(a[5], at::kFloat);
-  p->kv_lens = (const int32_t*)vec(a[6], at::kInt);
+  p->k_scale = (const float*)vec(k_scale, at::kFloat), p->v_scale = (const float*)vec(v_scale, at::kFloat);
+  p->kv_lens = (const int32_t*)vec(kv_lens, at::kInt);
   p->lse = lse.defined() ? (float*)lse.mutable_data_ptr() : nullptr;
   p->q_dtype = dtype_id(query.scalar_type());
-  p->scale = (float)PyFloat_AsDouble(a[10]);
-  p->num_splits = (int32_t)PyLong_AsLong(a[11]);
-  if (PyErr_Occurred()) return nullptr;
+  p->scale = scale, p->num_splits = num_splits;
   return result({out, lse}, hold);
   END_HANDLE_TH_ERRORS
 }
@@ -188,10 +212,7 @@ PyObject* validate(PyObject*, PyObject* const* a, Py_ssize_t n) {
   fill(k, d.k_dim, d.k_size, d.k_dtype, d.k_last_stride);
   fill(v, d.v_dim, d.v_size, d.v_dtype, d.v_last_stride);
   d.on_device = q.is_cuda() && k.is_cuda() && v.is_cuda();
-  d.has_attn_bias = PyObject_IsTrue(a[3]);
-  d.dropout_p = (float)PyFloat_AsDouble(a[4]);
-  d.is_causal = PyObject_IsTrue(a[5]);
-  if (PyErr_Occurred()) return nullptr;
+  d.has_attn_bias = truth(a[3]), d.dropout_p = real(a[4]), d.is_causal = truth(a[5]);
   char msg[512];
   if (mi355_sdpa_validate(&d, msg, sizeof(msg)) != MI355_SDPA_OK) return PyErr_SetString(PyExc_RuntimeError, msg), nullptr;
   Py_RETURN_NONE;
