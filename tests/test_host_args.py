@@ -45,6 +45,13 @@ def test_refuses_a_scale_that_is_no_number(amd):
         amd._lib.host().validate(t, t, t, False, "0", False)
 
 
+def test_takes_whole_numbers_of_any_type(amd):
+    p, t = amd._lib.FwdParams(), torch.zeros(1, 1, 2, 8)
+    for n in (2, 2.0, True, torch.tensor(2)):
+        with pytest.raises(ValueError, match="GPU tensor"):  # (past the conversions)
+            amd._lib.host().forward(C.addressof(p), t, t, t, None, True, False, torch.tensor(1.0), n, False)
+
+
 def test_placeholders_made_under_inference_mode_serve_training(amd, monkeypatch):
     from torch_neuronx_amd.python_ops import scaled_dot_product_fused_attention as ops
 

@@ -46,8 +46,11 @@ float real(PyObject* o) {
   if (PyErr_Occurred()) throw python_error();
   return (float)x;
 }
-int32_t whole(PyObject* o) {
-  const long x = PyLong_AsLong(o);
+int32_t whole(PyObject* o) {  // (whatever int() takes)
+  PyObject* const i = PyNumber_Long(o);
+  if (!i) throw python_error();
+  const long x = PyLong_AsLong(i);
+  Py_DECREF(i);
   if (PyErr_Occurred()) throw python_error();
   return (int32_t)x;
 }
