@@ -104,3 +104,16 @@ def test_the_debug_mask_of_a_call_is_its_own(amd, gpu_device):
     assert first.is_inference() and not second.is_inference()
     second.resize_(3)
     assert call().shape == (0,)
+
+
+@pytest.mark.gpu
+def test_a_lazily_cloned_output_is_written_alone(amd, gpu_device):
+    """torch._lazy_clone shares memory until one side is written: a call's output is written."""
+    q = torch.randn(2, 4, 1, 64, device=gpu_device, dtype=torch.bfloat16)
+    kv = torch.randn(2, 2, 40, 64, device=gpu_device).to(torch.float8_e4m3fn)
+    one = torch.ones(2, device=gpu_device)
+    want, _ = amd.decode_fp8kv(q, kv, kv, one, one)
+    base = torch.zeros_like(want)
+    got, _ = amd.decode_fp8kv(q, kv, kv, one, one, out=torch._lazy_clone(base))
+    same, untouched = torch.equal(got, want), not bool(base.any())
+    assert same and untouched

@@ -74,10 +74,11 @@ at::Tensor unit_last(const at::Tensor& t, std::vector<at::Tensor>& hold) {
   return hold.back();
 }
 
-void put(mi355_sdpa_tensor& d, const at::Tensor& t) {
+// (written: a tensor that the call writes, whose memory must be nobody else's, a lazy clone's for instance)
+void put(mi355_sdpa_tensor& d, const at::Tensor& t, bool written = false) {
   if (!t.defined()) return;
   four_dims(t);
-  d.data = const_cast<void*>(t.const_data_ptr());
+  d.data = written ? t.mutable_data_ptr() : const_cast<void*>(t.const_data_ptr());
   for (int i = 0; i < 4; ++i) d.size[i] = t.sizes()[i], d.stride[i] = t.strides()[i];
 }
 
@@ -126,7 +127,7 @@ PyObject* forward(PyObject*, PyObject* const* a, Py_ssize_t n) {
   const at::Tensor out = like(query, {B, H, L, v.size(3)}, seq_major);
   at::Tensor lse;
   if (need_lse) lse = at::empty({B, H, L}, query.options().dtype(at::kFloat));
-  put(p->q, q), put(p->k, k), put(p->v, v), put(p->out, out), put(p->bias, bias);
+  put(p->q, q), put(p->k, k), put(p->v, v), put(p->out, out, true), put(p->bias, bias);
   p->lse = lse.defined() ? (float*)lse.mutable_data_ptr() : nullptr;
   p->bias_dtype = bias.defined() ? dtype_id(bias.scalar_type()) : 0;
   p->dtype = dtype_id(query.scalar_type());
@@ -155,7 +156,7 @@ PyObject* backward(PyObject*, PyObject* const* a, Py_ssize_t n) {
   const int64_t B = q.size(0), Hq = q.size(1), L = q.size(2), E = q.size(3), Hkv = k.size(1), S = k.size(2), Dv = v.size(3);
   const at::Tensor dq = like(query, {B, Hq, L, E}, seq_major), dk = like(key, {B, Hkv, S, E}, seq_major), dv = like(value, {B, Hkv, S, Dv}, seq_major);
   put(p->grad_out, go), put(p->q, q), put(p->k, k), put(p->v, v), put(p->out, o);
-  put(p->grad_q, dq), put(p->grad_k, dk), put(p->grad_v, dv), put(p->bias, bias), put(p->grad_bias, dbias);
+  put(p->grad_q, dq, true), put(p->grad_k, dk, true), put(p->grad_v, dv, true), put(p->bias, bias), put(p->grad_bias, dbias, true);
   p->lse = (const float*)lse.const_data_ptr();
   p->bias_dtype = bias.defined() ? dtype_id(bias.scalar_type()) : 0;
   p->dtype = dtype_id(query.scalar_type());
@@ -190,7 +191,7 @@ PyObject* decode(PyObject*, PyObject* const* a, Py_ssize_t n) {
                     "decode_fp8kv: out must have shape (B, Hq, Lq, D) and the query's dtype");
   TORCH_CHECK_VALUE(!lse.defined() || (lse.sizes() == at::IntArrayRef({B, H, L}) && lse.scalar_type() == at::kFloat && lse.is_contiguous()),
                     "decode_fp8kv: lse must be a contiguous float32 (B, Hq, Lq) tensor");
-  put(p->q, q), put(p->k, k), put(p->v, v), put(p->out, out);
+  put(p->q, q), put(p->k, k), put(p->v, v), put(p->out, out, true);
   p->k_scale = (const float*)vec(k_scale, at::kFloat), p->v_scale = (const float*)vec(v_scale, at::kFloat);
   p->kv_lens = (const int32_t*)vec(kv_lens, at::kInt);
   p->lse = lse.defined() ? (float*)lse.mutable_data_ptr() : nullptr;
