@@ -1,6 +1,9 @@
 """The native argument marshalling: what it refuses, and the block it writes against the tensors it was given."""
 
 import ctypes as C
+import sys
+import threading
+import time
 
 import pytest
 import torch
@@ -117,3 +120,26 @@ def test_a_lazily_cloned_output_is_written_alone(amd, gpu_device):
     got, _ = amd.decode_fp8kv(q, kv, kv, one, one, out=torch._lazy_clone(base))
     same, untouched = torch.equal(got, want), not bool(base.any())
     assert same and untouched
+
+
+@pytest.mark.gpu
+def test_other_threads_run_while_a_call_allocates(amd, gpu_device):
+    """A thread that waits for the interpreter gets it while a call's outputs are allocated (which waits for the
+    GPU where memory is short).  No thread is made to give it up by time here, and the outputs are kept (freeing a
+    tensor lets others in), so only the allocation can."""
+    q = torch.randn(1, 2, 64, 64, device=gpu_device, dtype=torch.bfloat16)
+    p, host, go, ran, kept = amd._lib.FwdParams(), amd._lib.host(), threading.Event(), [], []
+    thread = threading.Thread(target=lambda: (go.wait(), ran.append(True)))
+    interval = sys.getswitchinterval()
+    sys.setswitchinterval(1000.0)
+    try:
+        thread.start()
+        go.set()
+        end = time.monotonic() + 3.0
+        while not ran and time.monotonic() < end and len(kept) < 20000:
+            kept.append(host.forward(C.addressof(p), q, q, q, None, True, False, 1.0, 0, False))
+        in_time = bool(ran)
+    finally:
+        sys.setswitchinterval(interval)
+        thread.join()
+    assert in_time

@@ -59,6 +59,12 @@ bool truth(PyObject* o) {
   if (x < 0) throw python_error();
   return x;
 }
+// Other Python threads run while this lives: what allocates or copies may wait for the GPU (an allocator short of
+// memory does).  The caller's tensors are held by value then, whatever those threads do to their Python objects.
+struct Unlocked {
+  PyThreadState* const state = PyEval_SaveThread();
+  ~Unlocked() { PyEval_RestoreThread(state); }
+};
 at::Tensor optional(PyObject* o) { return o == Py_None ? at::Tensor() : tensor(o); }
 
 void on_gpu(const at::Tensor& t, const char* name) {
@@ -116,18 +122,21 @@ PyObject* forward(PyObject*, PyObject* const* a, Py_ssize_t n) {
   HANDLE_TH_ERRORS
   arity(n, 10, "forward");
   auto* p = block<mi355_sdpa_fwd_params>(a[0]);
-  const at::Tensor &query = tensor(a[1]), &key = tensor(a[2]), &value = tensor(a[3]), bias = optional(a[4]);
+  const at::Tensor query = tensor(a[1]), key = tensor(a[2]), value = tensor(a[3]), bias = optional(a[4]);
   const bool need_lse = truth(a[5]), is_causal = truth(a[6]), seq_major = truth(a[9]);
   const float scale = real(a[7]);
   const int32_t force_kernel = whole(a[8]);
   on_gpu(query, "query"), on_gpu(key, "key"), on_gpu(value, "value");
   std::vector<at::Tensor> hold;
-  const at::Tensor q = unit_last(query, hold), k = unit_last(key, hold), v = unit_last(value, hold);
-  const int64_t B = q.size(0), H = q.size(1), L = q.size(2);
-  const at::Tensor out = like(query, {B, H, L, v.size(3)}, seq_major);
-  at::Tensor lse;
-  if (need_lse) lse = at::empty({B, H, L}, query.options().dtype(at::kFloat));
-  put(p->q, q), put(p->k, k), put(p->v, v), put(p->out, out, true), put(p->bias, bias);
+  at::Tensor out, lse;
+  {
+    const Unlocked unlocked;
+    const at::Tensor q = unit_last(query, hold), k = unit_last(key, hold), v = unit_last(value, hold);
+    const int64_t B = q.size(0), H = q.size(1), L = q.size(2);
+    out = like(query, {B, H, L, v.size(3)}, seq_major);
+    if (need_lse) lse = at::empty({B, H, L}, query.options().dtype(at::kFloat));
+    put(p->q, q), put(p->k, k), put(p->v, v), put(p->out, out, true), put(p->bias, bias);
+  }
   p->lse = lse.defined() ? (float*)lse.mutable_data_ptr() : nullptr;
   p->bias_dtype = bias.defined() ? dtype_id(bias.scalar_type()) : 0;
   p->dtype = dtype_id(query.scalar_type());
@@ -142,7 +151,7 @@ PyObject* backward(PyObject*, PyObject* const* a, Py_ssize_t n) {
   HANDLE_TH_ERRORS
   arity(n, 13, "backward");
   auto* p = block<mi355_sdpa_bwd_params>(a[0]);
-  const at::Tensor &grad_out = tensor(a[1]), &query = tensor(a[2]), &key = tensor(a[3]), &value = tensor(a[4]), &out = tensor(a[5]),
+  const at::Tensor grad_out = tensor(a[1]), query = tensor(a[2]), key = tensor(a[3]), value = tensor(a[4]), out = tensor(a[5]),
                    bias = optional(a[7]), dbias = optional(a[8]);
   at::Tensor lse = tensor(a[6]);
   const bool is_causal = truth(a[9]), seq_major = truth(a[12]);
@@ -150,13 +159,17 @@ PyObject* backward(PyObject*, PyObject* const* a, Py_ssize_t n) {
   const int32_t force_kernel = whole(a[11]);
   on_gpu(grad_out, "grad_out"), on_gpu(query, "query"), on_gpu(key, "key"), on_gpu(value, "value");
   std::vector<at::Tensor> hold;
-  const at::Tensor go = unit_last(grad_out, hold), q = unit_last(query, hold), k = unit_last(key, hold), v = unit_last(value, hold),
-                   o = unit_last(out, hold);
-  if (lse.scalar_type() != at::kFloat || !lse.is_contiguous()) hold.push_back(lse = lse.to(at::kFloat).contiguous());
-  const int64_t B = q.size(0), Hq = q.size(1), L = q.size(2), E = q.size(3), Hkv = k.size(1), S = k.size(2), Dv = v.size(3);
-  const at::Tensor dq = like(query, {B, Hq, L, E}, seq_major), dk = like(key, {B, Hkv, S, E}, seq_major), dv = like(value, {B, Hkv, S, Dv}, seq_major);
-  put(p->grad_out, go), put(p->q, q), put(p->k, k), put(p->v, v), put(p->out, o);
-  put(p->grad_q, dq, true), put(p->grad_k, dk, true), put(p->grad_v, dv, true), put(p->bias, bias), put(p->grad_bias, dbias, true);
+  at::Tensor dq, dk, dv;
+  {
+    const Unlocked unlocked;
+    const at::Tensor go = unit_last(grad_out, hold), q = unit_last(query, hold), k = unit_last(key, hold), v = unit_last(value, hold),
+                     o = unit_last(out, hold);
+    if (lse.scalar_type() != at::kFloat || !lse.is_contiguous()) hold.push_back(lse = lse.to(at::kFloat).contiguous());
+    const int64_t B = q.size(0), Hq = q.size(1), L = q.size(2), E = q.size(3), Hkv = k.size(1), S = k.size(2), Dv = v.size(3);
+    dq = like(query, {B, Hq, L, E}, seq_major), dk = like(key, {B, Hkv, S, E}, seq_major), dv = like(value, {B, Hkv, S, Dv}, seq_major);
+    put(p->grad_out, go), put(p->q, q), put(p->k, k), put(p->v, v), put(p->out, o);
+    put(p->grad_q, dq, true), put(p->grad_k, dk, true), put(p->grad_v, dv, true), put(p->bias, bias), put(p->grad_bias, dbias, true);
+  }
   p->lse = (const float*)lse.const_data_ptr();
   p->bias_dtype = bias.defined() ? dtype_id(bias.scalar_type()) : 0;
   p->dtype = dtype_id(query.scalar_type());
@@ -170,7 +183,7 @@ PyObject* decode(PyObject*, PyObject* const* a, Py_ssize_t n) {
   HANDLE_TH_ERRORS
   arity(n, 12, "decode");
   auto* p = block<mi355_sdpa_decode_params>(a[0]);
-  const at::Tensor &query = tensor(a[1]), &key = tensor(a[2]), &value = tensor(a[3]);
+  const at::Tensor query = tensor(a[1]), key = tensor(a[2]), value = tensor(a[3]);
   const at::Tensor k_scale = optional(a[4]), v_scale = optional(a[5]), kv_lens = optional(a[6]);
   at::Tensor out = optional(a[7]), lse = optional(a[8]);
   const bool need_lse = truth(a[9]);
@@ -178,22 +191,25 @@ PyObject* decode(PyObject*, PyObject* const* a, Py_ssize_t n) {
   const int32_t num_splits = whole(a[11]);
   on_gpu(query, "query"), on_gpu(key, "key"), on_gpu(value, "value");
   std::vector<at::Tensor> hold;
-  const at::Tensor q = unit_last(query, hold), k = unit_last(key, hold), v = unit_last(value, hold);
-  auto vec = [&](at::Tensor t, at::ScalarType dt) -> const void* {  // contiguous, on the query's device
-    if (!t.defined()) return nullptr;
-    if (t.scalar_type() != dt || !t.is_contiguous() || t.device() != query.device()) hold.push_back(t = t.to(query.device(), dt).contiguous());
-    return t.const_data_ptr();
-  };
-  const int64_t B = q.size(0), H = q.size(1), L = q.size(2), D = v.size(3);
-  if (!out.defined()) out = at::empty({B, H, L, D}, query.options());
-  if (!lse.defined() && need_lse) lse = at::empty({B, H, L}, query.options().dtype(at::kFloat));
-  TORCH_CHECK_VALUE(out.sizes() == at::IntArrayRef({B, H, L, D}) && out.scalar_type() == query.scalar_type(),
-                    "decode_fp8kv: out must have shape (B, Hq, Lq, D) and the query's dtype");
-  TORCH_CHECK_VALUE(!lse.defined() || (lse.sizes() == at::IntArrayRef({B, H, L}) && lse.scalar_type() == at::kFloat && lse.is_contiguous()),
-                    "decode_fp8kv: lse must be a contiguous float32 (B, Hq, Lq) tensor");
-  put(p->q, q), put(p->k, k), put(p->v, v), put(p->out, out, true);
-  p->k_scale = (const float*)vec(k_scale, at::kFloat), p->v_scale = (const float*)vec(v_scale, at::kFloat);
-  p->kv_lens = (const int32_t*)vec(kv_lens, at::kInt);
+  {
+    const Unlocked unlocked;
+    const at::Tensor q = unit_last(query, hold), k = unit_last(key, hold), v = unit_last(value, hold);
+    auto vec = [&](at::Tensor t, at::ScalarType dt) -> const void* {  // contiguous, on the query's device
+      if (!t.defined()) return nullptr;
+      if (t.scalar_type() != dt || !t.is_contiguous() || t.device() != query.device()) hold.push_back(t = t.to(query.device(), dt).contiguous());
+      return t.const_data_ptr();
+    };
+    const int64_t B = q.size(0), H = q.size(1), L = q.size(2), D = v.size(3);
+    if (!out.defined()) out = at::empty({B, H, L, D}, query.options());
+    if (!lse.defined() && need_lse) lse = at::empty({B, H, L}, query.options().dtype(at::kFloat));
+    TORCH_CHECK_VALUE(out.sizes() == at::IntArrayRef({B, H, L, D}) && out.scalar_type() == query.scalar_type(),
+                      "decode_fp8kv: out must have shape (B, Hq, Lq, D) and the query's dtype");
+    TORCH_CHECK_VALUE(!lse.defined() || (lse.sizes() == at::IntArrayRef({B, H, L}) && lse.scalar_type() == at::kFloat && lse.is_contiguous()),
+                      "decode_fp8kv: lse must be a contiguous float32 (B, Hq, Lq) tensor");
+    put(p->q, q), put(p->k, k), put(p->v, v), put(p->out, out, true);
+    p->k_scale = (const float*)vec(k_scale, at::kFloat), p->v_scale = (const float*)vec(v_scale, at::kFloat);
+    p->kv_lens = (const int32_t*)vec(kv_lens, at::kInt);
+  }
   p->lse = lse.defined() ? (float*)lse.mutable_data_ptr() : nullptr;
   p->q_dtype = dtype_id(query.scalar_type());
   p->scale = scale, p->num_splits = num_splits;
