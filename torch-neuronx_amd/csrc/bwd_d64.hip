@@ -1,5 +1,6 @@
 // Flash-attention backward for gfx950 at head dims up to 64, bf16/f16: plain and causal calls, per-batch
-// key counts, dropout.  (Calls with a bias, a window or a score functor: bwd_dq_w32.hip, bwd_dkdv_w32.hip.)
+// key counts, dropout.  (Calls with a bias, a window or a score functor, and causal ones with too few workgroups
+// here, see w32_dkdv: bwd_dq_w32.hip, bwd_dkdv_w32.hip.)
 //
 //   bwd_d64_dq_kernel     128 query rows per workgroup (4 wavefronts x 32), 64-key tiles:
 //                           S^T = K Q^T, dP^T = V dO^T, dS^T = P^T (dP^T - delta), dQ^T += K^T dS^T
@@ -14,8 +15,9 @@
 // to two thousand): what bounds them is neither pipe but the chain score - probability - dS - product of
 // one wavefront and the waits around it.  So nothing here is pipelined by hand; the registers are kept
 // to a third of the file (168) instead, three workgroups share a compute unit, and the chain of one
-// wavefront runs under the other two's.  A wavefront keeps all four products of its keys (at head dim 128
-// they do not fit and are split over two wavefronts that exchange P through LDS).
+// wavefront runs under the other two's (dK/dV with dropout or of at most 512 workgroups: two, see OCC).
+// A wavefront keeps all four products of its keys (at head dim 128 they do not fit and are split over two
+// wavefronts that exchange P through LDS).
 //
 // Tiles go from global memory straight into LDS (row-major, XOR swizzled, see tile_swz), three buffers,
 // two tiles ahead, one barrier per tile; transposed operands come out of the transposing LDS read.
@@ -324,7 +326,7 @@ __global__ __launch_bounds__(256, 3) void bwd_d64_dq_kernel(BwdM p, uint32_t* ke
 // OCC: workgroups per compute unit that the registers are kept to.  Three is better where there are that many
 // (B=32, 12 heads, S=512: 123 us for the whole backward against 127 with two, B=4, 32 heads, S=4096 causal 997
 // / 1033), two where there are not (B=4, 12 heads, S=1024 causal, 384 workgroups: 54 / 58; at three a few
-// values go to scratch) and with dropout (147 / 177: it needs 213 registers).
+// values go to scratch) and with dropout (193 registers; B=32, 12 heads, S=512 155 / 161, B=4, 16, S=2048 causal 198 / 229).
 template <typename T, bool DROP, int OCC>
 __global__ __launch_bounds__(256, OCC) void bwd_d64_dkdv_kernel(BwdM p, const uint32_t* keep_bits, int chunk) {
   __shared__ __attribute__((aligned(16))) uint16_t q_t[3][TILE];
@@ -528,11 +530,31 @@ int stream_chunk(const BwdM& g, int64_t rows) {
   return (int)std::max<int64_t>(1, std::min<int64_t>(streams / 8, (2 << 20) / (rows * D * 4)));
 }
 
+// Causal calls whose workgroups (tiles times streams) are too few to hide the longest of them: a key block of the first
+// keys sees every query row, the last one a few, all of them are on the chip at once, and at the end the long ones' chains
+// run with nobody beside them.  The kernels of 8 wavefronts per workgroup (bwd_dq_w32.hip, bwd_dkdv_w32.hip) have the shorter
+// chain.  Below 384 key blocks their items are split (bwd_dkdv_w32_plan), above 1024 the rest of the grid hides it.
+// Backward, us, both kernels here / dQ here and dK/dV there / both there (D=64):
+//   grouped heads, 384 blocks: B=3, 32/8 heads, S=2048 337 / 253 / 263;  B=6, 64/8, S=1024 344 / 263 / 291
+//     512: B=2, 32/8, S=4096 700 / 554 / 569;  B=8, 32/8, S=1024 200 / 170 / 194;  1024: B=8, 32/8, S=2048 626 / 580 / 639
+//   dQ's own grid (B * Hq query tiles), 576: B=6, 12 heads, S=1024 83 / 78 / 72;  768: B=2, 12, S=4096 277 / 261 / 243
+//     512: B=2, 8, S=4096 176 / 165 / 184;  768, S=512 (8 tiles): B=16, 12 53 / 57 / 56.  With key counts or narrow rows
+//     the other dQ kernel is its masked variant: B=3, 12, S=2048 with key counts 109 here / 122 there, D=48 103 / 115
+bool w32_dkdv(const BwdM& g) {
+  const int64_t blocks = (int64_t)g.B * g.Hkv * g.n_kt;
+  return g.causal && g.keep_scale == 0.f && g.Hq > g.Hkv && blocks >= 384 && blocks <= 1024;
+}
+bool w32_both(const BwdM& g) {
+  const int64_t tiles = (int64_t)g.B * g.Hq * g.n_qt;
+  return g.causal && g.keep_scale == 0.f && !g.kv_lens && g.d_real == D && (int64_t)g.B * g.Hkv * g.n_kt >= 384 && tiles > 512 && tiles <= 768 && g.L > 14 * BQ;
+}
+
 template <typename T, bool DROP>
 int launch_t(const BwdM& g, uint32_t* bits, hipStream_t s) {
   hipLaunchKernelGGL((bwd_d64_dq_kernel<T, DROP>), dim3((unsigned)((int64_t)g.B * g.Hq * g.n_qt)), dim3(256), 0, s, g, bits, stream_chunk(g, g.S));
   int rc = check_launch("bwd_d64_dq_kernel");
   if (rc) return rc;
+  if (!DROP && w32_dkdv(g)) return launch_bwd_dkdv_w32(g, std::is_same<T, bf16_t>::value ? MI355_SDPA_BF16 : MI355_SDPA_F16, 64, s);
   const int64_t blocks = (int64_t)g.B * g.Hkv * g.n_kt * g.parts;
   const int chunk = stream_chunk(g, (int64_t)g.L * (g.Hq / g.Hkv));
 #define DKDV(OCC) hipLaunchKernelGGL((bwd_d64_dkdv_kernel<T, DROP, OCC>), dim3((unsigned)blocks), dim3(256), 0, s, g, (const uint32_t*)bits, chunk)
@@ -548,7 +570,7 @@ int launch_t(const BwdM& g, uint32_t* bits, hipStream_t s) {
 
 bool bwd_d64_takes(const BwdM& g) {
   if (g.Hkv < 1) return false;  // (asked for the size of a workspace before anything is checked)
-  if (g.d_real > 64 || g.dv_real != g.d_real || g.bias_kind || g.gbias || g.window > 0 || g.sm.any || g.dq_split_tiles) return false;
+  if (g.d_real > 64 || g.dv_real != g.d_real || g.bias_kind || g.gbias || g.window > 0 || g.sm.any || g.dq_split_tiles || w32_both(g)) return false;
   // (32-bit byte offsets from the start of a batch, and of a key block's keep bits; the latter are the smaller ones
   // but for heads expanded from one)
   return bwd_dkdv_w32_fits(g, 64) && bwd_dq_w32_fits(g, 64) && (g.keep_scale == 0.f || block_words(g) * 4 < (1ll << 32));

@@ -1,5 +1,6 @@
 // Flash-attention backward, dK and dV, for gfx950, head dim 64 or 128, bf16/f16 (at 64 the calls with a bias, a
-// window, a functor or split dQ keys: bwd_d64.hip has the others).
+// window, a functor or split dQ keys, and causal ones of some grid sizes: bwd_d64.hip, which says which, has the others
+// within 32-bit offsets).
 //
 // One workgroup = 8 wavefronts = 128 keys of one (batch, kv head); it loops over the query
 // heads of the group (the GQA sum of decompositions.py:2595-2598 happens in registers) and over
