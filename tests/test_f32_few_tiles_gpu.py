@@ -31,6 +31,8 @@ def amd(gpu_device):
     (2, 2, 2, 150, 500, 104, 8, False),
     (1, 4, 4, 1000, 1000, 64, 64, True),
     (20, 4, 4, 130, 130, 64, 64, False),   # 160 workgroups of 128 rows: the last size here
+    (128, 1, 1, 128, 128, 64, 64, False),  # 512 workgroups of 32 rows: the last size here
+    (103, 1, 1, 129, 129, 64, 64, False),  # ... and past it
     (23, 4, 4, 129, 129, 64, 64, False),   # ... and past it
     (15, 8, 8, 150, 150, 64, 64, True),    # 240, causal
 ])

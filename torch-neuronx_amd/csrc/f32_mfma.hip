@@ -806,9 +806,12 @@ void fwd_f32_plan(FwdM& g, const mi355_sdpa_fwd_params& p, int mode) {
 // many workgroups.  Measured, 128-row / 32-row in us (8 heads, D=64; D=128 gives the same ratios):
 //   B=2, 4 heads, S=128 (8) 14.9 / 8.2;  B=1, S=1024 (64) 92 / 35;  B=2, S=1024 (128) 93 / 66, causal 92 / 41;
 //   B=4, S=1024 (256) 97 / 126, causal 93 / 79;  B=8, S=512 (256) 52 / 74, causal 50 / 52;  B=8, S=1024 (512) 160 / 251
+// Without the causal mask the 32-row ones, all as long, must not need a third turn of the chip (two of them share a
+// compute unit): B=3, S=700 (528 of them) 66 / 72, D=128 115 / 131; S=300 (480) 33 / 29.
 // A single key tile has nothing to share out (S=16: 5.8 / 6.6).
 bool few_query_tiles(const FwdM& g) {
-  return g.S > BT && (int64_t)g.B * g.Hq * ((g.L + 127) / 128) <= (g.causal ? 240 : 160);
+  const int64_t heads = (int64_t)g.B * g.Hq, wide = heads * ((g.L + 127) / 128);
+  return g.S > BT && (g.causal ? wide <= 240 : wide <= 160 && heads * ((g.L + 31) / 32) <= 512);
 }
 
 void fwd_f32_fill(FwdM& g, const mi355_sdpa_fwd_params& p, int& mode) {
