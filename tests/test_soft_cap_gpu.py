@@ -34,6 +34,9 @@ CASES = [
     (2, 2, 1, 97, 225, 64, True, 50, [225, 96], 5.0, 2.0),
     (1, 3, 3, 200, 64, 40, False, None, None, 50.0, 8.0),
     (1, 1, 1, 2, 700, 256, False, None, None, 5.0, 1.0),
+    # short windows at width 64 from 512 workgroups on run in the general functor variant, longer ones do not
+    (64, 8, 8, 97, 97, 64, True, 40, None, 5.0, 1.0),
+    (64, 16, 8, 300, 300, 64, True, 257, [300 - i for i in range(64)], 50.0, 1.0),
 ]
 
 

@@ -1143,7 +1143,12 @@ int launch_fwd_mfma_w32(const FwdM& g0, int dtype, int head_dim, int waves, hipS
     return MI355_SDPA_ERR_UNSUPPORTED;
   }
   const bool cap_only = g.sm.softcap > 0.f && !g.sm.alibi && !g.sm.key_bias && !g.sm.key_weight && !g.sm.doc_q;
-  const int mask = cap_only ? 5 : g.sm.any ? 4 : g.keep_scale != 0.f ? 3 : g.bias_kind != 0 ? 2 : (g.kv_lens != nullptr || g.d_real != head_dim || g.dv_real != head_dim || g.window > 0 || g.sink_logit || g.split_tiles) ? 1 : 0;
+  // (a short window at width 64 on a full chip is mostly edge tiles, each masked score three instructions more under
+  // MASK 5, and the other wavefronts hide the block of MASK 4.  B=4, 32/8 heads, S=4096, MASK 5 / 4 in us: window 64
+  // 114 / 93, 256 149 / 131, 512 194 / 181, 1024 273 / 267; B=1 (512 workgroups) 33 / 32, 45 / 44, 59 / 60; B=4, S=1024,
+  // 16 heads, window 64 19.1 / 19.0, 256 25.7 / 26.8.  At width 128 MASK 5 is never the slower one.)
+  const bool short_window = head_dim == 64 && g.window > 0 && blocks >= 512 && g.window <= (blocks >= 1024 ? 512 : 256);
+  const int mask = cap_only && !short_window ? 5 : g.sm.any ? 4 : g.keep_scale != 0.f ? 3 : g.bias_kind != 0 ? 2 : (g.kv_lens != nullptr || g.d_real != head_dim || g.dv_real != head_dim || g.window > 0 || g.sink_logit || g.split_tiles) ? 1 : 0;
   int rc = dtype == MI355_SDPA_BF16 ? launch_dims<bf16_t>(g, head_dim, waves, mask, grid, s)
                                           : launch_dims<f16_t>(g, head_dim, waves, mask, grid, s);
   if (rc != MI355_SDPA_OK) return rc;
