@@ -129,8 +129,8 @@ constexpr WideOp dkdv_op(int k) {  // S steps and dP steps (in turns where both 
 // MODE 4 (CAP, dQ kernel only): MODE 2 with a soft cap and no other functor.  What bounds this kernel is one wavefront's
 // chain with nobody else on its SIMD; the block of MODE 2 between S and dP (nine instructions per score, two of
 // them quarter-rate) ran with the matrix pipe idle.  Here the cap is part of the probability and rides on the
-// dP products.  dQ, B=2, 16 heads, S=4096, cap 50, MODE 2 / MODE 4: D=256 with a window of 1024 416 / 319 us (forward and backward
-// 924 / 831), causal 715 / 528, 192/128 causal 592 / 397.
+// dP products.  dQ, B=2, 16 heads, S=4096, cap 50, MODE 2 / MODE 4: D=256 with a window of 1024 375 / 288 us, causal 645 / 483,
+// 192/128 causal 576 / 376.
 template <typename T, int ER, int DVR, int MODE>
 __global__ __launch_bounds__(256, 1) void bwd_wide_dq_kernel(BwdM p) {
   constexpr bool MASKED = MODE == 1 || MODE == 3, CAP = MODE == 4, FUNC = MODE == 2 || CAP, DROP = MODE == 3;
@@ -1060,7 +1060,8 @@ int launch_w(const BwdM& g, hipStream_t s) {
            : cap_only ? launch_t<T, 192, 128, 4>(g, s) : func ? launch_t<T, 192, 128, 2>(g, s) : masked ? launch_t<T, 192, 128, 1>(g, s) : launch_t<T, 192, 128, 0>(g, s);
   if (drop) return launch_t<T, 256, 256, 3>(g, s);
   if (cap_only) return launch_t<T, 256, 256, 4>(g, s);
-  // (key counts alone take the functor instance: its dQ kernel tests only the tiles at an edge, and its dK/dV is the pair kernel's)
+  // (key counts alone take the functor instance: its dQ kernel tests only the tiles at an edge, and its dK/dV is the pair kernel's.
+  // Backward, B=2, 16 heads, S=4096 2468 -> 1683 us, B=8, S=512 203 -> 151)
   if (!g.bias_kind) return func || g.kv_lens ? launch_t<T, 256, 256, 2>(g, s) : launch_t<T, 256, 256, 0>(g, s);
   if (g.parts > 1) return launch_t<T, 256, 256, 1, true>(g, s);  // (bwd_wide_parts: no skip table then)
   return launch_t<T, 256, 256, 1>(g, s);

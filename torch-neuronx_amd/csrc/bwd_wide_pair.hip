@@ -17,10 +17,10 @@
 // requested, B is done with item n - 2).  Products, packing and sums are those of bwd_wide_dkdv_kernel.
 //
 // B=2, 16 heads, S=4096, D=256, dK/dV before (one wavefront per SIMD, spilling up to 184 B/lane) and now: window 1024 with
-// a soft cap 577 -> 346 us, window alone 538 -> 344, soft cap 1060 -> 605, causal alone 794 -> 650 (850 TFLOP/s).
+// a soft cap 577 -> 350 us, window alone 500 -> 323, soft cap 1033 -> 598, causal alone 706 -> 564 (975 TFLOP/s).
 // What bounds it: every matrix op reads one 1 KB operand from LDS (a wavefront has registers for 32 keys, so none
-// is used twice), and the two wavefronts of a SIMD reach their products at the same time.  Without the tile loads it takes 305 us instead of
-// 345, without the softmax as well 300; more operands requested ahead change nothing.
+// is used twice), and the two wavefronts of a SIMD reach their products at the same time.  Without the tile loads window and cap took 305 us
+// instead of 345, without the softmax as well 300; more operands requested ahead change nothing.
 #include "bwd_wide.h"
 
 namespace mi355 {
