@@ -17,6 +17,9 @@ struct FwdM {
   int B, Hq, Hkv, L, S;
   int n_qt;    // query tiles per head
   int causal;
+  // A call that names its kernel sums a row's keys in order whatever the sizes, and so equals a longer call on its prefix;
+  // one with key counts or a verdict equals the call that those stand for, and is left to the sizes.
+  int whole_keys = 0;
   int xcd_map;  // 1: (batch, kv head) streams are pinned to XCDs
   float scale;
   // masked calls (fwd_mfma_w32.hip only): additive bias or bool keep-mask with unit stride on the

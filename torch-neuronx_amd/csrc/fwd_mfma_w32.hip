@@ -60,9 +60,11 @@ constexpr float kLazy = 8.f;  // log2 headroom before the accumulator is rescale
 // of MASK = 4 it ran with the matrix pipe idle, at head dim 256 with nobody on the SIMD to fill it (B=2, 16 heads,
 // S=4096, D=256, window 1024: 264 -> 206 us, the same call without a cap 180; causal, no window 411 -> 318; D=128,
 // 32 heads, causal 377 -> 327; D=64, 32 heads, causal 270 -> 247, 16 heads, S=1000, B=4 46.5 -> 37).
-template <typename T, int D, int WAVES, int MASK>
+// PARTS = 2: twice the wavefronts over the same rows, in two halves that take every other key tile of the
+// workgroup's stream from LDS buffers of their own and add up their rows in LDS at the end (see merge_halves).
+template <typename T, int D, int WAVES, int MASK, int PARTS>
 __device__ __forceinline__ void fwd_w32_body(const FwdM& p, const MaskArgs ma) {
-  constexpr int BM = 32 * WAVES, NT = 64 * WAVES;
+  constexpr int BM = 32 * WAVES;
   constexpr int KS = D / 16;      // matrix ops of S^T = K Q^T per tile (phase A)
   constexpr int DB = D / 32;      // 32-row blocks of O^T
   constexpr int NPV = 2 * DB;     // matrix ops of O^T += V^T P^T per tile (phase B)
@@ -73,7 +75,8 @@ __device__ __forceinline__ void fwd_w32_body(const FwdM& p, const MaskArgs ma) {
   // they take the launch's dynamic LDS instead; head dim 256 runs one wavefront per SIMD with the
   // 512-register budget)
   constexpr bool BIASED = MASK == 2 || MASK == 3, DROP = MASK == 3;  // a bias tile in LDS; ... and the tile of a dropout keep-mask beside it
-  constexpr bool DYN = D > 128 || BIASED;
+  constexpr bool DYN = D > 128 || BIASED || PARTS > 1;
+  static_assert(PARTS == 1 || (PARTS == 2 && MASK < 2 && D <= 128), "the variants that share out the keys of a workgroup");
   // Tiles go from global memory straight into LDS (see the staging section): four unpadded,
   // swizzled buffers per operand, tile t in buffer t % 4.
   // mask functors (window, sink keys, sink logit): in the masked variant without a bias
@@ -84,8 +87,11 @@ __device__ __forceinline__ void fwd_w32_body(const FwdM& p, const MaskArgs ma) {
   __shared__ __attribute__((aligned(16))) uint16_t k_static[DYN ? 8 : NBUF * TILE];
   __shared__ __attribute__((aligned(16))) uint16_t v_static[DYN ? 8 : NBUF * TILE];
   extern __shared__ __attribute__((aligned(16))) uint16_t dyn_lds[];
-  uint16_t* const k_dma = DYN ? dyn_lds : k_static;
-  uint16_t* const v_dma = DYN ? dyn_lds + NBUF * TILE : v_static;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave_id = __builtin_amdgcn_readfirstlane(tid >> 6);  // uniform: keeps per-wavefront tests on the scalar unit
+  const int wave = PARTS > 1 ? wave_id % WAVES : wave_id, part = PARTS > 1 ? wave_id / WAVES : 0;  // which rows, which key tiles
+  uint16_t* const k_dma = DYN ? dyn_lds + part * (2 * NBUF * TILE) : k_static;
+  uint16_t* const v_dma = DYN ? k_dma + NBUF * TILE : v_static;
   // bias tiles (MASK = 2): per wavefront two buffers of four 1 KB groups, every lane its own 16 bytes of each
   uint16_t* const bias_lds = dyn_lds + 2 * NBUF * TILE;
   // ... and, with a tile skip table, the list of the key tiles this workgroup walks (1024 entries and the count)
@@ -93,8 +99,6 @@ __device__ __forceinline__ void fwd_w32_body(const FwdM& p, const MaskArgs ma) {
   // (dropout, which never comes with a table, has a wavefront's 1 KB of keep bytes there)
   const unsigned char* const keep_lds = (const unsigned char*)(bias_lds + WAVES * 2048);
 
-  const int tid = threadIdx.x, lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // uniform: keeps per-wavefront tests on the scalar unit
   int b, h, qt;
   int wrow = wave * 32;  // this wavefront's first row within the workgroup's rows
   int split = 0;  // (grouped calls with split keys: which part of them)
@@ -233,6 +237,9 @@ __device__ __forceinline__ void fwd_w32_body(const FwdM& p, const MaskArgs ma) {
     return zm + __builtin_logf(zl);
   };
   auto tile_of = [&](int u) {
+    // (two halves: position u of a half's stream is position 2 u + part of the workgroup's; a half whose stream has
+    // ended goes over the last tile again and drops it)
+    if constexpr (PARTS > 1) u = min(PARTS * u + part, nt - 1);
     if constexpr (MASK == 2) return listed ? __builtin_amdgcn_readfirstlane((int)tile_list[u]) : u + skip;
     // (the pipeline also forms, and drops, the scores of the stream position behind a wavefront's last
     // one: walking down that would be tile -1, whose per-key vectors lie in front of their arrays)
@@ -287,7 +294,9 @@ __device__ __forceinline__ void fwd_w32_body(const FwdM& p, const MaskArgs ma) {
     }
   };
 
-  const int nt_w = (ma.causal && !backwards) ? min(nt, qw_last / BN + 1 - skip) : nt;
+  int nt_w = (ma.causal && !backwards) ? min(nt, qw_last / BN + 1 - skip) : nt;
+  int nt_end = nt;  // steps of the tile loop
+  if constexpr (PARTS > 1) nt_w = (nt_w + PARTS - 1 - part) / PARTS, nt_end = (nt + PARTS - 1) / PARTS;  // (as many steps, and barriers, in both halves)
 
   // K and V are read through buffer resources that end with the last key row of this (batch, head);
   // the whole offset travels in the vector offset, the part the hardware checks against that bound:
@@ -896,12 +905,54 @@ __device__ __forceinline__ void fwd_w32_body(const FwdM& p, const MaskArgs ma) {
     iteration(t, std::integral_constant<int, 3>{}, s_b, s_a, pk_b, pk_a, ps_b, ps_a);
     ++t;
   }
-  for (; t < nt; ++t) idle_step(t);
+  for (; t < nt_end; ++t) idle_step(t);
   // (no load into LDS may be in flight when the workgroup's LDS is handed to the next one)
   wait_all_tiles();
 
   // ---- epilogue ------------------------------------------------------------------------------------
-  const float l_tot = l_run + __shfl_xor(l_run, 32, 64);
+  float l_tot = l_run + __shfl_xor(l_run, 32, 64);
+  constexpr int OB = DB / PARTS;  // blocks of O^T that this wavefront writes: all of them, or its half's
+  auto merge_halves = [&]() {
+    // Each half hands the other one the blocks that the other writes, unnormalised in float32, and every lane its row's
+    // reference and sum.  (A half whose tiles held no live key for a row has no say in the reference.  Rows whose scores so
+    // far were all -inf carry a reference of 0.)
+    f32x4* const xch = (f32x4*)dyn_lds + (size_t)wave_id * (OB * 4 * 64) + lane;
+    u32x2* const stat = (u32x2*)((f32x4*)dyn_lds + (size_t)PARTS * WAVES * (OB * 4 * 64)) + wave_id * 64 + lane;
+    const ptrdiff_t other = (part ? -WAVES : WAVES) * 64;
+    const float m_me = l_tot == 0.f ? -INFINITY : m_run == -INFINITY ? 0.f : m_run;
+    __syncthreads();  // every wavefront is done with the K / V tiles
+#pragma unroll
+    for (int i = 0; i < OB; ++i)
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        f32x4 w;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const float lo = oacc[i][4 * g + e], hi = oacc[(OB + i) % DB][4 * g + e];
+          w[e] = part ? lo : hi;
+          oacc[i][4 * g + e] = part ? hi : lo;
+        }
+        xch[(i * 4 + g) * 64] = w;
+      }
+    *stat = u32x2{__builtin_bit_cast(uint32_t, m_me), __builtin_bit_cast(uint32_t, l_tot)};
+    __syncthreads();
+    const u32x2 st = stat[other];
+    const uint32_t st0 = st[0], st1 = st[1];
+    const float m_ot = __builtin_bit_cast(float, st0), l_ot = __builtin_bit_cast(float, st1);
+    m_run = fmaxf(m_me, m_ot);
+    const float a_me = l_tot == 0.f ? 0.f : __builtin_amdgcn_exp2f((m_me - m_run) * c);
+    const float a_ot = l_ot == 0.f ? 0.f : __builtin_amdgcn_exp2f((m_ot - m_run) * c);
+    l_tot = fmaf(l_tot, a_me, l_ot * a_ot);
+#pragma unroll
+    for (int i = 0; i < OB; ++i)
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        const f32x4 w = xch[other * (OB * 4) + (i * 4 + g) * 64];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) oacc[i][4 * g + e] = fmaf(oacc[i][4 * g + e], a_me, w[e] * a_ot);
+      }
+  };
+  if constexpr (PARTS > 1) merge_halves();
   float inv = l_tot > 0.f ? 1.f / l_tot : 0.f;
   float lse_row = l_tot > 0.f ? m_run * p.scale + __builtin_logf(l_tot) : -INFINITY;
   if constexpr (DROP) inv *= p.keep_scale;
@@ -919,7 +970,7 @@ __device__ __forceinline__ void fwd_w32_body(const FwdM& p, const MaskArgs ma) {
       }
     }
   }
-  if constexpr (SPLITS) {
+  if constexpr (SPLITS && PARTS == 1) {
     if (p.split_tiles) {  // split keys: this part's normalised rows and their log-sum-exp, in float32, for the merge
       if (qrow < p.L) {
         const int64_t prow = (((int64_t)b * p.Hq + h) * p.n_split + split) * p.L + qrow;
@@ -942,28 +993,34 @@ __device__ __forceinline__ void fwd_w32_body(const FwdM& p, const MaskArgs ma) {
   // which nothing overlaps, took 3 % of the kernel.  The tile goes through LDS instead (the
   // tile buffers are free now; 32 rows x D per wavefront, 16-byte chunks XOR-swizzled by row
   // against bank conflicts) and leaves as whole rows, 16 bytes per lane.
-  __syncthreads();  // every wavefront is done with the K / V tiles
-  uint16_t* ot = wave < WAVES / 2 ? k_dma + wave * 32 * D : v_dma + (wave - WAVES / 2) * 32 * D;
-  constexpr int SW = CH < 16 ? CH - 1 : 15;
+  constexpr int DO = D / PARTS, CHO = CH / PARTS;  // columns that this wavefront writes, and their chunks
+  uint16_t* ot;
+  if constexpr (PARTS > 1) {
+    ot = dyn_lds + PARTS * WAVES * 32 * D + PARTS * WAVES * 256 + wave_id * 32 * DO;  // (behind what the halves exchange)
+  } else {
+    __syncthreads();  // every wavefront is done with the K / V tiles
+    ot = wave < WAVES / 2 ? k_dma + wave * 32 * D : v_dma + (wave - WAVES / 2) * 32 * D;
+  }
+  constexpr int SW = CHO < 16 ? CHO - 1 : 15;
 #pragma unroll
-  for (int db = 0; db < DB; ++db)
+  for (int db = 0; db < OB; ++db)
 #pragma unroll
     for (int g = 0; g < 4; ++g) {
       u32x2 w;
       w[0] = Mma<T>::pack(oacc[db][g * 4 + 0] * inv, oacc[db][g * 4 + 1] * inv);
       w[1] = Mma<T>::pack(oacc[db][g * 4 + 2] * inv, oacc[db][g * 4 + 3] * inv);
-      *(u32x2*)(ot + col * D + (((db * 4 + g) ^ (col & SW)) << 3) + half * 4) = w;
+      *(u32x2*)(ot + col * DO + (((db * 4 + g) ^ (col & SW)) << 3) + half * 4) = w;
     }
-  constexpr int RPI = 64 / CH;  // rows per store instruction
-  const int rr = lane / CH, cc = lane % CH;
-  uint16_t* obase = (uint16_t*)p.out + b * p.o_sb + h * p.o_sh + cc * 8;
+  constexpr int RPI = 64 / CHO;  // rows per store instruction
+  const int rr = lane / CHO, cc = lane % CHO;
+  uint16_t* obase = (uint16_t*)p.out + b * p.o_sb + h * p.o_sh + part * DO + cc * 8;
 #pragma unroll
   for (int i = 0; i < 32 / RPI; ++i) {
     const int r = i * RPI + rr;
-    const u32x4 w = *(const u32x4*)(ot + r * D + ((cc ^ (r & SW)) << 3));
-    if (qw0 + r < p.L && (!MASK || cc * 8 < drv)) *(u32x4*)(obase + (int64_t)(qw0 + r) * p.o_sl) = w;
+    const u32x4 w = *(const u32x4*)(ot + r * DO + ((cc ^ (r & SW)) << 3));
+    if (qw0 + r < p.L && (!MASK || part * DO + cc * 8 < drv)) *(u32x4*)(obase + (int64_t)(qw0 + r) * p.o_sl) = w;
   }
-  if (qrow < p.L && p.lse && half == 0) p.lse[((int64_t)b * p.Hq + h) * p.L + qrow] = lse_row;
+  if (qrow < p.L && p.lse && half == 0 && part == 0) p.lse[((int64_t)b * p.Hq + h) * p.L + qrow] = lse_row;
 }
 
 // The kernel of a variant.  A call whose bias comes with a verdict about it (see MaskArgs) is launched
@@ -973,8 +1030,8 @@ __device__ __forceinline__ void fwd_w32_body(const FwdM& p, const MaskArgs ma) {
 // was made with the causal flag - and any other bias leaves that kernel's workgroups nothing to do.
 // (Two kernels rather than one that branches: both variants in one kernel need more scalar registers
 // than there are, and the variant with a bias pays for its bias slot even when the slot is empty.)
-template <typename T, int D, int WAVES, int MASK, bool PATTERN = false>
-__global__ __launch_bounds__(64 * WAVES, D > 128 ? 1 : 8 / WAVES) void fwd_w32_kernel(FwdM p) {
+template <typename T, int D, int WAVES, int MASK, bool PATTERN = false, int PARTS = 1>
+__global__ __launch_bounds__(64 * WAVES * PARTS, D > 128 ? 1 : 8 / (WAVES * PARTS)) void fwd_w32_kernel(FwdM p) {
   static_assert(!PATTERN || MASK == 1, "the pattern kernel is the variant with key counts");
   MaskArgs ma = mask_args_of(p);
   if constexpr (MASK == 2 || PATTERN) {
@@ -982,7 +1039,7 @@ __global__ __launch_bounds__(64 * WAVES, D > 128 ? 1 : 8 / WAVES) void fwd_w32_k
   } else if constexpr (MASK == 3) {
     verdict_pattern(p, ma);  // (dropout: one variant takes a bias or none, so the verdict is applied in place)
   }
-  fwd_w32_body<T, D, WAVES, MASK>(p, ma);
+  fwd_w32_body<T, D, WAVES, MASK, PARTS>(p, ma);
 }
 
 // Merge of the parts of a call whose keys were split (see split_merge.h): normalised rows and their
@@ -1023,26 +1080,63 @@ void launch_merge(const FwdM& g, hipStream_t s) {
 }
 
 // one instantiation; head dim 256 and the variant with a bias need more than the 64 KB of LDS a kernel may declare
-template <typename T, int D, int WAVES, int MASK, bool PATTERN = false>
+template <typename T, int D, int WAVES, int MASK, bool PATTERN = false, int PARTS = 1>
 int launch_one(const FwdM& g, dim3 grid, hipStream_t s) {
   int bytes = 0;
-  if constexpr (D > 128 || MASK == 2 || MASK == 3) {
+  if constexpr (D > 128 || MASK == 2 || MASK == 3 || PARTS > 1) {
     // (four buffers per operand, 4 KB of bias tile per wavefront, and the tile list of a call with a skip table)
-    constexpr int kBase = 2 * 4 * BN * D * 2 + (MASK == 2 || MASK == 3 ? WAVES * 4096 : 0) + (MASK == 3 ? WAVES * 1024 : 0);
+    constexpr int kBase = PARTS * 2 * 4 * BN * D * 2 + (MASK == 2 || MASK == 3 ? WAVES * 4096 : 0) + (MASK == 3 ? WAVES * 1024 : 0);
     constexpr int kBytes = kBase + (MASK == 2 ? 2048 + 16 : 0);
     static LdsOnce once;
-    const hipError_t attr = reserve_lds(once, (const void*)fwd_w32_kernel<T, D, WAVES, MASK, PATTERN>, kBytes);
+    const hipError_t attr = reserve_lds(once, (const void*)fwd_w32_kernel<T, D, WAVES, MASK, PATTERN, PARTS>, kBytes);
     if (attr != hipSuccess) {
       set_error("SDPA: cannot reserve %d bytes of LDS for fwd_w32_kernel: %s", kBytes, hipGetErrorString(attr));
       return MI355_SDPA_ERR_LAUNCH;
     }
     bytes = (MASK == 2 && g.live_tiles) ? kBytes : kBase;
   }
-  hipLaunchKernelGGL((fwd_w32_kernel<T, D, WAVES, MASK, PATTERN>), grid, dim3(64 * WAVES), bytes, s, g);
+  hipLaunchKernelGGL((fwd_w32_kernel<T, D, WAVES, MASK, PATTERN, PARTS>), grid, dim3(64 * WAVES * PARTS), bytes, s, g);
   return MI355_SDPA_OK;
 }
+// Rows per workgroup of the kernels whose halves share out the keys (PARTS = 2: 64 or 128), or 0 where they are not taken.
+// With few rows a call lasts as long as its longest chain of key tiles, about 0.5 us a tile at head dim 128 for a wavefront
+// that has its SIMD to itself, beside a start and an end of 5 us; two halves walk half the chain each.
+//   64 rows, four wavefronts, each on a SIMD of its own: where a compute unit gets one workgroup (their LDS leaves room for
+//   one at head dim 128, two at 64).  Whole keys / halves in us: 16/4 heads, S=1021, D=128 18.6 / 14.0; 32/8 heads, S=400
+//   11.0 / 9.7; 16 heads, S=256 10.6 / 8.0; D=64: 12 heads, S=1024 13.7 / 9.8, B=2 14.6 / 11.1, S=2048 27.7 / 25.6, not
+//   causal S=785 11.5 / 9.0, S=197 B=4 8.1 / 6.1 (there against one 256-row workgroup per head, see fwd_w32_plan).  Past that a
+//   second turn of workgroups pays the start again: 32/8 heads, S=700 15.2 / 15.7, S=1400 30 / 36; D=64, B=16, S=197 9.1 / 12.5.
+//   128 rows, two wavefronts a SIMD: a long causal chain in front of many short ones.  32/8 heads, D=128: S=1021 21.2 / 20.5,
+//   S=1400 29.7 / 27; 28/4, S=1400 29.2 / 26; 16/4, S=4000 79 / 74; S=2500 60 / 68, two turns.  The exchange costs 1.5 us: S=256 9.0 / 10.2.
+int share_keys(const FwdM& g, int head_dim) {
+  if (g.whole_keys || g.grouped > 1 || g.split_tiles || g.L <= 32) return 0;
+  int tiles = (g.S + BN - 1) / BN;
+  if (g.window > 0) tiles = std::min(tiles, (g.window + 128) / BN);
+  const int64_t heads = (int64_t)g.B * g.Hq, wg64 = heads * ((g.L + 63) / 64), wg128 = heads * ((g.L + 127) / 128);
+  if (tiles >= 4 && wg64 <= (head_dim == 64 && g.causal ? g.grouped ? 512 : std::max(256, std::min(768, 16 * tiles)) : 256)) return 64;
+  if (!g.grouped && head_dim == 128 && g.causal && tiles >= 24 && wg128 <= std::min(512, 8 * tiles)) return 128;
+  return 0;
+}
+template <typename T, int D, int MASK, bool PATTERN>
+int launch_halves(FwdM g, int rows, hipStream_t s) {
+  g.grouped = 0, g.n_qt = (g.L + rows - 1) / rows;
+  const dim3 grid((unsigned)((int64_t)g.B * g.Hq * g.n_qt));
+  if (rows == 64) return launch_one<T, D, 2, MASK, PATTERN, 2>(g, grid, s);
+  return launch_one<T, D, 4, MASK, PATTERN, 2>(g, grid, s);
+}
+
 template <typename T, int D, int WAVES>
 int launch_mask(const FwdM& g, int mask, dim3 grid, hipStream_t s) {
+  if constexpr (D <= 128) {
+    if (const int rows = WAVES == 4 || g.grouped ? share_keys(g, D) : 0) {
+      if (mask == 2 && g.verdict) {  // (see fwd_w32_kernel)
+        if (int rc = launch_halves<T, D, 1, true>(g, rows, s)) return rc;
+        return launch_one<T, D, WAVES, 2>(g, grid, s);
+      }
+      if (mask == 1) return launch_halves<T, D, 1, false>(g, rows, s);
+      if (mask == 0) return launch_halves<T, D, 0, false>(g, rows, s);
+    }
+  }
   if (mask == 5) return launch_one<T, D, WAVES, 5>(g, grid, s);
   if (mask == 4) return launch_one<T, D, WAVES, 4>(g, grid, s);
   if (mask == 3) return launch_one<T, D, WAVES, 3>(g, grid, s);
