@@ -105,6 +105,11 @@ __device__ __forceinline__ void decode_block(const FwdM& p, int& b, int& h, int&
 // head_dim 64, 128 or 256: the width the kernel is built for (g.d_real: the width of the data);
 // waves = 4 or 8 wavefronts (128 or 256 query rows) per workgroup, 4 only at head dim 256
 int launch_fwd_mfma_w32(const FwdM& g, int dtype, int head_dim, int waves, hipStream_t s);
+// decode steps (fwd_few_rows.hip): at most 16 query rows per kv head and nothing but key counts on the scores; the plan
+// sets split_tiles (steps of 32 keys per part) and n_split
+bool few_rows_supported(const FwdM& g, int head_dim);
+void few_rows_plan(FwdM& g);
+int launch_fwd_few_rows(const FwdM& g, int dtype, int head_dim, hipStream_t s);
 // adds up the parts that a call with split keys left in g.part_o / g.part_lse (any of the three dtypes)
 int launch_fwd_split_merge(const FwdM& g, int dtype, hipStream_t s);
 // bytes of workspace with which that launch would split the keys of the call (0: it would not)

@@ -1060,7 +1060,7 @@ __global__ __launch_bounds__(SLICES * TPR) void fwd_split_merge_kernel(FwdM p) {
       lds, p.n_split, [&](int c, float& m, float& w) { m = pl[(int64_t)c * p.L], w = 1.f; },
       [&](int c) { return *(const f32x4*)(po + c * part_stride); }, O, M, L);
   const int d = threadIdx.x;
-  if (d < p.dv_real) ((T*)p.out)[b * p.o_sb + h * p.o_sh + (int64_t)l * p.o_sl + d] = (T)(L > 0.f ? O / L : 0.f);
+  if (d < p.dv_real) ((T*)p.out)[b * p.o_sb + h * p.o_sh + (int64_t)l * p.o_sl + d] = (T)(L == 0.f ? 0.f : O / L);
   if (d == 0 && p.lse) p.lse[row] = L > 0.f ? M + __builtin_logf(L) : -INFINITY;
 }
 
@@ -1171,6 +1171,7 @@ void fwd_w32_plan(FwdM& g, int head_dim, int& waves) {
   if (head_dim == 256) waves = 4;
   const int rep = g.Hq / g.Hkv;
   g.grouped = 0, g.split_tiles = 0, g.n_split = 1;
+  if (few_rows_supported(g, head_dim)) return few_rows_plan(g);
   // (one head per kv head counts too: nothing is shared then, but such a call can split its keys)
   if ((g.bias_kind == 0 || g.bias_sh == 0) && g.keep_scale == 0.f && !g.live_tiles) {
     const int blocks32 = (g.L + 31) / 32;  // 32-row blocks per head
@@ -1219,6 +1220,11 @@ int launch_fwd_mfma_w32(const FwdM& g0, int dtype, int head_dim, int waves, hipS
     const size_t rows = (size_t)g.B * g.Hq * g.n_split * g.L;
     if (g.part_o && g.n_split <= 512 && g.part_bytes >= rows * (g.dv_real + 1) * sizeof(float)) g.part_lse = g.part_o + rows * g.dv_real;
     else g.split_tiles = 0, g.n_split = 1;
+  }
+  if (few_rows_supported(g, head_dim)) {
+    if ((int64_t)g.B * g.Hkv == 0) return MI355_SDPA_OK;
+    const int rc = launch_fwd_few_rows(g, dtype, head_dim, s);
+    return rc != MI355_SDPA_OK || !g.split_tiles ? rc : launch_fwd_split_merge(g, dtype, s);
   }
   const int64_t blocks = g.grouped ? (int64_t)g.B * (g.Hq / g.grouped) * g.n_split : (int64_t)g.B * g.Hq * g.n_qt;
   if (blocks == 0) return MI355_SDPA_OK;

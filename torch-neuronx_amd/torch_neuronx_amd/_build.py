@@ -17,7 +17,7 @@ LIB_PATH = os.path.join(LIB_DIR, "libmi355_sdpa.so")
 HOST_PATH = os.path.join(LIB_DIR, "_host_args.so")
 OBJ_DIR = os.path.join(LIB_DIR, "obj")
 
-SOURCES = ["api", "fwd_generic", "fwd_mfma", "fwd_mfma_w32", "bwd_generic", "bwd_mfma", "bwd_dkdv_w32", "bwd_dq_w32", "bwd_wide", "bwd_wide_pair", "bwd_d64", "decode_fp8kv", "mask_rows", "f32_mfma"]
+SOURCES = ["api", "fwd_generic", "fwd_mfma", "fwd_mfma_w32", "fwd_few_rows", "bwd_generic", "bwd_mfma", "bwd_dkdv_w32", "bwd_dq_w32", "bwd_wide", "bwd_wide_pair", "bwd_d64", "decode_fp8kv", "mask_rows", "f32_mfma"]
 
 # packed-fp32 VALU ops are switched off for all device code in this library
 HIPCC_FLAGS = [
