@@ -1030,7 +1030,7 @@ __device__ __forceinline__ void fwd_w32_body(const FwdM& p, const MaskArgs ma) {
 // was made with the causal flag - and any other bias leaves that kernel's workgroups nothing to do.
 // (Two kernels rather than one that branches: both variants in one kernel need more scalar registers
 // than there are, and the variant with a bias pays for its bias slot even when the slot is empty.)
-template <typename T, int D, int WAVES, int MASK, bool PATTERN = false, int PARTS = 1>
+template <typename T, int PARTS, int D, int WAVES, int MASK, bool PATTERN>
 __global__ __launch_bounds__(64 * WAVES * PARTS, D > 128 ? 1 : 8 / (WAVES * PARTS)) void fwd_w32_kernel(FwdM p) {
   static_assert(!PATTERN || MASK == 1, "the pattern kernel is the variant with key counts");
   MaskArgs ma = mask_args_of(p);
@@ -1088,14 +1088,14 @@ int launch_one(const FwdM& g, dim3 grid, hipStream_t s) {
     constexpr int kBase = PARTS * 2 * 4 * BN * D * 2 + (MASK == 2 || MASK == 3 ? WAVES * 4096 : 0) + (MASK == 3 ? WAVES * 1024 : 0);
     constexpr int kBytes = kBase + (MASK == 2 ? 2048 + 16 : 0);
     static LdsOnce once;
-    const hipError_t attr = reserve_lds(once, (const void*)fwd_w32_kernel<T, D, WAVES, MASK, PATTERN, PARTS>, kBytes);
+    const hipError_t attr = reserve_lds(once, (const void*)fwd_w32_kernel<T, PARTS, D, WAVES, MASK, PATTERN>, kBytes);
     if (attr != hipSuccess) {
       set_error("SDPA: cannot reserve %d bytes of LDS for fwd_w32_kernel: %s", kBytes, hipGetErrorString(attr));
       return MI355_SDPA_ERR_LAUNCH;
     }
     bytes = (MASK == 2 && g.live_tiles) ? kBytes : kBase;
   }
-  hipLaunchKernelGGL((fwd_w32_kernel<T, D, WAVES, MASK, PATTERN, PARTS>), grid, dim3(64 * WAVES * PARTS), bytes, s, g);
+  hipLaunchKernelGGL((fwd_w32_kernel<T, PARTS, D, WAVES, MASK, PATTERN>), grid, dim3(64 * WAVES * PARTS), bytes, s, g);
   return MI355_SDPA_OK;
 }
 // Rows per workgroup of the kernels whose halves share out the keys (PARTS = 2: 64 or 128), or 0 where they are not taken.
