@@ -94,9 +94,10 @@ def _host_flags():
 
     torch_lib = os.path.join(os.path.dirname(torch.__file__), "lib")
     compile_flags = ["-O2", "-std=c++17", "-fPIC", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
-                     *(f"-I{d}" for d in include_paths()), "-I" + sysconfig.get_path("include")]
+                     *(f"-I{d}" for d in include_paths()), "-I" + sysconfig.get_path("include"),
+                     "-D__HIP_PLATFORM_AMD__=1", "-I" + os.path.join(os.path.dirname(os.path.dirname(os.path.realpath(_hipcc()))), "include")]
     link_flags = ["-shared", "-L" + LIB_DIR, "-l:" + os.path.basename(LIB_PATH), "-Wl,-rpath,$ORIGIN",
-                  "-L" + torch_lib, "-ltorch_python", "-ltorch_cpu", "-lc10"]
+                  "-L" + torch_lib, "-ltorch_python", "-ltorch_cpu", "-lc10_hip", "-lc10"]
     return compile_flags, link_flags
 
 

@@ -151,7 +151,7 @@ def host():
         spec = importlib.util.spec_from_file_location("_host_args", HOST_PATH)
         mod = importlib.util.module_from_spec(spec)
         spec.loader.exec_module(mod)
-        if (mod.FWD_BYTES, mod.BWD_BYTES, mod.DECODE_BYTES) != (C.sizeof(FwdParams), C.sizeof(BwdParams), C.sizeof(DecodeParams)):
+        if not hasattr(mod, "register_operators") or (mod.FWD_BYTES, mod.BWD_BYTES, mod.DECODE_BYTES) != (C.sizeof(FwdParams), C.sizeof(BwdParams), C.sizeof(DecodeParams)):
             raise RuntimeError(f"{HOST_PATH} was built for other structures than this binding's: rebuild it")
         _host = mod
     return _host

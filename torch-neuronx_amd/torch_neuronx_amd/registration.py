@@ -13,6 +13,9 @@ by this package.
 * ``aten::_fused_sdp_choice``: reachable through ``torch._fused_sdp_choice``; rules of
   torch_neuronx/csrc/aten/SdpBackendSelection.cpp:14-68.
 
+The flash and memory-efficient pairs are registered natively (``csrc/host_args.cpp``): plain calls never enter the
+interpreter, the others arrive in the Python functions as before.
+
 Upstream's autograd formulas for these ops call the matching ``_backward`` op, so no
 autograd.Function is needed.
 """
@@ -24,7 +27,7 @@ import warnings
 
 import torch
 
-from . import _lib, python_ops as po
+from . import _lib, ops, python_ops as po
 from .python_ops import scaled_dot_product_fused_attention as impl
 
 _lib_handle = None
@@ -48,14 +51,21 @@ def register(override_aten: bool | None = None) -> list:
         ("_scaled_dot_product_fused_attention_overrideable_backward",
          po.scaled_dot_product_fused_attention_overrideable_backward),
     ]
+    native = False
     if override_aten:
+        table += [("_fused_sdp_choice", impl.fused_sdp_choice)]
+        try:
+            _registered.extend(_lib.host().register_operators(vars(ops), vars(impl)))
+            native = True
+        except (RuntimeError, OSError, ImportError):
+            pass  # (not built yet, or for other structures: the functions below say so when they are called)
+    if override_aten and not native:
         table += [
             ("_scaled_dot_product_flash_attention", po.scaled_dot_product_flash_attention),
             ("_scaled_dot_product_flash_attention_backward", po.scaled_dot_product_flash_attention_backward),
             ("_scaled_dot_product_efficient_attention", po.scaled_dot_product_efficient_attention),
             ("_scaled_dot_product_efficient_attention_backward",
              po.scaled_dot_product_efficient_attention_backward),
-            ("_fused_sdp_choice", impl.fused_sdp_choice),
         ]
     with warnings.catch_warnings():
         warnings.simplefilter("ignore")  # "overriding a previously registered kernel" is the point
@@ -72,6 +82,8 @@ def unregister() -> None:
     route_functional(False)
     if _lib_handle is not None:
         _lib_handle._destroy()
+        if _lib._host is not None:
+            _lib._host.unregister_operators()
         _lib_handle = None
         _registered.clear()
 
