@@ -349,10 +349,12 @@ bool fwd_mfma_supported(const mi355_sdpa_fwd_params& p, const char** why) {
     const int64_t S = p.k.size[2], L = p.q.size[2];
     const int gran = 4 / esz;  // elements per dword
     if (S > 1 && p.bias.stride[3] != 1) return *why = "attn_bias keys are not unit-stride", false;
-    if (((uintptr_t)p.bias.data & 3) != 0 || S % gran != 0) return *why = "attn_bias not dword aligned", false;
+    // (a 16-bit bias over an odd number of keys is read to the end of the dword that its last element starts; a bool
+    // mask per key is scanned in whole dwords)
+    if (((uintptr_t)p.bias.data & 3) != 0 || (esz != 2 && S % gran != 0)) return *why = "attn_bias not dword aligned", false;
     for (int i = 0; i < 3; ++i)
       if (p.bias.size[i] > 1 && (p.bias.stride[i] % gran) != 0) return *why = "attn_bias stride not dword aligned", false;
-    if ((31 * p.bias.stride[2] + S) * esz >= (1ll << 31)) return *why = "attn_bias rows beyond 32-bit offsets", false;
+    if ((31 * p.bias.stride[2] + S) * esz > (1ll << 31) - 4) return *why = "attn_bias rows beyond 32-bit offsets", false;
     (void)L;
   }
   if (p.dropout_p > 0.f) {

@@ -434,8 +434,8 @@ __device__ __forceinline__ void fwd_w32_body(const FwdM& p, const MaskArgs ma) {
     }
   };
   // Bias of the score tile: lane = query row, 4 groups of 4 consecutive keys.  The resource starts
-  // at this wavefront's first row of the (batch, head) plane and ends with its last one, so keys
-  // past S read as zero (they are masked anyway).  Folded into the RAW scores, s += bias / scale,
+  // at this wavefront's first row of the (batch, head) plane and ends with the last one's last dword, so keys
+  // past S read as another row's, or as zero (they are masked anyway).  Folded into the RAW scores, s += bias / scale,
   // so that everything downstream (reference tracking, lse) is the unbiased code.
   // A wavefront's 32 x 32 tile lands in its own 4 KB of LDS through the same kind of load as the
   // K / V tiles, 16 bytes per lane and instruction whatever the element size:
@@ -453,7 +453,7 @@ __device__ __forceinline__ void fwd_w32_body(const FwdM& p, const MaskArgs ma) {
   const int b_esz = bkind == 1 ? 4 : bkind == 4 ? 1 : 2;
   const int b_rows = min(32, p.L - qw0);
   const u32x4 b_rsrc = descriptor((const char*)p.bias + (bkind ? (b * p.bias_sb + h * p.bias_sh + (int64_t)qw0 * p.bias_sl) * b_esz : 0),
-                                  (bkind && b_rows > 0) ? (int)(((b_rows - 1) * p.bias_sl + p.S) * b_esz) : 0);
+                                  (bkind && b_rows > 0) ? (int)((((b_rows - 1) * p.bias_sl + p.S) * b_esz + 3) & ~3) : 0);
   const uint32_t b_voff = (uint32_t)((min(col, max(b_rows - 1, 0)) * p.bias_sl + half * (bkind == 1 ? 4 : bkind == 4 ? 16 : 8)) * b_esz);
   const int b_loads = bkind == 1 ? 4 : bkind == 4 ? 1 : 2;
   const unsigned char* const bias_w = (const unsigned char*)bias_lds + (BIASED ? wave * 4096 : 0);

@@ -79,7 +79,7 @@ def empty_like_layout(ref: torch.Tensor, shape, dtype=None) -> torch.Tensor:
     return torch.empty_strided(tuple(shape), st, dtype=dtype or ref.dtype, device=ref.device)
 
 
-def _bias_view(attn_bias, B, Hq, L, S, repack_for=None):
+def _bias_view(attn_bias, B, Hq, L, S, repack_for=None, any_tail=False):
     """``attn_bias`` expanded to ``(B,Hq,L,S)`` (stride 0 on broadcast dims) and its dtype id.
 
     ``repack_for``: the dtype of the query, for calls that may run in the matrix-op kernels.  Those read
@@ -88,14 +88,15 @@ def _bias_view(attn_bias, B, Hq, L, S, repack_for=None):
     number of keys that is no multiple of four) is copied once, over its own extents - broadcast dims
     stay broadcast - into a layout they take: the same dtype where that can be aligned, float32
     otherwise (an additive 0 / -inf tensor for a bool mask).  One pass over the bias, against a call
-    that would otherwise leave the matrix-op kernels altogether."""
+    that would otherwise leave the matrix-op kernels altogether.  ``any_tail``: a 16-bit bias over an odd
+    number of keys is taken as it is when its rows start on dwords (the forward for 16-bit inputs does)."""
     if attn_bias is None:
         return None, 0
     b = attn_bias
     while b.dim() < 4:
         b = b.unsqueeze(0)
     b = b.expand(B, Hq, L, S)
-    if repack_for is not None and not _dword_rows(b, S):
+    if repack_for is not None and not _dword_rows(b, S, any_tail and repack_for != torch.float32):
         own = b[tuple(slice(0, 1) if (b.stride(i) == 0 and b.size(i) > 1) else slice(None) for i in range(4))]
         if own.dtype == torch.bool:
             tgt = repack_for if (S % 2 == 0 and repack_for in (torch.float16, torch.bfloat16)) else torch.float32
@@ -135,13 +136,13 @@ def _keep_rows(keep, B, Hq, L, S, dtype):
     return out
 
 
-def _dword_rows(b, S) -> bool:
+def _dword_rows(b, S, any_tail=False) -> bool:
     if b.dtype not in (torch.bool, torch.float16, torch.bfloat16, torch.float32):
         return True  # (not a dtype the matrix-op kernels take: nothing to gain)
     gran = max(4 // b.element_size(), 1)
     if S > 1 and b.stride(3) != 1:
         return False
-    if b.data_ptr() % 4 != 0 or S % gran != 0:
+    if b.data_ptr() % 4 != 0 or (S % gran != 0 and not (any_tail and gran == 2)):
         return False
     return all(b.size(i) <= 1 or b.stride(i) % gran == 0 for i in range(3))
 
@@ -289,7 +290,8 @@ def sdpa_forward(query, key, value, attn_bias=None, is_causal=False, scale=None,
     bias = attn_bias
     if bias is not None:
         B, Hq, S = query.shape[0], query.shape[1], key.shape[2]
-        bias = _bias_view(attn_bias, B, Hq, L, S, repack_for=None if force_kernel == _lib.KERNEL_GENERIC else query.dtype)[0]
+        bias = _bias_view(attn_bias, B, Hq, L, S, repack_for=None if force_kernel == _lib.KERNEL_GENERIC else query.dtype,
+                          any_tail=True)[0]
     p = _lib.FwdParams()
     out, lse, _hold = _lib.host().forward(C.addressof(p), query, key, value, bias, need_lse, bool(is_causal), scale,  # noqa: F841
                                           force_kernel, seq_major_out)  # (_hold: copies that the launch reads)
