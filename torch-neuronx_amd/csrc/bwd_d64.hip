@@ -6,6 +6,7 @@
 //                           S^T = K Q^T, dP^T = V dO^T, dS^T = P^T (dP^T - delta), dQ^T += K^T dS^T
 //                         it also forms delta = rowsum(dO * O) and leaves it, with the log2-domain
 //                         log-sum-exp, in the workspace for the second kernel
+//                         (with few workgroups both run in one launch, behind one that forms these: see together)
 //   bwd_d64_dkdv_kernel   128 keys per workgroup (4 wavefronts x 32 keys), 64-row query tiles of every head
 //                         of the group (the GQA sum of decompositions.py:2595-2598 happens in registers):
 //                           S = Q K^T, dP = dO V^T, dV^T += dO^T P, dK^T += Q^T dS
@@ -163,12 +164,11 @@ __device__ __forceinline__ BlockMap block_map(int bid, int streams, int n_tiles,
   return m;
 }
 
-template <typename T, bool DROP>
-__global__ __launch_bounds__(256, 3) void bwd_d64_dq_kernel(BwdM p, uint32_t* keep_bits, int chunk) {
-  __shared__ __attribute__((aligned(16))) uint16_t k_t[3][TILE];
-  __shared__ __attribute__((aligned(16))) uint16_t v_t[3][TILE];
+// (TERMS: leaves delta and the log2-domain log-sum-exp behind)
+template <typename T, bool DROP, bool TERMS>
+__device__ __forceinline__ void dq_body(const BwdM& p, uint32_t* keep_bits, int bid, int chunk, uint16_t (*k_t)[TILE], uint16_t (*v_t)[TILE]) {
   const int rep = p.Hq / p.Hkv;
-  const BlockMap bm = block_map(blockIdx.x, p.B * p.Hkv, p.n_qt, rep, chunk);
+  const BlockMap bm = block_map(bid, p.B * p.Hkv, p.n_qt, rep, chunk);
   const int qt = p.n_qt - 1 - bm.tile, b = bm.stream / p.Hkv, hk = bm.stream % p.Hkv, h = hk * rep + bm.unit;  // heavy query tiles first
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -237,7 +237,7 @@ __global__ __launch_bounds__(256, 3) void bwd_d64_dq_kernel(BwdM p, uint32_t* ke
     dl = dsum + __shfl_xor(dsum, 32, 64);
     // +inf turns exp2(x - lse) into 0 for rows past L and for rows without a live key
     lse2 = (qrow < p.L && l != -INFINITY) ? l * kLog2eF : INFINITY;
-    if (qrow < p.L && half == 0) p.delta[idx] = dl, p.lse2[idx] = lse2;
+    if (TERMS && qrow < p.L && half == 0) p.delta[idx] = dl, p.lse2[idx] = lse2;
   }
   TileReads rd;
   rd.init(lane);
@@ -323,26 +323,28 @@ __global__ __launch_bounds__(256, 3) void bwd_d64_dq_kernel(BwdM p, uint32_t* ke
   store_rows<T>(acc, p.scale, &k_t[0][0] + wave * 32 * D, lane, (uint16_t*)p.gq + b * p.gq_sb + h * p.gq_sh, p.gq_sl, qw0, p.L, dr);
 }
 
-// OCC: workgroups per compute unit that the registers are kept to.  Three is better where there are that many
-// (B=32, 12 heads, S=512: 123 us for the whole backward against 127 with two, B=4, 32 heads, S=4096 causal 997
-// / 1033), two where there are not (B=4, 12 heads, S=1024 causal, 384 workgroups: 54 / 58; at three a few
-// values go to scratch) and with dropout (193 registers; B=32, 12 heads, S=512 155 / 161, B=4, 16, S=2048 causal 198 / 229).
-template <typename T, bool DROP, int OCC>
-__global__ __launch_bounds__(256, OCC) void bwd_d64_dkdv_kernel(BwdM p, const uint32_t* keep_bits, int chunk) {
-  __shared__ __attribute__((aligned(16))) uint16_t q_t[3][TILE];
-  __shared__ __attribute__((aligned(16))) uint16_t do_t[3][TILE];
-  __shared__ __attribute__((aligned(16))) float lse_s[3][BQ], dl_s[3][BQ];
-  __shared__ __attribute__((aligned(16))) uint32_t bit_s[DROP ? 3 : 1][DROP ? 4 : 1][BQ];  // [buffer][wavefront's 32 keys][row]
+template <typename T, bool DROP>
+__global__ __launch_bounds__(256, 3) void bwd_d64_dq_kernel(BwdM p, uint32_t* keep_bits, int chunk) {
+  __shared__ __attribute__((aligned(16))) uint16_t k_t[3][TILE];
+  __shared__ __attribute__((aligned(16))) uint16_t v_t[3][TILE];
+  dq_body<T, DROP, true>(p, keep_bits, blockIdx.x, chunk, k_t, v_t);
+}
+
+template <bool DROP>
+using KeepTile = uint32_t[DROP ? 4 : 1][BQ];  // [wavefront's 32 keys][row]
+template <typename T, bool DROP>
+__device__ __forceinline__ void dkdv_body(const BwdM& p, const uint32_t* keep_bits, int bid, int chunk, uint16_t (*q_t)[TILE], uint16_t (*do_t)[TILE],
+                                          float (*lse_s)[BQ], float (*dl_s)[BQ], KeepTile<DROP>* bit_s) {
   const int streams = p.B * p.Hkv;
   // (the launch order and the split of a key block's items over workgroups: see bwd_dkdv_w32.hip)
   int kt, st, ph = 0, pq = 0;
   if (p.parts > 1) {
     const int vstreams = streams * p.parts_h;
-    const int v = blockIdx.x % vstreams, rest = blockIdx.x / vstreams;
+    const int v = bid % vstreams, rest = bid / vstreams;
     kt = rest % p.n_kt, pq = rest / p.n_kt;
     st = v / p.parts_h, ph = v % p.parts_h;
   } else {
-    const BlockMap bm = block_map(blockIdx.x, streams, p.n_kt, 1, chunk);
+    const BlockMap bm = block_map(bid, streams, p.n_kt, 1, chunk);
     kt = bm.tile, st = bm.stream;  // low key tiles see the most queries under a causal mask: first
   }
   const int b = st / p.Hkv, hk = st % p.Hkv;
@@ -523,6 +525,54 @@ __global__ __launch_bounds__(256, OCC) void bwd_d64_dkdv_kernel(BwdM p, const ui
   store_rows<T>(dv, DROP ? p.keep_scale : 1.f, &do_t[0][0] + wave * 32 * D, lane, (uint16_t*)p.gv + b * p.gv_sb + hk * p.gv_sh, p.gv_sl, kw0, p.S, dr);
 }
 
+// OCC: workgroups per compute unit that the registers are kept to.  Three is better where there are that many
+// (B=32, 12 heads, S=512: 123 us for the whole backward against 127 with two, B=4, 32 heads, S=4096 causal 997
+// / 1033), two where there are not (B=4, 12 heads, S=1024 causal, 384 workgroups: 54 / 58; at three a few
+// values go to scratch) and with dropout (193 registers; B=32, 12 heads, S=512 155 / 161, B=4, 16, S=2048 causal 198 / 229).
+template <typename T, bool DROP, int OCC>
+__global__ __launch_bounds__(256, OCC) void bwd_d64_dkdv_kernel(BwdM p, const uint32_t* keep_bits, int chunk) {
+  __shared__ __attribute__((aligned(16))) uint16_t q_t[3][TILE];
+  __shared__ __attribute__((aligned(16))) uint16_t do_t[3][TILE];
+  __shared__ __attribute__((aligned(16))) float lse_s[3][BQ], dl_s[3][BQ];
+  __shared__ __attribute__((aligned(16))) KeepTile<DROP> bit_s[DROP ? 3 : 1];
+  dkdv_body<T, DROP>(p, keep_bits, blockIdx.x, chunk, q_t, do_t, lse_s, dl_s, bit_s);
+}
+
+// Both in one launch, behind bwd_d64_terms_kernel: a dK/dV and a dQ workgroup by turns, eight of each (the XCDs), the
+// heaviest of both first.  (See together for where.)
+template <typename T>
+__global__ __launch_bounds__(256, 3) void bwd_d64_both_kernel(BwdM p, int dq_blocks, int dkdv_blocks, int dq_chunk, int dkdv_chunk) {
+  __shared__ __attribute__((aligned(16))) uint16_t a_t[3][TILE];
+  __shared__ __attribute__((aligned(16))) uint16_t b_t[3][TILE];
+  __shared__ __attribute__((aligned(16))) float lse_s[3][BQ], dl_s[3][BQ];
+  const int eight = blockIdx.x >> 3, in = blockIdx.x & 7, turns = min(dq_blocks + 7, dkdv_blocks + 7) >> 3;
+  const bool dq = eight < 2 * turns ? (eight & 1) != 0 : dq_blocks > dkdv_blocks;
+  const int bid = (eight < 2 * turns ? eight >> 1 : eight - turns) * 8 + in;
+  if (bid >= (dq ? dq_blocks : dkdv_blocks)) return;
+  if (dq) dq_body<T, false, false>(p, nullptr, bid, dq_chunk, a_t, b_t);
+  else dkdv_body<T, false>(p, nullptr, bid, dkdv_chunk, a_t, b_t, lse_s, dl_s, nullptr);
+}
+
+// delta and the log2-domain log-sum-exp of 32 rows per wavefront, the sums in dq_body's order
+template <typename T>
+__global__ __launch_bounds__(256) void bwd_d64_terms_kernel(BwdM p, int blocks32) {
+  const int lane = threadIdx.x & 63, col = lane & 31, half = lane >> 5;
+  const int64_t w = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6), bh = w / blocks32;
+  const int row = (int)(w % blocks32) * 32 + col;
+  if (bh >= (int64_t)p.B * p.Hq || row >= p.L) return;  // (both halves of a row, which the shuffle pairs)
+  const int b = (int)(bh / p.Hq), h = (int)(bh % p.Hq);
+  const uint16_t* gr = (const uint16_t*)p.go + b * p.go_sb + h * p.go_sh + (int64_t)row * p.go_sl + half * 8;
+  const uint16_t* orow = (const uint16_t*)p.out + b * p.o_sb + h * p.o_sh + (int64_t)row * p.o_sl + half * 8;
+  float dsum = 0.f;
+#pragma unroll
+  for (int ks = 0; ks < KS; ++ks)
+    if (half * 8 + ks * 16 < p.d_real) dsum += dot8<T>(*(const u32x4*)(gr + ks * 16), *(const u32x4*)(orow + ks * 16));
+  const float dl = dsum + __shfl_xor(dsum, 32, 64);
+  const int64_t idx = bh * p.L + row;
+  const float l = p.lse[idx];
+  if (half == 0) p.delta[idx] = dl, p.lse2[idx] = l != -INFINITY ? l * kLog2eF : INFINITY;
+}
+
 // streams of an XCD whose two tensors of `rows` rows fill half of its 4 MB of L2
 int stream_chunk(const BwdM& g, int64_t rows) {
   const int streams = g.B * g.Hkv;
@@ -549,8 +599,39 @@ bool w32_both(const BwdM& g) {
   return g.causal && g.keep_scale == 0.f && !g.kv_lens && g.d_real == D && (int64_t)g.B * g.Hkv * g.n_kt >= 384 && tiles > 512 && tiles <= 768 && g.L > 14 * BQ;
 }
 
+// Calls whose two kernels leave the chip half empty, each for as long as its longest chain of tiles: one launch of both.
+// Up to one workgroup per compute unit in all, nobody shares anything; beyond it a causal call's long workgroups run
+// beside short ones, up to three per compute unit, where the chains are long enough to pay for the third kernel in front
+// (4 us) and for the registers (168, some in scratch).  Workgroups in all and us, two launches / one (12 heads, D=64):
+//   up to 256: S=64, 6 heads 11.0 / 10.4;  B=4, S=197 not causal 19.8 / 17.9;  B=2, S=512 not causal 28.7 / 24.0;  B=1, S=1024 46.8 / 38.8
+//     336: B=2, S=785 not causal 43.2 / 42.8;  384: B=8, S=197 not causal 20.5 / 21.9
+//   causal, 384: B=16, 6 heads, S=200 19.3 / 18.3;  B=16, S=128 16.2 / 16.7;  grouped, 384: 16/4 heads, S=1021 47.6 / 41.1
+//     512: B=4, 16/4, S=500 42.8 / 38.6;  1536: B=2, 32/8, S=1000 77.2 / 78.3;  768: B=16, S=256 25.6 / 26.9;  B=8, S=512 34.9 / 32.7;  B=4, S=1024 55.1 / 49.6
+//     1024: B=8, 16 heads, S=512 39.0 / 44.8;  B=4, 16, S=1024 58.3 / 55.5;  B=2, 16, S=2048 96.2 / 85.5;  1152: B=12, S=512 56.0 / 57.9
+bool together(const BwdM& g) {
+  if (g.keep_scale != 0.f || w32_dkdv(g)) return false;
+  const int64_t all = (int64_t)g.B * g.Hq * g.n_qt + (int64_t)g.B * g.Hkv * g.n_kt * g.parts;
+  return all <= (!g.causal || g.L < 3 * BQ ? 256 : g.L < 7 * BQ ? 384 : g.Hq > g.Hkv ? 512 : g.L <= 14 * BQ ? 768 : 1024);
+}
+
+template <typename T>
+int launch_together(const BwdM& g, hipStream_t s) {
+  const int blocks32 = (g.L + 31) / 32;
+  hipLaunchKernelGGL((bwd_d64_terms_kernel<T>), dim3((unsigned)(((int64_t)g.B * g.Hq * blocks32 + 3) / 4)), dim3(256), 0, s, g, blocks32);
+  if (int rc = check_launch("bwd_d64_terms_kernel")) return rc;
+  const int dq = g.B * g.Hq * g.n_qt, dkdv = g.B * g.Hkv * g.n_kt * g.parts;
+  const int grid = ((dq + 7) / 8 + (dkdv + 7) / 8) * 8;
+  hipLaunchKernelGGL((bwd_d64_both_kernel<T>), dim3(grid), dim3(256), 0, s, g, dq, dkdv, stream_chunk(g, g.S), stream_chunk(g, (int64_t)g.L * (g.Hq / g.Hkv)));
+  return check_launch("bwd_d64_both_kernel");
+}
+
 template <typename T, bool DROP>
 int launch_t(const BwdM& g, uint32_t* bits, hipStream_t s) {
+  if (!DROP && together(g)) {
+    const int rc = launch_together<T>(g, s);
+    if (rc || g.parts == 1) return rc;
+    return launch_bwd_dkdv_merge(g, std::is_same<T, bf16_t>::value ? MI355_SDPA_BF16 : MI355_SDPA_F16, s);
+  }
   hipLaunchKernelGGL((bwd_d64_dq_kernel<T, DROP>), dim3((unsigned)((int64_t)g.B * g.Hq * g.n_qt)), dim3(256), 0, s, g, bits, stream_chunk(g, g.S));
   int rc = check_launch("bwd_d64_dq_kernel");
   if (rc) return rc;
