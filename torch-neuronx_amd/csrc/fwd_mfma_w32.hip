@@ -1158,6 +1158,24 @@ int launch_dims(const FwdM& g, int head_dim, int waves, int mask, dim3 grid, hip
 
 }  // namespace
 
+// 129 to 256 rows and one head per kv head: two workgroups of four wavefronts a head instead of one of eight.  Such a call is
+// bound by the start and end of its workgroups, at most eight key tiles apart.  The heads share no K / V, and the second
+// workgroup of a head finds them in L2.  One of eight / two of four in us, self-attention, B x heads:
+//   Head dim up to 64: nothing overlaps with the one workgroup of eight that a compute unit holds; of four the registers leave
+//   room for three, and fewer wavefronts idle (197 rows are four and three).  S=197 not causal: 96 9.4 / 7.8, 192 10.4 / 10.0,
+//   384 17.9 / 14.2, 768 30.1 / 26.4, 2048 71.3 / 63.9;  causal, 768 28.3 / 23.9;  S=145, 768 22.4 / 19.9;  D=56, S=197, 768 29.5 / 25.0.
+//   S=256: 128 10.2 / 8.4, 384 19.3 / 15.8, 768 causal 31.9 / 29.0, not causal 34.3 / 37.9: eight full wavefronts in three whole
+//   turns, so there it stays one past 224 rows.  (Four wavefronts per SIMD, in 128 registers with scratch: 35.1 at S=197, 768.)
+//   Head dim up to 128, where a compute unit holds eight wavefronts either way: as long as each workgroup has one to itself.
+//   D=128: 128 heads, S=145 10.7 / 9.5, S=256 13.6 / 11.9;  256 heads 13.1 / 14.3, 19.5 / 21.2.
+// Calls whose halves share out the keys (share_keys) or whose keys would be split keep the one workgroup.
+static bool two_workgroups(const FwdM& g, int head_dim) {
+  if (g.Hq != g.Hkv || g.bias_kind != 0 || g.L <= 128 || g.L > 256) return false;
+  const int64_t heads = (int64_t)g.B * g.Hq, wg64 = heads * ((g.L + 63) / 64);
+  if (wg64 <= (head_dim == 64 && g.causal ? 512 : 256) || (heads < 256 && g.S > 480)) return false;
+  return head_dim == 64 ? g.causal || g.L <= 224 || heads <= 512 : head_dim == 128 && heads <= 128;
+}
+
 // Grouped mode: every head of a kv group in one workgroup when their rows fit its wavefronts (four
 // wavefronts where they do, eight otherwise; for up to 32 query rows also a share of the group's
 // heads per workgroup) and there is no dropout mask and no bias that depends
@@ -1176,6 +1194,7 @@ void fwd_w32_plan(FwdM& g, int head_dim, int& waves) {
   if ((g.bias_kind == 0 || g.bias_sh == 0) && g.keep_scale == 0.f && !g.live_tiles) {
     const int blocks32 = (g.L + 31) / 32;  // 32-row blocks per head
     if (4 % rep == 0 && blocks32 * rep <= 4) waves = 4, g.grouped = rep;
+    else if (two_workgroups(g, head_dim)) waves = 4;
     else if (head_dim != 256 && 8 % rep == 0 && blocks32 * rep <= 8) waves = 8, g.grouped = rep;
     else if (blocks32 == 1) {
       // a decode step with more heads per kv head than wavefronts, or a number of them that does not
