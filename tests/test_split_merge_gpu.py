@@ -5,6 +5,7 @@ Bounds: a probability and an output element are each rounded to the input dtype 
 bfloat16), which in the 2-norm of a row stays below 2 * 2^-9 = 4e-3 with room for the sums; float32 rows carry
 the exponent's rounding, 2e-7 per unit of a log-sum-exp of about 10, and 1e-5 covers it."""
 
+import ctypes
 import math
 
 import pytest
@@ -95,3 +96,46 @@ def test_nan_keys_of_the_fp8_decode_are_not_dropped(amd, gpu_device, B, S, part,
     one = torch.ones(B, 8, device=gpu_device)
     out, lse = amd.decode_fp8kv(q, k, v, one, one)
     assert not out.any() and torch.isneginf(lse).all()
+
+
+@pytest.mark.parametrize("dtype,Hq,Hkv,L,D,biased", [
+    (torch.bfloat16, 8, 4, 1, 128, False),   # at most 16 rows a kv head
+    (torch.float16, 8, 8, 2, 64, False),
+    (torch.bfloat16, 8, 4, 1, 128, True),
+    (torch.float16, 8, 4, 1, 96, False),
+    (torch.bfloat16, 4, 4, 40, 128, False),  # 32 query rows a wavefront
+    (torch.bfloat16, 8, 8, 1, 256, False),
+    (torch.float32, 8, 4, 1, 64, False),
+])
+@pytest.mark.parametrize("where", ["a query row", "a key", "every key"])
+def test_a_nan_stays_in_its_row_with_and_without_parts(amd, gpu_device, dtype, Hq, Hkv, L, D, biased, where):
+    """Rows that a NaN reaches are NaN with lse = -inf, whether the keys are split (the NaN in one part of them) or not; the
+    other rows are those of the call without it, bit for bit."""
+    S = 2048
+    g = torch.Generator(device=gpu_device).manual_seed(D)
+    q, k, v = (torch.randn(1, h, n, D, generator=g, device=gpu_device).to(dtype) for h, n in ((Hq, L), (Hkv, S), (Hkv, S)))
+    bias = torch.randn(1, 1, 1, S, generator=g, device=gpu_device).expand(1, Hq, L, S) if biased else None
+
+    def call(workspace):
+        p = amd._lib.FwdParams()
+        out, lse, _ = amd._lib.host().forward(ctypes.addressof(p), q, k, v, bias, True, False, D**-0.5, 0, False)
+        lib = amd._lib.load()
+        need = lib.mi355_sdpa_fwd_workspace_bytes(ctypes.byref(p))
+        assert need > 0  # (the keys are split)
+        ws = torch.empty(need if workspace else 0, dtype=torch.uint8, device=gpu_device)
+        if workspace:
+            p.workspace, p.workspace_bytes = ws.data_ptr(), need
+        amd._lib.check(lib.mi355_sdpa_fwd(ctypes.byref(p), amd._lib.current_stream(q.device)))
+        return out, lse
+
+    clean = [call(w) for w in (True, False)]
+    reached = torch.zeros(1, Hq, L, dtype=torch.bool, device=gpu_device)
+    if where == "a query row":
+        q[0, 1, L - 1] = math.nan
+        reached[0, 1, L - 1] = True
+    else:
+        k[0, 0, 1500 if where == "a key" else slice(None)] = math.nan
+        reached[0, : Hq // Hkv] = True
+    for (want, want_lse), (out, lse) in zip(clean, [call(w) for w in (True, False)]):
+        assert bool(out[reached].isnan().all()) and bool((lse[reached] == -math.inf).all())
+        assert torch.equal(out[~reached], want[~reached]) and torch.equal(lse[~reached], want_lse[~reached])

@@ -23,6 +23,7 @@
 //                         sum of decompositions.py:2569-2599 happens in registers) and 32-row tiles
 #include "bwd_mfma.h"
 #include "fwd_mfma.h"
+#include "split_merge.h"
 
 namespace mi355 {
 namespace {
@@ -287,7 +288,7 @@ __global__ __launch_bounds__(64 * WAVES, 1) void fwd_f32_kernel(FwdM p) {
           *(f32x4*)(orow + d) = f32x4{oacc[db][g * 4] * inv, oacc[db][g * 4 + 1] * inv, oacc[db][g * 4 + 2] * inv, oacc[db][g * 4 + 3] * inv};
       }
     if (part) {
-      if (half == 0) p.part_lse[prow] = lse_row;
+      if (half == 0) p.part_lse[prow] = part_lse_of(l_tot, lse_row);
     } else if (p.lse && half == 0) {
       p.lse[((int64_t)b * p.Hq + h) * p.L + qrow] = lse_row;
     }

@@ -20,6 +20,7 @@
 #include <algorithm>
 
 #include "fwd_mfma.h"
+#include "split_merge.h"
 
 namespace mi355 {
 namespace {
@@ -205,8 +206,7 @@ __global__ __launch_bounds__(64 * kWaves, 2) void fwd_few_rows_kernel(FwdM p) {
     if (p.n_split > 1) {
       const int64_t prow = (((int64_t)b * p.Hq + h) * p.n_split + split) * p.L + l;
       *(f32x4*)(p.part_o + prow * D + d) = o * inv;
-      // (a sum that is NaN keeps its part in the merge, whose row is NaN then)
-      if (d == 0) p.part_lse[prow] = L == 0.f || L > 0.f ? lse : 0.f;
+      if (d == 0) p.part_lse[prow] = part_lse_of(L, lse);
     } else {
       *(u32x2*)((T*)p.out + b * p.o_sb + h * p.o_sh + l * p.o_sl + d) = u32x2{Mma<T>::pack(o[0] * inv, o[1] * inv), Mma<T>::pack(o[2] * inv, o[3] * inv)};
       if (d == 0 && p.lse) p.lse[((int64_t)b * p.Hq + h) * p.L + l] = lse;

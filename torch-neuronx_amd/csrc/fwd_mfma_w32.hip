@@ -983,7 +983,7 @@ __device__ __forceinline__ void fwd_w32_body(const FwdM& p, const MaskArgs ma) {
             if (d < drv)
               *(f32x4*)(po + d) = f32x4{oacc[db][g * 4] * inv, oacc[db][g * 4 + 1] * inv, oacc[db][g * 4 + 2] * inv, oacc[db][g * 4 + 3] * inv};
           }
-        if (half == 0) p.part_lse[prow] = lse_row;
+        if (half == 0) p.part_lse[prow] = part_lse_of(l_tot, lse_row);
       }
       return;
     }

@@ -19,6 +19,11 @@ namespace mi355 {
 constexpr int kMergeFew = 4, kMergeMany = 16;
 static inline int merge_slices_for(int64_t parts) { return parts > 16 ? kMergeMany : kMergeFew; }
 
+// What a part of a forward call leaves as its row's log-sum-exp, l being the sum behind it.  A row whose sum is NaN has
+// lse = -inf like one without a live key, but must not pass for one here, or the parts without the NaN would be the result:
+// it leaves the NaN, and the merged row is NaN too (with lse = -inf), as it is where the keys are not split.
+__device__ __forceinline__ float part_lse_of(float l, float lse) { return l == l ? lse : l; }
+
 template <int SLICES, int TPR>
 struct MergeLds {
   float o[SLICES][TPR * 4];
@@ -26,10 +31,11 @@ struct MergeLds {
 };
 
 // ml(c, m, l): statistics of part c, m in the log2 domain or (LN) the natural one (m = -inf: a part without
-// keys, its row is never used whatever it holds).  (The domain is the caller's: a log-sum-exp turned into the other
-// one and back takes two roundings of its own size, lse 4.1e-7 -> 4.4e-7 off at float32, 8 heads, S=2048; here only
-// differences are converted.)  row(c): this thread's four columns of part c.  Workgroup of SLICES * TPR threads;
-// on return thread d < 4 * TPR holds column d of the weighted sum (O), and M and L are those of the row.
+// keys, its row is never used whatever it holds; m = NaN: the merged row is NaN).  (The domain is the caller's: a
+// log-sum-exp turned into the other one and back takes two roundings of its own size, lse 4.1e-7 -> 4.4e-7 off at
+// float32, 8 heads, S=2048; here only differences are converted.)  row(c): this thread's four columns of part c.
+// Workgroup of SLICES * TPR threads; on return thread d < 4 * TPR holds column d of the weighted sum (O), and M and L are
+// those of the row.
 template <bool LN, int SLICES, int TPR, typename ML, typename ROW>
 __device__ __forceinline__ void merge_parts(MergeLds<SLICES, TPR>& lds, int np, ML ml, ROW row, float& O, float& M, float& L) {
   static_assert(SLICES >= 4, "one thread per column at the end");
@@ -73,11 +79,11 @@ __device__ __forceinline__ void merge_parts(MergeLds<SLICES, TPR>& lds, int np, 
   M = -INFINITY, L = 0.f, O = 0.f;
 #pragma unroll
   for (int s = 0; s < SLICES; ++s) M = fmaxf(M, lds.m[s]);
-  if (M == -INFINITY) return;
+  const float ref = M == -INFINITY ? 0.f : M;  // (as above: no part with a score, or none but those with a NaN)
   const int d = min((int)threadIdx.x, 4 * TPR - 1);
 #pragma unroll
   for (int s = 0; s < SLICES; ++s) {
-    const float w = weight(lds.m[s] - M);
+    const float w = weight(lds.m[s] - ref);
     L = fmaf(lds.l[s], w, L);
     O = fmaf(lds.o[s][d], w, O);
   }
