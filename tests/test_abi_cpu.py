@@ -348,3 +348,15 @@ def test_hot_kernels_use_no_scratch_and_keep_their_occupancy():
     for name, r in fwd.items():
         d = int(re.search(r"Li(\d+)ELi\d+ELi\d+E(?:Lb[01]E)?E", name).group(1))
         assert int(r["Occupancy_[waves/SIMD]"]) >= (1 if d > 128 else 2), name
+
+
+@pytest.mark.parametrize("B,Hq,Hkv,L,S,D,split", [
+    (8, 32, 8, 1, 2049, 128, True), (1, 32, 8, 1, 1000, 64, True), (40, 32, 8, 1, 4096, 128, True),
+    (64, 12, 12, 16, 383, 128, False),  # 768 sequences' heads of 16 rows fill the chip: 48 us in two parts each, 29 in one
+    (64, 12, 12, 1, 512, 64, False), (96, 64, 8, 2, 1000, 128, False),
+    (24, 64, 8, 2, 640, 128, False), (12, 32, 8, 1, 400, 128, False),
+])
+def test_a_decode_step_splits_its_keys_where_the_merge_is_the_smaller_part(amd, B, Hq, Hkv, L, S, D, split):
+    t = lambda h, n: amd._lib.Tensor4(4096, (C.c_int64 * 4)(B, h, n, D), (C.c_int64 * 4)(h * n * D, n * D, D, 1))
+    p = amd._lib.FwdParams(q=t(Hq, L), k=t(Hkv, S), v=t(Hkv, S), out=t(Hq, L), dtype=amd._lib.BF16, scale=0.125)
+    assert (amd._lib.load().mi355_sdpa_fwd_workspace_bytes(C.byref(p)) > 0) == split

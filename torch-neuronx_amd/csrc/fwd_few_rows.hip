@@ -226,19 +226,34 @@ bool few_rows_supported(const FwdM& g, int head_dim) {
 // turn that fills the chip in part leaves bandwidth unused (2048 keys: B=20 in 160 workgroups 41.5, 480 34.4; B=40 in 320 71,
 // 640 64, 960 59.6).  At least four steps, one per wavefront, and twelve in all, for less the second launch weighs more
 // (32/8 heads, 1000 keys: 8 parts 8.7, 4 parts 10.0, 2 parts 13.3; 512 keys, B=4: 4 parts 8.9, one 9.9).
+//   No parts at all where what they save, at 6.3 TB/s or 1.75 us a step of a workgroup (head dim 128), is less than the merge
+// costs: 3 us, and 2.5 more per thousand rows (1.75 at head dim 64), a workgroup each, whose parts go to memory and back in
+// float32.  Keys from memory, as planned above / one part, us, D=128: 96 kv heads in all of 16 rows, S=383 12.7 / 11.7, S=2049
+// 26.4 / 38.1;  192 of 16, S=1000 29.9 / 22.7, of one row 24.0 / 22.1;  288 of one row, S=1000 32.2 / 37.8, S=383 18.7 / 18.0;
+// 768 of 16, S=383 48.3 / 29.3, S=1000 88.3 / 65.3, of one row 65.2 / 63.0.  D=64: 288 of 16, S=1000 25.3 / 21.6, S=2049
+// 37.5 / 38.7.  (Beyond 512 workgroups the turns overlap: an unfilled one costs half its idle part.)
 void few_rows_plan(FwdM& g) {
   const int64_t groups = (int64_t)g.B * g.Hkv;
   const int steps = (g.S + kStep - 1) / kStep;
   g.split_tiles = 0, g.n_split = 1;
   if (steps < 12) return;
+  auto filled = [&](int n) {  // share of the chip's turns that `n` parts fill
+    const int64_t wgs = groups * n, slots = wgs <= 256 ? 256 : 512;
+    return (double)wgs / (double)(slots * ((wgs + slots - 1) / slots));
+  };
   int best = 1;
   double best_use = 0.;
   for (int n = 1; n <= std::min(steps / 4, 256) && (n - 1) * groups <= 1024; ++n) {
-    const int64_t wgs = groups * n, slots = wgs <= 256 ? 256 : 512;
-    const double use = (double)wgs / (double)(slots * ((wgs + slots - 1) / slots)) - 0.02 * (n * groups > 256) * (n - 1);
+    const double use = filled(n) - 0.02 * (n * groups > 256) * (n - 1);
     if (use > best_use) best_use = use, best = n;
   }
-  if (best >= 2) {
+  const double width = g.d_real / 128.;
+  auto us = [&](int n) {  // estimated, without the merge
+    const double f = filled(n), use = groups * n <= 512 ? f : 0.5 + 0.5 * f;
+    const int per = (steps + n - 1) / n;
+    return std::max((double)groups * g.S * g.d_real * 4 / 6.3e6 / use, 2.5 + 1.75 * width * ((per + kWaves - 1) / kWaves));
+  };
+  if (best >= 2 && us(1) - us(best) > 3. + (1e-3 + 1.5e-3 * width) * (double)g.B * g.Hq * g.L) {
     g.split_tiles = (steps + best - 1) / best;
     g.n_split = (steps + g.split_tiles - 1) / g.split_tiles;
   }
