@@ -19,6 +19,9 @@ pytestmark = pytest.mark.gpu
     (2, 6, 6, 129, 300, 48, False, [300, 17]),
     (3, 4, 2, 33, 200, 64, True, [0, 200, 64]),  # a batch without a key
     (1, 16, 4, 1021, 1021, 64, True, None),     # parts
+    (2, 12, 4, 192, 192, 64, True, None),       # three heads a kv head: two launches
+    (1, 28, 4, 150, 150, 64, True, None),
+    (1, 16, 2, 193, 193, 56, True, [150]),      # ... parts, past three query tiles: one
     (4, 32, 32, 129, 130, 64, False, None),     # 256 query and 256 key blocks: two launches
     (2, 32, 32, 256, 256, 64, False, None),     # 256 in all are 2 * 32 * 2 * 2
     (8, 12, 12, 511, 511, 64, True, None),      # 768 in all

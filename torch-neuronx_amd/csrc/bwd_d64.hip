@@ -608,8 +608,13 @@ bool w32_both(const BwdM& g) {
 //   causal, 384: B=16, 6 heads, S=200 19.3 / 18.3;  B=16, S=128 16.2 / 16.7;  grouped, 384: 16/4 heads, S=1021 47.6 / 41.1
 //     512: B=4, 16/4, S=500 42.8 / 38.6;  1536: B=2, 32/8, S=1000 77.2 / 78.3;  768: B=16, S=256 25.6 / 26.9;  B=8, S=512 34.9 / 32.7;  B=4, S=1024 55.1 / 49.6
 //     1024: B=8, 16 heads, S=512 39.0 / 44.8;  B=4, 16, S=1024 58.3 / 55.5;  B=2, 16, S=2048 96.2 / 85.5;  1152: B=12, S=512 56.0 / 57.9
+// Three heads per kv head and more, whole chains in dK/dV (three query tiles, or items that are not split): dK/dV walks as
+// many times dQ's tiles, dQ under it saves little, and its chain is the slower one in these registers.  Causal, two launches /
+// one: B=2, 12/4 heads, S=400 46.3 / 47.6;  16/4, S=200 36.9 / 39.7, split, S=400 43.2 / 41.7;  28/4, S=100 33.6 / 36.8, S=150 43.8 / 49.5,
+// split, S=200 34.5 / 33.8;  16/2, S=64 22.8 / 24.9, split, S=150 34.1 / 35.7, S=200 29.9 / 29.1.  (Two heads: 12/6, S=64 13.4 / 12.9, S=400 36.2 / 35.2.)
 bool together(const BwdM& g) {
   if (g.keep_scale != 0.f || w32_dkdv(g)) return false;
+  if (g.Hq >= 3 * g.Hkv && (g.parts == 1 || g.L <= 3 * BQ)) return false;
   const int64_t all = (int64_t)g.B * g.Hq * g.n_qt + (int64_t)g.B * g.Hkv * g.n_kt * g.parts;
   return all <= (!g.causal || g.L < 3 * BQ ? 256 : g.L < 7 * BQ ? 384 : g.Hq > g.Hkv ? 512 : g.L <= 14 * BQ ? 768 : 1024);
 }
