@@ -284,6 +284,24 @@ def test_registered_operator_surface(amd):
     assert hasattr(torch.ops.mi355_kernels, "sdpa_decode_fp8kv")
 
 
+def test_an_extension_that_does_not_register_its_operators_fails_loudly(amd, monkeypatch):
+    class Host:
+        def register_operators(self, *_):
+            raise RuntimeError("no such operator")
+
+    names = sorted(amd.registered_ops())
+    amd.unregister()
+    try:
+        with monkeypatch.context() as m:
+            m.setattr(amd._lib, "host", Host)
+            with pytest.raises(RuntimeError, match="no such operator"):
+                amd.register()
+            assert amd.registered_ops() == []
+    finally:
+        amd.register()
+    assert sorted(amd.registered_ops()) == names
+
+
 def test_missing_library_fails_loudly(amd, monkeypatch):
     from torch_neuronx_amd import _lib
 

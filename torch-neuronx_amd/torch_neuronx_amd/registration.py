@@ -51,15 +51,14 @@ def register(override_aten: bool | None = None) -> list:
         ("_scaled_dot_product_fused_attention_overrideable_backward",
          po.scaled_dot_product_fused_attention_overrideable_backward),
     ]
-    native = False
+    host = None
     if override_aten:
-        table += [("_fused_sdp_choice", impl.fused_sdp_choice)]
         try:
-            _registered.extend(_lib.host().register_operators(vars(ops), vars(impl)))
-            native = True
+            host = _lib.host()
         except (RuntimeError, OSError, ImportError):
             pass  # (not built yet, or for other structures: the functions below say so when they are called)
-    if override_aten and not native:
+        table += [("_fused_sdp_choice", impl.fused_sdp_choice)]
+    if override_aten and host is None:
         table += [
             ("_scaled_dot_product_flash_attention", po.scaled_dot_product_flash_attention),
             ("_scaled_dot_product_flash_attention_backward", po.scaled_dot_product_flash_attention_backward),
@@ -67,11 +66,18 @@ def register(override_aten: bool | None = None) -> list:
             ("_scaled_dot_product_efficient_attention_backward",
              po.scaled_dot_product_efficient_attention_backward),
         ]
-    with warnings.catch_warnings():
-        warnings.simplefilter("ignore")  # "overriding a previously registered kernel" is the point
-        for name, fn in table:
-            lib.impl(name, fn, "CUDA")
-            _registered.append(name)
+    try:
+        with warnings.catch_warnings():
+            warnings.simplefilter("ignore")  # "overriding a previously registered kernel" is the point
+            for name, fn in table:
+                lib.impl(name, fn, "CUDA")
+                _registered.append(name)
+        if host is not None:
+            _registered.extend(host.register_operators(vars(ops), vars(impl)))
+    except BaseException:
+        lib._destroy()
+        _registered.clear()
+        raise
     _lib_handle = lib
     return list(_registered)
 
