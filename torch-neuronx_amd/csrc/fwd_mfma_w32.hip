@@ -1121,8 +1121,10 @@ template <typename T, int D, int MASK, bool PATTERN>
 int launch_halves(FwdM g, int rows, hipStream_t s) {
   g.grouped = 0, g.n_qt = (g.L + rows - 1) / rows;
   const dim3 grid((unsigned)((int64_t)g.B * g.Hq * g.n_qt));
-  if (rows == 64) return launch_one<T, D, 2, MASK, PATTERN, 2>(g, grid, s);
-  return launch_one<T, D, 4, MASK, PATTERN, 2>(g, grid, s);
+  if constexpr (D == 128) {  // (128 rows: this width only)
+    if (rows == 128) return launch_one<T, D, 4, MASK, PATTERN, 2>(g, grid, s);
+  }
+  return launch_one<T, D, 2, MASK, PATTERN, 2>(g, grid, s);
 }
 
 template <typename T, int D, int WAVES>
