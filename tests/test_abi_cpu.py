@@ -342,9 +342,14 @@ def test_hot_kernels_use_no_scratch_and_keep_their_occupancy():
     # waits for every load at once (no counted waits), so a spill there costs time, not correctness.
     known = re.compile(r"bwd_wide_dkdv_kernelIDF16[b_]Li256ELi256ELi([0123])ELb([01])EE")
     for name, r in rows.items():
-        if r["src"] not in ("fwd_mfma_w32.hip", "bwd_dq_w32.hip", "bwd_dkdv_w32.hip", "bwd_wide.hip", "decode_fp8kv.hip"):
+        if r["src"] not in ("fwd_mfma_w32.hip", "fwd_few_rows.hip", "bwd_dq_w32.hip", "bwd_dkdv_w32.hip", "bwd_wide.hip", "bwd_d64.hip", "decode_fp8kv.hip"):
             continue
         scratch = int(r["ScratchSize_[bytes/lane]"])
+        if re.search(r"bwd_d64_(both_kernel|dkdv_kernelIDF16[b_]Lb0ELi3E)", name):
+            # three workgroups per compute unit want 168 registers: a few values beyond that go to scratch, which measured
+            # better than two (the file waits for every load at once, no counted waits)
+            assert scratch <= 48, (name, scratch)
+            continue
         if "decode_kernelIfLi256ELi1ELi3EE" in name:  # float32 queries at head dim 256, 9-16 rows: a dozen bytes, no counted waits there
             assert scratch <= 16, (name, scratch)
             continue

@@ -95,3 +95,19 @@ def test_an_infinite_or_nan_row_stays_its_own(amd, gpu_device):
     out, _ = amd.sdpa_forward(q, k, v)
     bad = out.isnan().any(-1)
     assert bool(bad[0, 0, 5]) and int(bad.sum()) == 1
+
+
+def test_a_long_causal_call_and_its_prefix(amd, gpu_device):
+    """The first rows depend on the first keys only.  A call that names its kernel sums them in the same order whatever
+    follows; one that does not may share them out differently, which moves a result by its rounding (the bounds above)."""
+    g = torch.Generator(device=gpu_device).manual_seed(8)
+    q, k, v = (torch.randn(1, h, 16384, 128, generator=g, device=gpu_device).to(torch.bfloat16) for h in (4, 1, 1))
+    n = 2048
+    for force, bits in ((amd._lib.KERNEL_MFMA, True), (0, False)):
+        out, lse = amd.sdpa_forward(q, k, v, is_causal=True, force_kernel=force)
+        pre, pre_lse = amd.sdpa_forward(q[:, :, :n], k[:, :, :n], v[:, :, :n], is_causal=True, force_kernel=force)
+        a, b = out[:, :, :n].double(), pre.double()
+        if bits:
+            assert torch.equal(a, b) and torch.equal(lse[:, :, :n], pre_lse)
+        assert float((a - b).norm() / b.norm()) <= 4e-3
+        assert float((lse[:, :, :n] - pre_lse).abs().max()) <= 4e-5  # (2e-5 of each)

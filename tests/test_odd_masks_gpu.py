@@ -41,6 +41,26 @@ def test_forward_takes_an_odd_number_of_keys(amd, gpu_device, dtype, bound, L, S
     assert float((lse.double() - torch.logsumexp(s, -1)).abs().max()) <= 2e-5
 
 
+@pytest.mark.parametrize("dtype,bound", [(torch.bfloat16, 4e-3), (torch.float16, 5e-4)])
+@pytest.mark.parametrize("L,S,pitch,D", [(33, 31, 32, 64), (130, 33, 34, 128), (65, 999, 1008, 128), (5, 97, 98, 64), (40, 129, 130, 256)])
+def test_forward_with_dropout_over_an_odd_number_of_keys(amd, gpu_device, dtype, bound, L, S, pitch, D):
+    """... together with a keep-mask, whose rows are padded to dwords as well."""
+    g = torch.Generator(device=gpu_device).manual_seed(S + 1)
+    B, Hq, Hkv, p = 2, 4, 2, 0.25
+    q, k, v = (torch.randn(B, h, n, D, generator=g, device=gpu_device).to(dtype) for h, n in ((Hq, L), (Hkv, S), (Hkv, S)))
+    rows = torch.full((B, Hq, L, pitch), math.nan, dtype=dtype, device=gpu_device)
+    bias = rows[..., :S]
+    bias.copy_(torch.randn(B, Hq, L, S, generator=g, device=gpu_device))
+    bias[..., 2::3] = -math.inf
+    keep = amd.ops.padded_keep_mask(B, Hq, L, S, q.device).bernoulli_(1 - p, generator=g)
+    out, lse = amd.sdpa_forward(q, k, v, attn_bias=bias, dropout_p=p, dropout_keep=keep, force_kernel=amd._lib.KERNEL_MFMA)
+    kd, vd = (t.double().repeat_interleave(2, 1) for t in (k, v))
+    s = q.double() @ kd.transpose(-1, -2).contiguous() / math.sqrt(D) + bias.double()
+    want = (torch.softmax(s, -1) * keep.double() / (1 - p)) @ vd
+    assert float((out.double() - want).norm() / want.norm()) <= bound
+    assert float((lse.double() - torch.logsumexp(s, -1)).abs().max()) <= 2e-5
+
+
 @pytest.mark.parametrize("dtype", [torch.bool, torch.float16, torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("S,pitch,offset", [(1, 1, 0), (7, 9, 1), (16, 16, 3), (65, 67, 5), (999, 1008, 0), (1030, 1031, 15)])
 def test_row_summaries_from_any_address(amd, gpu_device, dtype, S, pitch, offset):

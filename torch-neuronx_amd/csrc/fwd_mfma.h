@@ -17,8 +17,10 @@ struct FwdM {
   int B, Hq, Hkv, L, S;
   int n_qt;    // query tiles per head
   int causal;
-  // A call that names its kernel sums a row's keys in order whatever the sizes, and so equals a longer call on its prefix;
-  // one with key counts or a verdict equals the call that those stand for, and is left to the sizes.
+  // A call that names its kernel takes no halves (share_keys, fwd_mfma_w32.hip): a causal one so sums each row's keys in order
+  // whatever the sizes, and equals a longer call on its prefix bit for bit.  One with key counts or a verdict equals the call
+  // that those stand for, and is left to the sizes.  Not asked where keys are split or shared out for few rows: such
+  // calls have no causal flag, and a longer one is no prefix of theirs.
   int whole_keys = 0;
   int xcd_map;  // 1: (batch, kv head) streams are pinned to XCDs
   float scale;
