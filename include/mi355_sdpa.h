@@ -164,7 +164,13 @@ typedef struct mi355_sdpa_fwd_params {
                              this boundary: the reference's operator only ever sees additive
                              masks, because its caller turns a bool mask into 0 / -inf first
                              (decompositions.py:2101-2102); here that conversion, a pass over
-                             L*S elements, is left out and the kernels read the bytes        */
+                             L*S elements, is left out and the kernels read the bytes.
+                             The matrix-op forward for 16-bit inputs takes an F16 / BF16
+                             bias over an odd number of keys, in rows that start on 4-byte
+                             words, as it is: it reads each row to the end of the word that
+                             its last element starts, so the two bytes behind that element
+                             must be readable, behind the last row too (they are in any
+                             allocation of whole words; what they hold is not used)          */
   int32_t bias_dtype;     /* F32/F16/BF16/BOOL                                        */
   const int32_t* kv_lens; /* optional (B,): key j of batch b takes part iff j<kv_lens[b] */
   const uint8_t* dropout_keep; /* optional (B,Hq,L,S), 1 = keep: contiguous, or with rows

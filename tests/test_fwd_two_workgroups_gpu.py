@@ -18,8 +18,8 @@ pytestmark = pytest.mark.gpu
     (128, 4, 225, 225, 64, False, None, 0),   # 512 heads past 224 rows: two
     (129, 4, 225, 225, 64, False, None, 0),   # ... 516: one
     (129, 4, 256, 256, 64, True, None, 0),
-    (43, 6, 197, 700, 64, False, None, 0),    # 258 heads, more keys than rows, no split
-    (40, 6, 197, 700, 64, False, None, 0),    # 240 heads: keys in parts, one workgroup
+    (43, 6, 197, 700, 64, False, None, 0),    # 258 heads, more keys than rows: two
+    (40, 6, 197, 700, 64, False, None, 0),    # 240 heads over more than 480 keys: one workgroup
     (48, 8, 200, 200, 56, False, list(range(0, 48 * 4, 4)), 0),
     (65, 4, 255, 255, 64, True, None, 33),
     (32, 4, 193, 193, 128, True, None, 0),    # 128 heads

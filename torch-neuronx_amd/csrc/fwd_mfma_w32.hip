@@ -1106,8 +1106,13 @@ int launch_one(const FwdM& g, dim3 grid, hipStream_t s) {
 //   11.0 / 9.7; 16 heads, S=256 10.6 / 8.0; D=64: 12 heads, S=1024 13.7 / 9.8, B=2 14.6 / 11.1, S=2048 27.7 / 25.6, not
 //   causal S=785 11.5 / 9.0, S=197 B=4 8.1 / 6.1 (there against one 256-row workgroup per head, see fwd_w32_plan).  Past that a
 //   second turn of workgroups pays the start again: 32/8 heads, S=700 15.2 / 15.7, S=1400 30 / 36; D=64, B=16, S=197 9.1 / 12.5.
-//   128 rows, two wavefronts a SIMD: a long causal chain in front of many short ones.  32/8 heads, D=128: S=1021 21.2 / 20.5,
-//   S=1400 29.7 / 27; 28/4, S=1400 29.2 / 26; 16/4, S=4000 79 / 74; S=2500 60 / 68, two turns.  The exchange costs 1.5 us: S=256 9.0 / 10.2.
+//   128 rows, two wavefronts a SIMD: a long causal chain in front of many short ones, in one turn of two workgroups a compute
+//   unit.  D=128: 32/8 heads, S=1021 19.7 / 18.8, S=1407 28.6 / 25.8; 28/4, S=1407 27.2 / 24.0; 24/8 25.7 / 22.5; 16/4, S=4000
+//   80.7 / 69.3.  More than 512 workgroups: 32/8, S=2057 46.3 / 50.7, S=2500 59.5 / 66.0; 24/8, S=3000 65.0 / 68.0.  The exchange
+//   costs 1.5 us: S=256 9.0 / 10.2.  The bound of 8 * tiles keeps out calls of so many heads that short chains hide each other:
+//   64/8 heads, S=707 19.2 / 22.1, S=1021 26.9 / 29.0.  It is tighter than that needs: of 32 heads it takes the lengths whose last
+//   128 rows are full or nearly so, and those between would gain too (S=907 19.1 / 18.6, 1107 23.0 / 20.2, 1307 26.1 / 25.3,
+//   1907 41.9 / 39.0); 16, 24 and 28 heads are taken throughout.
 int share_keys(const FwdM& g, int head_dim) {
   if (g.whole_keys || g.grouped > 1 || g.split_tiles || g.L <= 32) return 0;
   int tiles = (g.S + BN - 1) / BN;
@@ -1161,8 +1166,8 @@ int launch_dims(const FwdM& g, int head_dim, int waves, int mask, dim3 grid, hip
 }  // namespace
 
 // 129 to 256 rows and one head per kv head: two workgroups of four wavefronts a head instead of one of eight.  Such a call is
-// bound by the start and end of its workgroups, at most eight key tiles apart.  The heads share no K / V, and the second
-// workgroup of a head finds them in L2.  One of eight / two of four in us, self-attention, B x heads:
+// bound by the start and end of its workgroups: in self-attention they are at most eight key tiles apart.  The heads share no
+// K / V, and the second workgroup of a head finds them in L2.  One of eight / two of four in us, self-attention, B x heads:
 //   Head dim up to 64: nothing overlaps with the one workgroup of eight that a compute unit holds; of four the registers leave
 //   room for three, and fewer wavefronts idle (197 rows are four and three).  S=197 not causal: 96 9.4 / 7.8, 192 10.4 / 10.0,
 //   384 17.9 / 14.2, 768 30.1 / 26.4, 2048 71.3 / 63.9;  causal, 768 28.3 / 23.9;  S=145, 768 22.4 / 19.9;  D=56, S=197, 768 29.5 / 25.0.
@@ -1170,7 +1175,11 @@ int launch_dims(const FwdM& g, int head_dim, int waves, int mask, dim3 grid, hip
 //   turns, so there it stays one past 224 rows.  (Four wavefronts per SIMD, in 128 registers with scratch: 35.1 at S=197, 768.)
 //   Head dim up to 128, where a compute unit holds eight wavefronts either way: as long as each workgroup has one to itself.
 //   D=128: 128 heads, S=145 10.7 / 9.5, S=256 13.6 / 11.9;  256 heads 13.1 / 14.3, 19.5 / 21.2.
-// Calls whose halves share out the keys (share_keys) or whose keys would be split keep the one workgroup.
+//   More keys than rows, 197 rows, head dim 64: 384 heads, S=700 33.4 / 25.7, S=1500 62.8 / 45.0, 768 heads 114 / 97.
+// Calls whose halves share out the keys (share_keys) keep the one workgroup.  So do fewer than 256 heads over more than 480
+// keys: without it causal ones fall to share_keys's 64-row kernels, too many turns of them (132 heads of 197 rows, S=1500,
+// head dim 64 9.4 / 11.0, 128 12.1 / 18.9), and at head dim 128 two are the slower form past 72 heads (132 heads, S=700 21.0 / 26.8).
+// (Not causal at head dim 64 two would be the better one there as well: 72 heads, S=700 16.0 / 12.2, 192 17.9 / 17.0.)
 static bool two_workgroups(const FwdM& g, int head_dim) {
   if (g.Hq != g.Hkv || g.bias_kind != 0 || g.L <= 128 || g.L > 256) return false;
   const int64_t heads = (int64_t)g.B * g.Hq, wg64 = heads * ((g.L + 63) / 64);

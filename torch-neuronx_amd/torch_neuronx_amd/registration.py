@@ -13,8 +13,9 @@ by this package.
 * ``aten::_fused_sdp_choice``: reachable through ``torch._fused_sdp_choice``; rules of
   torch_neuronx/csrc/aten/SdpBackendSelection.cpp:14-68.
 
-The flash and memory-efficient pairs are registered natively (``csrc/host_args.cpp``): plain calls never enter the
-interpreter, the others arrive in the Python functions as before.
+The flash and memory-efficient pairs are registered natively (``csrc/host_args.cpp``): plain calls enter the interpreter only
+to ask which kernel they are bound to (the environment switch and replaced functions are honoured on every call), the
+others arrive in the Python functions as before.
 
 Upstream's autograd formulas for these ops call the matching ``_backward`` op, so no
 autograd.Function is needed.
