@@ -184,3 +184,30 @@ def test_every_row_of_the_gradient_in_one_place(amd, gpu_device, L):
     out, lse = amd.sdpa_forward(q, k, v)
     for a, w in zip(amd.sdpa_backward(do, q, k, v, out, lse)[:3], amd.sdpa_backward(do.contiguous(), q, k, v, out, lse)[:3]):
         assert torch.equal(a, w)
+
+
+@pytest.mark.parametrize("p", [0.0, 0.25])
+@pytest.mark.parametrize("Hq,Hkv,L,S,lens", [
+    (1, 1, 3, 2, None), (3, 1, 32, 32, None), (2, 2, 33, 64, None), (2, 1, 64, 96, None), (3, 1, 96, 65, None), (2, 2, 160, 128, [128, 97]),
+    (6, 2, 193, 193, [193, 33]), (8, 1, 640, 129, None),  # (the last: the items of a key block go to several workgroups)
+])
+def test_causal_blocks_in_two_phases_and_one_by_one(amd, gpu_device, Hq, Hkv, L, S, lens, p):
+    """dK/dV takes items whose blocks are all live for a wavefront one block ahead, the others (the diagonal) block by block:
+    none of the first kind, none of the second, both; a first item of fewer than 64 rows."""
+    _check(amd, gpu_device, 2, Hq, Hkv, L, S, 64, True, torch.bfloat16, lens, p)
+
+
+def test_rows_that_a_key_does_not_see_do_not_reach_it(amd, gpu_device):
+    """Under a causal mask a NaN in rows of Q and dO stays with the blocks of 32 keys that have a key which sees them."""
+    B, Hq, Hkv, L, D = 1, 4, 2, 320, 64
+    g = torch.Generator(device=gpu_device).manual_seed(9)
+    q, k, v, do = (torch.randn(B, h, L, D, generator=g, device=gpu_device).to(torch.bfloat16) for h in (Hq, Hkv, Hkv, Hq))
+    out, lse = amd.sdpa_forward(q, k, v, is_causal=True)
+    want = amd.sdpa_backward(do, q, k, v, out, lse, is_causal=True)[:3]
+    for row in (5, 70, 130, 200):
+        qn, dn = q.clone(), do.clone()
+        qn[:, :, row], dn[:, :, row] = math.nan, math.inf
+        got = amd.sdpa_backward(dn, qn, k, v, out, lse, is_causal=True)[:3]
+        clean = (row // 32 + 1) * 32
+        for name, a, w in zip(("dk", "dv"), got[1:], want[1:]):
+            assert torch.equal(a[:, :, clean:], w[:, :, clean:]), (name, row)

@@ -14,9 +14,11 @@
 // At this width a 32 x 32 score block is 16 (dK/dV) or 12 (dQ) matrix ops of 32 cycles against about a
 // hundred vector instructions, and the calls are short (heads of 64 go with sequences of a few hundred
 // to two thousand): what bounds them is neither pipe but the chain score - probability - dS - product of
-// one wavefront and the waits around it.  So nothing here is pipelined by hand; the registers are kept
-// to a third of the file (168) instead, three workgroups share a compute unit, and the chain of one
-// wavefront runs under the other two's (dK/dV with dropout or of at most 512 workgroups: two, see OCC).
+// one wavefront, the instructions it issues one after the other and the waits around them.  The dQ kernel keeps its
+// registers to a third of the file (168), and the chain of one wavefront runs under the other two's of its SIMD; nothing
+// in it is pipelined by hand (in the two phases of the dK/dV kernel it measured the same, 986 / 1004 us for the backward of
+// B=4, 32 heads, S=4096 causal, within 1 % elsewhere, with dropout 2 % slower).  The dK/dV kernel, which holds
+// 128 registers of operands and accumulators, works on two blocks at a time instead (see dkdv_body).
 // A wavefront keeps all four products of its keys (at head dim 128 they do not fit and are split over two
 // wavefronts that exchange P through LDS).
 //
@@ -355,7 +357,6 @@ __device__ __forceinline__ void dkdv_body(const BwdM& p, const uint32_t* keep_bi
   const int k0 = kt * 128, kw0 = k0 + wave * 32, key = kw0 + col;
   const int dr = p.d_real;
   const int S = p.kv_lens ? min(p.S, max(p.kv_lens[b], 0)) : p.S;
-  const int first_q = key >= S ? INT_MAX : p.causal ? key : INT_MIN;  // the first query row that sees this lane's key
   const int nqs = (p.L + BQ - 1) / BQ, qs_begin = p.causal ? min(k0 / BQ, nqs) : 0;
   int n_items = k0 >= S ? 0 : rep * (nqs - qs_begin);  // no live key in this block: zeros
   int it0 = 0;
@@ -364,41 +365,60 @@ __device__ __forceinline__ void dkdv_body(const BwdM& p, const uint32_t* keep_bi
     n_items = max(min(n_items - it0, p.chunk_items), 0);
     if (n_items == 0 && pq > 0) return;  // (bwd_dkdv_merge_kernel counts the filled shares in the same way)
   }
-  // items: query tile by query tile from the last one down, the group's heads inside
-  const uint32_t rep_inv = (uint32_t)((0x100000000ull + (uint32_t)rep - 1) / (uint32_t)rep);
-  auto item_tile = [&](int it) { return rep == 1 ? it + it0 : (int)__umulhi((uint32_t)(it + it0), rep_inv); };
-  auto item_head = [&](int it) { return h0 + (it + it0 - item_tile(it) * rep); };
-  auto item_q0 = [&](int it) { return (nqs - 1 - item_tile(it)) * BQ; };
-
+  // items: query tile by query tile from the last one down, the group's heads inside.  Where the next item to fetch lies:
+  // byte offsets that follow from item to item by one addition each (worked out from an item's number they are a hundred
+  // scalar instructions per item, which the wavefronts issue one after the other like any others)
+  const int t0 = nqs - 1 - it0 / rep, hl0 = it0 % rep;
+  struct {
+    int hl;
+    uint32_t q, go, bit;
+    int64_t stat;
+    uint32_t q_bytes, go_bytes, rows4;  // (the buffers end with the head's last row)
+  } at;
+  const uint32_t q_head = (uint32_t)(p.q_sh * 2), go_head = (uint32_t)(p.go_sh * 2), bit_head = (uint32_t)p.L * 16;
+  const int64_t st_head = (int64_t)p.L * 4;
+  const uint32_t q_tile = (uint32_t)(p.q_sl * BQ * 2), go_tile = (uint32_t)(p.go_sl * BQ * 2);
+  {
+    const int rows = min(p.L - t0 * BQ, BQ);
+    at.hl = hl0;
+    at.q = hl0 * q_head + t0 * q_tile, at.go = hl0 * go_head + t0 * go_tile;
+    at.stat = hl0 * st_head + t0 * (BQ * 4), at.bit = (ph * rep + hl0) * bit_head + t0 * (BQ * 16);
+    at.q_bytes = (uint32_t)((rows - 1) * p.q_sl + dr) * 2, at.go_bytes = (uint32_t)((rows - 1) * p.go_sl + dr) * 2, at.rows4 = rows * 4;
+  }
   const u32x4 bit_rsrc = descriptor(DROP ? keep_bits + ((int64_t)st * p.n_kt + kt) * block_words(p) : nullptr, DROP ? block_words(p) * 4 : 0);
   uint32_t q_off[NCH], go_off[NCH];
   chunk_offsets(q_off, tid, p.q_sl, dr);
   chunk_offsets(go_off, tid, p.go_sl, dr);
   const uint32_t lds_q = lds_address(q_t) + wave * 1024, lds_do = lds_address(do_t) + wave * 1024;
+  const char* const q_base = (const char*)((const uint16_t*)p.q + b * p.q_sb + h0 * p.q_sh);
+  const char* const go_base = (const char*)((const uint16_t*)p.go + b * p.go_sb + h0 * p.go_sh);
+  const char* const stat_base = (const char*)((wave == 0 ? p.lse2 : p.delta) + ((int64_t)b * p.Hq + h0) * p.L);  // (wavefronts 0 and 1)
+  const uint32_t lds_stat = wave == 0 ? lds_address(lse_s) : lds_address(dl_s);
   // (the buffers of an item are its tile's own and end with the head's last row: a row past L must not be another
   // head's, whose NaN would survive the zero probabilities)
-  auto load_item = [&](int it, int buf) {
-    const int h = item_head(it), q0 = item_q0(it), rows = min(p.L - q0, BQ);
-    const u32x4 q_rsrc = descriptor((const uint16_t*)p.q + b * p.q_sb + h * p.q_sh + (int64_t)q0 * p.q_sl, ((int64_t)(rows - 1) * p.q_sl + dr) * 2);
-    const u32x4 go_rsrc = descriptor((const uint16_t*)p.go + b * p.go_sb + h * p.go_sh + (int64_t)q0 * p.go_sl, ((int64_t)(rows - 1) * p.go_sl + dr) * 2);
+  auto load_item = [&](int buf) {
+    const u32x4 q_rsrc = descriptor(q_base + at.q, at.q_bytes), go_rsrc = descriptor(go_base + at.go, at.go_bytes);
 #pragma unroll
     for (int n = 0; n < NCH; ++n) {
       lds_load16(q_rsrc, q_off[n], lds_q + (uint32_t)(buf * TILE_BYTES + n * 4096));
       lds_load16(go_rsrc, go_off[n], lds_do + (uint32_t)(buf * TILE_BYTES + n * 4096));
     }
-    if (wave < 2) {  // the rows' statistics: wavefront 0 log-sum-exps, wavefront 1 deltas
-      const u32x4 st_rsrc = descriptor((wave == 0 ? p.lse2 : p.delta) + ((int64_t)b * p.Hq + h) * p.L + q0, rows * 4);
-      lds_load4(st_rsrc, lane * 4, wave == 0 ? lds_address(lse_s[buf]) : lds_address(dl_s[buf]));
+    if (wave < 2) lds_load4(descriptor(stat_base + at.stat, at.rows4), lane * 4, lds_stat + buf * (BQ * 4));  // log-sum-exps, deltas
+    if constexpr (DROP) lds_load4(bit_rsrc, at.bit + lane * 16 + wave * 4, lds_address(bit_s) + (uint32_t)((buf * 4 + wave) * (BQ * 4)));
+    const bool wrap = ++at.hl == rep;
+    at.q += q_head, at.go += go_head, at.stat += st_head, at.bit += bit_head;
+    if (wrap) {
+      at.hl = 0;
+      at.q -= rep * q_head + q_tile, at.go -= rep * go_head + go_tile, at.stat -= rep * st_head + BQ * 4, at.bit -= rep * bit_head + BQ * 16;
+      at.q_bytes = (uint32_t)((BQ - 1) * p.q_sl + dr) * 2, at.go_bytes = (uint32_t)((BQ - 1) * p.go_sl + dr) * 2, at.rows4 = BQ * 4;
     }
-    if constexpr (DROP) lds_load4(bit_rsrc, (uint32_t)((h - hk * rep_all) * p.L + q0 + lane) * 16 + wave * 4, lds_address(bit_s[buf][wave]));
   };
   // rows past L: no probability whatever stands there (wavefront 0, which loaded the values it writes over and has
   // waited for them)
-  auto finish_item = [&](int it, int buf) {
-    const int q0 = item_q0(it);
+  auto finish_item = [&](int q0, int buf) {
     if (q0 + BQ > p.L && tid < BQ && q0 + tid >= p.L) lse_s[buf][tid] = INFINITY;
   };
-  if (n_items > 0) load_item(0, 0);
+  if (n_items > 0) load_item(0);
   u32x4 kf[KS], vf[KS];  // this lane's key as B operand
   {
     const int kc = max(min(key, S - 1), 0);  // (a live row: rows past the batch's keys may hold anything)
@@ -418,95 +438,204 @@ __device__ __forceinline__ void dkdv_body(const BwdM& p, const uint32_t* keep_bi
 #pragma unroll
   for (int i = 0; i < DB; ++i) zero(dk[i]), zero(dv[i]);
   const float c = p.scale * kLog2eF;
+  int q0 = t0 * BQ, hl = hl0, buf = 0, before = 0, next = 1;  // the item that is computed, and the buffers of it and its neighbours
+  // item `it + 1` is there for everyone, and the buffer of item it - 1, which everyone is done with, is filled again
+  auto publish = [&](int it) {
+    wait_loads();
+    if (it + 1 < n_items) finish_item(hl + 1 == rep ? q0 - BQ : q0, next);
+    __syncthreads();
+    if (it + 2 < n_items) load_item(next == 2 ? 0 : next + 1);
+  };
+  auto advance = [&]() {
+    if (++hl == rep) hl = 0, q0 -= BQ;
+    before = buf, buf = next, next = next == 2 ? 0 : next + 1;
+  };
+  auto mask = [&](f32x16& s, int qb) {  // scores of a block of 32 rows that not every key of the wavefront takes part in
+    if (__builtin_expect((p.causal && qb < kw0 + 31) || kw0 + 31 >= S, 0)) {
+      // this lane's key takes no part in the block's first `dead` rows (one register, not one per row kept across the loop)
+      int dead = (key >= S ? 32 : p.causal ? key - qb : 0) - half * 4;
+      asm volatile("" : "+v"(s), "+v"(dead));
+#pragma unroll
+      for (int r = 0; r < 16; ++r) s[r] = (r >> 2) * 8 + (r & 3) < dead ? -INFINITY : s[r];
+    }
+  };
+  // items with both blocks of 32 rows live for this wavefront (under a causal mask the others come last)
+  int n_main = kw0 < S ? n_items : 0;
+  if (p.causal) n_main = max(min(n_main, rep * (nqs - (kw0 + 32) / BQ) - it0), 0);
   if (n_items > 0) {
     wait_loads();
-    finish_item(0, 0);
+    finish_item(q0, 0);
     __syncthreads();
-    if (n_items > 1) load_item(1, 1);
+    if (n_items > 1) load_item(1);
   }
-  auto step = [&](int it, auto buf_c) {
-    constexpr int buf = decltype(buf_c)::value;
-    const int q0 = item_q0(it);
+
+  // A block of 32 query rows in two phases of eight slots, a matrix op and the vector work on two scores each: P, under the
+  // products dP of this block and dK of the block before; then dS, under the scores of the next block and dV of this one.
+  // So every product has vector work of its own wavefront to run under, and one register tile each of scores and dP is
+  // enough.  Operands are requested four ops ahead of their use, statistics of four rows four slots ahead, across the phases.
+  int it = 0;
+  if (n_main > 0) {
+    f32x16 s, dp;
+    uint32_t pk[8], bs[8];  // P and dS in pairs
+    u32x4 ring[4];
+    f32x4 rs[2];
+    u32x4 wd[DROP ? 2 : 1];
+    const lds_bytes q_l = (lds_bytes)&q_t[0][0], do_l = (lds_bytes)&do_t[0][0], lse_l = (lds_bytes)&lse_s[0][0] + half * 16, dl_l = (lds_bytes)&dl_s[0][0] + half * 16;
+    const lds_bytes bit_l = DROP ? (lds_bytes)&bit_s[0][0][0] + wave * (BQ * 4) + half * 16 : nullptr;
+    uint32_t row_a[KS], col_a[2][DB];  // byte offsets in a tile
 #pragma unroll
+    for (int ks = 0; ks < KS; ++ks) row_a[ks] = rd.row_off[ks] * 2;
+#pragma unroll
+    for (int i = 0; i < 2 * DB; ++i) col_a[i >> 1][i & 1] = rd.tr_off[i >> 1][i & 1] * 2;
+    auto rows = [&](lds_bytes tiles, int b, int mb, int ks) { return *(const __attribute__((address_space(3))) u32x4*)(tiles + (row_a[ks] + b * TILE_BYTES) + mb * 32 * D * 2); };
+    auto cols = [&](lds_bytes tiles, int b, int mb, int i) {
+      typedef s16x4 __attribute__((address_space(3)))* ptr;
+      const int st = 2 * mb + (i >> 1), db = i & 1;
+      const u32x2 lo = __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((ptr)(tiles + (col_a[0][db] + b * TILE_BYTES) + st * 16 * D * 2)));
+      const u32x2 hi = __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((ptr)(tiles + (col_a[1][db] + b * TILE_BYTES) + st * 16 * D * 2)));
+      return u32x4{lo[0], lo[1], hi[0], hi[1]};
+    };
+    auto stat_of = [&](lds_bytes rows_l, int b, int mb, int g) { return *(const __attribute__((address_space(3))) f32x4*)(rows_l + b * (BQ * 4) + (mb * 32 + g * 8) * 4); };
+    auto words_of = [&](int b, int mb, int g) { return *(const __attribute__((address_space(3))) u32x4*)(bit_l + b * (BQ * 16) + (mb * 32 + g * 8) * 4); };
+    auto add_rows = [&](f32x16 (&acc)[DB], const uint32_t (&w)[8], const u32x4& a, int i) {  // i = 2 * 16-row step + column block
+      const int sg = i >> 1;
+      acc[i & 1] = Mma<T>::run(a, u32x4{w[4 * sg], w[4 * sg + 1], w[4 * sg + 2], w[4 * sg + 3]}, acc[i & 1]);
+    };
+    auto phase_p = [&](int mb, int b_before, int b_next) {
+      zero(dp);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        const u32x4 a = ring[i % 4];
+        if (i < KS) dp = Mma<T>::run(a, vf[i], dp);
+        else add_rows(dk, bs, a, i - KS);
+        ring[i % 4] = i < KS ? cols(q_l, b_before, mb ^ 1, i) : rows(q_l, b_next, mb ^ 1, i - KS);
+        const int e = (2 * i) & 3, g = i >> 1;
+        const f32x4& l4 = rs[g & 1];
+        pk[i] = Mma<T>::pack(__builtin_amdgcn_exp2f(fmaf(s[2 * i], c, -l4[e])), __builtin_amdgcn_exp2f(fmaf(s[2 * i + 1], c, -l4[e + 1])));
+        asm volatile("" : "+v"(pk[i]));  // (here: the compiler would move it behind the next branch)
+        if (i & 1) rs[g & 1] = g < 2 ? stat_of(lse_l, buf, mb, g + 2) : stat_of(dl_l, buf, mb, g - 2);
+        if constexpr (DROP) {
+          if (i >= 6) wd[i & 1] = words_of(buf, mb, i - 6);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    };
+    // dS is formed from P as the matrix pipe gets it, rounded to the input dtype (as in the kernels that
+    // exchange P through LDS: a mask given as a tensor runs there, and the same mask as a flag here)
+    auto phase_ds = [&](int mb, int b_next) {
+      uint32_t pm[DROP ? 8 : 1];
+      zero(s);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        const u32x4 a = ring[i % 4];
+        if (i < KS) s = Mma<T>::run(a, kf[i], s);
+        else if constexpr (DROP) add_rows(dv, pm, a, i - KS);
+        else add_rows(dv, pk, a, i - KS);
+        ring[i % 4] = i < KS ? cols(do_l, buf, mb, i) : rows(do_l, b_next, mb ^ 1, i - KS);
+        if constexpr (DROP) {
+          // the first four slots: this key's bit of each row's word, as a mask of all ones or zeros, on dP and on the P that dV gets
+          if (i < 4) {
+            const u32x4 w4 = wd[i & 1];
+#pragma unroll
+            for (int j = 2 * i; j < 2 * i + 2; ++j) {
+              const int e = (2 * j) & 3;
+              const uint32_t m0 = (uint32_t)__builtin_amdgcn_sbfe((int)w4[e], (uint32_t)col, 1u), m1 = (uint32_t)__builtin_amdgcn_sbfe((int)w4[e + 1], (uint32_t)col, 1u);
+              const float dp0 = dp[2 * j], dp1 = dp[2 * j + 1];  // (copied out: a bit cast of a vector element reads element 0)
+              dp[2 * j] = __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, dp0) & m0);
+              dp[2 * j + 1] = __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, dp1) & m1);
+              pm[j] = pk[j] & __builtin_amdgcn_perm(m1, m0, 0x05040100u);
+            }
+            if (i < 2) wd[i & 1] = words_of(buf, mb, i + 2);
+          } else {
+            const int g = i - 4;
+            const f32x4 d4 = rs[g & 1];
+#pragma unroll
+            for (int j = 2 * g; j < 2 * g + 2; ++j) {
+              const int e = (2 * j) & 3;
+              bs[j] = Mma<T>::pack(Mma<T>::unpack(pk[j], 0) * fmaf(dp[2 * j], p.keep_scale, -d4[e]), Mma<T>::unpack(pk[j], 1) * fmaf(dp[2 * j + 1], p.keep_scale, -d4[e + 1]));
+              asm volatile("" : "+v"(bs[j]));
+            }
+            rs[g & 1] = g < 2 ? stat_of(dl_l, buf, mb, g + 2) : stat_of(lse_l, b_next, mb ^ 1, g - 2);
+          }
+        } else {
+          const int e = (2 * i) & 3, g = i >> 1;
+          const f32x4& d4 = rs[g & 1];
+          bs[i] = Mma<T>::pack(Mma<T>::unpack(pk[i], 0) * (dp[2 * i] - d4[e]), Mma<T>::unpack(pk[i], 1) * (dp[2 * i + 1] - d4[e + 1]));
+          asm volatile("" : "+v"(bs[i]));
+          if (i & 1) rs[g & 1] = g < 2 ? stat_of(dl_l, buf, mb, g + 2) : stat_of(lse_l, b_next, mb ^ 1, g - 2);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    };
+    // (no block in front of the first one: the dK that its first phase adds is of zero dS, with the other rows of the same
+    // tile, which every key of the wavefront sees anyway)
+#pragma unroll
+    for (int i = 0; i < 8; ++i) bs[i] = 0u;
+    zero(s);
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) s = Mma<T>::run(rows(q_l, 0, 0, ks), kf[ks], s);
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) ring[ks] = rows(do_l, 0, 0, ks);
+    rs[0] = stat_of(lse_l, 0, 0, 0), rs[1] = stat_of(lse_l, 0, 0, 1);
+#pragma nounroll
+    do {
+      mask(s, q0);
+      phase_p(0, before, buf);
+      phase_ds(0, buf);
+      publish(it);
+      mask(s, q0 + 32);
+      phase_p(1, buf, next);
+      phase_ds(1, next);  // (behind the last item the scores of a tile that nobody asked for, and nobody uses)
+      advance();
+    } while (++it < n_main);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) add_rows(dk, bs, cols(q_l, before, 1, i), i);
+  }
+  // the rest, block by block: nothing of a block that no key of the wavefront sees is computed, whatever its rows hold
+#pragma nounroll
+  for (; it < n_items; ++it) {
+    publish(it);
     for (int mb = 0; mb < 2; ++mb) {
       const int qb = q0 + mb * 32;
-      if ((p.causal && qb + 31 < kw0) || kw0 >= S) continue;  // (uniform per wavefront)
+      if (kw0 >= S || (p.causal && qb + 31 < kw0)) continue;  // (uniform per wavefront)
+      const uint16_t *const qt = q_t[buf] + mb * 32 * D, *const dot = do_t[buf] + mb * 32 * D;
       f32x16 s, dp;
       zero(s), zero(dp);
 #pragma unroll
-      for (int ks = 0; ks < KS; ++ks) s = Mma<T>::run(rd.rows(q_t[buf], mb, ks), kf[ks], s);
+      for (int ks = 0; ks < KS; ++ks) s = Mma<T>::run(rd.rows(qt, 0, ks), kf[ks], s);
 #pragma unroll
-      for (int ks = 0; ks < KS; ++ks) dp = Mma<T>::run(rd.rows(do_t[buf], mb, ks), vf[ks], dp);
-      if (__builtin_expect((p.causal && qb < kw0 + 31) || kw0 + 31 >= S, 0)) {
-        asm volatile("" : "+v"(s));
+      for (int ks = 0; ks < KS; ++ks) dp = Mma<T>::run(rd.rows(dot, 0, ks), vf[ks], dp);
+      mask(s, qb);
+      uint32_t pm[8], ds[8];
 #pragma unroll
-        for (int r = 0; r < 16; ++r) s[r] = qb + (r >> 2) * 8 + half * 4 + (r & 3) < first_q ? -INFINITY : s[r];
-      }
-      // dS is formed from P as the matrix pipe gets it, rounded to the input dtype (as in the kernels that
-      // exchange P through LDS: a mask given as a tensor runs there, and the same mask as a flag here)
-      uint32_t pk[8], pm[DROP ? 8 : 1];  // P in pairs; (dropout) the kept ones, for dV
-#pragma unroll
-      for (int g = 0; g < 4; ++g) {
-        const f32x4 l4 = *(const f32x4*)(&lse_s[buf][mb * 32 + g * 8 + half * 4]), d4 = *(const f32x4*)(&dl_s[buf][mb * 32 + g * 8 + half * 4]);
-        u32x4 w4 = {0u, 0u, 0u, 0u};
-        if constexpr (DROP) w4 = *(const u32x4*)(&bit_s[buf][wave][mb * 32 + g * 8 + half * 4]);
-        const uint32_t words_e[4] = {w4[0], w4[1], w4[2], w4[3]};
-        float x[4];
-#pragma unroll
-        for (int e = 0; e < 4; ++e) x[e] = __builtin_amdgcn_exp2f(fmaf(s[4 * g + e], c, -l4[e]));
-#pragma unroll
-        for (int j = 0; j < 2; ++j) {
-          pk[2 * g + j] = Mma<T>::pack(x[2 * j], x[2 * j + 1]);
-          if constexpr (DROP) pm[2 * g + j] = 0u;
-#pragma unroll
-          for (int e = 0; e < 2; ++e) {
-            const int r = 4 * g + 2 * j + e;
-            const float pr = Mma<T>::unpack(pk[2 * g + j], e);
-            if constexpr (DROP) {
-              // this key's bit of the row's word, as a mask of all ones or zeros
-              const uint32_t m = (uint32_t)__builtin_amdgcn_sbfe((int)words_e[2 * j + e], (uint32_t)col, 1u);
-              const float dpr = dp[r];  // (copied out: a bit cast of a vector element reads element 0)
-              const float dpk = __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, dpr) & m);
-              dp[r] = pr * fmaf(dpk, p.keep_scale, -d4[2 * j + e]);
-              pm[2 * g + j] |= m & (e ? 0xffff0000u : 0xffffu);
-            } else {
-              dp[r] = pr * (dp[r] - d4[2 * j + e]);
-            }
-          }
-          if constexpr (DROP) pm[2 * g + j] &= pk[2 * g + j];
+      for (int i = 0; i < 8; ++i) {
+        const int r0 = mb * 32 + (i >> 1) * 8 + half * 4 + (i & 1) * 2;  // the rows of scores 2 i and 2 i + 1
+        const float l0 = lse_s[buf][r0], l1 = lse_s[buf][r0 + 1], d0 = dl_s[buf][r0], d1 = dl_s[buf][r0 + 1];
+        const uint32_t pk = Mma<T>::pack(__builtin_amdgcn_exp2f(fmaf(s[2 * i], c, -l0)), __builtin_amdgcn_exp2f(fmaf(s[2 * i + 1], c, -l1)));
+        float g0 = dp[2 * i], g1 = dp[2 * i + 1];
+        pm[i] = pk;
+        if constexpr (DROP) {
+          const uint32_t m0 = (uint32_t)__builtin_amdgcn_sbfe((int)bit_s[buf][wave][r0], (uint32_t)col, 1u), m1 = (uint32_t)__builtin_amdgcn_sbfe((int)bit_s[buf][wave][r0 + 1], (uint32_t)col, 1u);
+          pm[i] &= __builtin_amdgcn_perm(m1, m0, 0x05040100u);
+          g0 = fmaf(m0 ? g0 : 0.f, p.keep_scale, -d0), g1 = fmaf(m1 ? g1 : 0.f, p.keep_scale, -d1);
+        } else {
+          g0 -= d0, g1 -= d1;
         }
+        ds[i] = Mma<T>::pack(Mma<T>::unpack(pk, 0) * g0, Mma<T>::unpack(pk, 1) * g1);
       }
 #pragma unroll
-      for (int sg = 0; sg < 2; ++sg) {
-        u32x4 bP;
-        if constexpr (DROP) bP = u32x4{pm[4 * sg], pm[4 * sg + 1], pm[4 * sg + 2], pm[4 * sg + 3]};
-        else bP = u32x4{pk[4 * sg], pk[4 * sg + 1], pk[4 * sg + 2], pk[4 * sg + 3]};
-        float ds[8];
+      for (int sg = 0; sg < 2; ++sg)
 #pragma unroll
-        for (int r = 0; r < 8; ++r) ds[r] = dp[8 * sg + r];
-        const u32x4 bS = pack8<T>(ds);
-#pragma unroll
-        for (int db = 0; db < DB; ++db) dv[db] = Mma<T>::run(rd.cols(do_t[buf], 2 * mb + sg, db), bP, dv[db]);
-#pragma unroll
-        for (int db = 0; db < DB; ++db) dk[db] = Mma<T>::run(rd.cols(q_t[buf], 2 * mb + sg, db), bS, dk[db]);
-      }
+        for (int db = 0; db < DB; ++db) {
+          dv[db] = Mma<T>::run(rd.cols(dot, sg, db), u32x4{pm[4 * sg], pm[4 * sg + 1], pm[4 * sg + 2], pm[4 * sg + 3]}, dv[db]);
+          dk[db] = Mma<T>::run(rd.cols(qt, sg, db), u32x4{ds[4 * sg], ds[4 * sg + 1], ds[4 * sg + 2], ds[4 * sg + 3]}, dk[db]);
+        }
     }
-    constexpr int nb = (buf + 1) % 3;
-    wait_loads();
-    if (it + 1 < n_items) finish_item(it + 1, nb);
-    __syncthreads();
-    // (the buffer of item it - 1: its last readers passed the barrier above)
-    if (it + 2 < n_items) load_item(it + 2, (buf + 2) % 3);
-  };
-  for (int it = 0;;) {
-    if (it >= n_items) break;
-    step(it, std::integral_constant<int, 0>{});
-    if (++it >= n_items) break;
-    step(it, std::integral_constant<int, 1>{});
-    if (++it >= n_items) break;
-    step(it, std::integral_constant<int, 2>{});
-    ++it;
+    advance();
   }
+  if (p.parts == 1 && n_items > 0) __syncthreads();  // (the rows leave through the tiles, which others may still read)
   if (p.parts > 1) {
     if (key >= p.S) return;  // float32 rows for bwd_dkdv_merge_kernel, which also applies the factors
     const int64_t row = ((((int64_t)(pq * p.parts_h + ph)) * p.B + b) * p.Hkv + hk) * p.S + key;
@@ -525,12 +654,12 @@ __device__ __forceinline__ void dkdv_body(const BwdM& p, const uint32_t* keep_bi
   store_rows<T>(dv, DROP ? p.keep_scale : 1.f, &do_t[0][0] + wave * 32 * D, lane, (uint16_t*)p.gv + b * p.gv_sb + hk * p.gv_sh, p.gv_sl, kw0, p.S, dr);
 }
 
-// OCC: workgroups per compute unit that the registers are kept to.  Three is better where there are that many
-// (B=32, 12 heads, S=512: 123 us for the whole backward against 127 with two, B=4, 32 heads, S=4096 causal 997
-// / 1033), two where there are not (B=4, 12 heads, S=1024 causal, 384 workgroups: 54 / 58; at three a few
-// values go to scratch) and with dropout (193 registers; B=32, 12 heads, S=512 155 / 161, B=4, 16, S=2048 causal 198 / 229).
-template <typename T, bool DROP, int OCC>
-__global__ __launch_bounds__(256, OCC) void bwd_d64_dkdv_kernel(BwdM p, const uint32_t* keep_bits, int chunk) {
+// Two workgroups per compute unit: the two phases of a block hold 221 registers (242 with dropout).  (The four products one
+// after the other in 168 registers, a third workgroup hiding the chain, is what this replaced: B=4, 12 heads, S=512, not
+// causal, the whole backward 32.2 -> 27.5 us, B=1, S=1024 causal 39.1 -> 30.1, B=64, S=197 79.6 -> 77.7, B=4, 32 heads, S=4096
+// causal 1027 -> 1004; with dropout B=32, S=512 148 -> 139, with key counts as well 158 -> 148.)
+template <typename T, bool DROP>
+__global__ __launch_bounds__(256, 2) void bwd_d64_dkdv_kernel(BwdM p, const uint32_t* keep_bits, int chunk) {
   __shared__ __attribute__((aligned(16))) uint16_t q_t[3][TILE];
   __shared__ __attribute__((aligned(16))) uint16_t do_t[3][TILE];
   __shared__ __attribute__((aligned(16))) float lse_s[3][BQ], dl_s[3][BQ];
@@ -541,7 +670,7 @@ __global__ __launch_bounds__(256, OCC) void bwd_d64_dkdv_kernel(BwdM p, const ui
 // Both in one launch, behind bwd_d64_terms_kernel: a dK/dV and a dQ workgroup by turns, eight of each (the XCDs), the
 // heaviest of both first.  (See together for where.)
 template <typename T>
-__global__ __launch_bounds__(256, 3) void bwd_d64_both_kernel(BwdM p, int dq_blocks, int dkdv_blocks, int dq_chunk, int dkdv_chunk) {
+__global__ __launch_bounds__(256, 2) void bwd_d64_both_kernel(BwdM p, int dq_blocks, int dkdv_blocks, int dq_chunk, int dkdv_chunk) {
   __shared__ __attribute__((aligned(16))) uint16_t a_t[3][TILE];
   __shared__ __attribute__((aligned(16))) uint16_t b_t[3][TILE];
   __shared__ __attribute__((aligned(16))) float lse_s[3][BQ], dl_s[3][BQ];
@@ -585,38 +714,36 @@ int stream_chunk(const BwdM& g, int64_t rows) {
 // run with nobody beside them.  The kernels of 8 wavefronts per workgroup (bwd_dq_w32.hip, bwd_dkdv_w32.hip) have the shorter
 // chain.  Below 384 key blocks their items are split (bwd_dkdv_w32_plan), above 1024 the rest of the grid hides it.
 // Backward, us, both kernels here / dQ here and dK/dV there / both there (D=64):
-//   grouped heads, 384 blocks: B=3, 32/8 heads, S=2048 337 / 253 / 263;  B=6, 64/8, S=1024 344 / 263 / 291
-//     512: B=2, 32/8, S=4096 700 / 554 / 569;  B=8, 32/8, S=1024 200 / 170 / 194;  1024: B=8, 32/8, S=2048 626 / 580 / 639
-//   dQ's own grid (B * Hq query tiles), 576: B=6, 12 heads, S=1024 83 / 78 / 72;  768: B=2, 12, S=4096 277 / 261 / 243
-//     512: B=2, 8, S=4096 176 / 165 / 184;  768, S=512 (8 tiles): B=16, 12 53 / 57 / 56.  With key counts or narrow rows
-//     the other dQ kernel is its masked variant: B=3, 12, S=2048 with key counts 109 here / 122 there, D=48 103 / 115
+//   grouped heads, 384 blocks: B=3, 32/8 heads, S=2048 294 / 248 / 263;  B=6, 64/8, S=1024 307 / 261 / 291
+//     512: B=2, 32/8, S=4096 632 / 562 / 569;  B=8, 32/8, S=1024 184 / 172 / 194;  1024: B=8, 32/8, S=2048 595 / 600 / 639
+//   dQ's own grid (B * Hq query tiles), 576: B=6, 12 heads, S=1024 77 / - / 73;  720: B=5, 12, S=1500 93 / - / 113;  768: B=4,
+//     12, S=2048 135 / - / 144, B=6, 16, S=1024 85 / - / 91, B=2, 12, S=4096 239 / - / 241;  512: B=2, 8, S=4096 149 here, 153 before
 bool w32_dkdv(const BwdM& g) {
   const int64_t blocks = (int64_t)g.B * g.Hkv * g.n_kt;
   return g.causal && g.keep_scale == 0.f && g.Hq > g.Hkv && blocks >= 384 && blocks <= 1024;
 }
 bool w32_both(const BwdM& g) {
   const int64_t tiles = (int64_t)g.B * g.Hq * g.n_qt;
-  return g.causal && g.keep_scale == 0.f && !g.kv_lens && g.d_real == D && (int64_t)g.B * g.Hkv * g.n_kt >= 384 && tiles > 512 && tiles <= 768 && g.L > 14 * BQ;
+  return g.causal && g.keep_scale == 0.f && !g.kv_lens && g.d_real == D && (int64_t)g.B * g.Hkv * g.n_kt >= 384 && tiles > 512 && tiles <= 640 && g.L > 14 * BQ;
 }
 
-// Calls whose two kernels leave the chip half empty, each for as long as its longest chain of tiles: one launch of both.
-// Up to one workgroup per compute unit in all, nobody shares anything; beyond it a causal call's long workgroups run
-// beside short ones, up to three per compute unit, where the chains are long enough to pay for the third kernel in front
-// (4 us) and for the registers (168, some in scratch).  Workgroups in all and us, two launches / one (12 heads, D=64):
-//   up to 256: S=64, 6 heads 11.0 / 10.4;  B=4, S=197 not causal 19.8 / 17.9;  B=2, S=512 not causal 28.7 / 24.0;  B=1, S=1024 46.8 / 38.8
-//     336: B=2, S=785 not causal 43.2 / 42.8;  384: B=8, S=197 not causal 20.5 / 21.9
-//   causal, 384: B=16, 6 heads, S=200 19.3 / 18.3;  B=16, S=128 16.2 / 16.7;  grouped, 384: 16/4 heads, S=1021 47.6 / 41.1
-//     512: B=4, 16/4, S=500 42.8 / 38.6;  1536: B=2, 32/8, S=1000 77.2 / 78.3;  768: B=16, S=256 25.6 / 26.9;  B=8, S=512 34.9 / 32.7;  B=4, S=1024 55.1 / 49.6
-//     1024: B=8, 16 heads, S=512 39.0 / 44.8;  B=4, 16, S=1024 58.3 / 55.5;  B=2, 16, S=2048 96.2 / 85.5;  1152: B=12, S=512 56.0 / 57.9
-// Three heads per kv head and more, whole chains in dK/dV (three query tiles, or items that are not split): dK/dV walks as
-// many times dQ's tiles, dQ under it saves little, and its chain is the slower one in these registers.  Causal, two launches /
-// one: B=2, 12/4 heads, S=400 46.3 / 47.6;  16/4, S=200 36.9 / 39.7, split, S=400 43.2 / 41.7;  28/4, S=100 33.6 / 36.8, S=150 43.8 / 49.5,
-// split, S=200 34.5 / 33.8;  16/2, S=64 22.8 / 24.9, split, S=150 34.1 / 35.7, S=200 29.9 / 29.1.  (Two heads: 12/6, S=64 13.4 / 12.9, S=400 36.2 / 35.2.)
+// Calls whose two kernels leave the chip half empty, each for as long as its longest chain of tiles: one launch of both,
+// behind the one that forms the row terms (4 us).  The line is the number of workgroups in all (two of them share a compute
+// unit), by the length of a chain, which is what the second launch would wait for.  Two launches / one, us, 12 heads and
+// D=64 where not said:
+//   not causal, 192: B=2, S=512 26.4 / 20.4;  384: B=8, S=197 20.3 / 20.2, B=4, S=512 29.9 / 27.5;  448: B=2, 16 heads, S=785 41.1 / 38.9
+//     768: B=3, 16, S=1000 71.7 / 68.9;  3072: B=64, S=197 78 / 92
+//   causal, up to six 64-row tiles, 192: B=16, 6 heads, S=128 14.9 / 12.8;  384: B=16, 6, S=200 20.0 / 17.2, S=256 21.2 / 17.8
+//     432: B=6, 12/6 heads, S=400 35.5 / 30.2;  576: B=6, S=400 27.8 / 23.7, B=12, S=256 24.3 / 27.7;  768: B=8, S=400 29.8 / 31.4
+//     three heads a kv head and more: B=2, 12/4, S=400 39.2 / 34.1, 16/4, S=200 31.7 / 28.4, 28/4, S=150 36.8 / 34.8, B=8, 28/4, S=100 29.6 / 27.2
+//   seven tiles and more, 480: B=4, S=600 33.2 / 25.8;  648: B=6, 12/6, S=700 51.3 / 43.4;  720: B=6, S=600 36.5 / 35.7
+//     768: B=8, S=512 34.7 / 35.5, B=4, S=1024 51.1 / 47.7;  864: B=6, S=700 39.4 / 40.9;  1120: B=5, 16, S=777 50.6 / 54.4
+//     grouped beyond 768: B=4, 32/8, S=700 77.5 / 80.2
+//   fifteen and more, 1024: B=4, 16, S=1024 65.2 / 57.5, B=2, 16, S=2048 90.5 / 88.7;  2048: B=4, 16, S=2048 154 / 157
 bool together(const BwdM& g) {
   if (g.keep_scale != 0.f || w32_dkdv(g)) return false;
-  if (g.Hq >= 3 * g.Hkv && (g.parts == 1 || g.L <= 3 * BQ)) return false;
   const int64_t all = (int64_t)g.B * g.Hq * g.n_qt + (int64_t)g.B * g.Hkv * g.n_kt * g.parts;
-  return all <= (!g.causal || g.L < 3 * BQ ? 256 : g.L < 7 * BQ ? 384 : g.Hq > g.Hkv ? 512 : g.L <= 14 * BQ ? 768 : 1024);
+  return all <= (!g.causal ? 768 : g.L < 7 * BQ ? 512 : g.Hq > g.Hkv || g.L <= 14 * BQ ? 768 : 1024);
 }
 
 template <typename T>
@@ -643,10 +770,7 @@ int launch_t(const BwdM& g, uint32_t* bits, hipStream_t s) {
   if (!DROP && w32_dkdv(g)) return launch_bwd_dkdv_w32(g, std::is_same<T, bf16_t>::value ? MI355_SDPA_BF16 : MI355_SDPA_F16, 64, s);
   const int64_t blocks = (int64_t)g.B * g.Hkv * g.n_kt * g.parts;
   const int chunk = stream_chunk(g, (int64_t)g.L * (g.Hq / g.Hkv));
-#define DKDV(OCC) hipLaunchKernelGGL((bwd_d64_dkdv_kernel<T, DROP, OCC>), dim3((unsigned)blocks), dim3(256), 0, s, g, (const uint32_t*)bits, chunk)
-  if (DROP || blocks <= 512) DKDV(2);
-  else if constexpr (!DROP) DKDV(3);
-#undef DKDV
+  hipLaunchKernelGGL((bwd_d64_dkdv_kernel<T, DROP>), dim3((unsigned)blocks), dim3(256), 0, s, g, (const uint32_t*)bits, chunk);
   rc = check_launch("bwd_d64_dkdv_kernel");
   if (rc || g.parts == 1) return rc;
   return launch_bwd_dkdv_merge(g, std::is_same<T, bf16_t>::value ? MI355_SDPA_BF16 : MI355_SDPA_F16, s);
