@@ -56,3 +56,22 @@ def test_key_counts(amd, gpu_device, causal):
             continue
         ro, rl = oracle_fwd(q[b:b + 1], k[b:b + 1, :, :n], v[b:b + 1, :, :n], is_causal=causal)
         assert max_abs(out[b:b + 1], ro) <= 1e-5 and max_abs(lse[b:b + 1], rl) <= 1e-5
+
+
+@pytest.mark.parametrize("B,Hq,Hkv,L,S,E,Dv,causal", [
+    (1, 2, 2, 1, 1, 64, 64, False),
+    (1, 2, 1, 15, 16, 64, 64, True),
+    (1, 2, 2, 17, 15, 8, 8, False),
+    (2, 2, 1, 16, 129, 72, 24, True),     # a ninth block of 16 keys
+    (1, 3, 1, 47, 128, 128, 128, False),
+    (1, 2, 2, 250, 250, 128, 128, True),
+    (32, 4, 4, 32, 40, 64, 64, False),    # 256 workgroups of 16 rows: the last size without the causal mask, and past it
+    (32, 4, 4, 33, 40, 64, 64, False),
+    (8, 8, 8, 128, 128, 128, 128, True),  # 512 with it
+    (8, 8, 8, 129, 129, 128, 128, True),
+    (8, 8, 8, 208, 208, 64, 64, True),    # 832 of short chains
+    (2, 16, 16, 401, 401, 64, 64, True),  # ... and of longer ones
+])
+def test_sixteen_rows_against_the_oracle(amd, gpu_device, B, Hq, Hkv, L, S, E, Dv, causal):
+    """The same in workgroups of 16 rows whose eight wavefronts take every eighth block of 16 keys."""
+    test_against_the_oracle(amd, gpu_device, B, Hq, Hkv, L, S, E, Dv, causal)

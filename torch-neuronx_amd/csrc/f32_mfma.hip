@@ -17,6 +17,7 @@
 //
 //   fwd_f32_kernel        128 query rows per workgroup (4 wavefronts x 32), 32-key tiles
 //   fwd_f32_few_kernel    32 query rows per workgroup, its wavefronts share out the key tiles (few query tiles)
+//   fwd_f32_rows16_kernel 16 query rows per workgroup and the 16 x 16 x 4 op (fewer still)
 //   bwd_f32_dq_kernel     the same shape; also leaves delta = rowsum(dO * O) and the log2-domain
 //                         log-sum-exp in the workspace
 //   bwd_f32_dkdv_kernel   128 keys per workgroup; loops over the query heads of the group (the GQA
@@ -293,6 +294,128 @@ __global__ __launch_bounds__(64 * WAVES, 1) void fwd_f32_kernel(FwdM p) {
       p.lse[((int64_t)b * p.Hq + h) * p.L + qrow] = lse_row;
     }
   }
+}
+
+// Sixteen query rows per workgroup and eight wavefronts that take every eighth block of 16 keys each, on the 16 x 16 x 4 op: the
+// calls whose 32-row workgroups (fwd_f32_few_kernel) would leave most compute units empty.  Such a call lasts as long
+// as one chain - Q and the first keys from memory, the matrix ops of a block, the meeting in LDS - and a block of 16 keys is a
+// quarter of a 32 x 32 one's ops.  (Lane (n, g), n = lane % 16, g = lane / 16: row n of the query rows, of K quarter g of row
+// n, of V elements 16 db + n of the keys 4 g + i; register i of the score tile is key 4 g + i of row n.)
+// Against the 32-row workgroups: B=2, 4 heads, S=128, D=64 8.7 -> 6.5 us, 8 heads, S=64, D=128 12.3 -> 7.5, S=512 causal
+// 19.0 -> 12.4, S=700 causal, D=128 46 -> 30 (where each pays: sixteen_rows).
+template <int D>
+__global__ __launch_bounds__(512, 1) void fwd_f32_rows16_kernel(FwdM p) {
+  constexpr int KW = 8, R = 16, DB = D / 16, PITCH = D + 4;
+  __shared__ float m_s[KW][R], l_s[KW][R];
+  __shared__ __attribute__((aligned(16))) float o_st[D > 64 ? 4 : KW * R * PITCH];
+  float* const o_s = D > 64 ? wide_f32_lds : o_st;  // [KW][R][PITCH]
+  const int n_rb = (p.L + R - 1) / R;
+  const int rb = n_rb - 1 - blockIdx.x / (p.B * p.Hq);  // heavy row blocks first
+  const int bh = blockIdx.x % (p.B * p.Hq), b = bh / p.Hq, h = bh % p.Hq, hk = h / (p.Hq / p.Hkv);
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, n = lane & 15, g = lane >> 4;
+  const int q0 = rb * R, qrow = q0 + n, qc = min(qrow, p.L - 1);
+  const float* kp = (const float*)p.k + b * p.k_sb + hk * p.k_sh;
+  const float* vp = (const float*)p.v + b * p.v_sb + hk * p.v_sh;
+  const int S = p.kv_lens ? min(p.S, max(p.kv_lens[b], 0)) : p.S;
+  int nt = (S + R - 1) / R;
+  if (p.causal) nt = min(nt, (min(q0 + R, p.L) - 1) / R + 1);
+  const int lim = p.causal ? min(qrow, S - 1) : S - 1;
+  const float c = p.scale * kLog2eF;
+  auto quarter_row = [&](float (&f)[D / 4], const float* row) {  // elements g * D/4 .. +D/4-1, zeros beyond the row's width
+#pragma unroll
+    for (int i = 0; i < D / 16; ++i) {
+      const int d = g * (D / 4) + i * 4;
+      const f32x4 w = d < p.d_real ? *(const f32x4*)(row + d) : f32x4{0.f, 0.f, 0.f, 0.f};
+      f[i * 4] = w[0], f[i * 4 + 1] = w[1], f[i * 4 + 2] = w[2], f[i * 4 + 3] = w[3];
+    }
+  };
+  float qf[D / 4], kf[D / 4], vf[4][DB];
+  auto fetch_k = [&](int t) { quarter_row(kf, kp + (int64_t)min(t * R + n, S - 1) * p.k_sl); };  // (rows past the keys: the last one again, masked)
+  auto fetch_v = [&](int t) {  // (... and zeros, which the zero probabilities leave finite)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int kv = t * R + 4 * g + i;
+      const float* row = vp + (int64_t)kv * p.v_sl + n;
+#pragma unroll
+      for (int db = 0; db < DB; ++db) vf[i][db] = (kv < S && db * 16 + n < p.dv_real) ? row[db * 16] : 0.f;
+    }
+  };
+  auto mma16 = [](float x, float y, f32x4 acc) { return __builtin_amdgcn_mfma_f32_16x16x4f32(x, y, acc, 0, 0, 0); };
+  f32x4 oacc[DB];
+#pragma unroll
+  for (int i = 0; i < DB; ++i) oacc[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+  float m_run = -INFINITY, l_run = 0.f;
+  if (wave < nt) fetch_k(wave);
+  quarter_row(qf, (const float*)p.q + b * p.q_sb + h * p.q_sh + (int64_t)qc * p.q_sl);
+  if (wave < nt) fetch_v(wave);
+  for (int t = wave; t < nt; t += KW) {
+    f32x4 s0 = {0.f, 0.f, 0.f, 0.f}, s1 = s0;  // (two chains: an op's result is the next one's input)
+#pragma unroll
+    for (int i = 0; i < D / 4; i += 2) s0 = mma16(kf[i], qf[i], s0), s1 = mma16(kf[i + 1], qf[i + 1], s1);
+    if (t + KW < nt) fetch_k(t + KW);
+    float s[4], tm = -INFINITY;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      s[i] = t * R + 4 * g + i > lim ? -INFINITY : s0[i] + s1[i];
+      tm = fmaxf(tm, s[i]);
+    }
+    tm = fmaxf(tm, __shfl_xor(tm, 16, 64));
+    tm = fmaxf(tm, __shfl_xor(tm, 32, 64));
+    const float m_new = fmaxf(m_run, tm);
+    const float m_use = m_new == -INFINITY ? 0.f : m_new;
+    const float alpha = __builtin_amdgcn_exp2f((m_run - m_use) * c);
+    m_run = m_new;
+    float psum = 0.f;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      s[i] = __builtin_amdgcn_exp2f((s[i] - m_use) * c);
+      psum += s[i];
+    }
+    l_run = l_run * alpha + psum;
+#pragma unroll
+    for (int db = 0; db < DB; ++db) oacc[db] *= alpha;
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int db = 0; db < DB; ++db) oacc[db] = mma16(vf[i][db], s[i], oacc[db]);
+    if (t + KW < nt) fetch_v(t + KW);
+  }
+  // the eight parts of a row: every wavefront leaves (maximum, sum, O) and a row is put together by 32 threads
+  float l_tot = l_run + __shfl_xor(l_run, 16, 64);
+  l_tot += __shfl_xor(l_tot, 32, 64);
+  if (g == 0) m_s[wave][n] = m_run, l_s[wave][n] = l_tot;
+  float* const o_w = o_s + (wave * R + n) * PITCH + g * 4;
+#pragma unroll
+  for (int db = 0; db < DB; ++db) *(f32x4*)(o_w + db * 16) = oacc[db];
+  __syncthreads();
+  const int r = tid >> 5, j = tid & 31;
+  float mt = -INFINITY, lt = 0.f, w[KW];
+#pragma unroll
+  for (int i = 0; i < KW; ++i) mt = fmaxf(mt, m_s[i][r]);
+#pragma unroll
+  for (int i = 0; i < KW; ++i) {
+    w[i] = mt == -INFINITY ? 0.f : __builtin_amdgcn_exp2f((m_s[i][r] - mt) * c);
+    lt = fmaf(l_s[i][r], w[i], lt);
+  }
+  const float inv = lt > 0.f ? 1.f / lt : 0.f;
+  if (q0 + r >= p.L) return;
+  float* const orow = (float*)p.out + b * p.o_sb + h * p.o_sh + (int64_t)(q0 + r) * p.o_sl;
+#pragma unroll
+  for (int d0 = 0; d0 < D; d0 += 64) {
+    const int d = d0 + j * 2;
+    float a0 = 0.f, a1 = 0.f;
+#pragma unroll
+    for (int i = 0; i < KW; ++i) {
+      const float* x = o_s + (i * R + r) * PITCH + d;
+      a0 = fmaf(x[0], w[i], a0), a1 = fmaf(x[1], w[i], a1);
+    }
+    if (d < p.dv_real) {
+      typedef __attribute__((ext_vector_type(2))) float f32x2;
+      *(f32x2*)(orow + d) = f32x2{a0 * inv, a1 * inv};
+    }
+  }
+  if (p.lse && j == 0)
+    p.lse[((int64_t)b * p.Hq + h) * p.L + q0 + r] = lt > 0.f ? mt * p.scale + __builtin_logf(lt) : -INFINITY;
 }
 
 // Few query tiles (a small batch, short sequences): 128-row workgroups would leave compute units empty and
@@ -815,6 +938,19 @@ bool few_query_tiles(const FwdM& g) {
   return g.S > BT && (g.causal ? wide <= 240 : wide <= 160 && heads * ((g.L + 31) / 32) <= 512);
 }
 
+// ... and which in fwd_f32_rows16_kernel.  Its workgroups cost twice the trips to K and V and have half the chain: up to one per
+// compute unit the chain is all that counts; under a causal mask, where most are shorter than the longest, up to two, and
+// up to 832 where even that one is short.  By their number, 32-row / 16-row in us (8 heads, D=64; the first also
+// against the 128-row kernel, which had single tiles):
+//   8: S=16 6.3 / 4.9, D=128 9.2 / 6.4;  256: B=4, S=128 8.9 / 7.0, B=2, S=256, D=128 21.2 / 16.2, S=512 19.5 / 13.2
+//   not causal, 336: B=7, S=100 8.5 / 9.7, B=3, S=201, 8/2 heads, D=72 17.9 / 14.7;  384: B=3, S=256 12.4 / 13.8;  400: B=2, S=400 19.0 / 18.7
+//   causal, 352: S=700, D=128 46 / 30;  512: B=4, S=256 12.4 / 12.0, S=1021, D=128 58 / 47;  704: B=2, S=700 25.9 / 25.9, D=128 46 / 49
+//     600: B=3, S=400 18.6 / 16.2;  800: B=4, S=400 22.6 / 20.5;  832: B=8, S=200 18.0 / 15.0;  1024: B=2, S=1021 40 / 44
+bool sixteen_rows(const FwdM& g) {
+  const int64_t blocks = (int64_t)g.B * g.Hq * ((g.L + 15) / 16);
+  return blocks <= (!g.causal ? 256 : g.d_real <= 64 && g.L <= 400 ? 832 : 512);
+}
+
 void fwd_f32_fill(FwdM& g, const mi355_sdpa_fwd_params& p, int& mode) {
   g.q = p.q.data, g.k = p.k.data, g.v = p.v.data, g.out = p.out.data, g.lse = p.lse;
   g.q_sb = p.q.stride[0], g.q_sh = p.q.stride[1], g.q_sl = p.q.stride[2];
@@ -862,7 +998,7 @@ int launch_fwd_f32_mfma(const mi355_sdpa_fwd_params& p, hipStream_t s) {
     else
       g.split_tiles = 0, g.n_split = 1;
   }
-  if (mode == 0 && !g.split_tiles && g.d_real <= 128 && few_query_tiles(g)) {
+  if (mode == 0 && !g.split_tiles && g.d_real <= 128 && (sixteen_rows(g) || few_query_tiles(g))) {
 #define LAUNCH_FEW(DD)                                                                                          \
   do {                                                                                                          \
     constexpr int kLds = 4 * 32 * (DD + 4) * (int)sizeof(float);                                                \
@@ -874,6 +1010,22 @@ int launch_fwd_f32_mfma(const mi355_sdpa_fwd_params& p, hipStream_t s) {
     }                                                                                                           \
     hipLaunchKernelGGL((fwd_f32_few_kernel<DD>), dim3((unsigned)((int64_t)g.B * g.Hq * ((g.L + 31) / 32))), dim3(256), kLds, s, g); \
   } while (0)
+    if (sixteen_rows(g)) {
+      const dim3 grid((unsigned)((int64_t)g.B * g.Hq * ((g.L + 15) / 16)));
+      if (g.d_real <= 64) {
+        hipLaunchKernelGGL((fwd_f32_rows16_kernel<64>), grid, dim3(512), 0, s, g);
+      } else {
+        constexpr int kLds = 8 * 16 * (128 + 4) * (int)sizeof(float);
+        static LdsOnce once;
+        const hipError_t e = reserve_lds(once, (const void*)fwd_f32_rows16_kernel<128>, kLds);
+        if (e != hipSuccess) {
+          set_error("SDPA: cannot reserve %d bytes of LDS for fwd_f32_rows16_kernel: %s", kLds, hipGetErrorString(e));
+          return MI355_SDPA_ERR_LAUNCH;
+        }
+        hipLaunchKernelGGL((fwd_f32_rows16_kernel<128>), grid, dim3(512), kLds, s, g);
+      }
+      return check_launch("fwd_f32_rows16_kernel");
+    }
     if (g.d_real <= 64) LAUNCH_FEW(64);
     else LAUNCH_FEW(128);
 #undef LAUNCH_FEW
