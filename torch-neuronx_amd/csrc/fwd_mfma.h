@@ -22,7 +22,7 @@ struct FwdM {
   // that those stand for, and is left to the sizes.  Not asked where keys are split or shared out for few rows: such
   // calls have no causal flag, and a longer one is no prefix of theirs.
   int whole_keys = 0;
-  int xcd_map;  // 1: (batch, kv head) streams are pinned to XCDs
+  int xcd_map;  // > 0: (batch, kv head) streams are pinned to XCDs, each of which takes them in chunks of so many
   float scale;
   // masked calls (fwd_mfma_w32.hip only): additive bias or bool keep-mask with unit stride on the
   // key dim, strides in elements (0 on broadcast dims), and per-batch key counts
@@ -85,11 +85,17 @@ __device__ __forceinline__ void decode_block(const FwdM& p, int& b, int& h, int&
     const int streams = p.B * p.Hkv;  // multiple of 8
     const int per_xcd = streams / 8;
     const int xcd = bid & 7;
-    int r = bid >> 3;  // index within this XCD: [qt desc][stream in xcd][head in group]
+    int r = bid >> 3;  // index within this XCD: [chunk of streams][qt desc][stream in chunk][head in group]
     const int hg = r % rep;
     r /= rep;
-    const int sl = r % per_xcd;
-    r /= per_xcd;
+    int first = 0, n = per_xcd;
+    if (p.xcd_map < per_xcd) {
+      const int c = r / (p.xcd_map * p.n_qt);
+      first = c * p.xcd_map, n = min(p.xcd_map, per_xcd - first);
+      r -= first * p.n_qt;
+    }
+    const int sl = first + r % n;
+    r /= n;
     qt = p.n_qt - 1 - r;
     const int stream = sl * 8 + xcd;
     b = stream / p.Hkv;

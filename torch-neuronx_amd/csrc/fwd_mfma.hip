@@ -399,7 +399,7 @@ static int launch_or_size(const mi355_sdpa_fwd_params& p, hipStream_t s, size_t*
   g.B = (int)p.q.size[0], g.Hq = (int)p.q.size[1], g.Hkv = (int)p.k.size[1];
   g.L = (int)p.q.size[2], g.S = (int)p.k.size[2];
   g.causal = p.is_causal, g.scale = p.scale, g.whole_keys = p.force_kernel != 0 && !p.kv_lens && !p.mask.mask_verdict;
-  g.xcd_map = ((g.B * g.Hkv) % 8 == 0) ? 1 : 0;
+  g.xcd_map = ((g.B * g.Hkv) % 8 == 0) ? g.B * g.Hkv / 8 : 0;
   g.kv_lens = p.kv_lens;
   if (p.bias.data) {
     g.bias = p.bias.data;

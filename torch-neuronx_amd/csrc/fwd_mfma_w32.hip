@@ -1243,9 +1243,26 @@ int launch_fwd_split_merge(const FwdM& g, int dtype, hipStream_t s) {
   return check_launch("fwd_split_merge_kernel");
 }
 
+// How many of its streams (a (batch, kv head)'s keys and values) an XCD takes at a time, all their query tiles before the
+// next ones.  Query tile by query tile over all of them, as is best while they fit its 4 MB of L2, every pass over the
+// tiles brings K and V from memory again (B=32, 12 heads, S=512: 234 MB fetched for 115).  In chunks of 1 MB without the
+// causal mask (a keep-mask and Q pass through the same L2); with it in chunks of the whole L2 and only where there are eight or
+// more: the first tiles of a chunk are the long ones, and the last chunk's start late.  All streams / in chunks, us:
+//   not causal, 4.6 MB: B=64, 12 heads, S=197, D=64 25.9 / 24.4;  5.7: B=40, 12, S=384 35.0 / 31.7;  6: B=32, 12, S=512 42.6 / 38.9, with dropout and
+//     key counts 51.0 / 46.3;  8: B=8, 16, S=1024, D=128 74.2 / 72.2;  16: B=4, 32, S=2048, D=128 240.6 / 237.8;  below: 4.4: B=30, 8, S=600 35.7 / 36.4
+//   causal, 8 chunks: B=4, 64 heads, S=4096, D=64 638 / 580, B=16, 32/8, S=4096, D=128 1989 / 1912, B=8, 32, S=2048 304 / 279, B=16, S=1024 220 / 190
+//     fewer: 4: B=8, 16, S=2048, D=64 82 / 85, B=4, 32, S=999, D=128 with key counts 48 / 50;  2: B=4, 16, S=2048, D=128 72 / 71
+static int stream_chunk(const FwdM& g) {
+  const int64_t per_xcd = (int64_t)g.B * g.Hkv / 8, bytes = std::max<int64_t>(1, (int64_t)g.S * (g.d_real + g.dv_real) * 2);
+  if (g.bias_kind || g.window > 0 || per_xcd * bytes <= (9 << 19)) return (int)per_xcd;
+  const int64_t chunk = std::min(per_xcd, std::max<int64_t>(1, (g.causal ? 4 << 20 : 1 << 20) / bytes));
+  return (int)(g.causal && per_xcd < 8 * chunk ? per_xcd : chunk);
+}
+
 int launch_fwd_mfma_w32(const FwdM& g0, int dtype, int head_dim, int waves, hipStream_t s) {
   FwdM g = g0;
   fwd_w32_plan(g, head_dim, waves);
+  if (g.xcd_map) g.xcd_map = stream_chunk(g);
   if (g.split_tiles) {  // (the caller's workspace: too small or absent, and the call runs unsplit)
     const size_t rows = (size_t)g.B * g.Hq * g.n_split * g.L;
     if (g.part_o && g.n_split <= 512 && g.part_bytes >= rows * (g.dv_real + 1) * sizeof(float)) g.part_lse = g.part_o + rows * g.dv_real;
