@@ -1,0 +1,73 @@
+"""Forward calls whose streams (a (batch, kv head)'s keys and values) an XCD takes in chunks: every (batch, head, row) is
+computed, once, also where the last chunk is a smaller one.
+
+Bound, against the same attention in float64 on the kernel's inputs: P and the output are each rounded once to bf16,
+2^-9 relative, which adds up to at most twice that in the 2-norm: 4e-3; the log-sum-exp is a float32 sum, 1e-5."""
+
+import math
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("B,Hq,Hkv,S,D,causal", [
+    (24, 12, 12, 577, 64, False),   # 36 streams an XCD in chunks of 7
+    (11, 32, 16, 333, 104, False),  # 22 in chunks of 7, two heads a kv head
+    (43, 24, 24, 1024, 64, True),   # 129 in chunks of 16: eight and a last one of a single stream
+    (19, 16, 8, 2048, 128, True),   # 19 in chunks of 4 are fewer than eight chunks: one after the other
+    (35, 16, 8, 2048, 128, True),   # 35: nine
+])
+def test_every_stream_is_computed(gpu_device, B, Hq, Hkv, S, D, causal):
+    import torch_neuronx_amd as amd
+
+    g = torch.Generator(device=gpu_device).manual_seed(S)
+    q, k, v = (torch.randn(B, h, S, D, generator=g, device=gpu_device).to(torch.bfloat16) for h in (Hq, Hkv, Hkv))
+    out, lse = amd.sdpa_forward(q, k, v, is_causal=causal)
+    dead = ~torch.ones(S, S, dtype=torch.bool, device=gpu_device).tril() if causal else None
+    for b in range(B):
+        K, V = (t[b].double().repeat_interleave(Hq // Hkv, 0) for t in (k, v))
+        s = q[b].double() @ K.transpose(-1, -2).contiguous() / math.sqrt(D)
+        if causal:
+            s.masked_fill_(dead, -math.inf)
+        far = (lse[b] - torch.logsumexp(s, -1)).abs().amax(-1)
+        assert float(far.max()) <= 1e-5, b
+        ref = torch.softmax(s, -1) @ V
+        far = (out[b].double() - ref).norm(dim=(-2, -1)) / ref.norm(dim=(-2, -1))
+        assert float(far.max()) <= 4e-3, (b, far)
+
+
+@pytest.mark.parametrize("B,Hq,Hkv,L,S,D,causal,lens", [
+    (57, 8, 8, 1100, 1100, 128, True, None),    # 57 streams an XCD in chunks of 7, in both kernels
+    (9, 16, 8, 3000, 300, 104, False, None),    # 9 one by one in dK/dV, which walks Q and dO of two heads
+    (13, 48, 48, 1000, 1000, 128, False, 1000), # 78 in chunks of 8, key counts
+    (11, 16, 16, 1024, 1024, 64, True, None),   # 22 in chunks of 16 at head dim 64
+    (25, 8, 8, 900, 900, 64, False, None),      # 25 in chunks of 4
+])
+def test_every_gradient_is_computed(gpu_device, B, Hq, Hkv, L, S, D, causal, lens):
+    """The same in the backward.  P, dS, O and the gradients are rounded once each: 8e-3, as in test_bwd_d64_gpu.py."""
+    import torch_neuronx_amd as amd
+
+    g = torch.Generator(device=gpu_device).manual_seed(S)
+    q, k, v, do = (torch.randn(B, h, n, D, generator=g, device=gpu_device).to(torch.bfloat16) for h, n in ((Hq, L), (Hkv, S), (Hkv, S), (Hq, L)))
+    kw = dict(is_causal=causal)
+    if lens:
+        kw["kv_lens"] = torch.tensor([lens - 37 * i for i in range(B)], dtype=torch.int32, device=gpu_device)
+    out, lse = amd.sdpa_forward(q, k, v, **kw)
+    grads = amd.sdpa_backward(do, q, k, v, out, lse, **kw)[:3]
+    rep = Hq // Hkv
+    for b in range(B):
+        n = lens - 37 * b if lens else S
+        Q, DO = q[b].double(), do[b].double()
+        K, V = (t[b, :, :n].double().repeat_interleave(rep, 0) for t in (k, v))
+        s = Q @ K.transpose(-1, -2).contiguous() / math.sqrt(D)
+        if causal:
+            s.masked_fill_(~torch.ones(L, n, dtype=torch.bool, device=gpu_device).tril(), -math.inf)
+        P = torch.softmax(s, -1)
+        dS = P * (DO @ V.transpose(-1, -2).contiguous() - (DO * (P @ V)).sum(-1, keepdim=True)) / math.sqrt(D)
+        want = (dS @ K, (dS.transpose(-1, -2).contiguous() @ Q).view(Hkv, rep, n, D).sum(1), (P.transpose(-1, -2).contiguous() @ DO).view(Hkv, rep, n, D).sum(1))
+        for name, a, r in zip(("dq", "dk", "dv"), grads, want):
+            got = a[b] if name == "dq" else a[b, :, :n]
+            far = (got.double() - r).norm(dim=(-2, -1)) / r.norm(dim=(-2, -1))
+            assert float(far.max()) <= 8e-3, (name, b, far)

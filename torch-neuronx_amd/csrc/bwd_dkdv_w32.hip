@@ -70,8 +70,13 @@ __device__ __forceinline__ void bwd_dkdv_w32_body(const BwdM& p, const MaskArgs 
     kt = rest % p.n_kt, pq = rest / p.n_kt;
     st = v / p.parts_h, ph = v % p.parts_h;
   } else {
-    kt = blockIdx.x / streams;  // low key tiles see the most queries under a causal mask: first
-    st = blockIdx.x % streams;
+    // (low key tiles see the most queries under a causal mask: first)
+    if (p.dkdv_chunk) {
+      chunk_place(blockIdx.x >> 3, streams / 8, p.dkdv_chunk, p.n_kt, st, kt);
+      st = st * 8 + (blockIdx.x & 7);
+    } else {
+      kt = blockIdx.x / streams, st = blockIdx.x % streams;
+    }
   }
   const int part = pq * p.parts_h + ph;  // its rows among the partial results
   const int b = st / p.Hkv, hk = st % p.Hkv;
@@ -959,6 +964,7 @@ int launch_bwd_dkdv_w32(const BwdM& g0, int dtype, int head_dim, hipStream_t s) 
   g.dv_real = g.d_real;
   if (!bwd_dkdv_plan_parts(g)) return MI355_SDPA_ERR_INVALID;
   if (!g.sm.doc_sorted || g.n_kt > 1024) g.kt_order = nullptr;  // (the ranking kernel holds 1024 weights)
+  if (!g.causal || g.Hq == g.Hkv) g.dkdv_chunk = bwd_stream_chunk(g, (int64_t)g.L * (g.Hq / g.Hkv));
   if (head_dim == 128) return dtype == MI355_SDPA_BF16 ? launch_m<bf16_t, 128>(g, s) : launch_m<f16_t, 128>(g, s);
   return dtype == MI355_SDPA_BF16 ? launch_m<bf16_t, 64>(g, s) : launch_m<f16_t, 64>(g, s);
 }

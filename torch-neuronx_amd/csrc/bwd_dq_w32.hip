@@ -65,9 +65,9 @@ __device__ __forceinline__ void bwd_dq_w32_body(const BwdM& p, const MaskArgs ma
       int r = bid >> 3;
       const int hg = r % rep;
       r /= rep;
-      const int sl = r % per_xcd;
-      r /= per_xcd;
-      qt = n_qt - 1 - r;
+      int sl, tile;
+      chunk_place(r, per_xcd, p.dq_chunk, n_qt, sl, tile);
+      qt = n_qt - 1 - tile;
       const int stream = sl * 8 + xcd;
       b = stream / p.Hkv, h = (stream % p.Hkv) * rep + hg;
     } else {
@@ -785,7 +785,9 @@ bool bwd_dq_w32_fits(const BwdM& g, int head_dim) {
   return (int64_t)(g.S + BN) * g.k_sl * 2 < (1ll << 31) && (int64_t)(g.S + BN) * g.v_sl * 2 < (1ll << 31) && g.k_sl >= 0 && g.v_sl >= 0;
 }
 
-int launch_bwd_dq_w32(const BwdM& g, int dtype, int head_dim, hipStream_t s) {
+int launch_bwd_dq_w32(const BwdM& g0, int dtype, int head_dim, hipStream_t s) {
+  BwdM g = g0;
+  g.dq_chunk = bwd_stream_chunk(g, g.S);
   const int64_t blocks = (int64_t)g.B * g.Hq * ((g.L + BM - 1) / BM);
   const dim3 grid((unsigned)blocks, (unsigned)(g.dq_split_tiles ? g.dq_n_split : 1)), block(512);
   const bool bf = dtype == MI355_SDPA_BF16;

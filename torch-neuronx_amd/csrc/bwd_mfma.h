@@ -1,6 +1,8 @@
 // Parameter block shared by the MFMA backward kernels.
 #pragma once
 
+#include <algorithm>
+
 #include "mfma_common.h"
 #include "score_mod.h"
 
@@ -17,6 +19,9 @@ struct BwdM {
   int B, Hq, Hkv, L, S;
   int n_qt, n_kt;
   int causal, xcd_map;
+  // Streams, (batch, kv head) pairs, that an XCD takes at a time, all tiles of them before the next ones (0: all of its
+  // streams; only where they divide over the XCDs): the dQ kernel of bwd_dq_w32.hip, the dK/dV kernel of bwd_dkdv_w32.hip
+  int dq_chunk = 0, dkdv_chunk = 0;
   float scale;
   // masked calls (the two-wavefronts-per-SIMD kernels only): a bias or bool keep-mask (unit stride
   // over keys; strides in elements; bias_sl = 0 for one that does not depend on the query row)
@@ -84,6 +89,18 @@ struct BwdM {
   const int32_t* verdict = nullptr;
 };
 
+// dq_chunk / dkdv_chunk of a call whose streams are two tensors of `rows` rows each: as many as fill an XCD's 4 MB of L2, past
+// which every pass over the tiles of all of them brings the tensors from memory again (see stream_chunk, fwd_mfma_w32.hip).
+// Where there are eight chunks or more; with fewer the long tiles that start late cost what the L2 saves.  The whole backward
+// in us, all streams / chunks (D=128, causal): B=8, 32 heads, S=4096 4504 / 4074, B=8, S=2048 1249 / 1189, B=16, S=1024 811 / 773;  fewer:
+// B=4, S=4096 2054 / 2073, B=4, S=2048 not causal 983 / 1001.  Chunks of a quarter of the L2 lose up to 12 %.  Grouped heads share Q and dO
+// tiles in another order in dK/dV: B=8, 32/8 heads, S=1024 307 us, in chunks 366 (bwd_dkdv_w32.hip takes none there).
+inline int bwd_stream_chunk(const BwdM& g, int64_t rows) {
+  const int64_t streams = (int64_t)g.B * g.Hkv, bytes = std::max<int64_t>(1, rows * g.d_real * 4);
+  if (streams % 8 != 0 || g.bias_kind || g.gbias || g.window > 0 || g.sm.any) return 0;
+  const int64_t chunk = std::max<int64_t>(1, (4 << 20) / bytes);
+  return streams / 8 >= 8 * chunk ? (int)chunk : 0;
+}
 // parts the dK/dV kernel of bwd_dkdv_w32.hip / of bwd_wide.hip would use for this call
 int bwd_dkdv_w32_parts(const BwdM& g);
 int bwd_wide_parts(const BwdM& g);
@@ -103,6 +120,16 @@ __device__ __forceinline__ float dot8(u32x4 a, u32x4 b) {
   return s;
 }
 
+
+// a workgroup's place in its XCD's order -> stream of the XCD and tile of the stream
+__device__ __forceinline__ void chunk_place(int r, int per_xcd, int chunk, int n_tiles, int& stream, int& tile) {
+  int first = 0, n = per_xcd;
+  if (chunk > 0 && chunk < per_xcd) {
+    first = r / (chunk * n_tiles) * chunk, n = min(chunk, per_xcd - first);
+    r -= first * n_tiles;
+  }
+  stream = first + r % n, tile = r / n;
+}
 
 // bias element as a float (bool: 0 or -inf)
 __device__ __forceinline__ float bias_value(const void* base, int64_t idx, int kind) {
