@@ -1,5 +1,5 @@
 """Forward calls whose streams (a (batch, kv head)'s keys and values) an XCD takes in chunks: every (batch, head, row) is
-computed, once, also where the last chunk is a smaller one.
+computed, once, also where the last chunk is a smaller one or some XCDs serve a stream less than others.
 
 Bound, against the same attention in float64 on the kernel's inputs: P and the output are each rounded once to bf16,
 2^-9 relative, which adds up to at most twice that in the 2-norm: 4e-3; the log-sum-exp is a float32 sum, 1e-5."""
@@ -18,6 +18,9 @@ pytestmark = pytest.mark.gpu
     (43, 24, 24, 1024, 64, True),   # 129 in chunks of 16: eight and a last one of a single stream
     (19, 16, 8, 2048, 128, True),   # 19 in chunks of 4 are fewer than eight chunks: one after the other
     (35, 16, 8, 2048, 128, True),   # 35: nine
+    (31, 12, 12, 512, 64, False),   # 372 streams: the last four XCDs serve one less, in chunks of 8
+    (21, 28, 4, 512, 128, True),    # 84, seven heads a kv head, no chunks
+    (9, 12, 12, 785, 64, False),    # 108 would need a turn of workgroups more: not pinned
 ])
 def test_every_stream_is_computed(gpu_device, B, Hq, Hkv, S, D, causal):
     import torch_neuronx_amd as amd
@@ -44,6 +47,10 @@ def test_every_stream_is_computed(gpu_device, B, Hq, Hkv, S, D, causal):
     (13, 48, 48, 1000, 1000, 128, False, 1000), # 78 in chunks of 8, key counts
     (11, 16, 16, 1024, 1024, 64, True, None),   # 22 in chunks of 16 at head dim 64
     (25, 8, 8, 900, 900, 64, False, None),      # 25 in chunks of 4
+    (31, 12, 12, 512, 512, 64, False, None),    # 372 streams: the last four XCDs serve one less
+    (15, 12, 12, 500, 500, 64, True, None),     # 180
+    (5, 12, 4, 300, 300, 64, True, None),       # 20: not pinned
+    (29, 12, 4, 300, 300, 64, True, None),      # 116, three heads a kv head
 ])
 def test_every_gradient_is_computed(gpu_device, B, Hq, Hkv, L, S, D, causal, lens):
     """The same in the backward.  P, dS, O and the gradients are rounded once each: 8e-3, as in test_bwd_d64_gpu.py."""

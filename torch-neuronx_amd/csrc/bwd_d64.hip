@@ -149,13 +149,13 @@ struct BlockMap {
 };
 __device__ __forceinline__ BlockMap block_map(int bid, int streams, int n_tiles, int units, int chunk) {
   BlockMap m;
-  if (chunk == 0) {  // (streams do not divide over the XCDs)
+  if (chunk == 0) {  // (streams that are not pinned to XCDs)
     m.tile = bid / (streams * units);
     const int r = bid % (streams * units);
     m.stream = r / units, m.unit = r % units;
     return m;
   }
-  const int per_xcd = streams / 8, xcd = bid & 7;
+  const int per_xcd = (streams + 7) / 8, xcd = bid & 7;
   int r = bid >> 3;
   const int c = r / (chunk * n_tiles * units), in_chunk = min(chunk, per_xcd - c * chunk);
   r -= c * chunk * n_tiles * units;
@@ -171,6 +171,7 @@ template <typename T, bool DROP, bool TERMS>
 __device__ __forceinline__ void dq_body(const BwdM& p, uint32_t* keep_bits, int bid, int chunk, uint16_t (*k_t)[TILE], uint16_t (*v_t)[TILE]) {
   const int rep = p.Hq / p.Hkv;
   const BlockMap bm = block_map(bid, p.B * p.Hkv, p.n_qt, rep, chunk);
+  if (bm.stream >= p.B * p.Hkv) return;  // (their number is no multiple of eight)
   const int qt = p.n_qt - 1 - bm.tile, b = bm.stream / p.Hkv, hk = bm.stream % p.Hkv, h = hk * rep + bm.unit;  // heavy query tiles first
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -348,6 +349,7 @@ __device__ __forceinline__ void dkdv_body(const BwdM& p, const uint32_t* keep_bi
   } else {
     const BlockMap bm = block_map(bid, streams, p.n_kt, 1, chunk);
     kt = bm.tile, st = bm.stream;  // low key tiles see the most queries under a causal mask: first
+    if (st >= streams) return;
   }
   const int b = st / p.Hkv, hk = st % p.Hkv;
   const int rep_all = p.Hq / p.Hkv, rep = p.parts > 1 ? rep_all / p.parts_h : rep_all, h0 = hk * rep_all + ph * rep;
@@ -707,12 +709,32 @@ __global__ __launch_bounds__(256) void bwd_d64_terms_kernel(BwdM p, int blocks32
 // of it without one (a keep-mask and the rows that are written pass through the same L2).  Against half of it throughout,
 // backward in us: causal B=16, 12 heads, S=512 67.0 -> 63.3, B=8, 16, S=2048 280 -> 272, B=4, 32, S=4096 1005 -> 979;  not causal
 // B=64, 12, S=197 76.0 -> 74.5, B=60, 16, S=256 103 -> 101, with dropout B=32, 12, S=512 142 -> 140, B=64, S=250 95.2 -> 93.4
-int stream_chunk(const BwdM& g, int64_t rows) {
-  const int streams = g.B * g.Hkv;
-  if (streams % 8 != 0) return 0;
-  const int64_t bytes = rows * D * 4, all = streams / 8;
+// (units: workgroups per stream.  A number of streams that does not divide over the XCDs: see stream_chunk, fwd_mfma_w32.hip;
+// backward, anywhere / pinned, us: B=31, 12 heads, S=512 137 / 131, B=21, 6, S=785 120 / 115, B=15, 12, S=512 causal 55.5 / 53.7)
+int stream_chunk(const BwdM& g, int64_t rows, int64_t units) {
+  const int64_t streams = (int64_t)g.B * g.Hkv, bytes = rows * D * 4, all = (streams + 7) / 8;
+  if (streams % 8 != 0) {
+    if (units == 1 || (all * 8 - streams) * 15 > streams) return 0;
+    for (int slots = 32; slots <= 96; slots += 32)
+      if ((all * units + slots - 1) / slots > (streams * units + 8 * slots - 1) / (8 * slots)) return 0;
+  }
   if (all * bytes <= (9 << 19)) return (int)all;
   return (int)std::max<int64_t>(1, std::min<int64_t>(all, (g.causal ? 4 << 20 : 1 << 20) / bytes));
+}
+// the two grids: a chunk (0: streams are not pinned) and the workgroups
+struct Grid {
+  int chunk;
+  int64_t blocks;
+};
+Grid dq_grid(const BwdM& g) {
+  const int64_t units = (int64_t)(g.Hq / g.Hkv) * g.n_qt, streams = (int64_t)g.B * g.Hkv;
+  const int chunk = stream_chunk(g, g.S, units);
+  return {chunk, (chunk ? (streams + 7) / 8 * 8 : streams) * units};
+}
+Grid dkdv_grid(const BwdM& g) {
+  const int64_t streams = (int64_t)g.B * g.Hkv;
+  const int chunk = g.parts > 1 ? 0 : stream_chunk(g, (int64_t)g.L * (g.Hq / g.Hkv), g.n_kt);
+  return {chunk, (chunk ? (streams + 7) / 8 * 8 : streams) * g.n_kt * g.parts};
 }
 
 // Causal calls whose workgroups (tiles times streams) are too few to hide the longest of them: a key block of the first
@@ -757,9 +779,9 @@ int launch_together(const BwdM& g, hipStream_t s) {
   const int blocks32 = (g.L + 31) / 32;
   hipLaunchKernelGGL((bwd_d64_terms_kernel<T>), dim3((unsigned)(((int64_t)g.B * g.Hq * blocks32 + 3) / 4)), dim3(256), 0, s, g, blocks32);
   if (int rc = check_launch("bwd_d64_terms_kernel")) return rc;
-  const int dq = g.B * g.Hq * g.n_qt, dkdv = g.B * g.Hkv * g.n_kt * g.parts;
-  const int grid = ((dq + 7) / 8 + (dkdv + 7) / 8) * 8;
-  hipLaunchKernelGGL((bwd_d64_both_kernel<T>), dim3(grid), dim3(256), 0, s, g, dq, dkdv, stream_chunk(g, g.S), stream_chunk(g, (int64_t)g.L * (g.Hq / g.Hkv)));
+  const Grid dq = dq_grid(g), dkdv = dkdv_grid(g);
+  const int grid = (int)((dq.blocks + 7) / 8 + (dkdv.blocks + 7) / 8) * 8;
+  hipLaunchKernelGGL((bwd_d64_both_kernel<T>), dim3(grid), dim3(256), 0, s, g, (int)dq.blocks, (int)dkdv.blocks, dq.chunk, dkdv.chunk);
   return check_launch("bwd_d64_both_kernel");
 }
 
@@ -770,13 +792,12 @@ int launch_t(const BwdM& g, uint32_t* bits, hipStream_t s) {
     if (rc || g.parts == 1) return rc;
     return launch_bwd_dkdv_merge(g, std::is_same<T, bf16_t>::value ? MI355_SDPA_BF16 : MI355_SDPA_F16, s);
   }
-  hipLaunchKernelGGL((bwd_d64_dq_kernel<T, DROP>), dim3((unsigned)((int64_t)g.B * g.Hq * g.n_qt)), dim3(256), 0, s, g, bits, stream_chunk(g, g.S));
+  const Grid dq = dq_grid(g), dkdv = dkdv_grid(g);
+  hipLaunchKernelGGL((bwd_d64_dq_kernel<T, DROP>), dim3((unsigned)dq.blocks), dim3(256), 0, s, g, bits, dq.chunk);
   int rc = check_launch("bwd_d64_dq_kernel");
   if (rc) return rc;
   if (!DROP && w32_dkdv(g)) return launch_bwd_dkdv_w32(g, std::is_same<T, bf16_t>::value ? MI355_SDPA_BF16 : MI355_SDPA_F16, 64, s);
-  const int64_t blocks = (int64_t)g.B * g.Hkv * g.n_kt * g.parts;
-  const int chunk = stream_chunk(g, (int64_t)g.L * (g.Hq / g.Hkv));
-  hipLaunchKernelGGL((bwd_d64_dkdv_kernel<T, DROP>), dim3((unsigned)blocks), dim3(256), 0, s, g, (const uint32_t*)bits, chunk);
+  hipLaunchKernelGGL((bwd_d64_dkdv_kernel<T, DROP>), dim3((unsigned)dkdv.blocks), dim3(256), 0, s, g, (const uint32_t*)bits, dkdv.chunk);
   rc = check_launch("bwd_d64_dkdv_kernel");
   if (rc || g.parts == 1) return rc;
   return launch_bwd_dkdv_merge(g, std::is_same<T, bf16_t>::value ? MI355_SDPA_BF16 : MI355_SDPA_F16, s);

@@ -110,7 +110,7 @@ __device__ __forceinline__ void fwd_w32_body(const FwdM& p, const MaskArgs ma) {
     b = bhk / p.Hkv, h = (bhk % p.Hkv) * rep + (bhc % chunks) * hpw + wave % hpw, qt = 0;
     wrow = (wave / hpw) * 32;
   } else {
-    decode_block(p, b, h, qt);
+    if (!decode_block(p, b, h, qt)) return;
   }
   const int hk = h / (p.Hq / p.Hkv);
   const int col = lane & 31, half = lane >> 5;
@@ -1125,7 +1125,7 @@ int share_keys(const FwdM& g, int head_dim) {
 template <typename T, int D, int MASK, bool PATTERN>
 int launch_halves(FwdM g, int rows, hipStream_t s) {
   g.grouped = 0, g.n_qt = (g.L + rows - 1) / rows;
-  const dim3 grid((unsigned)((int64_t)g.B * g.Hq * g.n_qt));
+  const dim3 grid((unsigned)tile_blocks(g));
   if constexpr (D == 128) {  // (128 rows: this width only)
     if (rows == 128) return launch_one<T, D, 4, MASK, PATTERN, 2>(g, grid, s);
   }
@@ -1253,7 +1253,19 @@ int launch_fwd_split_merge(const FwdM& g, int dtype, hipStream_t s) {
 //   causal, 8 chunks: B=4, 64 heads, S=4096, D=64 638 / 580, B=16, 32/8, S=4096, D=128 1989 / 1912, B=8, 32, S=2048 304 / 279, B=16, S=1024 220 / 190
 //     fewer: 4: B=8, 16, S=2048, D=64 82 / 85, B=4, 32, S=999, D=128 with key counts 48 / 50;  2: B=4, 16, S=2048, D=128 72 / 71
 static int stream_chunk(const FwdM& g) {
-  const int64_t per_xcd = (int64_t)g.B * g.Hkv / 8, bytes = std::max<int64_t>(1, (int64_t)g.S * (g.d_real + g.dv_real) * 2);
+  const int64_t streams = (int64_t)g.B * g.Hkv, per_xcd = (streams + 7) / 8;
+  if (streams % 8 != 0) {
+    // Some XCDs serve a stream less than others.  Unless they idle for more than a fifteenth, or the others need a turn of
+    // workgroups more than all would, one to three of which share a compute unit, that costs less than the K and V that every XCD
+    // brings for itself.  Anywhere / pinned in us: B=31, 12 heads, S=512 41.8 / 38.5, B=21, 6, S=785 36.3 / 34.3, B=41, 6, S=400 24.9 / 22.5,
+    // B=63, 12, S=197 24.5 / 23.1, B=15, 12, S=512 causal 17.3 / 16.5, B=21, 28/4, S=512, D=128 causal 82.3 / 74.1;  a turn more: B=9, 12, S=785 27.7 / 34.1.
+    // (One workgroup a stream shares nothing: 1 to 2 % slower.)
+    const int64_t units = (int64_t)(g.Hq / g.Hkv) * g.n_qt;
+    if (units == 1 || (per_xcd * 8 - streams) * 15 > streams) return 0;
+    for (int slots = 32; slots <= 96; slots += 32)
+      if ((per_xcd * units + slots - 1) / slots > (streams * units + 8 * slots - 1) / (8 * slots)) return 0;
+  }
+  const int64_t bytes = std::max<int64_t>(1, (int64_t)g.S * (g.d_real + g.dv_real) * 2);
   if (g.bias_kind || g.window > 0 || per_xcd * bytes <= (9 << 19)) return (int)per_xcd;
   const int64_t chunk = std::min(per_xcd, std::max<int64_t>(1, (g.causal ? 4 << 20 : 1 << 20) / bytes));
   return (int)(g.causal && per_xcd < 8 * chunk ? per_xcd : chunk);
@@ -1262,7 +1274,7 @@ static int stream_chunk(const FwdM& g) {
 int launch_fwd_mfma_w32(const FwdM& g0, int dtype, int head_dim, int waves, hipStream_t s) {
   FwdM g = g0;
   fwd_w32_plan(g, head_dim, waves);
-  if (g.xcd_map) g.xcd_map = stream_chunk(g);
+  g.xcd_map = stream_chunk(g);
   if (g.split_tiles) {  // (the caller's workspace: too small or absent, and the call runs unsplit)
     const size_t rows = (size_t)g.B * g.Hq * g.n_split * g.L;
     if (g.part_o && g.n_split <= 512 && g.part_bytes >= rows * (g.dv_real + 1) * sizeof(float)) g.part_lse = g.part_o + rows * g.dv_real;
@@ -1273,7 +1285,7 @@ int launch_fwd_mfma_w32(const FwdM& g0, int dtype, int head_dim, int waves, hipS
     const int rc = launch_fwd_few_rows(g, dtype, head_dim, s);
     return rc != MI355_SDPA_OK || !g.split_tiles ? rc : launch_fwd_split_merge(g, dtype, s);
   }
-  const int64_t blocks = g.grouped ? (int64_t)g.B * (g.Hq / g.grouped) * g.n_split : (int64_t)g.B * g.Hq * g.n_qt;
+  const int64_t blocks = g.grouped ? (int64_t)g.B * (g.Hq / g.grouped) * g.n_split : tile_blocks(g);
   if (blocks == 0) return MI355_SDPA_OK;
   if (blocks > 0x7fffffff) {
     set_error("SDPA: too many query tiles (%lld)", (long long)blocks);
