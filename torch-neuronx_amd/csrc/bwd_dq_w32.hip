@@ -250,7 +250,9 @@ __device__ __forceinline__ void bwd_dq_w32_body(const BwdM& p, const MaskArgs ma
     if constexpr (MASK == 2) return listed ? __builtin_amdgcn_readfirstlane((int)tile_list[u]) : u;
     else return FUNC ? u + (u >= n_lead ? skip : 0) : u;
   };
-  const int nt_w = ma.causal ? min(nt, (qw0 + 31) / BN + 1 - skip) : nt;  // tiles with work for this wavefront
+  // (none past the last row, up to seven of eight wavefronts, which left to walk every tile took matrix ops from the others.  The whole
+  // backward, D=128 causal: B=2, 28/4 heads, S=1800 238.8 -> 229.4 us, B=8, 32/8, S=300 79.4 -> 76.5, B=2, S=1050 137.8 -> 135.4)
+  const int nt_w = qw0 >= p.L ? 0 : ma.causal ? min(nt, (qw0 + 31) / BN + 1 - skip) : nt;  // tiles with work for this wavefront
   // first tile that needs masking: the one that reaches this wavefront's first row on the causal
   // diagonal (qw0 is a multiple of BN), or a ragged last tile; with a window also every tile that
   // reaches below the window of the wavefront's last row and is not made of sink keys alone
