@@ -57,6 +57,9 @@ def _want(q, k, v, causal, lens, window, sink):
     (1, 28, 4, 1055, 1055, 128, 128, True, None, 0, False),
     (2, 28, 4, 800, 800, 128, 128, True, None, 0, False),   # 392 > 8 x 25: whole keys
     (1, 24, 24, 1055, 1055, 104, 104, True, [777], 0, True),
+    (1, 32, 8, 801, 801, 128, 128, True, None, 0, False),   # 32 heads, whose last 128 rows are a quarter and three quarters full
+    (2, 16, 4, 993, 993, 128, 128, True, [990, 400], 0, False),
+    (1, 33, 11, 801, 801, 128, 128, True, None, 0, False),  # 231 > 8 x 28
 ])
 def test_halves_of_a_workgroup(amd, gpu_device, dtype, B, Hq, Hkv, L, S, D, Dv, causal, lens, window, sink):
     g = torch.Generator(device=gpu_device).manual_seed(L + S + D)

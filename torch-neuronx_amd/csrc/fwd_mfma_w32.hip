@@ -1113,17 +1113,18 @@ int launch_one(const FwdM& g, dim3 grid, hipStream_t s) {
 //   128 rows, two wavefronts a SIMD: a long causal chain in front of many short ones, in one turn of two workgroups a compute
 //   unit.  D=128: 32/8 heads, S=1021 19.7 / 18.8, S=1407 28.6 / 25.8; 28/4, S=1407 27.2 / 24.0; 24/8 25.7 / 22.5; 16/4, S=4000
 //   80.7 / 69.3.  More than 512 workgroups: 32/8, S=2057 46.3 / 50.7, S=2500 59.5 / 66.0; 24/8, S=3000 65.0 / 68.0.  The exchange
-//   costs 1.5 us: S=256 9.0 / 10.2.  The bound of 8 * tiles keeps out calls of so many heads that short chains hide each other:
-//   64/8 heads, S=707 19.2 / 22.1, S=1021 26.9 / 29.0.  It is tighter than that needs: of 32 heads it takes the lengths whose last
-//   128 rows are full or nearly so, and those between would gain too (S=907 19.1 / 18.6, 1107 23.0 / 20.2, 1307 26.1 / 25.3,
-//   1907 41.9 / 39.0); 16, 24 and 28 heads are taken throughout.
+//   costs 1.5 us: S=256 9.0 / 10.2.  The bound of 8 workgroups a key tile, 32 heads, keeps out calls of
+//   so many that short chains hide each other: 64/8 heads, S=707 19.2 / 22.1, S=1021 26.9 / 29.0, 48/8, S=820 19.8 / 22.3, 40/8
+//   18.5 / 19.4.  A last, partial block of 128 rows counts whole: 32/8, S=830 16.3 / 15.9, 907 17.9 / 17.3, 1030 21.0 / 19.5, 1107
+//   22.5 / 20.2, 1307 26.4 / 25.3, 1700 36.1 / 34.8, 1907 39.8 / 39.7, at head dim 104 1100 22.8 / 20.3.  Fewer than 24 tiles: 520
+//   12.4 / 12.8, 580 13.2 / 13.0, 760 15.4 / 15.3.
 int share_keys(const FwdM& g, int head_dim) {
   if (g.whole_keys || g.grouped > 1 || g.split_tiles || g.L <= 32) return 0;
   int tiles = (g.S + BN - 1) / BN;
   if (g.window > 0) tiles = std::min(tiles, (g.window + 128) / BN);
   const int64_t heads = (int64_t)g.B * g.Hq, wg64 = heads * ((g.L + 63) / 64), wg128 = heads * ((g.L + 127) / 128);
   if (tiles >= 4 && wg64 <= (head_dim == 64 && g.causal ? g.grouped ? 512 : std::max(256, std::min(768, 16 * tiles)) : 256)) return 64;
-  if (!g.grouped && head_dim == 128 && g.causal && tiles >= 24 && wg128 <= std::min(512, 8 * tiles)) return 128;
+  if (!g.grouped && head_dim == 128 && g.causal && tiles >= 24 && wg128 <= std::min(512, 8 * ((tiles + 3) & ~3))) return 128;
   return 0;
 }
 template <typename T, int D, int MASK, bool PATTERN>
