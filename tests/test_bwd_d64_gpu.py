@@ -1,4 +1,4 @@
-"""Backward at head dims up to 64 (the pair of kernels that keeps three workgroups on a compute unit): sizes around
+"""Backward at head dims up to 64 (the kernels of 128-row and 128-key workgroups): sizes around
 its 32-row blocks and 64-row tiles, narrow rows, grouped heads, key counts, dropout over numbers of keys that
 are no multiple of four or of a word of keep bits, items shared out over workgroups, many streams per XCD.
 
