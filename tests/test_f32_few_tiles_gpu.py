@@ -75,3 +75,18 @@ def test_key_counts(amd, gpu_device, causal):
 def test_sixteen_rows_against_the_oracle(amd, gpu_device, B, Hq, Hkv, L, S, E, Dv, causal):
     """The same in workgroups of 16 rows whose eight wavefronts take every eighth block of 16 keys."""
     test_against_the_oracle(amd, gpu_device, B, Hq, Hkv, L, S, E, Dv, causal)
+
+
+@pytest.mark.parametrize("B,Hq,Hkv,L,S,E,Dv", [
+    (10, 4, 2, 128, 128, 128, 128), (41, 1, 1, 128, 170, 128, 128),  # under the mask, head dims above 64: 320 of them of 33 to 128 rows, and past it
+    (14, 4, 4, 129, 129, 104, 104), (19, 3, 3, 129, 140, 104, 104),  # 512 from 129 rows on
+    (32, 4, 4, 32, 32, 128, 72), (43, 3, 1, 32, 90, 128, 128),       # 256 up to 32 rows
+    (128, 4, 4, 16, 16, 128, 128), (171, 3, 3, 16, 16, 128, 128),    # 512 up to 16
+    (64, 4, 4, 32, 32, 64, 64), (257, 1, 1, 20, 32, 64, 64),         # head dims up to 64: 512 of 17 to 32 rows
+    (11, 3, 3, 400, 400, 64, 64), (17, 2, 2, 400, 400, 48, 48),      # 832 up to 400 rows
+    (25, 1, 1, 160, 97, 64, 64), (13, 2, 2, 160, 97, 128, 128),      # more rows than keys: 256 as without the mask,
+    (32, 1, 1, 400, 47, 64, 64), (128, 2, 2, 64, 32, 64, 64),        # but for up to 96 keys at head dims up to 64
+    (24, 6, 2, 38, 38, 128, 128), (32, 4, 4, 38, 38, 128, 128),      # 288 of 32 rows, and 256
+])
+def test_on_both_sides_of_the_lines_of_sixteen_rows(amd, gpu_device, B, Hq, Hkv, L, S, E, Dv):
+    test_against_the_oracle(amd, gpu_device, B, Hq, Hkv, L, S, E, Dv, True)
