@@ -211,3 +211,20 @@ def test_rows_that_a_key_does_not_see_do_not_reach_it(amd, gpu_device):
         clean = (row // 32 + 1) * 32
         for name, a, w in zip(("dk", "dv"), got[1:], want[1:]):
             assert torch.equal(a[:, :, clean:], w[:, :, clean:]), (name, row)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("B,Hq,Hkv,L,S,D,causal,lens", [
+    (64, 8, 8, 64, 64, 64, False, None), (65, 8, 8, 64, 64, 64, False, None),    # 512 key blocks, and 520 block by block
+    (96, 8, 8, 33, 31, 64, True, None), (97, 8, 8, 33, 31, 64, True, None),      # 768, and past them
+    (48, 8, 8, 17, 200, 48, False, None),                                        # one item, two key blocks
+    (96, 32, 8, 40, 40, 64, False, None),                                        # four heads' items of one query tile
+    (80, 8, 8, 128, 128, 64, False, None), (80, 8, 8, 129, 128, 64, False, None),  # two items, three
+    (42, 16, 8, 65, 140, 64, True, [140 - 3 * i for i in range(42)]),            # causal: eight items at the most, above 640
+    (41, 8, 8, 190, 200, 64, True, [0, 33] * 20 + [200]),
+    (20, 8, 8, 460, 460, 64, True, None), (21, 8, 8, 512, 512, 64, True, None), (21, 8, 8, 513, 512, 64, True, None),
+])
+def test_a_third_workgroup_on_a_compute_unit(amd, gpu_device, B, Hq, Hkv, L, S, D, causal, lens, dtype):
+    """More key blocks than two per compute unit and at most three, of few items: dK/dV block by block, on both sides of the
+    lines of that."""
+    _check(amd, gpu_device, B, Hq, Hkv, L, S, D, causal, dtype, lens, 0.0)

@@ -336,7 +336,8 @@ __global__ __launch_bounds__(256, 3) void bwd_d64_dq_kernel(BwdM p, uint32_t* ke
 
 template <bool DROP>
 using KeepTile = uint32_t[DROP ? 4 : 1][BQ];  // [wavefront's 32 keys][row]
-template <typename T, bool DROP>
+// AHEAD: the items whose blocks are all live for a wavefront in two phases, one block ahead; without it every item block by block
+template <typename T, bool DROP, bool AHEAD>
 __device__ __forceinline__ void dkdv_body(const BwdM& p, const uint32_t* keep_bits, int bid, int chunk, uint16_t (*q_t)[TILE], uint16_t (*do_t)[TILE],
                                           float (*lse_s)[BQ], float (*dl_s)[BQ], KeepTile<DROP>* bit_s) {
   const int streams = p.B * p.Hkv;
@@ -463,7 +464,7 @@ __device__ __forceinline__ void dkdv_body(const BwdM& p, const uint32_t* keep_bi
     }
   };
   // items with both blocks of 32 rows live for this wavefront (under a causal mask the others come last)
-  int n_main = kw0 < S ? n_items : 0;
+  int n_main = AHEAD && kw0 < S ? n_items : 0;
   if (p.causal) n_main = max(min(n_main, rep * (nqs - (kw0 + 32) / BQ) - it0), 0);
   if (n_items > 0) {
     wait_loads();
@@ -477,7 +478,7 @@ __device__ __forceinline__ void dkdv_body(const BwdM& p, const uint32_t* keep_bi
   // So every product has vector work of its own wavefront to run under, and one register tile each of scores and dP is
   // enough.  Operands are requested four ops ahead of their use, statistics of four rows four slots ahead, across the phases.
   int it = 0;
-  if (n_main > 0) {
+  if (AHEAD && n_main > 0) {
     f32x16 s, dp;
     uint32_t pk[8], bs[8];  // P and dS in pairs
     u32x4 ring[4];
@@ -612,15 +613,21 @@ __device__ __forceinline__ void dkdv_body(const BwdM& p, const uint32_t* keep_bi
       for (int ks = 0; ks < KS; ++ks) dp = Mma<T>::run(rd.rows(dot, 0, ks), vf[ks], dp);
       mask(s, qb);
       uint32_t pm[8], ds[8];
+      f32x4 l4, d4;  // (with dropout four rows' at a time; without, in the kernel of 168 registers, that sends some to scratch)
+      u32x4 w4;
 #pragma unroll
       for (int i = 0; i < 8; ++i) {
-        const int r0 = mb * 32 + (i >> 1) * 8 + half * 4 + (i & 1) * 2;  // the rows of scores 2 i and 2 i + 1
-        const float l0 = lse_s[buf][r0], l1 = lse_s[buf][r0 + 1], d0 = dl_s[buf][r0], d1 = dl_s[buf][r0 + 1];
+        const int e = (2 * i) & 3, r0 = mb * 32 + (i >> 1) * 8 + half * 4 + e;  // the rows of scores 2 i and 2 i + 1
+        if constexpr (DROP) {
+          if (e == 0) l4 = *(const f32x4*)&lse_s[buf][r0], d4 = *(const f32x4*)&dl_s[buf][r0], w4 = *(const u32x4*)&bit_s[buf][wave][r0];
+        }
+        const float l0 = DROP ? l4[e] : lse_s[buf][r0], l1 = DROP ? l4[e + 1] : lse_s[buf][r0 + 1];
+        const float d0 = DROP ? d4[e] : dl_s[buf][r0], d1 = DROP ? d4[e + 1] : dl_s[buf][r0 + 1];
         const uint32_t pk = Mma<T>::pack(__builtin_amdgcn_exp2f(fmaf(s[2 * i], c, -l0)), __builtin_amdgcn_exp2f(fmaf(s[2 * i + 1], c, -l1)));
         float g0 = dp[2 * i], g1 = dp[2 * i + 1];
         pm[i] = pk;
         if constexpr (DROP) {
-          const uint32_t m0 = (uint32_t)__builtin_amdgcn_sbfe((int)bit_s[buf][wave][r0], (uint32_t)col, 1u), m1 = (uint32_t)__builtin_amdgcn_sbfe((int)bit_s[buf][wave][r0 + 1], (uint32_t)col, 1u);
+          const uint32_t m0 = (uint32_t)__builtin_amdgcn_sbfe((int)w4[e], (uint32_t)col, 1u), m1 = (uint32_t)__builtin_amdgcn_sbfe((int)w4[e + 1], (uint32_t)col, 1u);
           pm[i] &= __builtin_amdgcn_perm(m1, m0, 0x05040100u);
           g0 = fmaf(m0 ? g0 : 0.f, p.keep_scale, -d0), g1 = fmaf(m1 ? g1 : 0.f, p.keep_scale, -d1);
         } else {
@@ -657,17 +664,17 @@ __device__ __forceinline__ void dkdv_body(const BwdM& p, const uint32_t* keep_bi
   store_rows<T>(dv, DROP ? p.keep_scale : 1.f, &do_t[0][0] + wave * 32 * D, lane, (uint16_t*)p.gv + b * p.gv_sb + hk * p.gv_sh, p.gv_sl, kw0, p.S, dr);
 }
 
-// Two workgroups per compute unit: the two phases of a block hold 221 registers (242 with dropout).  (The four products one
-// after the other in 168 registers, a third workgroup hiding the chain, is what this replaced: B=4, 12 heads, S=512, not
-// causal, the whole backward 32.2 -> 27.5 us, B=1, S=1024 causal 39.1 -> 30.1, B=64, S=197 79.6 -> 77.7, B=4, 32 heads, S=4096
-// causal 1027 -> 1004; with dropout B=32, S=512 148 -> 139, with key counts as well 158 -> 148.)
-template <typename T, bool DROP>
-__global__ __launch_bounds__(256, 2) void bwd_d64_dkdv_kernel(BwdM p, const uint32_t* keep_bits, int chunk) {
+// One block ahead: two workgroups per compute unit, the two phases of a block hold 211 to 240 registers.  (Against the four
+// products one after the other in 168 registers, three workgroups: B=4, 12 heads, S=512, not causal, the whole backward 32.2 -> 27.5 us,
+// B=1, S=1024 causal 39.1 -> 30.1, B=64, S=197 79.6 -> 77.7, B=4, 32 heads, S=4096 causal 1027 -> 1004; with dropout B=32, S=512
+// 148 -> 139, with key counts as well 158 -> 148.  Where those are still taken: three_per_cu.)
+template <typename T, bool DROP, bool AHEAD>
+__global__ __launch_bounds__(256, AHEAD ? 2 : 3) void bwd_d64_dkdv_kernel(BwdM p, const uint32_t* keep_bits, int chunk) {
   __shared__ __attribute__((aligned(16))) uint16_t q_t[3][TILE];
   __shared__ __attribute__((aligned(16))) uint16_t do_t[3][TILE];
   __shared__ __attribute__((aligned(16))) float lse_s[3][BQ], dl_s[3][BQ];
   __shared__ __attribute__((aligned(16))) KeepTile<DROP> bit_s[DROP ? 3 : 1];
-  dkdv_body<T, DROP>(p, keep_bits, blockIdx.x, chunk, q_t, do_t, lse_s, dl_s, bit_s);
+  dkdv_body<T, DROP, AHEAD>(p, keep_bits, blockIdx.x, chunk, q_t, do_t, lse_s, dl_s, bit_s);
 }
 
 // Both in one launch, behind bwd_d64_terms_kernel: a dK/dV and a dQ workgroup by turns, eight of each (the XCDs), the
@@ -682,7 +689,7 @@ __global__ __launch_bounds__(256, 2) void bwd_d64_both_kernel(BwdM p, int dq_blo
   const int bid = (eight < 2 * turns ? eight >> 1 : eight - turns) * 8 + in;
   if (bid >= (dq ? dq_blocks : dkdv_blocks)) return;
   if (dq) dq_body<T, false, false>(p, nullptr, bid, dq_chunk, a_t, b_t);
-  else dkdv_body<T, false>(p, nullptr, bid, dkdv_chunk, a_t, b_t, lse_s, dl_s, nullptr);
+  else dkdv_body<T, false, true>(p, nullptr, bid, dkdv_chunk, a_t, b_t, lse_s, dl_s, nullptr);
 }
 
 // delta and the log2-domain log-sum-exp of 32 rows per wavefront, the sums in dq_body's order
@@ -775,6 +782,21 @@ bool together(const BwdM& g) {
   return all <= (!g.causal ? 768 : g.L < 7 * BQ ? 512 : g.Hq > g.Hkv || g.L <= 14 * BQ ? 768 : 1024);
 }
 
+// Calls whose dK/dV runs block by block, three workgroups per compute unit: more key blocks than two per compute unit, but
+// not than three, which then take one turn instead of two, and so few items each that the second turn is longer than what
+// the two phases save.  A block ahead / block by block, the whole backward in us, D=64:
+//   one item, 576 blocks: B=72, 8 heads, S=32 18.7 / 16.4, S=64 21.4 / 19.8;  768: S=32 18.9 / 17.0, S=64 22.9 / 21.8, causal 23.8 / 22.2, 32/8 heads, S=32 40.4 / 36.7
+//     512: S=32 13.8 / 14.5, S=64 16.8 / 17.5;  832: S=32 22.8 / 22.8, S=64 28.0 / 28.5
+//   two: 640, S=128 35.0 / 34.0, causal 35.9 / 34.2;  832: 44.5 / 44.1, causal 45.2 / 45.7;  three: S=160 31.0 / 30.7, S=192 35.2 / 34.5
+//   causal, up to eight: 576, S=160 27.5 / 27.8, S=320 30.6 / 32.1;  704: S=256 41.0 / 38.0, S=320 36.7 / 34.0, S=384 42.7 / 38.5, S=512 56.1 / 54.2
+//     768: S=256 42.6 / 39.8, S=384 45.6 / 41.1, S=512 53.6 / 51.0;  ten: S=640 54.4 / 53.9
+// (With dropout, whose kernel takes more registers, a block ahead everywhere: B=64, 12 heads, S=64 25.0 / 26.7, S=100 39.2 / 42.0.)
+bool three_per_cu(const BwdM& g) {
+  const int64_t blocks = (int64_t)g.B * g.Hkv * g.n_kt;
+  const int tiles = (g.L + BQ - 1) / BQ, items = g.Hq / g.Hkv * tiles;
+  return blocks > 512 && blocks <= 768 && (tiles <= 1 || items <= 2 || (g.causal && items <= 8 && blocks > 640));
+}
+
 template <typename T>
 int launch_together(const BwdM& g, hipStream_t s) {
   const int blocks32 = (g.L + 31) / 32;
@@ -798,7 +820,8 @@ int launch_t(const BwdM& g, uint32_t* bits, hipStream_t s) {
   int rc = check_launch("bwd_d64_dq_kernel");
   if (rc) return rc;
   if (!DROP && w32_dkdv(g)) return launch_bwd_dkdv_w32(g, std::is_same<T, bf16_t>::value ? MI355_SDPA_BF16 : MI355_SDPA_F16, 64, s);
-  hipLaunchKernelGGL((bwd_d64_dkdv_kernel<T, DROP>), dim3((unsigned)dkdv.blocks), dim3(256), 0, s, g, (const uint32_t*)bits, dkdv.chunk);
+  if (!DROP && three_per_cu(g)) hipLaunchKernelGGL((bwd_d64_dkdv_kernel<T, false, false>), dim3((unsigned)dkdv.blocks), dim3(256), 0, s, g, nullptr, dkdv.chunk);
+  else hipLaunchKernelGGL((bwd_d64_dkdv_kernel<T, DROP, true>), dim3((unsigned)dkdv.blocks), dim3(256), 0, s, g, (const uint32_t*)bits, dkdv.chunk);
   rc = check_launch("bwd_d64_dkdv_kernel");
   if (rc || g.parts == 1) return rc;
   return launch_bwd_dkdv_merge(g, std::is_same<T, bf16_t>::value ? MI355_SDPA_BF16 : MI355_SDPA_F16, s);
