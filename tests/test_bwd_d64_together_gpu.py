@@ -27,6 +27,14 @@ pytestmark = pytest.mark.gpu
     (8, 12, 12, 511, 511, 64, True, None),      # 768 in all
     (2, 16, 16, 1100, 700, 40, True, [700, 699]),
     (4, 16, 16, 1024, 1024, 64, True, None),    # 1024 in all
+    # not causal, up to five query tiles 512 in all, from six and with three heads a kv head 768, 704 with two, and past each
+    (32, 8, 8, 128, 100, 64, False, None), (33, 8, 8, 127, 128, 64, False, [128 - i for i in range(33)]),
+    (16, 8, 8, 321, 321, 64, False, None), (17, 8, 8, 384, 300, 48, False, None), (16, 8, 8, 320, 320, 64, False, None),
+    (7, 16, 8, 400, 400, 64, False, None), (8, 16, 8, 400, 500, 64, False, None),
+    (38, 16, 4, 65, 65, 64, False, None), (39, 16, 4, 65, 65, 64, False, None), (48, 12, 4, 65, 65, 64, False, None),
+    # causal: three workgroups a compute unit above 640 and up to 768, up to ten query tiles
+    (10, 8, 8, 448, 448, 64, True, None), (11, 8, 8, 448, 448, 64, True, None), (12, 8, 8, 500, 512, 40, True, [512 - 40 * i for i in range(12)]),
+    (12, 8, 8, 512, 513, 64, True, None), (9, 8, 8, 640, 630, 64, True, None), (9, 8, 8, 641, 630, 64, True, None),
 ])
 def test_gradients(gpu_device, dtype, bound, B, Hq, Hkv, L, S, D, causal, lens):
     import torch_neuronx_amd as amd

@@ -679,8 +679,8 @@ __global__ __launch_bounds__(256, AHEAD ? 2 : 3) void bwd_d64_dkdv_kernel(BwdM p
 
 // Both in one launch, behind bwd_d64_terms_kernel: a dK/dV and a dQ workgroup by turns, eight of each (the XCDs), the
 // heaviest of both first.  (See together for where.)
-template <typename T>
-__global__ __launch_bounds__(256, 2) void bwd_d64_both_kernel(BwdM p, int dq_blocks, int dkdv_blocks, int dq_chunk, int dkdv_chunk) {
+template <typename T, bool AHEAD>
+__global__ __launch_bounds__(256, AHEAD ? 2 : 3) void bwd_d64_both_kernel(BwdM p, int dq_blocks, int dkdv_blocks, int dq_chunk, int dkdv_chunk) {
   __shared__ __attribute__((aligned(16))) uint16_t a_t[3][TILE];
   __shared__ __attribute__((aligned(16))) uint16_t b_t[3][TILE];
   __shared__ __attribute__((aligned(16))) float lse_s[3][BQ], dl_s[3][BQ];
@@ -689,7 +689,7 @@ __global__ __launch_bounds__(256, 2) void bwd_d64_both_kernel(BwdM p, int dq_blo
   const int bid = (eight < 2 * turns ? eight >> 1 : eight - turns) * 8 + in;
   if (bid >= (dq ? dq_blocks : dkdv_blocks)) return;
   if (dq) dq_body<T, false, false>(p, nullptr, bid, dq_chunk, a_t, b_t);
-  else dkdv_body<T, false, true>(p, nullptr, bid, dkdv_chunk, a_t, b_t, lse_s, dl_s, nullptr);
+  else dkdv_body<T, false, AHEAD>(p, nullptr, bid, dkdv_chunk, a_t, b_t, lse_s, dl_s, nullptr);
 }
 
 // delta and the log2-domain log-sum-exp of 32 rows per wavefront, the sums in dq_body's order
@@ -767,19 +767,32 @@ bool w32_both(const BwdM& g) {
 // behind the one that forms the row terms (4 us).  The line is the number of workgroups in all (two of them share a compute
 // unit), by the length of a chain, which is what the second launch would wait for.  Two launches / one, us, 12 heads and
 // D=64 where not said:
-//   not causal, 192: B=2, S=512 26.4 / 20.4;  384: B=8, S=197 20.3 / 20.2, B=4, S=512 29.9 / 27.5;  448: B=2, 16 heads, S=785 41.1 / 38.9
-//     768: B=3, 16, S=1000 71.7 / 68.9;  3072: B=64, S=197 78 / 92
+//   not causal, 192: B=2, S=512 26.4 / 20.4;  384: B=8, S=197 20.3 / 20.2, B=4, S=512 29.9 / 27.5;  448: B=2, 16 heads, S=785 41.1 / 38.9;  3072: B=64, S=197 78 / 92
+//     beyond 512 by the number of tiles, 640, 8 heads: B=40, S=64 16.0 / 17.6, S=128 22.5 / 23.3, B=20, S=256 27.8 / 28.6;  720: B=15, S=320 29.3 / 30.2, S=384 34.0 / 33.3,
+//       B=9, S=640 45.6 / 43.8;  768: B=3, 16, S=1000 71.7 / 68.9;  816: B=17, S=384 34.7 / 39.2
+//     two heads a kv head, 576: 16/8, B=24, S=128 21.8 / 24.6, B=6, S=512 43.6 / 41.9;  768: 16/8, B=32, S=128 23.2 / 26.9, B=8, S=512 44.4 / 48.0
+//     three and more, 640: 32/8, B=16, S=100 27.8 / 25.1, S=128 27.2 / 25.7;  672: B=3, S=400 51.2 / 50.3;  704: 12/4, B=22, S=200 38.9 / 37.2;  768: B=16, S=330 51.2 / 49.5
 //   causal, up to six 64-row tiles, 192: B=16, 6 heads, S=128 14.9 / 12.8;  384: B=16, 6, S=200 20.0 / 17.2, S=256 21.2 / 17.8
 //     432: B=6, 12/6 heads, S=400 35.5 / 30.2;  576: B=6, S=400 27.8 / 23.7, B=12, S=256 24.3 / 27.7;  768: B=8, S=400 29.8 / 31.4
 //     three heads a kv head and more: B=2, 12/4, S=400 39.2 / 34.1, 16/4, S=200 31.7 / 28.4, 28/4, S=150 36.8 / 34.8, B=8, 28/4, S=100 29.6 / 27.2
 //   seven tiles and more, 480: B=4, S=600 33.2 / 25.8;  648: B=6, 12/6, S=700 51.3 / 43.4;  720: B=6, S=600 36.5 / 35.7
-//     768: B=8, S=512 34.7 / 35.5, B=4, S=1024 51.1 / 47.7;  864: B=6, S=700 39.4 / 40.9;  1120: B=5, 16, S=777 50.6 / 54.4
+//     768: B=4, S=1024 51.1 / 47.7;  864: B=6, S=700 39.4 / 40.9;  1120: B=5, 16, S=777 50.6 / 54.4
 //     grouped beyond 768: B=4, 32/8, S=700 77.5 / 80.2
 //   fifteen and more, 1024: B=4, 16, S=1024 65.2 / 57.5, B=2, 16, S=2048 90.5 / 88.7;  2048: B=4, 16, S=2048 154 / 157
 bool together(const BwdM& g) {
   if (g.keep_scale != 0.f || w32_dkdv(g)) return false;
   const int64_t all = (int64_t)g.B * g.Hq * g.n_qt + (int64_t)g.B * g.Hkv * g.n_kt * g.parts;
-  return all <= (!g.causal ? 768 : g.L < 7 * BQ ? 512 : g.Hq > g.Hkv || g.L <= 14 * BQ ? 768 : 1024);
+  if (!g.causal) return all <= (g.Hq >= 3 * g.Hkv ? 768 : g.L <= 5 * BQ ? 512 : g.Hq == g.Hkv ? 768 : 704);
+  return all <= (g.L < 7 * BQ ? 512 : g.Hq > g.Hkv || g.L <= 14 * BQ ? 768 : 1024);
+}
+// ... and which of them with dK/dV block by block, in three workgroups a compute unit: calls under the causal mask of more
+// than two and a half each, which then are one turn.  Two launches / one, a block ahead / one, block by block, us, 8 heads:
+//   576: S=512 32.5 / 28.3 / 29.4, S=640 36.1 / 29.3 / 31.9;  640: S=448 29.0 / 27.1 / 27.1, S=512 32.9 / 30.5 / 30.2, S=576 33.3 / 29.1 / 30.5
+//   704: S=512 32.7 / 33.0 / 30.6;  672, longer chains: S=768 - / 37.5 / 39.3, S=896 - / 39.0 / 44.2;  768: S=448 30.0 / 30.0 / 28.3, S=512 34.0 / 34.0 / 31.8
+//   grouped, 768: 16/8, S=512 41.7 / 37.3 / 43.6
+bool together_three_per_cu(const BwdM& g) {
+  const int64_t all = (int64_t)g.B * g.Hq * g.n_qt + (int64_t)g.B * g.Hkv * g.n_kt * g.parts;
+  return g.causal && g.Hq == g.Hkv && g.L <= 10 * BQ && all > 640 && all <= 768;
 }
 
 // Calls whose dK/dV runs block by block, three workgroups per compute unit: more key blocks than two per compute unit, but
@@ -804,7 +817,8 @@ int launch_together(const BwdM& g, hipStream_t s) {
   if (int rc = check_launch("bwd_d64_terms_kernel")) return rc;
   const Grid dq = dq_grid(g), dkdv = dkdv_grid(g);
   const int grid = (int)((dq.blocks + 7) / 8 + (dkdv.blocks + 7) / 8) * 8;
-  hipLaunchKernelGGL((bwd_d64_both_kernel<T>), dim3(grid), dim3(256), 0, s, g, (int)dq.blocks, (int)dkdv.blocks, dq.chunk, dkdv.chunk);
+  if (together_three_per_cu(g)) hipLaunchKernelGGL((bwd_d64_both_kernel<T, false>), dim3(grid), dim3(256), 0, s, g, (int)dq.blocks, (int)dkdv.blocks, dq.chunk, dkdv.chunk);
+  else hipLaunchKernelGGL((bwd_d64_both_kernel<T, true>), dim3(grid), dim3(256), 0, s, g, (int)dq.blocks, (int)dkdv.blocks, dq.chunk, dkdv.chunk);
   return check_launch("bwd_d64_both_kernel");
 }
 
