@@ -72,8 +72,8 @@ CASES = [
     (1, 8, 1, 700, 300, 64, True, None, 0.0),
     (8, 20, 20, 130, 520, 64, False, None, 0.1),  # 20 streams per XCD, chunks of 15
     (4, 10, 10, 600, 600, 64, True, None, 0.0),  # 5 streams per XCD; key blocks of 384 to 512 workgroups
-    # causal calls whose dK/dV (grouped heads, 384 to 1024 key blocks) or both kernels (513 to 768 query tiles of more
-    # than 14 x 64 rows) are those of bwd_dkdv_w32.hip / bwd_dq_w32.hip, and their neighbours that are not
+    # causal calls of grouped heads whose dK/dV is that of bwd_dkdv_w32.hip (384 to 1024 key blocks), and their neighbours that are
+    # not; one head per kv head, 513 to 768 query tiles of 15 and more of 64 rows
     (95, 8, 4, 65, 65, 64, True, None, 0.0),
     (96, 8, 4, 65, 65, 64, True, None, 0.0),
     (96, 8, 4, 65, 130, 40, True, [65 + i % 66 for i in range(96)], 0.0),
@@ -83,6 +83,7 @@ CASES = [
     (25, 3, 3, 896, 896, 64, True, None, 0.0),
     (24, 3, 3, 897, 897, 64, True, None, 0.0),
     (24, 3, 3, 897, 897, 64, True, [897 - 30 * i for i in range(24)], 0.0),
+    (19, 5, 5, 1020, 1020, 64, True, None, 0.0),
 ]
 
 

@@ -749,18 +749,14 @@ Grid dkdv_grid(const BwdM& g) {
 // keys sees every query row, the last one a few, all of them are on the chip at once, and at the end the long ones' chains
 // run with nobody beside them.  The kernels of 8 wavefronts per workgroup (bwd_dq_w32.hip, bwd_dkdv_w32.hip) have the shorter
 // chain.  Below 384 key blocks their items are split (bwd_dkdv_w32_plan), above 1024 the rest of the grid hides it.
-// Backward, us, both kernels here / dQ here and dK/dV there / both there (D=64):
-//   grouped heads, 384 blocks: B=3, 32/8 heads, S=2048 294 / 248 / 263;  B=6, 64/8, S=1024 307 / 261 / 291
-//     512: B=2, 32/8, S=4096 632 / 562 / 569;  B=8, 32/8, S=1024 184 / 172 / 194;  1024: B=8, 32/8, S=2048 595 / 600 / 639
-//   dQ's own grid (B * Hq query tiles), 576: B=6, 12 heads, S=1024 77 / - / 73;  720: B=5, 12, S=1500 93 / - / 113;  768: B=4,
-//     12, S=2048 135 / - / 144, B=6, 16, S=1024 85 / - / 91, B=2, 12, S=4096 239 / - / 241;  512: B=2, 8, S=4096 149 here, 153 before
+// Backward, us, both kernels here / dQ here and dK/dV there (D=64):
+//   grouped heads, 384 blocks: B=3, 32/8 heads, S=2048 294 / 248;  B=6, 64/8, S=1024 307 / 261
+//     512: B=2, 32/8, S=4096 632 / 562;  B=8, 32/8, S=1024 184 / 172;  1024: B=8, 32/8, S=2048 595 / 600
+// (dQ's kernel there, two wavefronts a SIMD, and its dK/dV lose to both here with one head per kv head: B=6, 12 heads, S=1024 63 / 73, B=5, S=1500
+// 90 / 107, B=4, S=2048 116 / 135, B=2, S=4096 203 / 245.)
 bool w32_dkdv(const BwdM& g) {
   const int64_t blocks = (int64_t)g.B * g.Hkv * g.n_kt;
   return g.causal && g.keep_scale == 0.f && g.Hq > g.Hkv && blocks >= 384 && blocks <= 1024;
-}
-bool w32_both(const BwdM& g) {
-  const int64_t tiles = (int64_t)g.B * g.Hq * g.n_qt;
-  return g.causal && g.keep_scale == 0.f && !g.kv_lens && g.d_real == D && (int64_t)g.B * g.Hkv * g.n_kt >= 384 && tiles > 512 && tiles <= 640 && g.L > 14 * BQ;
 }
 
 // Calls whose two kernels leave the chip half empty, each for as long as its longest chain of tiles: one launch of both,
@@ -845,7 +841,7 @@ int launch_t(const BwdM& g, uint32_t* bits, hipStream_t s) {
 
 bool bwd_d64_takes(const BwdM& g) {
   if (g.Hkv < 1) return false;  // (asked for the size of a workspace before anything is checked)
-  if (g.d_real > 64 || g.dv_real != g.d_real || g.bias_kind || g.gbias || g.window > 0 || g.sm.any || g.dq_split_tiles || w32_both(g)) return false;
+  if (g.d_real > 64 || g.dv_real != g.d_real || g.bias_kind || g.gbias || g.window > 0 || g.sm.any || g.dq_split_tiles) return false;
   // (32-bit byte offsets from the start of a batch, and of a key block's keep bits; the latter are the smaller ones
   // but for heads expanded from one)
   return bwd_dkdv_w32_fits(g, 64) && bwd_dq_w32_fits(g, 64) && (g.keep_scale == 0.f || block_words(g) * 4 < (1ll << 32));

@@ -1,5 +1,5 @@
 // Flash-attention backward, dK and dV, for gfx950, head dim 64 or 128, bf16/f16 (at 64 the calls with a bias, a
-// window, a functor or split dQ keys, and causal ones of some grid sizes: bwd_d64.hip, which says which, has the others
+// window, a functor or split dQ keys, and causal ones of some numbers of grouped heads: bwd_d64.hip, which says which, has the others
 // within 32-bit offsets).
 //
 // One workgroup = 8 wavefronts = 128 keys of one (batch, kv head); it loops over the query

@@ -1,6 +1,5 @@
 // Flash-attention backward, dQ, for gfx950, head dim 64 or 128, bf16/f16 (at 64 the calls with a bias, a window, a
-// functor or split keys, those whose Q or dO of one batch is beyond 32-bit offsets, and causal ones of some grid sizes:
-// bwd_d64.hip, which says which, has the others).
+// functor or split keys, and those whose Q or dO of one batch is beyond 32-bit offsets: bwd_d64.hip has the others).
 //
 // One workgroup = 8 wavefronts of 32 query rows each (256 rows of one (batch, query head)), one
 // workgroup per compute unit, two wavefronts per SIMD with 256 registers each; it walks the keys
