@@ -72,8 +72,7 @@ CASES = [
     (1, 8, 1, 700, 300, 64, True, None, 0.0),
     (8, 20, 20, 130, 520, 64, False, None, 0.1),  # 20 streams per XCD, chunks of 15
     (4, 10, 10, 600, 600, 64, True, None, 0.0),  # 5 streams per XCD; key blocks of 384 to 512 workgroups
-    # causal calls of grouped heads whose dK/dV is that of bwd_dkdv_w32.hip (384 to 1024 key blocks), and their neighbours that are
-    # not; one head per kv head, 513 to 768 query tiles of 15 and more of 64 rows
+    # causal calls of two heads a kv head and one of 384 and more key blocks; one of 513 to 768 query tiles, 15 and more of 64 rows
     (95, 8, 4, 65, 65, 64, True, None, 0.0),
     (96, 8, 4, 65, 65, 64, True, None, 0.0),
     (96, 8, 4, 65, 130, 40, True, [65 + i % 66 for i in range(96)], 0.0),
@@ -229,3 +228,15 @@ def test_a_third_workgroup_on_a_compute_unit(amd, gpu_device, B, Hq, Hkv, L, S, 
     """More key blocks than two per compute unit and at most three, of few items: dK/dV block by block, on both sides of the
     lines of that."""
     _check(amd, gpu_device, B, Hq, Hkv, L, S, D, causal, dtype, lens, 0.0)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("B,Hq,Hkv,L,S,D,lens", [
+    (63, 6, 2, 321, 321, 64, None), (64, 6, 2, 321, 321, 64, None), (64, 6, 2, 320, 320, 64, None),  # 378 key blocks, 384, of five query tiles
+    (43, 6, 2, 321, 700, 40, [700 - 15 * i for i in range(43)]),                                      # 516
+    (64, 12, 4, 330, 200, 64, [200 - 3 * i for i in range(64)]),                                      # 512
+    (65, 12, 4, 330, 200, 64, None), (64, 4, 2, 321, 321, 64, None),                                  # 520; two heads a kv head
+])
+def test_on_both_sides_of_the_lines_of_grouped_heads(amd, gpu_device, B, Hq, Hkv, L, S, D, lens, dtype):
+    """Causal calls whose dK/dV is that of bwd_dkdv_w32.hip: three heads a kv head, 384 to 512 key blocks, six query tiles."""
+    _check(amd, gpu_device, B, Hq, Hkv, L, S, D, True, dtype, lens, 0.0)

@@ -745,18 +745,20 @@ Grid dkdv_grid(const BwdM& g) {
   return {chunk, (chunk ? (streams + 7) / 8 * 8 : streams) * g.n_kt * g.parts};
 }
 
-// Causal calls whose workgroups (tiles times streams) are too few to hide the longest of them: a key block of the first
-// keys sees every query row, the last one a few, all of them are on the chip at once, and at the end the long ones' chains
-// run with nobody beside them.  The kernels of 8 wavefronts per workgroup (bwd_dq_w32.hip, bwd_dkdv_w32.hip) have the shorter
-// chain.  Below 384 key blocks their items are split (bwd_dkdv_w32_plan), above 1024 the rest of the grid hides it.
-// Backward, us, both kernels here / dQ here and dK/dV there (D=64):
-//   grouped heads, 384 blocks: B=3, 32/8 heads, S=2048 294 / 248;  B=6, 64/8, S=1024 307 / 261
-//     512: B=2, 32/8, S=4096 632 / 562;  B=8, 32/8, S=1024 184 / 172;  1024: B=8, 32/8, S=2048 595 / 600
+// Causal calls whose dK/dV workgroups are too few to hide the longest of them, which is long: a key block of the first keys sees
+// every query row of several heads, the last one a few, all of them are on the chip at once, and at the end the long ones'
+// chains run with nobody beside them.  The kernel of 8 wavefronts per workgroup (bwd_dkdv_w32.hip) has the shorter chain.  Below 384
+// key blocks the items are split (bwd_dkdv_w32_plan), above two workgroups of this file's per compute unit the rest of the grid
+// hides it.  Backward, us, dK/dV here / there (D=64):
+//   four heads a kv head, 384 blocks: B=12, 32/8, S=512 99 / 91, B=6, 64/8, S=1024 307 / 264, B=3, 32/8, S=2048 294 / 254;  512: B=16, S=512 115 / 113, B=8, S=1024 181 / 168,
+//     B=2, S=4096 630 / 563;  640: B=10, S=1024 204 / 218;  768: B=6, S=2048 422 / 459;  1024: B=8, S=2048 544 / 589;  short, 384: B=24, S=256 74 / 81
+//   three: 384: B=6, 24/8, S=1024 111 / 111;  512: B=8, S=1024 139 / 131, B=4, S=2048 254 / 230;  seven: 512: B=16, 28/4, S=1024 308 / 287;  640: 345 / 371
+//   two: 384: B=3, 16/8, S=2048 135 / 135;  512: B=4, S=2048 157 / 162, B=16, S=512 63 / 70
 // (dQ's kernel there, two wavefronts a SIMD, and its dK/dV lose to both here with one head per kv head: B=6, 12 heads, S=1024 63 / 73, B=5, S=1500
 // 90 / 107, B=4, S=2048 116 / 135, B=2, S=4096 203 / 245.)
 bool w32_dkdv(const BwdM& g) {
   const int64_t blocks = (int64_t)g.B * g.Hkv * g.n_kt;
-  return g.causal && g.keep_scale == 0.f && g.Hq > g.Hkv && blocks >= 384 && blocks <= 1024;
+  return g.causal && g.keep_scale == 0.f && g.Hq >= 3 * g.Hkv && g.L > 5 * BQ && blocks >= 384 && blocks <= 512;
 }
 
 // Calls whose two kernels leave the chip half empty, each for as long as its longest chain of tiles: one launch of both,
