@@ -45,12 +45,19 @@ def test_every_stream_is_computed(gpu_device, B, Hq, Hkv, S, D, causal):
     (57, 8, 8, 1100, 1100, 128, True, None),    # 57 streams an XCD in chunks of 7, in both kernels
     (9, 16, 8, 3000, 300, 104, False, None),    # 9 one by one in dK/dV, which walks Q and dO of two heads
     (13, 48, 48, 1000, 1000, 128, False, 1000), # 78 in chunks of 8, key counts
-    (11, 16, 16, 1024, 1024, 64, True, None),   # 22 in chunks of 16 at head dim 64
+    (11, 16, 16, 1024, 1024, 64, True, None),   # 22 at a time at head dim 64
     (25, 8, 8, 900, 900, 64, False, None),      # 25 in chunks of 4
     (31, 12, 12, 512, 512, 64, False, None),    # 372 streams: the last four XCDs serve one less
     (15, 12, 12, 500, 500, 64, True, None),     # 180
     (5, 12, 4, 300, 300, 64, True, None),       # 20: not pinned
     (29, 12, 4, 300, 300, 64, True, None),      # 116, three heads a kv head
+    (70, 8, 8, 200, 200, 64, True, None),       # causal, up to three key blocks: 70 (3.6 MB) in five chunks of 14, 64 at a time
+    (64, 8, 8, 200, 200, 64, True, None),
+    (35, 8, 8, 500, 500, 64, True, None),       # four: 35 (4.5 MB) in five of 7, 32 (4.1) at a time
+    (32, 8, 8, 500, 500, 64, True, None),
+    (19, 12, 12, 1100, 900, 64, True, None),    # 228: the last four XCDs serve one less than 29, at a time
+    (12, 16, 16, 700, 4100, 64, True, None),    # 24 of 4100 keys, more than 24 MB: in two chunks of 12 for dQ
+    (12, 16, 16, 4100, 700, 48, True, None),    # ... of 4100 rows for dK/dV
 ])
 def test_every_gradient_is_computed(gpu_device, B, Hq, Hkv, L, S, D, causal, lens):
     """The same in the backward.  P, dS, O and the gradients are rounded once each: 8e-3, as in test_bwd_d64_gpu.py."""

@@ -712,22 +712,36 @@ __global__ __launch_bounds__(256) void bwd_d64_terms_kernel(BwdM p, int blocks32
   if (half == 0) p.delta[idx] = dl, p.lse2[idx] = l != -INFINITY ? l * kLog2eF : INFINITY;
 }
 
-// Streams of an XCD that it takes at a time, their two tensors having `rows` rows: all of them where its 4 MB of L2 hold them,
-// otherwise as many as fill it under a causal mask, where the last chunk's long tiles should not start late, and a quarter
-// of it without one (a keep-mask and the rows that are written pass through the same L2).  Against half of it throughout,
-// backward in us: causal B=16, 12 heads, S=512 67.0 -> 63.3, B=8, 16, S=2048 280 -> 272, B=4, 32, S=4096 1005 -> 979;  not causal
-// B=64, 12, S=197 76.0 -> 74.5, B=60, 16, S=256 103 -> 101, with dropout B=32, 12, S=512 142 -> 140, B=64, S=250 95.2 -> 93.4
-// (units: workgroups per stream.  A number of streams that does not divide over the XCDs: see stream_chunk, fwd_mfma_w32.hip;
-// backward, anywhere / pinned, us: B=31, 12 heads, S=512 137 / 131, B=21, 6, S=785 120 / 115, B=15, 12, S=512 causal 55.5 / 53.7)
+// Streams of an XCD that it takes at a time, their two tensors having `rows` rows and `units` workgroups each, in equal chunks.
+// Without the causal mask all of them where its 4 MB of L2 hold them, otherwise as many as fill a quarter of it (a keep-mask and
+// the rows that are written pass through the same L2).  All / in chunks, backward in us, 8 heads: 3.1 MB: B=24, S=512 70 / 69;  4.0: B=20, S=785 127 / 131;
+// 4.2: B=64, S=256 61 / 58, with dropout 72 / 67, B=32, S=512 87 / 84;  4.7: B=48, S=384 83 / 81;  6.3: B=48, S=512 122 / 118
+// Under the mask the first workgroups of a chunk are the long ones, and the last chunk's should not start late:
+//   up to four workgroups a stream, where they differ little, from 3.25 MB (four workgroups: 4) on in chunks of 32 to 48 workgroups.  All / so: B=64, S=256 55 / 54, B=48, S=320 56 / 52, S=384
+//     69 / 62, S=448 81 / 80, S=512 95 / 89;  B=64, S=512 114 / 115, with dropout B=40, S=512 96 / 91;  less: B=32, S=256 with dropout 34 / 37, S=448 56 / 61, B=64, S=197 46 / 47.5, B=24, S=512 59 / 61
+//   otherwise none up to 24 MB, six times the L2: B=11, 12 heads, S=1948 235, in two chunks of eight and a last one of a single stream 284; B=8, 8 heads, S=2500 199, two
+//     of 4 MB 253, three of 2 MB 228; B=24, S=1024 120, 134, 127; B=8, 32/8, S=4096 (dK/dV: 33 MB) 1834, 1944, -.  Beyond it as many as the L2 holds, but 128 workgroups at
+//     least: B=64, S=2048 1133 / 1061, B=96, S=1500 1053 / 991, B=32, 32/8, S=2048 2120 / 1990
+// (A number of streams that does not divide over the XCDs: see stream_chunk, fwd_mfma_w32.hip; backward, anywhere / pinned, us:
+// B=31, 12 heads, S=512 137 / 131, B=21, 6, S=785 120 / 115, B=15, 12, S=512 causal 55.5 / 53.7)
 int stream_chunk(const BwdM& g, int64_t rows, int64_t units) {
-  const int64_t streams = (int64_t)g.B * g.Hkv, bytes = rows * D * 4, all = (streams + 7) / 8;
+  const int64_t streams = (int64_t)g.B * g.Hkv, bytes = std::max<int64_t>(1, rows * D * 4), all = (streams + 7) / 8;
   if (streams % 8 != 0) {
     if (units == 1 || (all * 8 - streams) * 15 > streams) return 0;
     for (int slots = 32; slots <= 96; slots += 32)
       if ((all * units + slots - 1) / slots > (streams * units + 8 * slots - 1) / (8 * slots)) return 0;
   }
-  if (all * bytes <= (9 << 19)) return (int)all;
-  return (int)std::max<int64_t>(1, std::min<int64_t>(all, (g.causal ? 4 << 20 : 1 << 20) / bytes));
+  int64_t chunk = all;
+  if (!g.causal)
+    chunk = all * bytes < (4 << 20) ? all : (1 << 20) / bytes;
+  else if (units <= 4)
+    chunk = all * bytes < (units == 4 ? 4 << 20 : 13 << 18) ? all : units == 4 ? 8 : 16;
+  else if (all * bytes > (24 << 20))
+    chunk = std::max<int64_t>((4 << 20) / bytes, 128 / units);
+  if (chunk < 1) chunk = 1;
+  if (chunk >= all) return (int)std::max<int64_t>(1, all);
+  const int64_t n = (all + chunk - 1) / chunk;
+  return (int)((all + n - 1) / n);
 }
 // the two grids: a chunk (0: streams are not pinned) and the workgroups
 struct Grid {
