@@ -15,8 +15,15 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("B,Hq,Hkv,S,D,causal", [
     (24, 12, 12, 577, 64, False),   # 36 streams an XCD in chunks of 7
     (11, 32, 16, 333, 104, False),  # 22 in chunks of 7, two heads a kv head
+    (12, 8, 8, 900, 128, False),    # 12 (5.5 MB) at a time, 12 of 1030 keys (6.3 MB) in chunks of four
+    (12, 8, 8, 1030, 128, False),
+    (11, 16, 8, 1100, 72, False),   # 11 in chunks of four, the last one of three
+    (10, 32, 8, 1100, 128, False),  # four heads a kv head: one by one
     (43, 24, 24, 1024, 64, True),   # 129 in chunks of 16: eight and a last one of a single stream
     (19, 16, 8, 2048, 128, True),   # 19 in chunks of 4 are fewer than eight chunks: one after the other
+    (9, 8, 8, 4096, 256, True),     # 9 of 4 MB each: at a time
+    (17, 8, 8, 2830, 128, True),    # 17, two of which fill the L2: in five chunks of four, the last one of a single stream
+    (35, 8, 8, 1500, 128, True),    # 35, chunks of five
     (35, 16, 8, 2048, 128, True),   # 35: nine
     (31, 12, 12, 512, 64, False),   # 372 streams: the last four XCDs serve one less, in chunks of 8
     (21, 28, 4, 512, 128, True),    # 84, seven heads a kv head, no chunks

@@ -1251,13 +1251,21 @@ int launch_fwd_split_merge(const FwdM& g, int dtype, hipStream_t s) {
 // How many of its streams (a (batch, kv head)'s keys and values) an XCD takes at a time, all their query tiles before the
 // next ones.  Query tile by query tile over all of them, as is best while they fit its 4 MB of L2, every pass over the
 // tiles brings K and V from memory again (B=32, 12 heads, S=512: 234 MB fetched for 115).  In chunks of 1 MB without the
-// causal mask (a keep-mask and Q pass through the same L2); with it in chunks of the whole L2 and only where there are eight or
-// more: the first tiles of a chunk are the long ones, and the last chunk's start late.  All streams / in chunks, us:
+// causal mask (a keep-mask and Q pass through the same L2), at head dims of 65 to 128 with up to two heads a kv head - a workgroup
+// has a compute unit to itself there, and one or two streams' are a fraction of the 32 of them - of four streams at least, and from three query tiles on
+// only beyond 6 MB.  All streams / in chunks, us:
 //   not causal, 4.6 MB: B=64, 12 heads, S=197, D=64 25.9 / 24.4;  5.7: B=40, 12, S=384 35.0 / 31.7;  6: B=32, 12, S=512 42.6 / 38.9, with dropout and
 //     key counts 51.0 / 46.3;  8: B=8, 16, S=1024, D=128 74.2 / 72.2;  16: B=4, 32, S=2048, D=128 240.6 / 237.8;  below: 4.4: B=30, 8, S=600 35.7 / 36.4
+//   D=128, 8 heads, all / 1 MB / four streams: 5.3: B=8, S=1284 60 / 66 / 65, B=12, S=900 46 / 52 / 47, B=12, S=785 40 / 43 / 43;  8.4: B=16, S=1030 78 / 84 / 77
+//     7.9: B=12, S=1284 89 / 98 / 88;  12.6: B=12, S=2052 194 / 202 / 189;  15.8: B=24, S=1284 172 / 174 / 163;  two query tiles: B=24, S=512 36 / 34 / 34
+//     16/8 heads: B=12, S=1284 165 / 173 / 165;  32/8: B=16, S=1030 302 / 288 / 294
+// With the mask in chunks of the whole L2, four streams at least, and only where there are eight or more, of two at least: the first tiles of a
+// chunk are the long ones, and the last chunk's start late (equal chunks: a small last one is the latest).
 //   causal, 8 chunks: B=4, 64 heads, S=4096, D=64 638 / 580, B=16, 32/8, S=4096, D=128 1989 / 1912, B=8, 32, S=2048 304 / 279, B=16, S=1024 220 / 190
 //     fewer: 4: B=8, 16, S=2048, D=64 82 / 85, B=4, 32, S=999, D=128 with key counts 48 / 50;  2: B=4, 16, S=2048, D=128 72 / 71
-static int stream_chunk(const FwdM& g) {
+//     of one stream, of two, of four: B=8, 8 heads, S=6000, D=128 486 / 517, 493, 488;  B=12, S=2829, D=256 467 / 467, 445, 454;  B=16, S=6000, D=64 575 / -, 592, 573;
+//       B=16, S=2000, D=256 331 / -, 328, 306;  B=16, S=2829, D=128 272 / -, 275, 255
+static int stream_chunk(const FwdM& g, int head_dim) {
   const int64_t streams = (int64_t)g.B * g.Hkv, per_xcd = (streams + 7) / 8;
   if (streams % 8 != 0) {
     // Some XCDs serve a stream less than others.  Unless they idle for more than a fifteenth, or the others need a turn of
@@ -1271,15 +1279,19 @@ static int stream_chunk(const FwdM& g) {
       if ((per_xcd * units + slots - 1) / slots > (streams * units + 8 * slots - 1) / (8 * slots)) return 0;
   }
   const int64_t bytes = std::max<int64_t>(1, (int64_t)g.S * (g.d_real + g.dv_real) * 2);
-  if (g.bias_kind || g.window > 0 || per_xcd * bytes <= (9 << 19)) return (int)per_xcd;
-  const int64_t chunk = std::min(per_xcd, std::max<int64_t>(1, (g.causal ? 4 << 20 : 1 << 20) / bytes));
-  return (int)(g.causal && per_xcd < 8 * chunk ? per_xcd : chunk);
+  const bool by_four = !g.causal && head_dim == 128 && g.Hq <= 2 * g.Hkv;
+  if (g.bias_kind || g.window > 0 || per_xcd * bytes <= (by_four && g.n_qt >= 3 ? 6 << 20 : 9 << 19)) return (int)per_xcd;
+  if (!g.causal) return (int)std::min(per_xcd, std::max<int64_t>(by_four ? 4 : 1, (1 << 20) / bytes));
+  const int64_t chunk = std::max<int64_t>(2, (4 << 20) / bytes);
+  if (per_xcd < 8 * chunk) return (int)per_xcd;
+  const int64_t n = (per_xcd + std::max<int64_t>(4, chunk) - 1) / std::max<int64_t>(4, chunk);
+  return (int)((per_xcd + n - 1) / n);
 }
 
 int launch_fwd_mfma_w32(const FwdM& g0, int dtype, int head_dim, int waves, hipStream_t s) {
   FwdM g = g0;
   fwd_w32_plan(g, head_dim, waves);
-  g.xcd_map = stream_chunk(g);
+  g.xcd_map = stream_chunk(g, head_dim);
   if (g.split_tiles) {  // (the caller's workspace: too small or absent, and the call runs unsplit)
     const size_t rows = (size_t)g.B * g.Hq * g.n_split * g.L;
     if (g.part_o && g.n_split <= 512 && g.part_bytes >= rows * (g.dv_real + 1) * sizeof(float)) g.part_lse = g.part_o + rows * g.dv_real;
