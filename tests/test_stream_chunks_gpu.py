@@ -51,6 +51,8 @@ def test_every_stream_is_computed(gpu_device, B, Hq, Hkv, S, D, causal):
 @pytest.mark.parametrize("B,Hq,Hkv,L,S,D,causal,lens", [
     (57, 8, 8, 1100, 1100, 128, True, None),    # 57 streams an XCD in chunks of 7, in both kernels
     (9, 16, 8, 3000, 300, 104, False, None),    # 9 one by one in dK/dV, which walks Q and dO of two heads
+    (18, 4, 4, 5000, 400, 128, True, None),     # 9, one of which fills the L2: in three chunks of three in dK/dV
+    (20, 8, 4, 400, 5000, 128, True, None),     # 10: four, four and two in dQ
     (13, 48, 48, 1000, 1000, 128, False, 1000), # 78 in chunks of 8, key counts
     (11, 16, 16, 1024, 1024, 64, True, None),   # 22 at a time at head dim 64
     (25, 8, 8, 900, 900, 64, False, None),      # 25 in chunks of 4

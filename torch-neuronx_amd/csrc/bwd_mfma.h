@@ -93,13 +93,20 @@ struct BwdM {
 // which every pass over the tiles of all of them brings the tensors from memory again (see stream_chunk, fwd_mfma_w32.hip).
 // Where there are eight chunks or more; with fewer the long tiles that start late cost what the L2 saves.  The whole backward
 // in us, all streams / chunks (D=128, causal): B=8, 32 heads, S=4096 4504 / 4074, B=8, S=2048 1249 / 1189, B=16, S=1024 811 / 773;  fewer:
-// B=4, S=4096 2054 / 2073, B=4, S=2048 not causal 983 / 1001.  Chunks of a quarter of the L2 lose up to 12 %.  Grouped heads share Q and dO
-// tiles in another order in dK/dV: B=8, 32/8 heads, S=1024 307 us, in chunks 366 (bwd_dkdv_w32.hip takes none there).
+// B=4, S=4096 2054 / 2073;  chunks of a quarter of the L2 lose up to 12 %.  Not causal, 8 heads: B=48, S=1400 1650 / 1465, B=24, S=3000 3350 / 2950,
+// B=64, S=1024 1220 / 1150;  fewer: B=4, 32 heads, S=2048 983 / 1001.  Under the mask four streams at least, in equal chunks: the
+// dQ workgroups of one stream of 5000 keys are 20 for 32 compute units (all / one / four): 8 heads, B=8, S=5000 1400 / 1510 / 1386, B=9 1595 / 1674 / 1580 (three),
+// B=20 3900 / 3720 / 3510.  Grouped heads share Q and dO tiles in another order in dK/dV: B=8, 32/8 heads, S=1024 307 us, in
+// chunks 366 (bwd_dkdv_w32.hip takes none there).
+// (The kernels for head dims up to 64, whose workgroups share a compute unit, have lines of their own: see bwd_d64.hip.)
 inline int bwd_stream_chunk(const BwdM& g, int64_t rows) {
   const int64_t streams = (int64_t)g.B * g.Hkv, bytes = std::max<int64_t>(1, rows * g.d_real * 4);
   if (streams % 8 != 0 || g.bias_kind || g.gbias || g.window > 0 || g.sm.any) return 0;
-  const int64_t chunk = std::max<int64_t>(1, (4 << 20) / bytes);
-  return streams / 8 >= 8 * chunk ? (int)chunk : 0;
+  const int64_t all = streams / 8, fill = std::max<int64_t>(1, (4 << 20) / bytes);
+  if (all < 8 * fill) return 0;
+  if (!g.causal) return (int)fill;
+  const int64_t n = (all + std::max<int64_t>(4, fill) - 1) / std::max<int64_t>(4, fill);
+  return (int)((all + n - 1) / n);
 }
 // parts the dK/dV kernel of bwd_dkdv_w32.hip / of bwd_wide.hip would use for this call
 int bwd_dkdv_w32_parts(const BwdM& g);
