@@ -84,8 +84,9 @@ def test_sixteen_rows_against_the_oracle(amd, gpu_device, B, Hq, Hkv, L, S, E, D
     (128, 4, 4, 16, 16, 128, 128), (171, 3, 3, 16, 16, 128, 128),    # 512 up to 16
     (64, 4, 4, 32, 32, 64, 64), (257, 1, 1, 20, 32, 64, 64),         # head dims up to 64: 512 of 17 to 32 rows
     (11, 3, 3, 400, 400, 64, 64), (17, 2, 2, 400, 400, 48, 48),      # 832 up to 400 rows
-    (25, 1, 1, 160, 97, 64, 64), (13, 2, 2, 160, 97, 128, 128),      # more rows than keys: 256 as without the mask,
-    (32, 1, 1, 400, 47, 64, 64), (128, 2, 2, 64, 32, 64, 64),        # but for up to 96 keys at head dims up to 64
+    (22, 1, 1, 210, 105, 128, 128), (23, 1, 1, 210, 105, 128, 128),  # half as many keys as rows: 320 at head dims above 64,
+    (36, 1, 1, 210, 150, 128, 128), (18, 1, 1, 311, 264, 128, 64),   # not with more keys
+    (32, 1, 1, 400, 47, 64, 64), (128, 2, 2, 64, 32, 64, 64),        # and not at head dims up to 64
     (24, 6, 2, 38, 38, 128, 128), (32, 4, 4, 38, 38, 128, 128),      # 288 of 32 rows, and 256
 ])
 def test_on_both_sides_of_the_lines_of_sixteen_rows(amd, gpu_device, B, Hq, Hkv, L, S, E, Dv):

@@ -940,11 +940,12 @@ bool few_query_tiles(const FwdM& g) {
 
 // ... and which in fwd_f32_rows16_kernel.  Its workgroups cost twice the trips to K and V and have half the chain.  Up to one
 // per compute unit the chain is all that counts.  Under a causal mask, where most are shorter than the longest, more of them
-// pay, the fewer the wider the head and the shorter the chain of min(L, S) keys - unless there are clearly fewer keys than rows,
-// all but the first of which then see every key.  By their number, 16-row / 32-row time (the 128-row kernel's for up to 32
+// pay, the fewer the wider the head and the shorter the chain of min(L, S) keys, and at head dims above 64 fewer again with half as many keys
+// as rows, most of which then see every key.  By their number, 16-row / 32-row time (the 128-row kernel's for up to 32
 // keys, a single tile, which has nothing to share out):
 //   not causal, 256: S=32 0.77, S=128 0.73, S=512 0.67, D=128 0.73 0.79 0.74;  288: S=64 0.93, S=128 1.15, S=512 1.14, D=128 1.10 1.37 1.25
-//   causal, more rows than keys: 400, L=800, S=200 1.08, D=128 1.29;  300, L=1600, S=128 1.12, D=128 1.36;  384, L=512, S=64 0.93, D=128 1.13;  768, L=375, S=47 0.83
+//   causal, more rows than keys, D=128: 280, L=200, S=100 0.96;  300, L=1600, S=128 1.36;  350, L=400, S=200 1.03;  400, L=800, S=200 1.29;  not twice as many: 360, L=311, S=264 0.75
+//     D=64: 400, L=800, S=200 1.08;  450, L=300, S=100 1.17, L=260, S=130 0.84, L=528, S=264 0.89;  768, L=375, S=47 0.83
 //   causal, D=64, 512: L=32 1.00, 832: 1.19;  832: L=64 0.84, L=128 0.89, L=256 0.95, L=400 0.93, 1024: L=64 1.22;  L=512, 512: 0.92, 640: 1.03;  L=1000, 504: 0.89, 756: 1.06
 //   causal, D=128, 256: L=32 0.71, 288: 1.18;  320: L=64 0.96, L=100 0.96, L=128 0.93, 384: 0.99 1.10 1.09;  512: L=130 1.00, L=160 0.99, L=200 0.98, L=256 1.00,
 //     L=512 0.86, 576, from L=160: 1.06 1.04 1.16 1.00;  up to 16 rows, any number: 0.65 to 0.75
@@ -954,10 +955,10 @@ bool sixteen_rows(const FwdM& g) {
   const int64_t heads = (int64_t)g.B * g.Hq, blocks = heads * ((g.L + 15) / 16);
   if (!g.causal) return blocks <= 256;
   if (blocks <= 512 && heads * ((g.L + 31) / 32) > 256) return true;
-  if (g.L > g.S && (g.d_real > 64 || g.S > 96)) return blocks <= 256;
   const int keys = std::min(g.L, g.S);
+  if (g.d_real > 64 && g.L / 2 >= g.S) return blocks <= 320;
   if (g.d_real <= 64) return blocks <= (g.L > 400 || (keys > 16 && keys <= 32) ? 512 : 832);
-  return blocks <= (g.L <= 16 || g.L > 128 ? 512 : g.L <= 32 ? 256 : 320);
+  return blocks <= (keys <= 16 || keys > 128 ? 512 : keys <= 32 ? 256 : 320);
 }
 
 void fwd_f32_fill(FwdM& g, const mi355_sdpa_fwd_params& p, int& mode) {
