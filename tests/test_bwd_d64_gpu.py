@@ -70,7 +70,7 @@ CASES = [
     (3, 2, 2, 130, 261, 48, False, [261, 33, 0], 0.25),
     (2, 8, 1, 500, 140, 64, False, None, 0.1),   # the items of a key block go to several workgroups
     (1, 8, 1, 700, 300, 64, True, None, 0.0),
-    (8, 20, 20, 130, 520, 64, False, None, 0.1),  # 20 streams per XCD, chunks of 15
+    (8, 20, 20, 130, 520, 64, False, None, 0.1),  # 20 streams per XCD
     (4, 10, 10, 600, 600, 64, True, None, 0.0),  # 5 streams per XCD; key blocks of 384 to 512 workgroups
     # causal calls of two heads a kv head and one of 384 and more key blocks; one of 513 to 768 query tiles, 15 and more of 64 rows
     (95, 8, 4, 65, 65, 64, True, None, 0.0),

@@ -1,5 +1,5 @@
-"""Forward calls whose streams (a (batch, kv head)'s keys and values) an XCD takes in chunks: every (batch, head, row) is
-computed, once, also where the last chunk is a smaller one or some XCDs serve a stream less than others.
+"""Calls whose streams (a (batch, kv head)'s keys and values) an XCD takes in chunks, forward, backward and with dropout: every
+(batch, head, row) is computed, once, also where the last chunk is a smaller one or some XCDs serve a stream less than others.
 
 Bound, against the same attention in float64 on the kernel's inputs: P and the output are each rounded once to bf16,
 2^-9 relative, which adds up to at most twice that in the 2-norm: 4e-3; the log-sum-exp is a float32 sum, 1e-5."""
@@ -90,6 +90,42 @@ def test_every_gradient_is_computed(gpu_device, B, Hq, Hkv, L, S, D, causal, len
         P = torch.softmax(s, -1)
         dS = P * (DO @ V.transpose(-1, -2).contiguous() - (DO * (P @ V)).sum(-1, keepdim=True)) / math.sqrt(D)
         want = (dS @ K, (dS.transpose(-1, -2).contiguous() @ Q).view(Hkv, rep, n, D).sum(1), (P.transpose(-1, -2).contiguous() @ DO).view(Hkv, rep, n, D).sum(1))
+        for name, a, r in zip(("dq", "dk", "dv"), grads, want):
+            got = a[b] if name == "dq" else a[b, :, :n]
+            far = (got.double() - r).norm(dim=(-2, -1)) / r.norm(dim=(-2, -1))
+            assert float(far.max()) <= 8e-3, (name, b, far)
+
+
+@pytest.mark.parametrize("lens", [False, True])
+@pytest.mark.parametrize("B,H,L,S,causal", [
+    (26, 8, 900, 700, False),   # 26 streams an XCD, in chunks of 5 and a last one of a single stream (dQ, by the keys) and of 4 and 2 (dK/dV, by the rows)
+    (31, 12, 512, 512, False),  # 372: the last four XCDs serve one less than 47, in chunks of 8
+    (13, 12, 300, 400, False),  # 156: 20 at a time, the last four 19
+    (45, 8, 500, 470, True),    # causal, four key blocks: 45 in chunks of 8 and 5
+    (23, 12, 300, 300, True),   # three: 276 of which the last four XCDs serve one less than 35
+])
+def test_keep_bits_reach_every_stream(gpu_device, B, H, L, S, causal, lens):
+    """With dropout: the dQ kernel leaves the keep bits that the dK/dV kernel reads, each in the order of its own chunks."""
+    import torch_neuronx_amd as amd
+
+    g = torch.Generator(device=gpu_device).manual_seed(S)
+    D, p = 64, 0.25
+    q, k, v, do = (torch.randn(B, H, n, D, generator=g, device=gpu_device).to(torch.bfloat16) for n in (L, S, S, L))
+    keep = amd.ops.padded_keep_mask(B, H, L, S, gpu_device).bernoulli_(1 - p, generator=g)
+    kw = dict(is_causal=causal, dropout_p=p, dropout_keep=keep)
+    if lens:
+        kw["kv_lens"] = torch.tensor([S - 9 * i for i in range(B)], dtype=torch.int32, device=gpu_device)
+    out, lse = amd.sdpa_forward(q, k, v, **kw)
+    grads = amd.sdpa_backward(do, q, k, v, out, lse, **kw)[:3]
+    for b in range(B):
+        n = S - 9 * b if lens else S
+        Q, DO, K, V, kp = q[b].double(), do[b].double(), k[b, :, :n].double(), v[b, :, :n].double(), keep[b, :, :, :n].double() / (1 - p)
+        s = Q @ K.transpose(-1, -2).contiguous() / math.sqrt(D)
+        if causal:
+            s.masked_fill_(~torch.ones(L, n, dtype=torch.bool, device=gpu_device).tril(), -math.inf)
+        P = torch.softmax(s, -1)
+        dS = P * ((DO @ V.transpose(-1, -2).contiguous()) * kp - (DO * ((P * kp) @ V)).sum(-1, keepdim=True)) / math.sqrt(D)
+        want = (dS @ K, dS.transpose(-1, -2).contiguous() @ Q, (P * kp).transpose(-1, -2).contiguous() @ DO)
         for name, a, r in zip(("dq", "dk", "dv"), grads, want):
             got = a[b] if name == "dq" else a[b, :, :n]
             far = (got.double() - r).norm(dim=(-2, -1)) / r.norm(dim=(-2, -1))
