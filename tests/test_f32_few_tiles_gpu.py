@@ -1,6 +1,7 @@
-"""Float32 forward with few query tiles: 32-row workgroups whose four wavefronts share out the key tiles.
-Sizes around a tile, around four tiles (one per wavefront) and around the number of workgroups at which the
-128-row kernel takes over, ragged key counts (none at all included), narrow V, grouped heads, L != S.
+"""Float32 forward with few query tiles: 32-row workgroups whose four wavefronts share out the key tiles, and with fewer
+still 16-row workgroups whose eight wavefronts share out blocks of 16 keys.  Sizes around a tile, around a round of all
+wavefronts and on both sides of the lines between the two and the 128-row kernel, and for each of the two ragged key
+counts (none at all included), head dims below the width a kernel is built for, narrow V, grouped heads, L != S.
 
 Bound: the tolerance of the float32 gate, 1e-5 on values of order 1 (float32 sums of at most 128 products and
 1000 keys: about 3e-7 relative measured, and the rows are compared absolutely)."""
@@ -91,3 +92,33 @@ def test_sixteen_rows_against_the_oracle(amd, gpu_device, B, Hq, Hkv, L, S, E, D
 ])
 def test_on_both_sides_of_the_lines_of_sixteen_rows(amd, gpu_device, B, Hq, Hkv, L, S, E, Dv):
     test_against_the_oracle(amd, gpu_device, B, Hq, Hkv, L, S, E, Dv, True)
+
+
+@pytest.mark.parametrize("B,Hq,Hkv,L,S,E,Dv,causal", [
+    (15, 4, 2, 97, 161, 64, 64, False),     # 420 of 16 rows, 240 of 32, 60 of 128
+    (17, 3, 1, 150, 129, 40, 8, False),
+    (20, 4, 4, 100, 40, 72, 24, False),
+    (10, 6, 2, 200, 700, 104, 104, False),
+    (16, 12, 4, 70, 97, 64, 40, True),      # causal, D <= 64: 960 of 16, 192 of 128
+    (50, 2, 1, 150, 333, 48, 48, True),
+    (12, 6, 2, 128, 257, 128, 72, True),    # 576 of 16, 72 of 128
+    (30, 4, 1, 130, 129, 80, 80, True),
+])
+def test_thirty_two_rows_against_the_oracle(amd, gpu_device, B, Hq, Hkv, L, S, E, Dv, causal):
+    """32-row workgroups where there are too many of 16 rows: grouped heads, narrow rows, L != S."""
+    test_against_the_oracle(amd, gpu_device, B, Hq, Hkv, L, S, E, Dv, causal)
+
+
+@pytest.mark.parametrize("B,H,S,D,causal", [(20, 2, 140, 64, False), (20, 5, 140, 64, True), (20, 3, 140, 104, True)])
+def test_key_counts_in_thirty_two_rows(amd, gpu_device, B, H, S, D, causal):
+    q, k, v = qkv(B, H, H, S, S, D, seed=6)
+    lens = torch.tensor([140, 0, 1, 97, 33] * 4, dtype=torch.int32)
+    for b in range(B):
+        k[b, :, lens[b]:], v[b, :, lens[b]:] = float("nan"), float("nan")
+    out, lse = amd.sdpa_forward(*(t.to(gpu_device) for t in (q, k, v)), is_causal=causal, kv_lens=lens.to(gpu_device))
+    for b, n in enumerate(lens.tolist()):
+        if n == 0:
+            assert not out[b].any() and torch.isneginf(lse[b]).all()
+            continue
+        ro, rl = oracle_fwd(q[b:b + 1], k[b:b + 1, :, :n], v[b:b + 1, :, :n], is_causal=causal)
+        assert max_abs(out[b:b + 1], ro) <= 1e-5 and max_abs(lse[b:b + 1], rl) <= 1e-5
