@@ -19,14 +19,19 @@ pytestmark = pytest.mark.gpu
     (2, 6, 6, 129, 300, 48, False, [300, 17]),
     (3, 4, 2, 33, 200, 64, True, [0, 200, 64]),  # a batch without a key
     (1, 16, 4, 1021, 1021, 64, True, None),     # parts
-    (2, 12, 4, 192, 192, 64, True, None),       # three heads a kv head: two launches
+    (2, 12, 4, 192, 192, 64, True, None),       # three heads a kv head
     (1, 28, 4, 150, 150, 64, True, None),
     (1, 16, 2, 193, 193, 56, True, [150]),      # ... parts, past three query tiles: one
-    (4, 32, 32, 129, 130, 64, False, None),     # 256 query and 256 key blocks: two launches
+    (4, 32, 32, 129, 130, 64, False, None),     # 256 query and 256 key blocks: 512 in all, the last size here
     (2, 32, 32, 256, 256, 64, False, None),     # 256 in all are 2 * 32 * 2 * 2
     (8, 12, 12, 511, 511, 64, True, None),      # 768 in all
     (2, 16, 16, 1100, 700, 40, True, [700, 699]),
     (4, 16, 16, 1024, 1024, 64, True, None),    # 1024 in all
+    # ... and past each: up to six query tiles 512, from seven 768, from fifteen 1024, with grouped heads 768
+    (32, 8, 8, 128, 128, 64, True, None), (33, 8, 8, 128, 100, 64, True, [100 - i for i in range(33)]),
+    (16, 8, 8, 256, 200, 56, True, None), (17, 8, 8, 256, 256, 64, True, None), (11, 8, 8, 384, 384, 64, True, None),
+    (13, 8, 8, 500, 500, 64, True, None), (8, 16, 8, 512, 512, 64, True, None), (9, 16, 8, 449, 449, 64, True, None),
+    (8, 8, 8, 896, 896, 64, True, None), (7, 8, 8, 896, 640, 64, True, None), (7, 8, 8, 1025, 1025, 64, True, None), (8, 8, 8, 1025, 1000, 48, True, None),
     # not causal, up to five query tiles 512 in all, from six and with three heads a kv head 768, 704 with two, and past each
     (32, 8, 8, 128, 100, 64, False, None), (33, 8, 8, 127, 128, 64, False, [128 - i for i in range(33)]),
     (16, 8, 8, 321, 321, 64, False, None), (17, 8, 8, 384, 300, 48, False, None), (16, 8, 8, 320, 320, 64, False, None),
