@@ -1,6 +1,6 @@
 // Flash-attention backward for gfx950 at head dims up to 64, bf16/f16: plain and causal calls, per-batch
-// key counts, dropout.  (Calls with a bias, a window or a score functor, and causal ones with too few workgroups
-// here, see w32_dkdv: bwd_dq_w32.hip, bwd_dkdv_w32.hip.)
+// key counts, dropout.  (Calls with a bias, a window or a score functor: bwd_dq_w32.hip, bwd_dkdv_w32.hip, and
+// dK/dV of causal calls of grouped heads with too few workgroups here: bwd_dkdv_w32.hip, see w32_dkdv.)
 //
 //   bwd_d64_dq_kernel     128 query rows per workgroup (4 wavefronts x 32), 64-key tiles:
 //                           S^T = K Q^T, dP^T = V dO^T, dS^T = P^T (dP^T - delta), dQ^T += K^T dS^T
@@ -18,7 +18,8 @@
 // registers to a third of the file (168), and the chain of one wavefront runs under the other two's of its SIMD; nothing
 // in it is pipelined by hand (in the two phases of the dK/dV kernel it measured the same, 986 / 1004 us for the backward of
 // B=4, 32 heads, S=4096 causal, within 1 % elsewhere, with dropout 2 % slower).  The dK/dV kernel, which holds
-// 128 registers of operands and accumulators, works on two blocks at a time instead (see dkdv_body).
+// 128 registers of operands and accumulators, works on two blocks at a time instead (see dkdv_body), but for calls of
+// just over two workgroups per compute unit and few items, which take it block by block in three (see three_per_cu).
 // A wavefront keeps all four products of its keys (at head dim 128 they do not fit and are split over two
 // wavefronts that exchange P through LDS).
 //
@@ -667,7 +668,8 @@ __device__ __forceinline__ void dkdv_body(const BwdM& p, const uint32_t* keep_bi
 // One block ahead: two workgroups per compute unit, the two phases of a block hold 211 to 240 registers.  (Against the four
 // products one after the other in 168 registers, three workgroups: B=4, 12 heads, S=512, not causal, the whole backward 32.2 -> 27.5 us,
 // B=1, S=1024 causal 39.1 -> 30.1, B=64, S=197 79.6 -> 77.7, B=4, 32 heads, S=4096 causal 1027 -> 1004; with dropout B=32, S=512
-// 148 -> 139, with key counts as well 158 -> 148.  Where those are still taken: three_per_cu.)
+// 148 -> 139, with key counts as well 158 -> 148.  Where those are still taken: three_per_cu.  Neither goes to scratch, but
+// both want more scalar registers than there are: 16 to 24 are kept in vector lanes, 74 to 108 in the launch of both kernels.)
 template <typename T, bool DROP, bool AHEAD>
 __global__ __launch_bounds__(256, AHEAD ? 2 : 3) void bwd_d64_dkdv_kernel(BwdM p, const uint32_t* keep_bits, int chunk) {
   __shared__ __attribute__((aligned(16))) uint16_t q_t[3][TILE];
