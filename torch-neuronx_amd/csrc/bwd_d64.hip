@@ -139,34 +139,6 @@ __device__ __forceinline__ void store_rows(const f32x16 (&acc)[DB], float scale,
   }
 }
 
-// blockIdx -> (tile, stream = (batch, kv head), unit within the stream's group of heads).  Workgroups of a
-// stream read the same K / V (dQ) or Q / dO (dK/dV) and should meet in one L2: the streams are dealt to the
-// XCDs (block i runs on XCD i % 8), and an XCD takes them in chunks whose tensors fit its 4 MB (stream_chunk),
-// all tiles of a chunk before the next one, heaviest tiles first within it.  (All streams of the XCD tile
-// by tile, 48 of them of 128 KB: B=32, 12 heads, S=512, every tile pass fetches K and V from memory
-// again, 274 MB for 126 MB of tensors, and the dQ kernel takes 142 thousand cycles instead of 130.)
-struct BlockMap {
-  int tile, stream, unit;
-};
-__device__ __forceinline__ BlockMap block_map(int bid, int streams, int n_tiles, int units, int chunk) {
-  BlockMap m;
-  if (chunk == 0) {  // (streams that are not pinned to XCDs)
-    m.tile = bid / (streams * units);
-    const int r = bid % (streams * units);
-    m.stream = r / units, m.unit = r % units;
-    return m;
-  }
-  const int per_xcd = (streams + 7) / 8, xcd = bid & 7;
-  int r = bid >> 3;
-  const int c = r / (chunk * n_tiles * units), in_chunk = min(chunk, per_xcd - c * chunk);
-  r -= c * chunk * n_tiles * units;
-  m.unit = r % units;
-  r /= units;
-  m.stream = (c * chunk + r % in_chunk) * 8 + xcd;
-  m.tile = r / in_chunk;
-  return m;
-}
-
 // (TERMS: leaves delta and the log2-domain log-sum-exp behind)
 template <typename T, bool DROP, bool TERMS>
 __device__ __forceinline__ void dq_body(const BwdM& p, uint32_t* keep_bits, int bid, int chunk, uint16_t (*k_t)[TILE], uint16_t (*v_t)[TILE]) {
@@ -669,7 +641,7 @@ __device__ __forceinline__ void dkdv_body(const BwdM& p, const uint32_t* keep_bi
 // products one after the other in 168 registers, three workgroups: B=4, 12 heads, S=512, not causal, the whole backward 32.2 -> 27.5 us,
 // B=1, S=1024 causal 39.1 -> 30.1, B=64, S=197 79.6 -> 77.7, B=4, 32 heads, S=4096 causal 1027 -> 1004; with dropout B=32, S=512
 // 148 -> 139, with key counts as well 158 -> 148.  Where those are still taken: three_per_cu.  Neither goes to scratch, but
-// both want more scalar registers than there are: 16 to 24 are kept in vector lanes, 74 to 108 in the launch of both kernels.)
+// both want more scalar registers than there are: 16 to 24 are kept in vector lanes, 73 to 90 in the launch of both kernels.)
 template <typename T, bool DROP, bool AHEAD>
 __global__ __launch_bounds__(256, AHEAD ? 2 : 3) void bwd_d64_dkdv_kernel(BwdM p, const uint32_t* keep_bits, int chunk) {
   __shared__ __attribute__((aligned(16))) uint16_t q_t[3][TILE];
@@ -724,15 +696,10 @@ __global__ __launch_bounds__(256) void bwd_d64_terms_kernel(BwdM p, int blocks32
 //   otherwise none up to 24 MB, six times the L2: B=11, 12 heads, S=1948 235, in two chunks of eight and a last one of a single stream 284; B=8, 8 heads, S=2500 199, two
 //     of 4 MB 253, three of 2 MB 228; B=24, S=1024 120, 134, 127; B=8, 32/8, S=4096 (dK/dV: 33 MB) 1834, 1944, -.  Beyond it as many as the L2 holds, but 128 workgroups at
 //     least: B=64, S=2048 1133 / 1061, B=96, S=1500 1053 / 991, B=32, 32/8, S=2048 2120 / 1990
-// (A number of streams that does not divide over the XCDs: see stream_chunk, fwd_mfma_w32.hip; backward, anywhere / pinned, us:
-// B=31, 12 heads, S=512 137 / 131, B=21, 6, S=785 120 / 115, B=15, 12, S=512 causal 55.5 / 53.7)
+// (A number of streams that does not divide over the XCDs: see pinned_streams, mfma_common.h)
 int stream_chunk(const BwdM& g, int64_t rows, int64_t units) {
   const int64_t streams = (int64_t)g.B * g.Hkv, bytes = std::max<int64_t>(1, rows * D * 4), all = (streams + 7) / 8;
-  if (streams % 8 != 0) {
-    if (units == 1 || (all * 8 - streams) * 15 > streams) return 0;
-    for (int slots = 32; slots <= 96; slots += 32)
-      if ((all * units + slots - 1) / slots > (streams * units + 8 * slots - 1) / (8 * slots)) return 0;
-  }
+  if (!pinned_streams(streams, units)) return 0;
   int64_t chunk = all;
   if (!g.causal)
     chunk = all * bytes < (4 << 20) ? all : (1 << 20) / bytes;
@@ -753,12 +720,12 @@ struct Grid {
 Grid dq_grid(const BwdM& g) {
   const int64_t units = (int64_t)(g.Hq / g.Hkv) * g.n_qt, streams = (int64_t)g.B * g.Hkv;
   const int chunk = stream_chunk(g, g.S, units);
-  return {chunk, (chunk ? (streams + 7) / 8 * 8 : streams) * units};
+  return {chunk, mapped_blocks(streams, units, chunk)};
 }
 Grid dkdv_grid(const BwdM& g) {
   const int64_t streams = (int64_t)g.B * g.Hkv;
   const int chunk = g.parts > 1 ? 0 : stream_chunk(g, (int64_t)g.L * (g.Hq / g.Hkv), g.n_kt);
-  return {chunk, (chunk ? (streams + 7) / 8 * 8 : streams) * g.n_kt * g.parts};
+  return {chunk, mapped_blocks(streams, (int64_t)g.n_kt * g.parts, chunk)};
 }
 
 // Causal calls whose dK/dV workgroups are too few to hide the longest of them, which is long: a key block of the first keys sees

@@ -71,12 +71,8 @@ __device__ __forceinline__ void bwd_dkdv_w32_body(const BwdM& p, const MaskArgs 
     st = v / p.parts_h, ph = v % p.parts_h;
   } else {
     // (low key tiles see the most queries under a causal mask: first)
-    if (p.dkdv_chunk) {
-      chunk_place(blockIdx.x >> 3, streams / 8, p.dkdv_chunk, p.n_kt, st, kt);
-      st = st * 8 + (blockIdx.x & 7);
-    } else {
-      kt = blockIdx.x / streams, st = blockIdx.x % streams;
-    }
+    const BlockMap m = block_map(blockIdx.x, streams, p.n_kt, 1, p.dkdv_chunk);
+    kt = m.tile, st = m.stream;
   }
   const int part = pq * p.parts_h + ph;  // its rows among the partial results
   const int b = st / p.Hkv, hk = st % p.Hkv;

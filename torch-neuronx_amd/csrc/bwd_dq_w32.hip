@@ -57,23 +57,9 @@ __device__ __forceinline__ void bwd_dq_w32_body(const BwdM& p, const MaskArgs ma
 
   int b, h, qt;
   {
-    const int bid = blockIdx.x, rep = p.Hq / p.Hkv;
-    const int n_qt = (p.L + BM - 1) / BM;
-    if (p.xcd_map) {
-      const int per_xcd = (p.B * p.Hkv) / 8, xcd = bid & 7;
-      int r = bid >> 3;
-      const int hg = r % rep;
-      r /= rep;
-      int sl, tile;
-      chunk_place(r, per_xcd, p.dq_chunk, n_qt, sl, tile);
-      qt = n_qt - 1 - tile;
-      const int stream = sl * 8 + xcd;
-      b = stream / p.Hkv, h = (stream % p.Hkv) * rep + hg;
-    } else {
-      const int heads = p.B * p.Hq;
-      qt = n_qt - 1 - bid / heads;
-      b = (bid % heads) / p.Hq, h = (bid % heads) % p.Hq;
-    }
+    const int rep = p.Hq / p.Hkv, n_qt = (p.L + BM - 1) / BM;
+    const BlockMap m = block_map(blockIdx.x, p.B * p.Hkv, n_qt, rep, p.dq_chunk);
+    b = m.stream / p.Hkv, h = (m.stream % p.Hkv) * rep + m.unit, qt = n_qt - 1 - m.tile;
   }
   const int hk = h / (p.Hq / p.Hkv);
   const int tid = threadIdx.x, lane = tid & 63;
@@ -788,7 +774,7 @@ bool bwd_dq_w32_fits(const BwdM& g, int head_dim) {
 
 int launch_bwd_dq_w32(const BwdM& g0, int dtype, int head_dim, hipStream_t s) {
   BwdM g = g0;
-  g.dq_chunk = bwd_stream_chunk(g, g.S);
+  if (const int chunk = bwd_stream_chunk(g, g.S)) g.dq_chunk = chunk;
   const int64_t blocks = (int64_t)g.B * g.Hq * ((g.L + BM - 1) / BM);
   const dim3 grid((unsigned)blocks, (unsigned)(g.dq_split_tiles ? g.dq_n_split : 1)), block(512);
   const bool bf = dtype == MI355_SDPA_BF16;

@@ -18,9 +18,9 @@ struct BwdM {
   int64_t o_sb, o_sh, o_sl, gq_sb, gq_sh, gq_sl, gk_sb, gk_sh, gk_sl, gv_sb, gv_sh, gv_sl;
   int B, Hq, Hkv, L, S;
   int n_qt, n_kt;
-  int causal, xcd_map;
-  // Streams, (batch, kv head) pairs, that an XCD takes at a time, all tiles of them before the next ones (0: all of its
-  // streams; only where they divide over the XCDs): the dQ kernel of bwd_dq_w32.hip, the dK/dV kernel of bwd_dkdv_w32.hip
+  int causal;
+  // Streams, (batch, kv head) pairs, that an XCD takes at a time, all tiles of them before the next ones (0: not pinned, see
+  // block_map): the dQ kernels of bwd_mfma.hip and bwd_dq_w32.hip, the dK/dV kernel of bwd_dkdv_w32.hip
   int dq_chunk = 0, dkdv_chunk = 0;
   float scale;
   // masked calls (the two-wavefronts-per-SIMD kernels only): a bias or bool keep-mask (unit stride
@@ -127,16 +127,6 @@ __device__ __forceinline__ float dot8(u32x4 a, u32x4 b) {
   return s;
 }
 
-
-// a workgroup's place in its XCD's order -> stream of the XCD and tile of the stream
-__device__ __forceinline__ void chunk_place(int r, int per_xcd, int chunk, int n_tiles, int& stream, int& tile) {
-  int first = 0, n = per_xcd;
-  if (chunk > 0 && chunk < per_xcd) {
-    first = r / (chunk * n_tiles) * chunk, n = min(chunk, per_xcd - first);
-    r -= first * n_tiles;
-  }
-  stream = first + r % n, tile = r / n;
-}
 
 // bias element as a float (bool: 0 or -inf)
 __device__ __forceinline__ float bias_value(const void* base, int64_t idx, int kind) {

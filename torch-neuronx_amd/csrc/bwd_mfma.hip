@@ -275,23 +275,9 @@ __global__ __launch_bounds__(256, 1) void bwd_dq_kernel(BwdM p) {
 
   int b, h, qt;
   {
-    const int bid = blockIdx.x, rep = p.Hq / p.Hkv;
-    const int n_qt = (p.L + BM - 1) / BM;
-    if (p.xcd_map) {
-      const int per_xcd = (p.B * p.Hkv) / 8, xcd = bid & 7;
-      int r = bid >> 3;
-      const int hg = r % rep;
-      r /= rep;
-      const int sl = r % per_xcd;
-      r /= per_xcd;
-      qt = n_qt - 1 - r;
-      const int stream = sl * 8 + xcd;
-      b = stream / p.Hkv, h = (stream % p.Hkv) * rep + hg;
-    } else {
-      const int heads = p.B * p.Hq;
-      qt = n_qt - 1 - bid / heads;
-      b = (bid % heads) / p.Hq, h = (bid % heads) % p.Hq;
-    }
+    const int rep = p.Hq / p.Hkv, n_qt = (p.L + BM - 1) / BM;
+    const BlockMap m = block_map(blockIdx.x, p.B * p.Hkv, n_qt, rep, p.dq_chunk);
+    b = m.stream / p.Hkv, h = (m.stream % p.Hkv) * rep + m.unit, qt = n_qt - 1 - m.tile;
   }
   const int hk = h / (p.Hq / p.Hkv);
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
@@ -528,7 +514,7 @@ static void fill(BwdM& g, const mi355_sdpa_bwd_params& p) {
   g.L = (int)p.q.size[2], g.S = (int)p.k.size[2];
   g.n_qt = (g.L + 127) / 128, g.n_kt = (g.S + 127) / 128;
   g.causal = p.is_causal, g.scale = p.scale;
-  g.xcd_map = ((g.B * g.Hkv) % 8 == 0) ? 1 : 0;
+  g.dq_chunk = (g.B * g.Hkv) % 8 == 0 ? g.B * g.Hkv / 8 : 0;
   g.kv_lens = p.kv_lens;
   g.d_real = (int)p.q.size[3], g.dv_real = (int)p.v.size[3];
   g.window = p.mask.window, g.sink_keys = p.mask.sink_keys;

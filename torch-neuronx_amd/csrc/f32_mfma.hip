@@ -1165,7 +1165,7 @@ int launch_bwd_f32_mfma(const mi355_sdpa_bwd_params& p, hipStream_t s) {
 #undef SET3
   g.B = (int)p.q.size[0], g.Hq = (int)p.q.size[1], g.Hkv = (int)p.k.size[1];
   g.L = (int)p.q.size[2], g.S = (int)p.k.size[2];
-  g.causal = p.is_causal, g.scale = p.scale, g.xcd_map = 0;
+  g.causal = p.is_causal, g.scale = p.scale;
   g.kv_lens = p.kv_lens;
   g.d_real = (int)p.q.size[3], g.dv_real = (int)p.v.size[3];
   set_score_mask(g, p);

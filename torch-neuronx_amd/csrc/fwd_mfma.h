@@ -75,46 +75,17 @@ struct FwdM {
 };
 
 // Decode blockIdx.x -> (batch, query head, query tile).  Tiles are issued heaviest first
-// (for causal attention the last query tile walks the most keys).  With xcd_map the eight
-// XCDs (blocks are dealt round-robin, block i -> XCD i % 8) each serve a fixed subset of
-// (batch, kv head) streams, so the K/V of a stream stay in one XCD's L2.  False: a workgroup of a stream that does not
-// exist, where their number is no multiple of eight.
+// (for causal attention the last query tile walks the most keys).  False: a workgroup of a stream that does not exist.
 __device__ __forceinline__ bool decode_block(const FwdM& p, int& b, int& h, int& qt) {
-  const int bid = blockIdx.x;
-  const int rep = p.Hq / p.Hkv;
-  if (p.xcd_map) {
-    const int streams = p.B * p.Hkv;
-    const int per_xcd = (streams + 7) / 8;
-    const int xcd = bid & 7;
-    int r = bid >> 3;  // index within this XCD: [chunk of streams][qt desc][stream in chunk][head in group]
-    const int hg = r % rep;
-    r /= rep;
-    int first = 0, n = per_xcd;
-    if (p.xcd_map < per_xcd) {
-      const int c = r / (p.xcd_map * p.n_qt);
-      first = c * p.xcd_map, n = min(p.xcd_map, per_xcd - first);
-      r -= first * p.n_qt;
-    }
-    const int sl = first + r % n;
-    r /= n;
-    qt = p.n_qt - 1 - r;
-    const int stream = sl * 8 + xcd;
-    if (stream >= streams) return false;
-    b = stream / p.Hkv;
-    h = (stream % p.Hkv) * rep + hg;
-  } else {
-    const int heads = p.B * p.Hq;
-    qt = p.n_qt - 1 - bid / heads;
-    const int bh = bid % heads;
-    b = bh / p.Hq;
-    h = bh % p.Hq;
-  }
-  return true;
+  const int rep = p.Hq / p.Hkv, streams = p.B * p.Hkv;
+  const BlockMap m = block_map(blockIdx.x, streams, p.n_qt, rep, p.xcd_map);
+  b = m.stream / p.Hkv;
+  h = (m.stream % p.Hkv) * rep + m.unit;
+  qt = p.n_qt - 1 - m.tile;
+  return m.stream < streams;
 }
 // the grid that it decodes
-inline int64_t tile_blocks(const FwdM& g) {
-  return g.xcd_map ? ((int64_t)g.B * g.Hkv + 7) / 8 * 8 * (g.Hq / g.Hkv) * g.n_qt : (int64_t)g.B * g.Hq * g.n_qt;
-}
+inline int64_t tile_blocks(const FwdM& g) { return mapped_blocks((int64_t)g.B * g.Hkv, (int64_t)(g.Hq / g.Hkv) * g.n_qt, g.xcd_map); }
 
 // head_dim 64, 128 or 256: the width the kernel is built for (g.d_real: the width of the data);
 // waves = 4 or 8 wavefronts (128 or 256 query rows) per workgroup, 4 only at head dim 256

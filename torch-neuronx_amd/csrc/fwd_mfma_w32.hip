@@ -1267,17 +1267,7 @@ int launch_fwd_split_merge(const FwdM& g, int dtype, hipStream_t s) {
 //       B=16, S=2000, D=256 331 / -, 328, 306;  B=16, S=2829, D=128 272 / -, 275, 255
 static int stream_chunk(const FwdM& g, int head_dim) {
   const int64_t streams = (int64_t)g.B * g.Hkv, per_xcd = (streams + 7) / 8;
-  if (streams % 8 != 0) {
-    // Some XCDs serve a stream less than others.  Unless they idle for more than a fifteenth, or the others need a turn of
-    // workgroups more than all would, one to three of which share a compute unit, that costs less than the K and V that every XCD
-    // brings for itself.  Anywhere / pinned in us: B=31, 12 heads, S=512 41.8 / 38.5, B=21, 6, S=785 36.3 / 34.3, B=41, 6, S=400 24.9 / 22.5,
-    // B=63, 12, S=197 24.5 / 23.1, B=15, 12, S=512 causal 17.3 / 16.5, B=21, 28/4, S=512, D=128 causal 82.3 / 74.1;  a turn more: B=9, 12, S=785 27.7 / 34.1.
-    // (One workgroup a stream shares nothing: 1 to 2 % slower.)
-    const int64_t units = (int64_t)(g.Hq / g.Hkv) * g.n_qt;
-    if (units == 1 || (per_xcd * 8 - streams) * 15 > streams) return 0;
-    for (int slots = 32; slots <= 96; slots += 32)
-      if ((per_xcd * units + slots - 1) / slots > (streams * units + 8 * slots - 1) / (8 * slots)) return 0;
-  }
+  if (!pinned_streams(streams, (int64_t)(g.Hq / g.Hkv) * g.n_qt)) return 0;
   const int64_t bytes = std::max<int64_t>(1, (int64_t)g.S * (g.d_real + g.dv_real) * 2);
   const bool by_four = !g.causal && head_dim == 128 && g.Hq <= 2 * g.Hkv;
   if (g.bias_kind || g.window > 0 || per_xcd * bytes <= (by_four && g.n_qt >= 3 ? 6 << 20 : 9 << 19)) return (int)per_xcd;

@@ -172,4 +172,51 @@ __device__ __forceinline__ int tile_swz(int r) {
   return D >= 128 ? (((r & 3) << 2) | ((r >> 2) & 3)) : ((((r >> 1) & 1) << 2) | ((r >> 2) & 3));
 }
 
+// blockIdx -> (tile, stream = (batch, kv head), unit within the stream's group of heads).  Workgroups of a stream read the same
+// K / V (forward, dQ) or Q / dO (dK/dV) and should meet in one L2: the streams are dealt to the XCDs (block i runs on XCD
+// i % 8), and an XCD takes them in chunks, all tiles of a chunk before the next one (each kernel's host code says how many).
+// chunk 0: streams that are not pinned.  Where their number is no multiple of eight, a pinned grid has workgroups whose
+// stream does not exist (stream >= streams): they leave at once.
+struct BlockMap {
+  int tile, stream, unit;
+};
+__device__ __forceinline__ BlockMap block_map(int bid, int streams, int n_tiles, int units, int chunk) {
+  BlockMap m;
+  if (chunk == 0) {
+    m.tile = bid / (streams * units);
+    const int r = bid % (streams * units);
+    m.stream = r / units, m.unit = r % units;
+    return m;
+  }
+  const int per_xcd = (streams + 7) / 8, xcd = bid & 7;
+  int r = bid >> 3, first = 0, n = per_xcd;  // index within this XCD: [chunk][tile][stream in chunk][unit]
+  m.unit = r % units;
+  r /= units;
+  if (chunk < per_xcd) {
+    first = r / (chunk * n_tiles) * chunk, n = min(chunk, per_xcd - first);
+    r -= first * n_tiles;
+  }
+  m.stream = (first + r % n) * 8 + xcd;
+  m.tile = r / n;
+  return m;
+}
+// The workgroups of such a grid.
+inline int64_t mapped_blocks(int64_t streams, int64_t units, int chunk) { return (chunk ? (streams + 7) / 8 * 8 : streams) * units; }
+
+// Whether streams of `units` workgroups each are pinned to XCDs.  Where their number is no multiple of eight, some XCDs serve a
+// stream less than others.  Unless they idle for more than a fifteenth, or the others need a turn of workgroups more than all
+// would, one to three of which share a compute unit, that costs less than the tensors that every XCD brings for itself.
+// Anywhere / pinned, forward in us: B=31, 12 heads, S=512 41.8 / 38.5, B=21, 6, S=785 36.3 / 34.3, B=41, 6, S=400 24.9 / 22.5,
+// B=63, 12, S=197 24.5 / 23.1, B=15, 12, S=512 causal 17.3 / 16.5, B=21, 28/4, S=512, D=128 causal 82.3 / 74.1;  a turn more: B=9, 12, S=785 27.7 / 34.1.
+// Backward at head dims up to 64: B=31, 12, S=512 137 / 131, B=21, 6, S=785 120 / 115, B=15, 12, S=512 causal 55.5 / 53.7.
+// (One workgroup a stream shares nothing: 1 to 2 % slower.)
+inline bool pinned_streams(int64_t streams, int64_t units) {
+  if (streams % 8 == 0) return true;
+  const int64_t all = (streams + 7) / 8;
+  if (units == 1 || (all * 8 - streams) * 15 > streams) return false;
+  for (int slots = 32; slots <= 96; slots += 32)
+    if ((all * units + slots - 1) / slots > (streams * units + 8 * slots - 1) / (8 * slots)) return false;
+  return true;
+}
+
 }  // namespace mi355
