@@ -72,7 +72,7 @@ CASES = [
     (1, 8, 1, 700, 300, 64, True, None, 0.0),
     (8, 20, 20, 130, 520, 64, False, None, 0.1),  # 20 streams per XCD
     (4, 10, 10, 600, 600, 64, True, None, 0.0),  # 5 streams per XCD; key blocks of 384 to 512 workgroups
-    # causal calls of two heads a kv head and one of 384 and more key blocks; one of 513 to 768 query tiles, 15 and more of 64 rows
+    # causal calls of 380 to 1032 key blocks: two heads a kv head, short; one, 525 to 760 query tiles of 14 to 16 items
     (95, 8, 4, 65, 65, 64, True, None, 0.0),
     (96, 8, 4, 65, 65, 64, True, None, 0.0),
     (96, 8, 4, 65, 130, 40, True, [65 + i % 66 for i in range(96)], 0.0),

@@ -98,6 +98,8 @@ struct BwdM {
 // dQ workgroups of one stream of 5000 keys are 20 for 32 compute units (all / one / four): 8 heads, B=8, S=5000 1400 / 1510 / 1386, B=9 1595 / 1674 / 1580 (three),
 // B=20 3900 / 3720 / 3510.  Grouped heads share Q and dO tiles in another order in dK/dV: B=8, 32/8 heads, S=1024 307 us, in
 // chunks 366 (bwd_dkdv_w32.hip takes none there).
+// (Stream counts that do not divide by eight are not pinned here.  Anywhere / pinned as the forward does: B=47, 1 head, S=2000 383 / 363 us, B=7, 9, S=2048
+// 491 / 473, causal 280 / 269, B=1, 31, S=4096 888 / 853;  B=31, 4, S=1024 280 / 276, B=21, 6, S=785 207 / 206, B=31, 12, S=512 275 / 278, B=63, 12, S=197 164 / 165.)
 // (The kernels for head dims up to 64, whose workgroups share a compute unit, have lines of their own: see bwd_d64.hip.)
 inline int bwd_stream_chunk(const BwdM& g, int64_t rows) {
   const int64_t streams = (int64_t)g.B * g.Hkv, bytes = std::max<int64_t>(1, rows * g.d_real * 4);
