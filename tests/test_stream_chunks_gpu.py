@@ -62,8 +62,16 @@ def test_every_stream_is_computed(gpu_device, B, Hq, Hkv, S, D, causal):
     (29, 12, 4, 300, 300, 64, True, None),      # 116, three heads a kv head
     (70, 8, 8, 200, 200, 64, True, None),       # causal, up to three key blocks: 70 (3.6 MB) in five chunks of 14, 64 at a time
     (64, 8, 8, 200, 200, 64, True, None),
-    (35, 8, 8, 500, 500, 64, True, None),       # four: 35 (4.5 MB) in five of 7, 32 (4.1) at a time
-    (32, 8, 8, 500, 500, 64, True, None),
+    (24, 8, 8, 500, 500, 64, True, None),       # four: 24 at a time, 25 and 31 in two chunks, 25 of 2.3 MB at a time
+    (25, 8, 8, 400, 390, 64, True, None),
+    (31, 8, 8, 385, 512, 64, True, None),
+    (25, 8, 8, 385, 360, 56, True, None),       # (three key blocks)
+    (32, 8, 8, 500, 500, 64, True, None),       # 32 of 4.1 MB in two of 16, of 3.9 at a time
+    (32, 8, 8, 480, 480, 64, True, None),
+    (33, 8, 8, 490, 490, 64, True, None),       # 33 and 42 in three, 43 in six
+    (42, 8, 8, 400, 400, 64, True, None),
+    (43, 8, 8, 400, 400, 64, True, None),
+    (28, 16, 8, 400, 400, 64, True, None),      # two heads a kv head: 28 of 5.7 MB for dK/dV in four
     (19, 12, 12, 1100, 900, 64, True, None),    # 228: the last four XCDs serve one less than 29, at a time
     (12, 16, 16, 700, 4100, 64, True, None),    # 24 of 4100 keys, more than 24 MB: in two chunks of 12 for dQ
     (12, 16, 16, 4100, 700, 48, True, None),    # ... of 4100 rows for dK/dV
@@ -102,6 +110,8 @@ def test_every_gradient_is_computed(gpu_device, B, Hq, Hkv, L, S, D, causal, len
     (31, 12, 512, 512, False),  # 372: the last four XCDs serve one less than 47, in chunks of 8
     (13, 12, 300, 400, False),  # 156: 20 at a time, the last four 19
     (45, 8, 500, 470, True),    # causal, four key blocks: 45 in chunks of 8 and 5
+    (29, 8, 450, 512, True),    # 29 in chunks of 15 and 14
+    (35, 8, 500, 460, True),    # 35 in chunks of 12 and 11
     (23, 12, 300, 300, True),   # three: 276 of which the last four XCDs serve one less than 35
 ])
 def test_keep_bits_reach_every_stream(gpu_device, B, H, L, S, causal, lens):

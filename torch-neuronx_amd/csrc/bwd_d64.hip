@@ -693,6 +693,9 @@ __global__ __launch_bounds__(256) void bwd_d64_terms_kernel(BwdM p, int blocks32
 // Under the mask the first workgroups of a chunk are the long ones, and the last chunk's should not start late:
 //   up to four workgroups a stream, where they differ little, from 3.25 MB (four workgroups: 4) on in chunks of 32 to 48 workgroups.  All / so: B=64, S=256 55 / 54, B=48, S=320 56 / 52, S=384
 //     69 / 62, S=448 81 / 80, S=512 95 / 89;  B=64, S=512 114 / 115, with dropout B=40, S=512 96 / 91;  less: B=32, S=256 with dropout 34 / 37, S=448 56 / 61, B=64, S=197 46 / 47.5, B=24, S=512 59 / 61
+//     four, 25 to 42 streams: two chunks, beyond 32 three.  All / eights / two / three: 25: S=390 47.9 / 51.9 / 45.0, S=512 58.1 / 65.3 / 57.9;  28: S=420 55.3 / 56.2 / 52.6, S=480 61.8 / 60.9 / 58.2, S=512 66.9 / 64.2 / 62.8,
+//       with dropout 76.0 / 76.6 / 73.6;  31: S=390 55.1 / 57.9 / 55.7, S=512 69.4 / 68.7 / 65.4;  32: S=420 54.0 / 59.4 / 57.2, S=480 63.2 / 65.2 / 63.0, S=512 67.9 / 69.2 / 66.4;  33: S=420 59.9 / 67.4 / 60.7 / -,
+//       S=480 69.0 / 70.7 / 67.0 / 66.0;  36: S=512 80.3 / 78.6 / 77.2 / 75.8;  38: S=512 with dropout 94.1 / 94.2 / 93.1 / 91.0;  40: S=512 with key counts 80.6 / 78.7 / 81.7 / 77.2
 //   otherwise none up to 24 MB, six times the L2: B=11, 12 heads, S=1948 235, in two chunks of eight and a last one of a single stream 284; B=8, 8 heads, S=2500 199, two
 //     of 4 MB 253, three of 2 MB 228; B=24, S=1024 120, 134, 127; B=8, 32/8, S=4096 (dK/dV: 33 MB) 1834, 1944, -.  Beyond it as many as the L2 holds, but 128 workgroups at
 //     least: B=64, S=2048 1133 / 1061, B=96, S=1500 1053 / 991, B=32, 32/8, S=2048 2120 / 1990
@@ -703,6 +706,8 @@ int stream_chunk(const BwdM& g, int64_t rows, int64_t units) {
   int64_t chunk = all;
   if (!g.causal)
     chunk = all * bytes < (4 << 20) ? all : (1 << 20) / bytes;
+  else if (units == 4 && g.Hq == g.Hkv && all > 24 && all <= 42 && all * bytes >= (all < 32 ? 9 << 18 : 4000000))
+    chunk = all <= 32 ? 16 : 14;
   else if (units <= 4)
     chunk = all * bytes < (units == 4 ? 4 << 20 : 13 << 18) ? all : units == 4 ? 8 : 16;
   else if (all * bytes > (24 << 20))
