@@ -62,6 +62,10 @@ def test_every_stream_is_computed(gpu_device, B, Hq, Hkv, S, D, causal):
     (29, 12, 4, 300, 300, 64, True, None),      # 116, three heads a kv head
     (70, 8, 8, 200, 200, 64, True, None),       # causal, up to three key blocks: 70 (3.6 MB) in five chunks of 14, 64 at a time
     (64, 8, 8, 200, 200, 64, True, None),
+    (32, 8, 8, 300, 288, 64, True, None),       # three, 32 at a time, 33 of 288 keys and rows in three chunks, of 287 at a time
+    (33, 8, 8, 288, 288, 64, True, None),
+    (33, 8, 8, 287, 290, 64, True, None),
+    (33, 16, 8, 300, 300, 64, True, None),      # two heads a kv head: 33 of 5 MB for dK/dV
     (24, 8, 8, 500, 500, 64, True, None),       # four: 24 at a time, 25 and 31 in two chunks, 25 of 2.3 MB at a time
     (25, 8, 8, 400, 390, 64, True, None),
     (31, 8, 8, 385, 512, 64, True, None),
@@ -110,6 +114,7 @@ def test_every_gradient_is_computed(gpu_device, B, Hq, Hkv, L, S, D, causal, len
     (31, 12, 512, 512, False),  # 372: the last four XCDs serve one less than 47, in chunks of 8
     (13, 12, 300, 400, False),  # 156: 20 at a time, the last four 19
     (45, 8, 500, 470, True),    # causal, four key blocks: 45 in chunks of 8 and 5
+    (37, 8, 300, 384, True),    # three: 37 in chunks of 13 and 11
     (29, 8, 450, 512, True),    # 29 in chunks of 15 and 14
     (35, 8, 500, 460, True),    # 35 in chunks of 12 and 11
     (23, 12, 300, 300, True),   # three: 276 of which the last four XCDs serve one less than 35
