@@ -36,6 +36,7 @@ pytestmark = pytest.mark.gpu
     (32, 8, 8, 128, 100, 64, False, None), (33, 8, 8, 127, 128, 64, False, [128 - i for i in range(33)]),
     (16, 8, 8, 321, 321, 64, False, None), (17, 8, 8, 384, 300, 48, False, None), (16, 8, 8, 320, 320, 64, False, None),
     (7, 16, 8, 400, 400, 64, False, None), (8, 16, 8, 400, 500, 64, False, None),
+    (6, 8, 4, 934, 934, 64, False, None), (2, 8, 4, 1498, 1498, 48, False, [1498, 1000]),  # ... 768 with split items
     (38, 16, 4, 65, 65, 64, False, None), (39, 16, 4, 65, 65, 64, False, None), (48, 12, 4, 65, 65, 64, False, None),
     # causal: three workgroups a compute unit above 640 and up to 768, up to ten query tiles
     (10, 8, 8, 448, 448, 64, True, None), (11, 8, 8, 448, 448, 64, True, None), (12, 8, 8, 500, 512, 40, True, [512 - 40 * i for i in range(12)]),

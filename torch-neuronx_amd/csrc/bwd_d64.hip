@@ -760,7 +760,7 @@ bool w32_dkdv(const BwdM& g) {
 //   not causal, 192: B=2, S=512 26.4 / 20.4;  384: B=8, S=197 20.3 / 20.2, B=4, S=512 29.9 / 27.5;  448: B=2, 16 heads, S=785 41.1 / 38.9;  3072: B=64, S=197 78 / 92
 //     beyond 512 by the number of tiles, 640, 8 heads: B=40, S=64 16.0 / 17.6, S=128 22.5 / 23.3, B=20, S=256 27.8 / 28.6;  720: B=15, S=320 29.3 / 30.2, S=384 34.0 / 33.3,
 //       B=9, S=640 45.6 / 43.8;  768: B=3, 16, S=1000 71.7 / 68.9;  816: B=17, S=384 34.7 / 39.2
-//     two heads a kv head, 576: 16/8, B=24, S=128 21.8 / 24.6, B=6, S=512 43.6 / 41.9;  768: 16/8, B=32, S=128 23.2 / 26.9, B=8, S=512 44.4 / 48.0
+//     two heads a kv head, 576: 16/8, B=24, S=128 21.8 / 24.6, B=6, S=512 43.6 / 41.9;  768: 16/8, B=32, S=128 23.2 / 26.9, B=8, S=512 44.4 / 48.0, split items B=6, 8/4, S=934 84.8 / 81.2, B=2, S=1498 79 / 70
 //     three and more, 640: 32/8, B=16, S=100 27.8 / 25.1, S=128 27.2 / 25.7;  672: B=3, S=400 51.2 / 50.3;  704: 12/4, B=22, S=200 38.9 / 37.2;  768: B=16, S=330 51.2 / 49.5
 //   causal, up to six 64-row tiles, 192: B=16, 6 heads, S=128 14.9 / 12.8;  384: B=16, 6, S=200 20.0 / 17.2, S=256 21.2 / 17.8
 //     432: B=6, 12/6 heads, S=400 35.5 / 30.2;  576: B=6, S=400 27.8 / 23.7, B=12, S=256 24.3 / 27.7;  768: B=8, S=400 29.8 / 31.4
@@ -772,7 +772,7 @@ bool w32_dkdv(const BwdM& g) {
 bool together(const BwdM& g) {
   if (g.keep_scale != 0.f || w32_dkdv(g)) return false;
   const int64_t all = (int64_t)g.B * g.Hq * g.n_qt + (int64_t)g.B * g.Hkv * g.n_kt * g.parts;
-  if (!g.causal) return all <= (g.Hq >= 3 * g.Hkv ? 768 : g.L <= 5 * BQ ? 512 : g.Hq == g.Hkv ? 768 : 704);
+  if (!g.causal) return all <= (g.Hq >= 3 * g.Hkv ? 768 : g.L <= 5 * BQ ? 512 : g.Hq == g.Hkv || g.parts > 1 ? 768 : 704);
   return all <= (g.L < 7 * BQ ? 512 : g.Hq > g.Hkv || g.L <= 14 * BQ ? 768 : 1024);
 }
 // ... and which of them with dK/dV block by block, in three workgroups a compute unit: calls under the causal mask of more
