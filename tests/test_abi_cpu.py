@@ -373,6 +373,8 @@ def test_hot_kernels_use_no_scratch_and_keep_their_occupancy():
     for name, r in d64.items():
         three = "bwd_d64_dq_kernel" in name or re.search(r"both_kernelIDF16[b_]Lb0E|dkdv_kernelIDF16[b_]Lb0ELb0E", name)
         assert int(r["Occupancy_[waves/SIMD]"]) == (3 if three else 2), name
+        if "both_kernel" in name:  # (either body's parameters fit the scalar registers, both together do not)
+            assert r["SGPRs_Spill"] == "0", name
 
 
 @pytest.mark.parametrize("B,Hq,Hkv,L,S,D,split", [

@@ -38,9 +38,11 @@ pytestmark = pytest.mark.gpu
     (7, 16, 8, 400, 400, 64, False, None), (8, 16, 8, 400, 500, 64, False, None),
     (6, 8, 4, 934, 934, 64, False, None), (2, 8, 4, 1498, 1498, 48, False, [1498, 1000]),  # ... 768 with split items
     (38, 16, 4, 65, 65, 64, False, None), (39, 16, 4, 65, 65, 64, False, None), (48, 12, 4, 65, 65, 64, False, None),
-    # causal: three workgroups a compute unit above 640 and up to 768, up to ten query tiles
+    # causal: three workgroups a compute unit above 640 and up to 768, up to eight query tiles
     (10, 8, 8, 448, 448, 64, True, None), (11, 8, 8, 448, 448, 64, True, None), (12, 8, 8, 500, 512, 40, True, [512 - 40 * i for i in range(12)]),
-    (12, 8, 8, 512, 513, 64, True, None), (9, 8, 8, 640, 630, 64, True, None), (9, 8, 8, 641, 630, 64, True, None),
+    (12, 8, 8, 512, 513, 64, True, None), (12, 8, 8, 513, 512, 64, True, None), (9, 8, 8, 640, 630, 64, True, None), (9, 8, 8, 641, 630, 64, True, None),
+    # ... and long chains a block ahead
+    (25, 2, 2, 1024, 1024, 64, True, None), (26, 2, 2, 1000, 1024, 48, True, [1024 - 30 * i for i in range(26)]), (24, 2, 2, 1217, 1280, 64, True, None), (11, 2, 2, 2561, 2500, 64, True, None),
 ])
 def test_gradients(gpu_device, dtype, bound, B, Hq, Hkv, L, S, D, causal, lens):
     import torch_neuronx_amd as amd

@@ -640,8 +640,8 @@ __device__ __forceinline__ void dkdv_body(const BwdM& p, const uint32_t* keep_bi
 // One block ahead: two workgroups per compute unit, the two phases of a block hold 211 to 240 registers.  (Against the four
 // products one after the other in 168 registers, three workgroups: B=4, 12 heads, S=512, not causal, the whole backward 32.2 -> 27.5 us,
 // B=1, S=1024 causal 39.1 -> 30.1, B=64, S=197 79.6 -> 77.7, B=4, 32 heads, S=4096 causal 1027 -> 1004; with dropout B=32, S=512
-// 148 -> 139, with key counts as well 158 -> 148.  Where those are still taken: three_per_cu.  Neither goes to scratch, but
-// both want more scalar registers than there are: 16 to 24 are kept in vector lanes, 73 to 90 in the launch of both kernels.)
+// 148 -> 139, with key counts as well 158 -> 148.  Where those are still taken: three_per_cu.  Neither goes to scratch;
+// 16 to 24 scalar registers are kept in vector lanes.)
 template <typename T, bool DROP, bool AHEAD>
 __global__ __launch_bounds__(256, AHEAD ? 2 : 3) void bwd_d64_dkdv_kernel(BwdM p, const uint32_t* keep_bits, int chunk) {
   __shared__ __attribute__((aligned(16))) uint16_t q_t[3][TILE];
@@ -651,10 +651,21 @@ __global__ __launch_bounds__(256, AHEAD ? 2 : 3) void bwd_d64_dkdv_kernel(BwdM p
   dkdv_body<T, DROP, AHEAD>(p, keep_bits, blockIdx.x, chunk, q_t, do_t, lse_s, dl_s, bit_s);
 }
 
+// The launch's parameters, read anew.  A workgroup of both kernels is one or the other; parameters that the compiler reads at
+// the top for either want 83 to 108 scalar registers more than there are, and come back lane by lane in the loops.  Read where
+// each body begins they all fit: causal, 4 heads, in us: B=7, S=2000 77.5 / 75.8, B=8, S=1700 67.2 / 63.1, B=10, S=1536 68.4 / 65.8;
+// 12 heads: B=4, S=1024 45.6 / 43.0, B=1, S=128 12.8 / 11.6, B=4, S=512, not causal 26.3 / 24.8.
+// (The kernels of their own hold 0 to 24 in vector lanes, outside their loops, and measure the same either way.)
+__device__ __forceinline__ const BwdM& own_args() {
+  auto args = (const __attribute__((address_space(4))) BwdM*)__builtin_amdgcn_kernarg_segment_ptr();
+  asm volatile("" : "+s"(args));
+  return *(const BwdM*)args;
+}
+
 // Both in one launch, behind bwd_d64_terms_kernel: a dK/dV and a dQ workgroup by turns, eight of each (the XCDs), the
 // heaviest of both first.  (See together for where.)
 template <typename T, bool AHEAD>
-__global__ __launch_bounds__(256, AHEAD ? 2 : 3) void bwd_d64_both_kernel(BwdM p, int dq_blocks, int dkdv_blocks, int dq_chunk, int dkdv_chunk) {
+__global__ __launch_bounds__(256, AHEAD ? 2 : 3) void bwd_d64_both_kernel(BwdM /* first: see own_args */, int dq_blocks, int dkdv_blocks, int dq_chunk, int dkdv_chunk) {
   __shared__ __attribute__((aligned(16))) uint16_t a_t[3][TILE];
   __shared__ __attribute__((aligned(16))) uint16_t b_t[3][TILE];
   __shared__ __attribute__((aligned(16))) float lse_s[3][BQ], dl_s[3][BQ];
@@ -662,8 +673,8 @@ __global__ __launch_bounds__(256, AHEAD ? 2 : 3) void bwd_d64_both_kernel(BwdM p
   const bool dq = eight < 2 * turns ? (eight & 1) != 0 : dq_blocks > dkdv_blocks;
   const int bid = (eight < 2 * turns ? eight >> 1 : eight - turns) * 8 + in;
   if (bid >= (dq ? dq_blocks : dkdv_blocks)) return;
-  if (dq) dq_body<T, false, false>(p, nullptr, bid, dq_chunk, a_t, b_t);
-  else dkdv_body<T, false, AHEAD>(p, nullptr, bid, dkdv_chunk, a_t, b_t, lse_s, dl_s, nullptr);
+  if (dq) dq_body<T, false, false>(own_args(), nullptr, bid, dq_chunk, a_t, b_t);
+  else dkdv_body<T, false, AHEAD>(own_args(), nullptr, bid, dkdv_chunk, a_t, b_t, lse_s, dl_s, nullptr);
 }
 
 // delta and the log2-domain log-sum-exp of 32 rows per wavefront, the sums in dq_body's order
@@ -776,13 +787,13 @@ bool together(const BwdM& g) {
   return all <= (g.L < 7 * BQ ? 512 : g.Hq > g.Hkv || g.L <= 14 * BQ ? 768 : 1024);
 }
 // ... and which of them with dK/dV block by block, in three workgroups a compute unit: calls under the causal mask of more
-// than two and a half each, which then are one turn.  Two launches / one, a block ahead / one, block by block, us, 8 heads:
-//   576: S=512 32.5 / 28.3 / 29.4, S=640 36.1 / 29.3 / 31.9;  640: S=448 29.0 / 27.1 / 27.1, S=512 32.9 / 30.5 / 30.2, S=576 33.3 / 29.1 / 30.5
-//   704: S=512 32.7 / 33.0 / 30.6;  672, longer chains: S=768 - / 37.5 / 39.3, S=896 - / 39.0 / 44.2;  768: S=448 30.0 / 30.0 / 28.3, S=512 34.0 / 34.0 / 31.8
+// than two and a half each and short chains, which then are one turn.  Two launches / one, a block ahead / one, block by block, us:
+//   576: S=448 29.8 / 23.5 / 26.5, S=512 33.7 / 27.5 / 29.9;  672: S=448 30.4 / 29.3 / 28.8, S=512 34.7 / 32.3 / 31.9;  768: S=448 31.3 / 31.1 / 29.2, S=512 35.3 / 33.2 / 32.0
+//   longer: 680: S=576 35.9 / 31.2 / 32.7, S=640 39.8 / 35.3 / 35.6;  768: S=700 40.5 / 35.3 / 37.9, S=1024 53.2 / 45.7 / 48.0;  960: S=1536 77.3 / 68.3 / 66.3, S=2048 91.5 / 83.3 / 83.7
 //   grouped, 768: 16/8, S=512 41.7 / 37.3 / 43.6
 bool together_three_per_cu(const BwdM& g) {
   const int64_t all = (int64_t)g.B * g.Hq * g.n_qt + (int64_t)g.B * g.Hkv * g.n_kt * g.parts;
-  return g.causal && g.Hq == g.Hkv && g.L <= 10 * BQ && all > 640 && all <= 768;
+  return g.causal && g.Hq == g.Hkv && g.L <= 8 * BQ && all > 640 && all <= 768;
 }
 
 // Calls whose dK/dV runs block by block, three workgroups per compute unit: more key blocks than two per compute unit, but
