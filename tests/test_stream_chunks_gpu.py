@@ -114,6 +114,7 @@ def test_every_gradient_is_computed(gpu_device, B, Hq, Hkv, L, S, D, causal, len
     (31, 12, 512, 512, False),  # 372: the last four XCDs serve one less than 47, in chunks of 8
     (13, 12, 300, 400, False),  # 156: 20 at a time, the last four 19
     (45, 8, 500, 470, True),    # causal, four key blocks: 45 in chunks of 8 and 5
+    (61, 8, 1000, 1000, True),  # more than 15 MB: 61 in chunks of 16 and 13
     (37, 8, 300, 384, True),    # three: 37 in chunks of 13 and 11
     (29, 8, 450, 512, True),    # 29 in chunks of 15 and 14
     (35, 8, 500, 460, True),    # 35 in chunks of 12 and 11

@@ -711,7 +711,7 @@ __global__ __launch_bounds__(256) void bwd_d64_terms_kernel(BwdM p, int blocks32
 //       S=480 69.0 / 70.7 / 67.0 / 66.0;  36: S=512 80.3 / 78.6 / 77.2 / 75.8;  38: S=512 with dropout 94.1 / 94.2 / 93.1 / 91.0;  40: S=512 with key counts 80.6 / 78.7 / 81.7 / 77.2
 //   otherwise none up to 24 MB, six times the L2: B=11, 12 heads, S=1948 235, in two chunks of eight and a last one of a single stream 284; B=8, 8 heads, S=2500 199, two
 //     of 4 MB 253, three of 2 MB 228; B=24, S=1024 120, 134, 127; B=8, 32/8, S=4096 (dK/dV: 33 MB) 1834, 1944, -.  Beyond it as many as the L2 holds, but 128 workgroups at
-//     least: B=64, S=2048 1133 / 1061, B=96, S=1500 1053 / 991, B=32, 32/8, S=2048 2120 / 1990
+//     least: B=64, S=2048 1133 / 1061, B=96, S=1500 1053 / 991, B=32, 32/8, S=2048 2120 / 1990;  with dropout beyond 15 MB: 22 MB: B=116, S=747 522 / 498;  16.4: B=64, S=1000 442 / 428;  15.4: B=100, S=600 315 / 315;  11: B=60, S=747 256 / 260
 // (A number of streams that does not divide over the XCDs: see pinned_streams, mfma_common.h)
 int stream_chunk(const BwdM& g, int64_t rows, int64_t units) {
   const int64_t streams = (int64_t)g.B * g.Hkv, bytes = std::max<int64_t>(1, rows * D * 4), all = (streams + 7) / 8;
@@ -725,7 +725,7 @@ int stream_chunk(const BwdM& g, int64_t rows, int64_t units) {
     chunk = 16;
   else if (units <= 4)
     chunk = all * bytes < (units == 4 ? 4 << 20 : 13 << 18) ? all : units == 4 ? 8 : 16;
-  else if (all * bytes > (24 << 20))
+  else if (all * bytes > (g.keep_scale != 0.f ? 15 << 20 : 24 << 20))
     chunk = std::max<int64_t>((4 << 20) / bytes, 128 / units);
   if (chunk < 1) chunk = 1;
   if (chunk >= all) return (int)std::max<int64_t>(1, all);
