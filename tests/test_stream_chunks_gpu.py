@@ -66,6 +66,8 @@ def test_every_stream_is_computed(gpu_device, B, Hq, Hkv, S, D, causal):
     (33, 8, 8, 288, 288, 64, True, None),
     (33, 8, 8, 287, 290, 64, True, None),
     (33, 16, 8, 300, 300, 64, True, None),      # two heads a kv head: 33 of 5 MB for dK/dV
+    (56, 8, 8, 270, 270, 64, True, None),       # 56 of 3.9 MB at a time, 62 of 4.3 in four chunks
+    (62, 8, 8, 270, 270, 64, True, None),
     (24, 8, 8, 500, 500, 64, True, None),       # four: 24 at a time, 25 and 31 in two chunks, 25 of 2.3 MB at a time
     (25, 8, 8, 400, 390, 64, True, None),
     (31, 8, 8, 385, 512, 64, True, None),

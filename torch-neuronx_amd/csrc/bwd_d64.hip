@@ -702,10 +702,10 @@ __global__ __launch_bounds__(256) void bwd_d64_terms_kernel(BwdM p, int blocks32
 // the rows that are written pass through the same L2).  All / in chunks, backward in us, 8 heads: 3.1 MB: B=24, S=512 70 / 69;  4.0: B=20, S=785 127 / 131;
 // 4.2: B=64, S=256 61 / 58, with dropout 72 / 67, B=32, S=512 87 / 84;  4.7: B=48, S=384 83 / 81;  6.3: B=48, S=512 122 / 118
 // Under the mask the first workgroups of a chunk are the long ones, and the last chunk's should not start late:
-//   up to four workgroups a stream, where they differ little, from 3.25 MB (four workgroups: 4) on in chunks of 32 to 48 workgroups.  All / so: B=64, S=256 55 / 54, B=48, S=320 56 / 52, S=384
+//   up to four workgroups a stream, where they differ little, from 3.25 MB (three and four workgroups: 4) on in chunks of 32 to 48 workgroups.  All / so: B=64, S=256 55 / 54, B=48, S=320 56 / 52, S=384
 //     69 / 62, S=448 81 / 80, S=512 95 / 89;  B=64, S=512 114 / 115, with dropout B=40, S=512 96 / 91;  less: B=32, S=256 with dropout 34 / 37, S=448 56 / 61, B=64, S=197 46 / 47.5, B=24, S=512 59 / 61
 //     three, more than 32 streams of 288 keys and more: sixteens.  All / so: 33: S=300 43.9 / 41.3, S=384 51.8 / 51.2;  36: S=300 47.0 / 42.7, S=330 50.8 / 47.5;  40: S=300 48.5 / 45.9, S=330 54.7 / 50.9;
-//       44: S=300 51.3 / 51.0, S=360 62.3 / 58.7;  48: S=330 61.5 / 57.0;  less: 32: S=300 37.9 / 37.4, S=384 46.7 / 45.3, 44: S=270 47.6 / 52.7
+//       44: S=300 51.3 / 51.0, S=360 62.3 / 58.7;  48: S=330 61.5 / 57.0;  less: 32: S=300 37.9 / 37.4, S=384 46.7 / 45.3, 44: S=270 47.6 / 52.7, 56: S=260 56.2 / 61.9, S=286 58.3 / 60.7
 //     four, 25 to 42 streams: two chunks, beyond 32 three.  All / eights / two / three: 25: S=390 47.9 / 51.9 / 45.0, S=512 58.1 / 65.3 / 57.9;  28: S=420 55.3 / 56.2 / 52.6, S=480 61.8 / 60.9 / 58.2, S=512 66.9 / 64.2 / 62.8,
 //       with dropout 76.0 / 76.6 / 73.6;  31: S=390 55.1 / 57.9 / 55.7, S=512 69.4 / 68.7 / 65.4;  32: S=420 54.0 / 59.4 / 57.2, S=480 63.2 / 65.2 / 63.0, S=512 67.9 / 69.2 / 66.4;  33: S=420 59.9 / 67.4 / 60.7 / -,
 //       S=480 69.0 / 70.7 / 67.0 / 66.0;  36: S=512 80.3 / 78.6 / 77.2 / 75.8;  38: S=512 with dropout 94.1 / 94.2 / 93.1 / 91.0;  40: S=512 with key counts 80.6 / 78.7 / 81.7 / 77.2
@@ -724,7 +724,7 @@ int stream_chunk(const BwdM& g, int64_t rows, int64_t units) {
   else if (units == 3 && g.Hq == g.Hkv && all > 32 && bytes >= 9 << 13)
     chunk = 16;
   else if (units <= 4)
-    chunk = all * bytes < (units == 4 ? 4 << 20 : 13 << 18) ? all : units == 4 ? 8 : 16;
+    chunk = all * bytes < (units == 4 || (units == 3 && g.Hq == g.Hkv) ? 4 << 20 : 13 << 18) ? all : units == 4 ? 8 : 16;
   else if (all * bytes > (g.keep_scale != 0.f ? 15 << 20 : 24 << 20))
     chunk = std::max<int64_t>((4 << 20) / bytes, 128 / units);
   if (chunk < 1) chunk = 1;
