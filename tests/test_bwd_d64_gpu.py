@@ -68,6 +68,7 @@ CASES = [
     (2, 2, 2, 64, 197, 64, False, None, 0.25),
     (1, 4, 2, 131, 131, 64, True, None, 0.25),
     (3, 2, 2, 130, 261, 48, False, [261, 33, 0], 0.25),
+    (19, 28, 4, 19, 1071, 64, True, None, 0.0),  # 684 key blocks, 76 of which have an item
     (2, 8, 1, 500, 140, 64, False, None, 0.1),   # the items of a key block go to several workgroups
     (1, 8, 1, 700, 300, 64, True, None, 0.0),
     (8, 20, 20, 130, 520, 64, False, None, 0.1),  # 20 streams per XCD

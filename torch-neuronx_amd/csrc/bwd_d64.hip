@@ -806,7 +806,7 @@ bool together_three_per_cu(const BwdM& g) {
 //     768: S=256 42.6 / 39.8, S=384 45.6 / 41.1, S=512 53.6 / 51.0;  ten: S=640 54.4 / 53.9
 // (With dropout, whose kernel takes more registers, a block ahead everywhere: B=64, 12 heads, S=64 25.0 / 26.7, S=100 39.2 / 42.0.)
 bool three_per_cu(const BwdM& g) {
-  const int64_t blocks = (int64_t)g.B * g.Hkv * g.n_kt;
+  const int64_t blocks = (int64_t)g.B * g.Hkv * (g.causal ? std::min(g.n_kt, (g.L + 127) / 128) : g.n_kt);  // (key blocks past the last row have no item)
   const int tiles = (g.L + BQ - 1) / BQ, items = g.Hq / g.Hkv * tiles;
   return blocks > 512 && blocks <= 768 && (tiles <= 1 || items <= 2 || (g.causal && items <= 8 && blocks > 640));
 }
